@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -334,7 +335,7 @@ int launch_stages(famrdp_plan* p, double dt, int flags, hipStream_t st, bool adj
         LAUNCH_CHECK();
       }
     } else if (flags & FAMRDP_STEP_BATCHED) {
-      k_viscous_flux_batched<false><<<p->persistent_grid, 256, 0, st>>>(dtab, p->d_tiles, p->ntiles, stage, p->gas);
+      k_viscous_flux_batched<<<p->persistent_grid, 256, 0, st>>>(dtab, p->d_tiles, p->ntiles, stage, p->gas);
       LAUNCH_CHECK();
       k_stage_batched<<<p->persistent_grid, 256, 0, st>>>(dtab, p->d_tiles, p->ntiles, p->gas.gamma,
                                                           p->limiter, dt, stage);

@@ -80,14 +80,6 @@ __device__ __forceinline__ void load_prim(const double* __restrict__ q, int64_t 
   cons_to_prim(qc, g, pv);
 }
 
-__device__ __forceinline__ void load_prim_fast(const double* __restrict__ q, int64_t N, int64_t c, double g,
-                                               double pv[5]) {
-  double qc[5];
-#pragma unroll
-  for (int v = 0; v < 5; ++v) qc[v] = q[v * N + c];
-  cons_to_prim_fast(qc, g, pv);
-}
-
 // XCD-aware order: workgroups are dealt round-robin to the 8 XCDs, so map
 // consecutive ids of one XCD onto consecutive tiles (neighbouring tiles share
 // halo lines in that XCD's L2).

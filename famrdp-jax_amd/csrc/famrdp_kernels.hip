@@ -92,8 +92,6 @@ __global__ void k_roe_flux(const double* __restrict__ UL, const double* __restri
 // ---------------------------------------------------------------------------
 
 // Viscous flux tensor G at cell c (rhs/viscous.py:30-108, roll wrap).
-// FAST selects the stage-kernel arithmetic (reciprocals, fast sqrt).
-template <bool FAST>
 __device__ __forceinline__ void cell_viscous_flux(const double* __restrict__ q, const double* __restrict__ kxyz,
                                                   double* __restrict__ G, int ni, int nj, int nk, int64_t N,
                                                   int64_t c, const Gas& gas) {
@@ -102,30 +100,24 @@ __device__ __forceinline__ void cell_viscous_flux(const double* __restrict__ q, 
   const int64_t cm[3] = {c + (wrap_m(i, ni) - i) * si, c + (wrap_m(j, nj) - j) * sj, c + (wrap_m(k, nk) - k)};
   const int64_t cp[3] = {c + (wrap_p(i, ni) - i) * si, c + (wrap_p(j, nj) - j) * sj, c + (wrap_p(k, nk) - k)};
   double pv[5];
-  if (FAST) load_prim_fast(q, N, c, gas.gamma, pv); else load_prim(q, N, c, gas.gamma, pv);
-  const double T = FAST ? temperature_fast(pv, gas.R) : temperature(pv, gas.R);
+  load_prim(q, N, c, gas.gamma, pv);
+  const double T = temperature(pv, gas.R);
   double d[3][4];
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
     double pp[5], pm[5];
-    if (FAST) {
-      load_prim_fast(q, N, cp[l], gas.gamma, pp);
-      load_prim_fast(q, N, cm[l], gas.gamma, pm);
-    } else {
-      load_prim(q, N, cp[l], gas.gamma, pp);
-      load_prim(q, N, cm[l], gas.gamma, pm);
-    }
+    load_prim(q, N, cp[l], gas.gamma, pp);
+    load_prim(q, N, cm[l], gas.gamma, pm);
     d[l][0] = 0.5 * (pp[1] - pm[1]);
     d[l][1] = 0.5 * (pp[2] - pm[2]);
     d[l][2] = 0.5 * (pp[3] - pm[3]);
-    d[l][3] = FAST ? 0.5 * (temperature_fast(pp, gas.R) - temperature_fast(pm, gas.R))
-                   : 0.5 * (temperature(pp, gas.R) - temperature(pm, gas.R));
+    d[l][3] = 0.5 * (temperature(pp, gas.R) - temperature(pm, gas.R));
   }
   double kk[9];
 #pragma unroll
   for (int m = 0; m < 9; ++m) kk[m] = kxyz[m * N + c];
   double g9[9];
-  if (FAST) viscous_flux_fast(pv, T, d, kk, gas, g9); else viscous_flux(pv, T, d, kk, gas, g9);
+  viscous_flux(pv, T, d, kk, gas, g9);
 #pragma unroll
   for (int m = 0; m < 9; ++m) G[m * N + c] = g9[m];
 }
@@ -226,15 +218,7 @@ __global__ void __launch_bounds__(256) k_viscous_flux(const double* __restrict__
                                                       double* __restrict__ G, int ni, int nj, int nk, Gas gas) {
   const int64_t N = (int64_t)ni * nj * nk;
   const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c < N) cell_viscous_flux<false>(q, kxyz, G, ni, nj, nk, N, c, gas);
-}
-
-__global__ void __launch_bounds__(256) k_viscous_flux_fast(const double* __restrict__ q,
-                                                           const double* __restrict__ kxyz, double* __restrict__ G,
-                                                           int ni, int nj, int nk, Gas gas) {
-  const int64_t N = (int64_t)ni * nj * nk;
-  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c < N) cell_viscous_flux<true>(q, kxyz, G, ni, nj, nk, N, c, gas);
+  if (c < N) cell_viscous_flux(q, kxyz, G, ni, nj, nk, N, c, gas);
 }
 
 __global__ void k_fastmath_probe(const double* __restrict__ x, double* __restrict__ r, double* __restrict__ s,
@@ -302,7 +286,6 @@ __global__ void k_axpby(double* __restrict__ out, double a, const double* __rest
 // every block of the plan (the block-offset table is `blocks`).
 // ---------------------------------------------------------------------------
 
-template <bool FAST>
 __global__ void __launch_bounds__(256) k_viscous_flux_batched(const BlockDesc* __restrict__ blocks,
                                                               const Tile* __restrict__ tiles, int ntiles, int stage,
                                                               Gas gas) {
@@ -314,7 +297,7 @@ __global__ void __launch_bounds__(256) k_viscous_flux_batched(const BlockDesc* _
       const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
       Gas gb = gas;
       gb.mu0 = b.mu0;
-      cell_viscous_flux<FAST>(qin, b.kxyz, b.G, b.ni, b.nj, b.nk, b.N, c, gb);
+      cell_viscous_flux(qin, b.kxyz, b.G, b.ni, b.nj, b.nk, b.N, c, gb);
     }
   }
 }
@@ -599,10 +582,11 @@ __global__ void __launch_bounds__(256) k_sum_parts(const double* __restrict__ pa
 //     exist only between cells 1..n-2 of their axis).
 //  2. Viscous flux tensor G (rhs/viscous.py:30-108) for the tile plus a
 //     one-cell cross halo into LDS; every cell takes its viscous divergence.
-//  3. For each axis in the reference's order (i, j, k): MUSCL-2 + Roe face
-//     fluxes of the tile's low faces plus one layer of high faces into an LDS
-//     face buffer (aliasing G), then -(F(c+1/2) - F(c-1/2)) / vol for cells
-//     with 2 <= c_d <= n_d - 3 (rhs/invscd.py:100-131).
+//  3. For each axis, j, k, then i (the order the marching kernel sums them
+//     in): MUSCL-2 + Roe face fluxes of the tile's low faces plus one layer
+//     of high faces into an LDS face buffer (aliasing G), then
+//     F(c+1/2) - F(c-1/2) for cells with 2 <= c_d <= n_d - 3
+//     (rhs/invscd.py:100-131).
 //  4. rhs = inv + vis and the Shu-Osher combination (solver/step.py:45-53).
 // ===========================================================================
 namespace famrdp {
@@ -615,10 +599,10 @@ namespace famrdp {
 // to the threads beyond the tile's cells, or after the low face when there
 // are none).  Face fluxes go to the LDS buffer s_f (axes i, j: f * Pd + o,
 // axis k: o * (TK + 1) + f, face f between local cells f-1 and f); after a
-// barrier every cell with 2 <= c <= n-3 along D takes -(F(c+1/2) -
-// F(c-1/2)) / vol.  Ends with a barrier (s_f is reused by the next axis).
+// barrier every cell with 2 <= c <= n-3 along D adds F(c+1/2) - F(c-1/2)
+// (fluxes doubled, see roe_flux2) to A.  Ends with a barrier (s_f is reused by the next axis).
 // ---------------------------------------------------------------------------
-// kxyz[D, :] of the left neighbour of cell c along D (the left cell of the
+// kxyz[D, :] / 2 of the left neighbour of cell c along D (the left cell of the
 // cell's own low face), loaded early so the face phase does not wait on it;
 // zero where that face does not exist.
 template <int D>
@@ -629,14 +613,15 @@ __device__ __forceinline__ void load_kl_own(const BlockDesc& b, int64_t c, int g
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
     const double v = b.kxyz[(D * 3 + m) * b.N + cl];
-    kl[m] = ok ? v : 0.0;
+    kl[m] = ok ? 0.5 * v : 0.0;
   }
 }
 
 template <int D, class T, int TI, int TJ, int TK, int NTH, int LIM>
 __device__ __forceinline__ void face_axis(const BlockDesc& b, int i0, int j0, int k0, const double* s_pv,
-                                          double* s_f, const double kk[9], const double kl_own[3], bool own, int t,
-                                          int x, int y, int z, double rvol, double g, double inv[5]) {
+                                          double* s_f, const double kkh[9], const double kl_own[3], bool own, int t,
+                                          int x, int y, int z, const StageGas& gas, double A[5]) {
+  EXACT_FP
   constexpr int NT = TI * TJ * TK;
   constexpr int Td = D == 0 ? TI : (D == 1 ? TJ : TK);
   constexpr int Pd = NT / Td;
@@ -664,11 +649,11 @@ __device__ __forceinline__ void face_axis(const BlockDesc& b, int i0, int j0, in
     double kl[3], kr[3];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-      kl[m] = kr_own ? kl_own[m] : b.kxyz[(D * 3 + m) * N + cl];
-      kr[m] = kr_own ? kk[D * 3 + m] : b.kxyz[(D * 3 + m) * N + cr];
+      kl[m] = kr_own ? kl_own[m] : 0.5 * b.kxyz[(D * 3 + m) * N + cl];
+      kr[m] = kr_own ? kkh[D * 3 + m] : 0.5 * b.kxyz[(D * 3 + m) * N + cr];
     }
     double Fa[5];
-    face_flux_prim<LIM>(p4[0], p4[1], p4[2], p4[3], kl, kr, g, Fa);
+    face_flux2<LIM>(p4[0], p4[1], p4[2], p4[3], kl, kr, gas, Fa);
 #pragma unroll
     for (int v = 0; v < 5; ++v) s_f[v * T::NF + slot] = Fa[v];
   };
@@ -688,7 +673,7 @@ __device__ __forceinline__ void face_axis(const BlockDesc& b, int i0, int j0, in
     const int lo = D == 2 ? o_own * (TK + 1) + loc_d : loc_d * Pd + o_own;
     const int hi = D == 2 ? lo + 1 : lo + Pd;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) inv[v] = inv[v] + (-(s_f[v * T::NF + hi] - s_f[v * T::NF + lo]) * rvol);
+    for (int v = 0; v < 5; ++v) A[v] = A[v] + (s_f[v * T::NF + hi] - s_f[v * T::NF + lo]);
   }
   __syncthreads();
 }
@@ -757,8 +742,9 @@ __device__ __forceinline__ void fused_stage_loads(const BlockDesc& b, const doub
 template <int TI, int TJ, int TK, int LIM, bool RS>
 __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0, int j0, int k0,
                                                       const double* __restrict__ qin, const double* q0, double* qout,
-                                                      const Gas& gas, double dt, int stage,
+                                                      const StageGas& gas, double dt, int stage,
                                                       const FusedCells<TI, TJ, TK>& fc, double qq[][5]) {
+  EXACT_FP
   using T = FusedGeom<TI, TJ, TK>;
   constexpr int NIT = FusedCells<TI, TJ, TK>::NIT;
   __shared__ double lds[RS ? T::NLDS_RS : T::NLDS];
@@ -769,10 +755,8 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
   const int t = threadIdx.x;
   const int ni = b.ni, nj = b.nj, nk = b.nk;
   const int64_t N = b.N;
-  const double g = gas.gamma;
-  Gas gb = gas;
-  gb.mu0 = b.mu0;
-  dt = dt * b.dt_scale;
+  const double cmu = uniform(gas.cmu * b.mu0);
+  const StageCoef sc = stage_coef(stage, dt * b.dt_scale);
   const int x = t / (TJ * TK), y = (t / TK) % TJ, z = t % TK;
   const int gi = i0 + x, gj = j0 + y, gk = k0 + z;
   const bool own = gi < ni && gj < nj && gk < nk;
@@ -784,24 +768,24 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
   for (int it = 0; it < NIT; ++it) {
     const int h = t + it * T::NT;
     if (h < T::NPV) {
-      double pp[5];
-      cons_to_prim_fast(qq[it], g, pp);
+      double pp[6];
+      prim_and_temp(qq[it], gas, pp);
 #pragma unroll
       for (int v = 0; v < 5; ++v) s_pv[v * T::NPV + h] = pp[v];
-      s_T[h] = temperature_fast(pp, gb.R);
+      s_T[h] = pp[5];
     }
   }
 
   // ---- metrics of the G cells --------------------------------------------------
-  double kk[9];
+  double kkh[9];   // kxyz / 2 of the thread's cell
 #pragma unroll
-  for (int m = 0; m < 9; ++m) kk[m] = b.kxyz[m * N + c];
+  for (int m = 0; m < 9; ++m) kkh[m] = 0.5 * b.kxyz[m * N + c];
   constexpr int NGIT = FusedCells<TI, TJ, TK>::NGIT;
   double kh[NGIT > 1 ? NGIT - 1 : 1][9];
 #pragma unroll
   for (int it = 1; it < NGIT; ++it) {
 #pragma unroll
-    for (int m = 0; m < 9; ++m) kh[it - 1][m] = b.kxyz[m * N + fc.gh[it - 1]];
+    for (int m = 0; m < 9; ++m) kh[it - 1][m] = 0.5 * b.kxyz[m * N + fc.gh[it - 1]];
   }
   __syncthreads();
 
@@ -815,22 +799,21 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
     const int lx = lc.x, ly = lc.y, lz = lc.z;
     double kc[9];
 #pragma unroll
-    for (int m = 0; m < 9; ++m) kc[m] = it == 0 ? kk[m] : kh[it > 0 ? it - 1 : 0][m];
+    for (int m = 0; m < 9; ++m) kc[m] = it == 0 ? kkh[m] : kh[it > 0 ? it - 1 : 0][m];
     double d[3][4];
     const int s0 = T::pv_slot(lx, ly, lz);
-    const double pv[5] = {0.0, s_pv[T::NPV + s0], s_pv[2 * T::NPV + s0], s_pv[3 * T::NPV + s0], 0.0};
-    const double Tc = s_T[s0];
+    const double uvwT[4] = {s_pv[T::NPV + s0], s_pv[2 * T::NPV + s0], s_pv[3 * T::NPV + s0], s_T[s0]};
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
       const int sp = T::pv_slot(lx + (l == 0), ly + (l == 1), lz + (l == 2));
       const int sm = T::pv_slot(lx - (l == 0), ly - (l == 1), lz - (l == 2));
-      d[l][0] = 0.5 * (s_pv[T::NPV + sp] - s_pv[T::NPV + sm]);
-      d[l][1] = 0.5 * (s_pv[2 * T::NPV + sp] - s_pv[2 * T::NPV + sm]);
-      d[l][2] = 0.5 * (s_pv[3 * T::NPV + sp] - s_pv[3 * T::NPV + sm]);
-      d[l][3] = 0.5 * (s_T[sp] - s_T[sm]);
+      d[l][0] = s_pv[T::NPV + sp] - s_pv[T::NPV + sm];
+      d[l][1] = s_pv[2 * T::NPV + sp] - s_pv[2 * T::NPV + sm];
+      d[l][2] = s_pv[3 * T::NPV + sp] - s_pv[3 * T::NPV + sm];
+      d[l][3] = s_T[sp] - s_T[sm];
     }
     double g9[9];
-    viscous_flux_fast(pv, Tc, d, kc, gb, g9);
+    viscous_flux_fast(uvwT, d, kc, cmu, gas, g9);
 #pragma unroll
     for (int m = 0; m < 9; ++m) {
       if constexpr (RS) gsave[it][m] = g9[m];
@@ -858,19 +841,18 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
   if (own) {
     const int sp[3] = {T::g_slot(x + 1, y, z), T::g_slot(x, y + 1, z), T::g_slot(x, y, z + 1)};
     const int sm[3] = {T::g_slot(x - 1, y, z), T::g_slot(x, y - 1, z), T::g_slot(x, y, z - 1)};
+    double gm[9], gp[9], dj[9], dk[9];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      double res = 0.0;
-#pragma unroll
-      for (int jj = 0; jj < 3; ++jj) {
-        const double* Gc = s_g + gidx(r, jj) * T::NG;
-        const double d0 = 0.5 * (Gc[sp[0]] - Gc[sm[0]]);
-        const double d1 = 0.5 * (Gc[sp[1]] - Gc[sm[1]]);
-        const double d2 = 0.5 * (Gc[sp[2]] - Gc[sm[2]]);
-        res = res + (d0 * kk[0 * 3 + jj] + d1 * kk[1 * 3 + jj] + d2 * kk[2 * 3 + jj]);
-      }
-      vis[r] = res;
+    for (int m = 0; m < 9; ++m) {
+      const double* Gc = s_g + m * T::NG;
+      gm[m] = Gc[sm[0]];
+      gp[m] = Gc[sp[0]];
+      dj[m] = Gc[sp[1]] - Gc[sm[1]];
+      dk[m] = Gc[sp[2]] - Gc[sm[2]];
     }
+    visc_div_im(gm, kkh, vis);
+    visc_div_jk(dj, dk, kkh, vis);
+    visc_div_ip(gp, kkh, vis);
   }
   __syncthreads();   // G space is reused by the face buffer (and the primitives)
   if constexpr (RS) {
@@ -878,8 +860,8 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
     for (int it = 0; it < NIT; ++it) {
       const int h = t + it * T::NT;
       if (h < T::NPV) {
-        double pp[5];
-        cons_to_prim_fast(qq[it], g, pp);
+        double pp[6];
+        prim_and_temp(qq[it], gas, pp);
 #pragma unroll
         for (int v = 0; v < 5; ++v) s_pv[v * T::NPV + h] = pp[v];
       }
@@ -892,20 +874,14 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
   load_kl_own<0>(b, c, gi, own, kl0);
   load_kl_own<1>(b, c, gj, own, kl1);
   load_kl_own<2>(b, c, gk, own, kl2);
-  double inv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  const double rvol = own ? rcp(b.vol[c] + 1e-300) : 0.0;
-  face_axis<0, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl0, own, t, x, y, z, rvol, g, inv);
-  face_axis<1, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl1, own, t, x, y, z, rvol, g, inv);
-  face_axis<2, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl2, own, t, x, y, z, rvol, g, inv);
+  double A[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const double rvh = own ? 0.5 * rcp(b.vol[c] + 1e-300) : 0.0;
+  face_axis<1, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl1, own, t, x, y, z, gas, A);
+  face_axis<2, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl2, own, t, x, y, z, gas, A);
+  face_axis<0, T, TI, TJ, TK, T::NT, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl0, own, t, x, y, z, gas, A);
   if (!own) return;
 
   // ---- 4. rhs and the RK3 combination ----------------------------------------
-  double rhs[5];
-  rhs[0] = inv[0] + 0.0;
-  rhs[1] = inv[1] + vis[0];
-  rhs[2] = inv[2] + vis[1];
-  rhs[3] = inv[3] + vis[2];
-  rhs[4] = inv[4] + vis[3];
   double qs[5], qq0[5];
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
@@ -913,13 +889,13 @@ __device__ __forceinline__ void stage_tile_fused_regs(const BlockDesc& b, int i0
     qq0[v] = stage == 1 ? 0.0 : q0[v * N + c];
   }
 #pragma unroll
-  for (int v = 0; v < 5; ++v) qout[v * N + c] = rk_combine(stage, qq0[v], qs[v], dt, rhs[v]);
+  for (int v = 0; v < 5; ++v) qout[v * N + c] = stage_update(sc, qq0[v], qs[v], A[v], rvh, v == 0 ? 0.0 : vis[v - 1]);
 }
 
 template <int TI, int TJ, int TK, int LIM, bool RS>
 __device__ __forceinline__ void stage_tile_fused(const BlockDesc& b, int i0, int j0, int k0,
                                                  const double* __restrict__ qin, const double* q0, double* qout,
-                                                 const Gas& gas, double dt, int stage) {
+                                                 const StageGas& gas, double dt, int stage) {
   FusedCells<TI, TJ, TK> fc;
   fused_cells<TI, TJ, TK>(b, i0, j0, k0, (int)threadIdx.x, fc);
   double qq[FusedCells<TI, TJ, TK>::NIT][5];
@@ -931,7 +907,7 @@ __device__ __forceinline__ void stage_tile_fused(const BlockDesc& b, int i0, int
 // form at 256 threads: three workgroups per CU, at most 168 VGPRs).
 template <int TI, int TJ, int TK, int LIM, bool RS, int WPE>
 __global__ void __launch_bounds__(TI * TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_stage_fused(BlockDesc b, int stage, Gas gas, double dt, int ntj, int ntk) {
+k_stage_fused(BlockDesc b, int stage, StageGas gas, double dt, int ntj, int ntk) {
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int tk = t % ntk, tj = (t / ntk) % ntj, ti = t / (ntk * ntj);
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
@@ -941,7 +917,7 @@ k_stage_fused(BlockDesc b, int stage, Gas gas, double dt, int ntj, int ntk) {
 
 template <int TI, int TJ, int TK, int LIM, bool RS, int WPE>
 __global__ void __launch_bounds__(TI * TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_stage_fused_batched(const BlockDesc* __restrict__ blocks, const Tile3* __restrict__ tiles, int stage, Gas gas,
+k_stage_fused_batched(const BlockDesc* __restrict__ blocks, const Tile3* __restrict__ tiles, int stage, StageGas gas,
                       double dt) {
   const Tile3 tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];
   const BlockDesc& b = blocks[tl.block];
@@ -1027,15 +1003,15 @@ struct SplitGeom {
 
 template <int TI, int TJ, int TK>
 __device__ __forceinline__ void visc_tile(const BlockDesc& b, int i0, int j0, int k0, const double* __restrict__ qin,
-                                          const Gas& gas) {
+                                          const StageGas& gas) {
+  EXACT_FP
   using T = FusedGeom<TI, TJ, TK>;       // g_slot / g_cell: tile + one-cell cross halo
   __shared__ double s_w[4 * T::NG];      // u, v, w, T
   const int t = threadIdx.x;
   const int ni = b.ni, nj = b.nj, nk = b.nk;
   const int64_t N = b.N;
   const int64_t si = (int64_t)nj * nk, sj = nk;
-  Gas gb = gas;
-  gb.mu0 = b.mu0;
+  const double cmu = uniform(gas.cmu * b.mu0);
   {
     constexpr int NIT = (T::NG + T::NT - 1) / T::NT;
     int cc[NIT];
@@ -1062,12 +1038,12 @@ __device__ __forceinline__ void visc_tile(const BlockDesc& b, int i0, int j0, in
     for (int it = 0; it < NIT; ++it) {
       const int h = t + it * T::NT;
       if (h < T::NG) {
-        double pp[5];
-        cons_to_prim_fast(qq[it], gas.gamma, pp);
+        double pp[6];
+        prim_and_temp(qq[it], gas, pp);
         s_w[h] = pp[1];
         s_w[T::NG + h] = pp[2];
         s_w[2 * T::NG + h] = pp[3];
-        s_w[3 * T::NG + h] = temperature_fast(pp, gb.R);
+        s_w[3 * T::NG + h] = pp[5];
       }
     }
   }
@@ -1077,21 +1053,20 @@ __device__ __forceinline__ void visc_tile(const BlockDesc& b, int i0, int j0, in
   if (gi >= ni || gj >= nj || gk >= nk) return;
   const int64_t c = (int64_t)gi * si + (int64_t)gj * sj + gk;
   const int s0 = T::g_slot(x, y, z);
-  const double pv[5] = {0.0, s_w[s0], s_w[T::NG + s0], s_w[2 * T::NG + s0], 0.0};
-  const double Tc = s_w[3 * T::NG + s0];
+  const double uvwT[4] = {s_w[s0], s_w[T::NG + s0], s_w[2 * T::NG + s0], s_w[3 * T::NG + s0]};
   double d[3][4];
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
     const int sp = T::g_slot(x + (l == 0), y + (l == 1), z + (l == 2));
     const int sm = T::g_slot(x - (l == 0), y - (l == 1), z - (l == 2));
 #pragma unroll
-    for (int v = 0; v < 4; ++v) d[l][v] = 0.5 * (s_w[v * T::NG + sp] - s_w[v * T::NG + sm]);
+    for (int v = 0; v < 4; ++v) d[l][v] = s_w[v * T::NG + sp] - s_w[v * T::NG + sm];
   }
   double kc[9];
 #pragma unroll
-  for (int m = 0; m < 9; ++m) kc[m] = b.kxyz[m * N + c];
+  for (int m = 0; m < 9; ++m) kc[m] = 0.5 * b.kxyz[m * N + c];
   double g9[9];
-  viscous_flux_fast(pv, Tc, d, kc, gb, g9);
+  viscous_flux_fast(uvwT, d, kc, cmu, gas, g9);
 #pragma unroll
   for (int m = 0; m < 9; ++m) b.G[m * N + c] = g9[m];
 }
@@ -1099,7 +1074,8 @@ __device__ __forceinline__ void visc_tile(const BlockDesc& b, int i0, int j0, in
 template <int TI, int TJ, int TK, int NTH, int LIM>
 __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int j0, int k0,
                                                  const double* __restrict__ qin, const double* q0, double* qout,
-                                                 const Gas& gas, double dt, int stage) {
+                                                 const StageGas& gas, double dt, int stage) {
+  EXACT_FP
   using T = SplitGeom<TI, TJ, TK>;
   static_assert(NTH >= T::NT && NTH % 64 == 0, "stage kernel needs a thread per cell");
   __shared__ double lds[T::NLDS];
@@ -1109,8 +1085,7 @@ __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int
   const int ni = b.ni, nj = b.nj, nk = b.nk;
   const int64_t N = b.N;
   const int64_t si = (int64_t)nj * nk, sj = nk;
-  const double g = gas.gamma;
-  dt = dt * b.dt_scale;
+  const StageCoef sc = stage_coef(stage, dt * b.dt_scale);
   // threads t < NT own cell (x, y, z) of the tile; all NTH threads compute faces
   const int x = t / (TJ * TK), y = (t / TK) % TJ, z = t % TK;
   const int gi = i0 + x, gj = j0 + y, gk = k0 + z;
@@ -1147,8 +1122,8 @@ __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int
     for (int it = 0; it < NIT; ++it) {
       const int h = t + it * NTH;
       if (h < T::NP) {
-        double pp[5];
-        cons_to_prim_fast(qq[it], g, pp);
+        double pp[6];
+        prim_and_temp(qq[it], gas, pp);
 #pragma unroll
         for (int v = 0; v < 5; ++v) s_pv[v * T::NP + h] = pp[v];
       }
@@ -1156,9 +1131,9 @@ __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int
   }
 
   // ---- 2. divergence of the viscous tensor (G of the six wrapped neighbours) ---
-  double kk[9];
+  double kkh[9];
 #pragma unroll
-  for (int m = 0; m < 9; ++m) kk[m] = own ? b.kxyz[m * N + c] : 0.0;
+  for (int m = 0; m < 9; ++m) kkh[m] = own ? 0.5 * b.kxyz[m * N + c] : 0.0;
   double kl0[3], kl1[3], kl2[3];
   load_kl_own<0>(b, c, gi, own, kl0);
   load_kl_own<1>(b, c, gj, own, kl1);
@@ -1169,38 +1144,30 @@ __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int
                            c + (wrap_p(gk, nk) - gk)};
     const int64_t cm[3] = {c + (int64_t)(wrap_m(gi, ni) - gi) * si, c + (int64_t)(wrap_m(gj, nj) - gj) * sj,
                            c + (wrap_m(gk, nk) - gk)};
-    const double* __restrict__ Gb = b.G;
+    double gm[9], gp[9], dj[9], dk[9];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      double res = 0.0;
-#pragma unroll
-      for (int jj = 0; jj < 3; ++jj) {
-        const double* Gc = Gb + gidx(r, jj) * N;
-        const double d0 = 0.5 * (Gc[cp[0]] - Gc[cm[0]]);
-        const double d1 = 0.5 * (Gc[cp[1]] - Gc[cm[1]]);
-        const double d2 = 0.5 * (Gc[cp[2]] - Gc[cm[2]]);
-        res = res + (d0 * kk[0 * 3 + jj] + d1 * kk[1 * 3 + jj] + d2 * kk[2 * 3 + jj]);
-      }
-      vis[r] = res;
+    for (int m = 0; m < 9; ++m) {
+      const double* __restrict__ Gc = b.G + m * N;
+      gm[m] = Gc[cm[0]];
+      gp[m] = Gc[cp[0]];
+      dj[m] = Gc[cp[1]] - Gc[cm[1]];
+      dk[m] = Gc[cp[2]] - Gc[cm[2]];
     }
+    visc_div_im(gm, kkh, vis);
+    visc_div_jk(dj, dk, kkh, vis);
+    visc_div_ip(gp, kkh, vis);
   }
   __syncthreads();
 
   // ---- 3. inviscid faces, axis by axis ---------------------------------------
-  double inv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  const double rvol = own ? rcp(b.vol[c] + 1e-300) : 0.0;
-  face_axis<0, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl0, own, t, x, y, z, rvol, g, inv);
-  face_axis<1, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl1, own, t, x, y, z, rvol, g, inv);
-  face_axis<2, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kk, kl2, own, t, x, y, z, rvol, g, inv);
+  double A[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const double rvh = own ? 0.5 * rcp(b.vol[c] + 1e-300) : 0.0;
+  face_axis<1, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl1, own, t, x, y, z, gas, A);
+  face_axis<2, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl2, own, t, x, y, z, gas, A);
+  face_axis<0, T, TI, TJ, TK, NTH, LIM>(b, i0, j0, k0, s_pv, s_f, kkh, kl0, own, t, x, y, z, gas, A);
   if (!own) return;
 
   // ---- 4. rhs and the RK3 combination ----------------------------------------
-  double rhs[5];
-  rhs[0] = inv[0] + 0.0;
-  rhs[1] = inv[1] + vis[0];
-  rhs[2] = inv[2] + vis[1];
-  rhs[3] = inv[3] + vis[2];
-  rhs[4] = inv[4] + vis[3];
   double qs[5], qq0[5];
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
@@ -1208,11 +1175,11 @@ __device__ __forceinline__ void stage_tile_split(const BlockDesc& b, int i0, int
     qq0[v] = stage == 1 ? 0.0 : q0[v * N + c];
   }
 #pragma unroll
-  for (int v = 0; v < 5; ++v) qout[v * N + c] = rk_combine(stage, qq0[v], qs[v], dt, rhs[v]);
+  for (int v = 0; v < 5; ++v) qout[v * N + c] = stage_update(sc, qq0[v], qs[v], A[v], rvh, v == 0 ? 0.0 : vis[v - 1]);
 }
 
 template <int TI, int TJ, int TK>
-__global__ void __launch_bounds__(TI * TJ * TK) k_visc_tensor(BlockDesc b, int stage, Gas gas, int ntj, int ntk) {
+__global__ void __launch_bounds__(TI * TJ * TK) k_visc_tensor(BlockDesc b, int stage, StageGas gas, int ntj, int ntk) {
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int tk = t % ntk, tj = (t / ntk) % ntj, ti = t / (ntk * ntj);
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
@@ -1220,7 +1187,7 @@ __global__ void __launch_bounds__(TI * TJ * TK) k_visc_tensor(BlockDesc b, int s
 }
 
 template <int TI, int TJ, int TK, int NTH, int LIM>
-__global__ void __launch_bounds__(NTH) k_stage_split(BlockDesc b, int stage, Gas gas, double dt, int ntj, int ntk) {
+__global__ void __launch_bounds__(NTH) k_stage_split(BlockDesc b, int stage, StageGas gas, double dt, int ntj, int ntk) {
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int tk = t % ntk, tj = (t / ntk) % ntj, ti = t / (ntk * ntj);
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
@@ -1231,7 +1198,7 @@ __global__ void __launch_bounds__(NTH) k_stage_split(BlockDesc b, int stage, Gas
 template <int TI, int TJ, int TK>
 __global__ void __launch_bounds__(TI * TJ * TK) k_visc_tensor_batched(const BlockDesc* __restrict__ blocks,
                                                                       const Tile3* __restrict__ tiles, int stage,
-                                                                      Gas gas) {
+                                                                      StageGas gas) {
   const Tile3 tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];
   const BlockDesc& b = blocks[tl.block];
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
@@ -1240,7 +1207,7 @@ __global__ void __launch_bounds__(TI * TJ * TK) k_visc_tensor_batched(const Bloc
 
 template <int TI, int TJ, int TK, int NTH, int LIM>
 __global__ void __launch_bounds__(NTH) k_stage_split_batched(const BlockDesc* __restrict__ blocks,
-                                                             const Tile3* __restrict__ tiles, int stage, Gas gas,
+                                                             const Tile3* __restrict__ tiles, int stage, StageGas gas,
                                                              double dt) {
   const Tile3 tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];
   const BlockDesc& b = blocks[tl.block];
@@ -1315,7 +1282,7 @@ inline void tile_dims(int v, int& ti, int& tj, int& tk) {
 // One stage of one block (plain launch) with variant v; the limiter is a
 // template parameter of the stage kernels (LIM_MINMOD / LIM_VANLEER).
 template <int LIM>
-inline void launch_stage_lim(int v, const BlockDesc& d, int stage, const Gas& gas, double dt, int ncu,
+inline void launch_stage_lim(int v, const BlockDesc& d, int stage, const StageGas& gas, double dt, int ncu,
                              hipStream_t st) {
   int TI, TJ, TK;
   tile_dims(v, TI, TJ, TK);
@@ -1343,17 +1310,24 @@ inline void launch_stage_lim(int v, const BlockDesc& d, int stage, const Gas& ga
   }
 }
 
+inline StageGas stage_gas(const Gas& g) {
+  const double gm1 = g.gamma - 1.0;
+  return StageGas{gm1, 0.5 * gm1, 2.0 * g.gamma / gm1, g.R, 1.0 / g.R, g.Ts, (g.T0 + g.Ts) / (g.T0 * std::sqrt(g.T0)),
+                  g.gamma * g.R / (gm1 * g.Pr_lam)};
+}
+
 inline void launch_fused(int v, const BlockDesc& d, int stage, const Gas& gas, int lim, double dt, int ncu,
                          hipStream_t st) {
-  if (lim == LIM_VANLEER) launch_stage_lim<LIM_VANLEER>(v, d, stage, gas, dt, ncu, st);
-  else launch_stage_lim<LIM_MINMOD>(v, d, stage, gas, dt, ncu, st);
+  const StageGas sg = stage_gas(gas);
+  if (lim == LIM_VANLEER) launch_stage_lim<LIM_VANLEER>(v, d, stage, sg, dt, ncu, st);
+  else launch_stage_lim<LIM_MINMOD>(v, d, stage, sg, dt, ncu, st);
 }
 
 // One stage of every block in one launch (two for the split pair) over a tile
 // table built for v.
 template <int LIM>
 inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3* tiles, int ntiles, int stage,
-                                     const Gas& gas, double dt, int ncu, hipStream_t st) {
+                                     const StageGas& gas, double dt, int ncu, hipStream_t st) {
   switch (v) {
 #define FAMRDP_TB(id, a, b, c, rs, w)                                                                       \
   case id:                                                                                                   \
@@ -1379,8 +1353,9 @@ inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3
 
 inline void launch_fused_batched(int v, const BlockDesc* blocks, const Tile3* tiles, int ntiles, int stage,
                                  const Gas& gas, int lim, double dt, int ncu, hipStream_t st) {
-  if (lim == LIM_VANLEER) launch_stage_batched_lim<LIM_VANLEER>(v, blocks, tiles, ntiles, stage, gas, dt, ncu, st);
-  else launch_stage_batched_lim<LIM_MINMOD>(v, blocks, tiles, ntiles, stage, gas, dt, ncu, st);
+  const StageGas sg = stage_gas(gas);
+  if (lim == LIM_VANLEER) launch_stage_batched_lim<LIM_VANLEER>(v, blocks, tiles, ntiles, stage, sg, dt, ncu, st);
+  else launch_stage_batched_lim<LIM_MINMOD>(v, blocks, tiles, ntiles, stage, sg, dt, ncu, st);
 }
 
 }  // namespace famrdp

@@ -5,32 +5,44 @@
 //
 // A workgroup owns a column of TJ x TK cells (one thread per (j, k) column)
 // over a segment [pA, pB) of planes along i, the slowest axis, and walks it
-// one plane per step.  Step s, for s = pA-1 .. pB:
+// one plane per step, with two barriers per step.  Step s, for s = pA-1 .. pB:
 //
-//   a. The primitives and temperature of plane s go to the LDS plane P: the
+//   A. The primitives and temperature of plane s go to the LDS plane P: the
 //      tile's columns and two halo rings (the second one without corners),
-//      at periodic (roll) coordinates.  They were converted in the previous
-//      step from loads issued a step before that.
-//   b. The i-face between planes s-1 and s of the thread's own column (its
-//      left state was reconstructed in the previous step; the right state
-//      and the next face's left state share one limited slope per
-//      variable), and the viscous flux tensor G of plane s at the column
-//      (j/k differences from P, i differences from the column's registers).
-//   c. The viscous divergence of plane s-1: j/k differences of G(s-1) from
-//      the LDS G plane, the i difference from G(s) and G(s-2) in registers.
-//   d. The inviscid terms of plane s-1 (i from the two i-faces around it,
-//      j and k from the LDS face buffer filled in the previous step) and the
-//      Shu-Osher combination; plane s-1 is written.
-//   e. G(s) replaces G(s-1) in LDS, with G of the tile's one-cell cross halo;
-//      the MUSCL-2 + Roe faces of plane s along j and k go to the face
-//      buffer (each thread its column's low j-face, then its low k-face,
-//      both with offsets fixed by the column; the last wave the far-end
-//      layer); the halo of plane s+1 is converted for the next step.
+//      at periodic (roll) coordinates; they were converted in the previous
+//      step.  Then what plane s-1 takes from LDS, left there by the previous
+//      step: the j and k differences of the viscous tensor G(s-1) and of the
+//      j and k face fluxes, and the column's own G(s-1), folded at once into
+//      the share the lower i-neighbour of plane s has in its divergence (four
+//      values carried instead of nine).  Then the i-face between planes s-1
+//      and s of the column, from registers (its left state was reconstructed
+//      in the previous step; the right state and the next face's left state
+//      share one limited slope per variable).
+//   -- barrier: P is in place, and every read of G(s-1) and of its faces done
+//   B. G of plane s at the column (j/k differences from P, i differences from
+//      the column's registers), which completes the divergence of plane s-1;
+//      the Shu-Osher update of plane s-1 is written.  G(s) goes over G(s-1) in
+//      LDS, with G of the tile's one-cell cross halo; the MUSCL-2 + Roe faces
+//      of plane s along j and k go to the face buffer (each thread its
+//      column's low j-face, then its low k-face, both with offsets fixed by
+//      the column; the last wave the far-end layer); the halo of plane s+1 is
+//      converted for the next step.
+//   -- barrier: G(s) and the faces of plane s are in place, P is free
 //
-// Loads are issued a phase or more before their use where registers allow:
-// the column's metrics of plane s before the barrier of phase a (and kept for
-// the next step's divergence), the update operands of plane s-1 and the
-// cross halo's metrics in phase b, the state of plane s+2 a step ahead.
+// Loads are issued a phase or more before their use and spread through the
+// arithmetic (march_spread): the next plane's metrics, the state of the plane
+// after it and the update operands through the faces of this plane, the halo's
+// state at the end of phase B, the metrics of the faces' other cells and of
+// the cross halo at the end of phase A.
+//
+// What bounds it (260^3 padded, stage 2, random smooth state): neither FP64
+// issue nor HBM alone.  The same launch with every load an L2 hit takes
+// 1.09 ms, its VALU instructions alone 0.64 ms, its bytes past L2 (6 GB, 1.8
+// times the compulsory 3.5 GB: halos, the re-read of the plane being updated)
+// 1.2 ms at the 4.9 TB/s of a large copy; at two waves per SIMD (255
+// registers, 77.7 KB of LDS) the three overlap to 1.40 ms (132^3: 209 us).
+// With three barriers per plane, conservative jumps in the Roe flux and the
+// far-end faces' loads inside their round: 1.51 ms (231 us).
 //
 // Each cell's primitives, viscous tensor and faces are computed once per
 // segment, apart from the tile's halo rings in j and k and the two extra
@@ -48,13 +60,6 @@
 #include "famrdp_march_geom.h"
 
 namespace famrdp {
-
-// primitives (rho, u, v, w, p) and temperature of one cell, as the fused
-// kernel stages them
-DF void march_prim(const double q[5], double g, double R, double pv[6]) {
-  cons_to_prim_fast(q, g, pv);
-  pv[5] = temperature_fast(pv, R);
-}
 
 // The arrays a march reads and writes, as buffer resources: a load or store
 // takes the element's 32-bit byte offset in a vector register and the
@@ -90,17 +95,14 @@ __host__ __device__ __forceinline__ bool march_fits(int64_t N) { return N * 72 <
 
 // Viscous flux tensor of the cell at P slot `sl` (rhs/viscous.py:30-108):
 // j/k neighbours from P, i neighbours (u, v, w, T) from um (plane s-1) and up
-// (plane s+1); kch = kxyz / 2 at the cell.  The fused kernel's expressions,
-// with the 1/2 of each central difference moved onto the metrics: halving
-// is exact, so every product d k of the gradients is the same number and
-// the tensor has the same bits, for 12 multiplies fewer.
+// (plane s+1); kch = kxyz / 2 at the cell.
 template <int TJ, int TK>
-DF void march_visc(const double* sP, int sl, const double um[4], const double up[4], const double kch[9],
-                   const Gas& gb, double g9[9]) {
+DF void march_visc(const double* sP, int sl, const double um[4], const double up[4], const double kch[9], double cmu,
+                   const StageGas& gas, double g9[9]) {
+  EXACT_FP
   using M = MarchGeom<TJ, TK>;
   constexpr int NP = M::NP;
-  const double pv[5] = {0.0, sP[NP + sl], sP[2 * NP + sl], sP[3 * NP + sl], 0.0};
-  const double Tc = sP[5 * NP + sl];
+  const double uvwT[4] = {sP[NP + sl], sP[2 * NP + sl], sP[3 * NP + sl], sP[5 * NP + sl]};
   double d[3][4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) d[0][s] = up[s] - um[s];
@@ -113,16 +115,15 @@ DF void march_visc(const double* sP, int sl, const double um[4], const double up
     d[l][2] = sP[3 * NP + sp] - sP[3 * NP + sm];
     d[l][3] = sP[5 * NP + sp] - sP[5 * NP + sm];
   }
-  viscous_flux_fast(pv, Tc, d, kch, gb, g9);
+  viscous_flux_fast(uvwT, d, kch, cmu, gas, g9);
 }
 
-// One j- or k-face of the plane (rhs/invscd.py:53-97) into face buffer slot
-// f: the four cells' primitives from P slots base + s str (s = 0..3), kxyz
-// of the face's axis at the cells either side (plane offsets cl, cr; the
-// axis's first row of kxyz at byte offset s0).
+// One j- or k-face of the plane (rhs/invscd.py:53-97, twice the flux) into
+// face buffer slot f: the four cells' primitives from P slots base + s str
+// (s = 0..3), kl, kr = kxyz / 2 of the face's axis at the cells either side.
 template <int TJ, int TK, int LIM>
-DF void march_face(const double* sP, double* sF, int base, int str, __amdgpu_buffer_rsrc_t rk, unsigned cl,
-                   unsigned cr, unsigned s0, unsigned nb, int f, double g) {
+DF void march_face(const double* sP, double* sF, int base, int str, const double kl[3], const double kr[3], int f,
+                   const StageGas& gas) {
   using M = MarchGeom<TJ, TK>;
   double p4[4][5];
 #pragma unroll
@@ -130,60 +131,10 @@ DF void march_face(const double* sP, double* sF, int base, int str, __amdgpu_buf
 #pragma unroll
     for (int v = 0; v < 5; ++v) p4[s4][v] = sP[v * M::NP + base + s4 * str];
   }
-  double kl[3], kr[3];
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    kl[m] = ldx(rk, cl, s0 + m * nb);
-    kr[m] = ldx(rk, cr, s0 + m * nb);
-  }
   double Fa[5];
-  face_flux_prim<LIM>(p4[0], p4[1], p4[2], p4[3], kl, kr, g, Fa);
+  face_flux2<LIM>(p4[0], p4[1], p4[2], p4[3], kl, kr, gas, Fa);
 #pragma unroll
   for (int v = 0; v < 5; ++v) sF[v * M::NFB + f] = Fa[v];
-}
-
-// A thread's own low j- or k-face (rounds 0 and 1): the right-hand cell is
-// the thread's column, whose kxyz / 2 of the plane (krh, rows s0 / nb ..) the
-// thread holds in registers; the left-hand row (plane offset cl) is loaded
-// and halved, which is exact, so the face has the bits of march_face.
-template <int TJ, int TK, int LIM>
-DF void march_face_own(const double* sP, double* sF, int base, int str, __amdgpu_buffer_rsrc_t rk, unsigned cl,
-                       unsigned s0, unsigned nb, const double krh[3], int f, double g) {
-  using M = MarchGeom<TJ, TK>;
-  double p4[4][5];
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) p4[s4][v] = sP[v * M::NP + base + s4 * str];
-  }
-  double klh[3];
-#pragma unroll
-  for (int m = 0; m < 3; ++m) klh[m] = 0.5 * ldx(rk, cl, s0 + m * nb);
-  double Fa[5];
-  face_flux_prim_h<LIM>(p4[0], p4[1], p4[2], p4[3], klh, krh, g, Fa);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) sF[v * M::NFB + f] = Fa[v];
-}
-
-// The far-end layer of the plane at offset `op` (face_of round 2: j-faces
-// past the tile's last row, k-faces past its last column), for the threads
-// of the last wave; j-face f (< NFJ) at (f / TK, f % TK) lies between local
-// rows f / TK - 1 and f / TK, k-face NFJ + r (TK + 1) + c between local
-// columns c - 1 and c of row r.  Faces exist between cells 1 .. n-2 of their
-// axis (left cell a in [1, n-3]) and never read a wrapped cell.
-template <int TJ, int TK, int LIM>
-DF void march_far_faces(const BlockDesc& b, __amdgpu_buffer_rsrc_t rk, unsigned nb, int j0, int k0, unsigned op,
-                        const double* sP, double* sF, double g, int t) {
-  using M = MarchGeom<TJ, TK>;
-  const int f = M::face_of(t, 2);
-  if (f < 0) return;
-  const int nj = b.nj, nk = b.nk;
-  const MarchFace fc = M::face(f, j0, k0, nj, nk);
-  if (!fc.ok) return;
-  const bool isj = fc.isj;
-  const unsigned cl = op + (isj ? (unsigned)fc.a * nk + fc.oc : (unsigned)fc.oc * nk + fc.a) + (isj ? 3u : 6u) * (unsigned)b.N;
-  const unsigned cr = cl + (isj ? (unsigned)nk : 1u);
-  march_face<TJ, TK, LIM>(sP, sF, fc.base, fc.str, rk, cl, cr, 0, nb, f, g);
 }
 
 // v, hidden from the optimiser: what is computed from it inside the march
@@ -193,22 +144,34 @@ __device__ __forceinline__ unsigned march_opaque(unsigned v) {
   return v;
 }
 
-// x as computed (rounded), hidden from the optimiser: the fused kernel
-// stages primitives, viscous tensors and face fluxes through LDS before
-// using them, so the compiler never contracts the multiply that produced a
-// value into the add that consumes it; values used here straight from
-// registers are held the same way, which keeps the bits equal
-DF void march_keep(double& x) { asm volatile("" : "+v"(x)); }
+// x is computed by here: the compiler moves arithmetic that only a later
+// phase consumes past barriers and scheduling fences, down to its use, and
+// then holds that arithmetic's many operands in registers instead of x
+DF void march_pin(double& x) { asm volatile("" : "+v"(x)); }
 template <int K>
-DF void march_keep(double (&x)[K]) {
+DF void march_pin(double (&x)[K]) {
 #pragma unroll
-  for (int i = 0; i < K; ++i) march_keep(x[i]);
+  for (int i = 0; i < K; ++i) march_pin(x[i]);
+}
+
+// Order for the scheduler: N loads, each followed by V arithmetic
+// instructions.  Issued back to back the loads of a phase hold every wave of
+// the workgroup at the address unit (about 16 cycles a load and CU, all four
+// waves in the same phase); spread through a face they cost their issue slot.
+template <int N, int V>
+DF void march_spread() {
+  if constexpr (N > 0) {
+    __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);   // a VMEM read
+    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);    // V VALU instructions
+    march_spread<N - 1, V>();
+  }
 }
 
 template <int TJ, int TK, int LIM>
 __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, int j0, int k0, int pA, int pB,
                                               const double* __restrict__ qin, const double* q0, double* qout,
-                                              const Gas& gas, double dt, int stage) {
+                                              const StageGas& gas, double dt, int stage) {
+  EXACT_FP
   using M = MarchGeom<TJ, TK>;
   double* sP = lds;                          // [6][NP]  rho u v w p T of plane s
   double* sG = sP + 6 * M::NP;               // [9][NGP] G of plane s-1 (then s)
@@ -219,21 +182,44 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
   const int ni = b.ni, nj = b.nj, nk = b.nk;
   const int64_t N = b.N;
   const unsigned si = (unsigned)nj * (unsigned)nk;
-  const double g = gas.gamma;
-  Gas gb = gas;
-  gb.mu0 = b.mu0;
-  dt = dt * b.dt_scale;
+  const double cmu = uniform(gas.cmu * b.mu0);
+  const StageCoef sc = stage_coef(stage, dt * b.dt_scale);
   const unsigned nb = (unsigned)N * 8u;     // bytes between variables
-  const __amdgpu_buffer_rsrc_t rq = march_rsrc(qin, 5 * N), r0 = march_rsrc(q0, 5 * N),
+  const __amdgpu_buffer_rsrc_t rq = march_rsrc(qin, 5 * N), r0 = march_rsrc(q0, stage == 1 ? 0 : 5 * N),   // stage 1 takes no q0: loads give 0
                                ro = march_rsrc(qout, 5 * N), rk = march_rsrc(b.kxyz, 9 * N),
                                rv = march_rsrc(b.vol, N);
 
   // ---- fixed per thread for the whole march --------------------------------
   const MarchThread th = M::thread(t, j0, k0, nj, nk);
   const int tj = th.tj, tk = th.tk, slot = th.slot, gslot = th.gslot, hs = th.hs;
-  const int hslot = th.hslot, hgslot = th.hgslot;
-  const bool own = th.own, jin = th.jin, kin = th.kin, fj = th.fj, fk = th.fk, hg = th.hg;
-  const unsigned col = th.col, hcol = th.hcol;
+  int hslot = th.hslot, hgslot = th.hgslot;
+  const bool own = th.own, jin = th.jin, kin = th.kin, hg = th.hg;
+  const unsigned col = th.col;
+  unsigned hcol = th.hcol, hcol2 = th.hcol;
+  // The last wave stages no halo; its threads take the far-end faces (face_of
+  // round 2: j-faces past the tile's last row, k-faces past its last column)
+  // instead.  The same registers hold their fixed places: hslot the P slot of
+  // the cell two before the face, hgslot the face buffer slot, hcol and hcol2
+  // the offsets in kxyz of the face's axis at the cells either side (hcol2
+  // less the three rows that follow), so the metrics of a far face and of a
+  // cross-halo cell are the same loads.
+  int fstr = 0;
+  const int ff = M::face_of(t, 2);
+  if (ff >= 0) {
+    const MarchFace fc = M::face(ff, j0, k0, nj, nk);
+    if (fc.ok) {
+      fstr = fc.str;
+      hslot = fc.base;
+      hgslot = ff;
+      const unsigned row = (fc.isj ? 3u : 6u) * (unsigned)N;
+      hcol = row + (fc.isj ? (unsigned)fc.a * nk + fc.oc : (unsigned)fc.oc * nk + fc.a);
+      hcol2 = hcol + (fc.isj ? (unsigned)nk : 1u) - 3u * (unsigned)N;
+    }
+  }
+  const bool hm = hg || fstr > 0;   // loads metrics for phase B's last part
+  // where the low faces' other cells lie (this cell where there is no face:
+  // a valid address, and a flux that no update reads)
+  const unsigned dfj = th.fj ? (unsigned)nk : 0u, dfk = th.fk ? 1u : 0u;
   auto plane = [&](int s) -> unsigned { return (unsigned)(s < 0 ? s + ni : (s >= ni ? s - ni : s)) * si; };
 
   // ---- warm-up: planes pA-2, pA-1 converted, pA loading ---------------------
@@ -241,14 +227,12 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
   {
     double qq[5], x[6];
     march_load5(rq, nb, plane(pA - 2) + col, qq);
-    march_prim(qq, g, gb.R, pm);
+    prim_and_temp(qq, gas, pm);
     march_load5(rq, nb, plane(pA - 1) + col, qq);
-    march_prim(qq, g, gb.R, pc);
-    march_keep(pm);
-    march_keep(pc);
+    prim_and_temp(qq, gas, pc);
     if (hg) {
       march_load5(rq, nb, plane(pA - 2) + hcol, qq);
-      march_prim(qq, g, gb.R, x);
+      prim_and_temp(qq, gas, x);
       sU[hs] = x[1];
       sU[M::NHG + hs] = x[2];
       sU[2 * M::NHG + hs] = x[3];
@@ -256,162 +240,139 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
     }
     if (hs >= 0) {
       march_load5(rq, nb, plane(pA - 1) + hcol, qq);
-      march_prim(qq, g, gb.R, x);
+      prim_and_temp(qq, gas, x);
 #pragma unroll
       for (int v = 0; v < 6; ++v) sH[v * M::NHS + hs] = x[v];
     }
   }
-  double qn[5], qnh[5] = {0, 0, 0, 0, 0};
+  double qn[5], kk[9];
   march_load5(rq, nb, plane(pA) + col, qn);
+#pragma unroll
+  for (int m = 0; m < 9; ++m) kk[m] = ldx(rk, plane(pA - 1) + col, m * nb);
+
+  // the update operands of the next step, and the state of its halo
+  double vl = 1.0, qs[5] = {0, 0, 0, 0, 0}, qq0[5] = {0, 0, 0, 0, 0}, qnh[5] = {0, 0, 0, 0, 0};
   if (hs >= 0) march_load5(rq, nb, plane(pA) + hcol, qnh);
 
   double kpvh[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // kxyz / 2 of the column at plane s-1
   double pLn[5] = {0, 0, 0, 0, 0};       // left state of the column's next i-face
   double Fm[5] = {0, 0, 0, 0, 0};        // i-face below plane s-1
-  double Gm2[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // G(s-2) of the column
+  double vism[4] = {0, 0, 0, 0};         // G(s-2)'s share of the divergence of plane s-1
 
   for (int s = pA - 1; s <= pB; ++s) {
     const unsigned op = plane(s), om = plane(s - 1);
     const unsigned c_s = op + march_opaque(col), c_m = om + march_opaque(col);
     const bool faces = s >= pA && s < pB;            // plane s is owned: its j/k faces
-    const bool upd = s > pA;                         // plane s-1 is owned: its update (s-1 < pB always)
-    // the column's metrics of plane s, loaded once (issued before the barrier,
-    // which covers their latency): the i-face takes its right-hand row from
-    // them, and they are kept for the next step's i-face (left-hand row) and
-    // divergence of G(s)
-    double kk[9];
-#pragma unroll
-    for (int m = 0; m < 9; ++m) kk[m] = ldx(rk, c_s, m * nb);
-    // ---- a. P <- plane s ------------------------------------------------------
+    const bool iin = s - 1 >= 2 && s - 1 <= ni - 3;  // plane s-1 takes its i-faces
+
+    // ---- A. P <- plane s -------------------------------------------------------
 #pragma unroll
     for (int v = 0; v < 6; ++v) sP[v * M::NP + slot] = pc[v];
     if (hs >= 0) {
 #pragma unroll
       for (int v = 0; v < 6; ++v) sP[v * M::NP + hslot] = sH[v * M::NHS + hs];
     }
-    __syncthreads();
-
-    // ---- b. i-face between planes s-1 and s; G of plane s at the column --------
-    double pn[6];
-    march_prim(qn, g, gb.R, pn);
-    march_keep(pn);
-    if (s + 2 <= pB + 1) march_load5(rq, nb, plane(s + 2) + march_opaque(col), qn);
-    // the metrics halved: the i-face normal is their sum, and the central
-    // differences of the viscous terms are taken without their 1/2
-    double kkh[9];
-#pragma unroll
-    for (int m = 0; m < 9; ++m) kkh[m] = 0.5 * kk[m];
-    double Fi[5] = {0, 0, 0, 0, 0};
+    __builtin_amdgcn_sched_barrier(0);
+    // what plane s-1 takes from LDS
+    double vis[4] = {vism[0], vism[1], vism[2], vism[3]};
+    double A[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     {
-      double pLs[5], pRs[5];
-      muscl_cell<LIM>(pm, pc, pn, pLs, pRs);
-      face_state_fence(pLn);
-      face_state_fence(pRs);
-      if (s >= pA && s - 1 >= 1 && s - 1 <= ni - 3) face_flux_lr_h(pLn, pRs, kpvh, kkh, g, Fi);
-      march_keep(Fi);
+      double dj[9], dk[9];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) pLn[v] = pLs[v];
-    }
-    // the update operands of plane s-1, issued before G(s) is computed
-    double qs[5] = {0, 0, 0, 0, 0}, qq0[5] = {0, 0, 0, 0, 0}, vl = 1.0;
-    if (upd && own) {
-      vl = ldx(rv, c_m, 0);
+      for (int m = 0; m < 9; ++m) {
+        const double* Gc = sG + m * M::NGP;
+        dj[m] = Gc[gslot + M::GK] - Gc[gslot - M::GK];
+        dk[m] = Gc[gslot + 1] - Gc[gslot - 1];
+      }
+      visc_div_jk(dj, dk, kpvh, vis);
+      const int lo = tj * TK + tk, lok = M::NFJ + tj * (TK + 1) + tk;
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        qs[v] = ldx(rq, c_m, v * nb);
-        qq0[v] = stage == 1 ? 0.0 : ldx(r0, c_m, v * nb);
+        const double* Fv = sF + v * M::NFB;
+        const double fj = Fv[lo + TK] - Fv[lo], fk = Fv[lok + 1] - Fv[lok];
+        A[v] = jin ? fj : 0.0;
+        A[v] = kin ? A[v] + fk : A[v];
       }
+      march_pin(vis);
+      march_pin(A);
     }
-    double g9[9];
-    {
-      const double um[4] = {pm[1], pm[2], pm[3], pm[5]}, up[4] = {pn[1], pn[2], pn[3], pn[5]};
-      march_visc<TJ, TK>(sP, slot, um, up, kkh, gb, g9);
-      march_keep(g9);
-    }
-    // metrics of the G cross-halo cell of plane s, for phase e
-    double kh[9];
-    if (hg) {
-      const unsigned ch = op + march_opaque(hcol);
+    double kkh[9];   // kxyz / 2 of plane s
 #pragma unroll
-      for (int m = 0; m < 9; ++m) kh[m] = ldx(rk, ch, m * nb);
+    for (int m = 0; m < 9; ++m) kkh[m] = 0.5 * kk[m];
+    {
+      double gm[9];
+#pragma unroll
+      for (int m = 0; m < 9; ++m) gm[m] = sG[m * M::NGP + gslot];
+      visc_div_im(gm, kkh, vism);
+      march_pin(vism);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the i-face between planes s-1 and s
+    double pn[6];
+    prim_and_temp(qn, gas, pn);
+    {
+      double pLs[5], pRs[5], Fi[5];
+      muscl_cell<LIM>(pm, pc, pn, pLs, pRs);
+      const double S[3] = {kpvh[0] + kkh[0], kpvh[1] + kkh[1], kpvh[2] + kkh[2]};
+      roe_flux2(pLn, pRs, S, gas, Fi);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) {
+        if (iin) A[v] = A[v] + (Fi[v] - Fm[v]);
+        Fm[v] = Fi[v];
+        pLn[v] = pLs[v];
+      }
+      march_pin(A);
+      march_pin(Fm);
+      march_pin(pLn);
+    }
+    // metrics of the faces' other cells, and of the cross halo or a far face
+    double kh[9], klj[3], klk[3];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      klj[m] = ldx(rk, c_s - dfj, (3 + m) * nb);
+      klk[m] = ldx(rk, c_s - dfk, (6 + m) * nb);
+    }
+    if (hm) {
+      const unsigned ch = op + march_opaque(hcol), ch2 = op + march_opaque(hcol2);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) kh[m] = ldx(rk, ch, m * nb);
+#pragma unroll
+      for (int m = 3; m < 9; ++m) kh[m] = ldx(rk, ch2, m * nb);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();   // P in place; G(s-1) and the faces of plane s-1 read
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- B. G(s), the update of plane s-1 ---------------------------------------
+    {
+      double g9[9];
+      const double um[4] = {pm[1], pm[2], pm[3], pm[5]}, up[4] = {pn[1], pn[2], pn[3], pn[5]};
+      march_visc<TJ, TK>(sP, slot, um, up, kkh, cmu, gas, g9);
+      visc_div_ip(g9, kpvh, vis);
+#pragma unroll
+      for (int m = 0; m < 9; ++m) sG[m * M::NGP + gslot] = g9[m];
+      march_pin(vis);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (s > pA && own) {   // plane s-1 is the segment's (s-1 < pB always)
+      const double rvh = 0.5 * rcp(vl + 1e-300);
+#pragma unroll
+      for (int v = 0; v < 5; ++v)
+        stx(ro, c_m, v * nb, stage_update(sc, qq0[v], qs[v], A[v], rvh, v == 0 ? 0.0 : vis[v - 1]));
     }
 #pragma unroll
     for (int v = 0; v < 6; ++v) {
       pm[v] = pc[v];
       pc[v] = pn[v];
     }
-
-    // ---- c. divergence of G(s-1) ------------------------------------------------
-    double vis[4] = {0.0, 0.0, 0.0, 0.0};
-    if (upd && own) {
-      const double* km = kpvh;   // the differences' 1/2 on the metrics, as in march_visc
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        double res = 0.0;
-#pragma unroll
-        for (int jj = 0; jj < 3; ++jj) {
-          const int c = gidx(r, jj);
-          const double* Gc = sG + c * M::NGP;
-          const double d0 = g9[c] - Gm2[c];
-          const double d1 = Gc[gslot + M::GK] - Gc[gslot - M::GK];
-          const double d2 = Gc[gslot + 1] - Gc[gslot - 1];
-          res = res + (d0 * km[0 * 3 + jj] + d1 * km[1 * 3 + jj] + d2 * km[2 * 3 + jj]);
-        }
-        vis[r] = res;
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < 9; ++m) Gm2[m] = sG[m * M::NGP + gslot];    // G(s-1): G(s'-2) of the next step
 #pragma unroll
     for (int m = 0; m < 9; ++m) kpvh[m] = kkh[m];
-
-    // ---- d. update of plane s-1 -------------------------------------------------
-    if (upd && own) {
-      march_keep(vl);
-      const double rvol = rcp(vl + 1e-300);
-      double inv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-      if (s - 1 >= 2 && s - 1 <= ni - 3) {
-#pragma unroll
-        for (int v = 0; v < 5; ++v) inv[v] = inv[v] + (-(Fi[v] - Fm[v]) * rvol);
-      }
-      if (jin) {
-        const int lo = tj * TK + tk;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) inv[v] = inv[v] + (-(sF[v * M::NFB + lo + TK] - sF[v * M::NFB + lo]) * rvol);
-      }
-      if (kin) {
-        const int lo = M::NFJ + tj * (TK + 1) + tk;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) inv[v] = inv[v] + (-(sF[v * M::NFB + lo + 1] - sF[v * M::NFB + lo]) * rvol);
-      }
-      double rhs[5];
-      rhs[0] = inv[0] + 0.0;
-      rhs[1] = inv[1] + vis[0];
-      rhs[2] = inv[2] + vis[1];
-      rhs[3] = inv[3] + vis[2];
-      rhs[4] = inv[4] + vis[3];
-      // loaded in phase b; held opaque here so that the combination below
-      // compiles with the same contractions as the fused kernel's, which
-      // loads these values right where it combines them
-      march_keep(qs);
-      march_keep(qq0);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        stx(ro, c_m, v * nb, rk_combine(stage, qq0[v], qs[v], dt, rhs[v]));
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 5; ++v) Fm[v] = Fi[v];
-    __syncthreads();   // every read of G(s-1) and of the faces of plane s-1 done
-
-    // ---- e. G(s) over G(s-1); G of the cross halo; faces of plane s; next halo --
-#pragma unroll
-    for (int m = 0; m < 9; ++m) sG[m * M::NGP + gslot] = g9[m];
+    __builtin_amdgcn_sched_barrier(0);
+    // G of the cross halo; the next plane's halo
     if (hs >= 0) {
       double x[6];
-      march_prim(qnh, g, gb.R, x);     // plane s+1 at the halo cell
-      march_keep(x);
-      if (s + 2 <= pB + 1) march_load5(rq, nb, plane(s + 2) + march_opaque(hcol), qnh);
+      prim_and_temp(qnh, gas, x);     // plane s+1 at the halo cell
 #pragma unroll
       for (int v = 0; v < 6; ++v) sH[v * M::NHS + hs] = x[v];
       if (hg) {
@@ -420,7 +381,7 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
         double khh[9], g9h[9];
 #pragma unroll
         for (int m = 0; m < 9; ++m) khh[m] = 0.5 * kh[m];
-        march_visc<TJ, TK>(sP, hslot, um, up, khh, gb, g9h);
+        march_visc<TJ, TK>(sP, hslot, um, up, khh, cmu, gas, g9h);
 #pragma unroll
         for (int m = 0; m < 9; ++m) sG[m * M::NGP + hgslot] = g9h[m];
         sU[hs] = sP[M::NP + hslot];
@@ -429,20 +390,56 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
         sU[3 * M::NHG + hs] = sP[5 * M::NP + hslot];
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    // the next plane's metrics and the state of the plane after it, and the
+    // update operands of plane s; loaded on either side of `faces`, so that no
+    // older value has to be kept for a step that does not need them
+    auto load_next = [&] {
+#pragma unroll
+      for (int m = 0; m < 9; ++m) kk[m] = ldx(rk, plane(s + 1) + march_opaque(col), m * nb);
+      march_load5(rq, nb, plane(s + 2) + march_opaque(col), qn);
+    };
+    auto load_operands = [&] {
+      vl = ldx(rv, op + march_opaque(col), 0);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) {
+        qs[v] = ldx(rq, op + march_opaque(col), v * nb);
+        qq0[v] = ldx(r0, op + march_opaque(col), v * nb);
+      }
+    };
+    if (!faces) load_next();
     if (faces) {
-      // round 0: the column's low j-face (cells gj-2 .. gj+1 of column gk;
-      // in the block wherever the face exists, so its plane offsets are
-      // those of the column and the column nk before it)
-      if (fj)
-        march_face_own<TJ, TK, LIM>(sP, sF, slot - 2 * M::PK, M::PK, rk, c_s - (unsigned)nk, 3 * nb, nb, kpvh + 3, t, g);
+      double klh[3];
+      // round 0: the column's low j-face (cells gj-2 .. gj+1 of column gk),
+      // between its instructions load_operands
+#pragma unroll
+      for (int m = 0; m < 3; ++m) klh[m] = 0.5 * klj[m];
+      load_operands();
+      march_face<TJ, TK, LIM>(sP, sF, slot - 2 * M::PK, M::PK, klh, kpvh + 3, t, gas);
+      march_spread<11, 16>();
       __builtin_amdgcn_sched_barrier(0);   // one face at a time: the rounds are not interleaved
-      // round 1: the column's low k-face
-      if (fk)
-        march_face_own<TJ, TK, LIM>(sP, sF, slot - 2, 1, rk, c_s - 1u, 6 * nb, nb, kpvh + 6, M::NFJ + tj * (TK + 1) + tk, g);
+      // round 1: the column's low k-face, between its instructions load_next
+#pragma unroll
+      for (int m = 0; m < 3; ++m) klh[m] = 0.5 * klk[m];
+      load_next();
+      march_face<TJ, TK, LIM>(sP, sF, slot - 2, 1, klh, kpvh + 6, M::NFJ + tj * (TK + 1) + tk, gas);
+      march_spread<14, 13>();
       __builtin_amdgcn_sched_barrier(0);
-      march_far_faces<TJ, TK, LIM>(b, rk, nb, j0, k0, op, sP, sF, g, (int)march_opaque((unsigned)t));
+      if (fstr > 0) {   // round 2: the far-end layer
+        double kl[3], kr[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+          kl[m] = 0.5 * kh[m];
+          kr[m] = 0.5 * kh[3 + m];
+        }
+        march_face<TJ, TK, LIM>(sP, sF, hslot, fstr, kl, kr, hgslot, gas);
+      }
     }
+    if (!faces) load_operands();
+    if (hs >= 0) march_load5(rq, nb, plane(s + 2) + march_opaque(hcol), qnh);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();   // G(s) and the faces of plane s in place; P free
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -451,7 +448,7 @@ __device__ __forceinline__ void march_segment(double* lds, const BlockDesc& b, i
 template <int TJ, int TK, int LIM>
 __device__ __forceinline__ void march_tile(double* lds, const BlockDesc& b, int tr, int j0, int k0, int pA,
                                            int pB, const double* __restrict__ qin, double* qout, int stage,
-                                           const Gas& gas, double dt) {
+                                           const StageGas& gas, double dt) {
   static_assert(MarchGeom<TJ, TK>::NLDS == MarchGeom<TK, TJ>::NLDS, "transposed tile LDS");
   if constexpr (TJ == TK) {
     march_segment<TJ, TK, LIM>(lds, b, j0, k0, pA, pB, qin, b.q, qout, gas, dt, stage);
@@ -465,7 +462,7 @@ __device__ __forceinline__ void march_tile(double* lds, const BlockDesc& b, int 
 // Segments split the block's planes evenly (lengths differ by at most one).
 template <int TJ, int TK, int L, int LIM, int WPE>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_stage_march(BlockDesc b, int stage, Gas gas, double dt) {
+k_stage_march(BlockDesc b, int stage, StageGas gas, double dt) {
   __shared__ double lds[MarchGeom<TJ, TK>::NLDS];
   const int w = xcd_remap(blockIdx.x, gridDim.x);
   const MarchTiling mt = march_tiling(TJ, TK, b.nj, b.nk);
@@ -482,7 +479,7 @@ k_stage_march(BlockDesc b, int stage, Gas gas, double dt) {
 // Batched launch over a tile table whose i0 is 2 x segment index + strip bit.
 template <int TJ, int TK, int L, int LIM, int WPE>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_stage_march_batched(const BlockDesc* __restrict__ blocks, const Tile3* __restrict__ tiles, int stage, Gas gas,
+k_stage_march_batched(const BlockDesc* __restrict__ blocks, const Tile3* __restrict__ tiles, int stage, StageGas gas,
                       double dt) {
   __shared__ double lds[MarchGeom<TJ, TK>::NLDS];
   const Tile3 tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];

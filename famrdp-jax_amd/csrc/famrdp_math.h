@@ -78,10 +78,16 @@ FD double limit(int lim, double a, double b) {
 // max(a,b) (the one nearer zero), mixed signs or a zero give 0 -- the
 // reference's value exactly, in four min/max, for non-NaN arguments.  A NaN
 // argument is dropped here (hardware min/max return the other operand; two
-// NaNs give 0); the face routine that calls it (face_flux_prim) restores the
-// reference's NaN propagation for the whole four-cell stencil instead, at two
-// instructions per face rather than two per limiter call.
+// NaNs give 0); the face states that use it restore the reference's NaN
+// propagation for the whole four-cell stencil instead, at two instructions
+// per face rather than two per limiter call.
 FD double minmod_fast(double a, double b) { return fmax(fmin(a, b), fmin(fmax(a, b), 0.0)); }
+
+// The same value as a clamped to the interval between 0 and b (b > 0: a in
+// [0, b]; b < 0: a in [b, 0]): the interval, two min/max, serves both slopes
+// of a face, whose cells share the difference b.
+FD void minmod_range(double b, double& lo, double& hi) { lo = fmin(b, 0.0); hi = fmax(b, 0.0); }
+FD double minmod_in(double a, double lo, double hi) { return fmin(fmax(a, lo), hi); }
 
 // flux/roe.py:5-18
 FD void physical_flux(const double U[5], const double n[3], double g, double F[5]) {
@@ -181,81 +187,74 @@ FD void face_flux(const double pv0[5], const double pv1[5], const double pv2[5],
 }
 
 // ---------------------------------------------------------------------------
-// Stage-kernel forms.  Same mathematics as above, arranged for throughput:
-// each divisor is inverted once and multiplied (x * (1/y) rounds at most one
-// ulp away from x / y), and the Roe flux takes the reconstructed primitives
-// directly instead of converting them to conservative variables and back
-// (the reference's prim_to_cons -> roe_flux round trip is the identity up to
-// rounding).
+// Stage-kernel forms: the mathematics above, arranged for throughput.
+//
+// The stage kernels are bound by FP64 issue, so what counts here is the
+// number of instructions.  Every product that feeds a sum is an explicit fma
+// and the compiler's own contraction is off (EXACT_FP), so a function gives
+// the same bits in whichever kernel it is inlined, and the fused and marching
+// kernels, which share these functions and the order of every sum, agree bit
+// for bit.
 // ---------------------------------------------------------------------------
 
 #define DF __device__ __forceinline__
+#define EXACT_FP _Pragma("clang fp contract(off)")
 
-// 1/x from the hardware reciprocal seed refined by two Newton-Raphson steps
-// (each squares the relative error), for finite non-zero x.
+// 1/x from the hardware reciprocal seed (relative error e below 2^-24) and
+// one cubic correction r (1 + e + e^2): rounding is all that is left (2^-72
+// otherwise), in three fma where two Newton steps take four.  For finite
+// non-zero x.
 DF double rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  return fma(r, e, r);
+  EXACT_FP
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
-// sqrt(x) from the hardware reciprocal square-root seed: one coupled
-// Newton step on (sqrt, 1/(2 sqrt)) and two residual corrections.  IEEE
-// special cases: +-0 and +inf are returned as they are (the seed gives inf
-// and 0 there), x < 0 and NaN give NaN (the seed is NaN, so g is).
+// sqrt(x) from the hardware reciprocal square-root seed and one cubic
+// correction s (1 + e/2 + 3 e^2 / 8), e = 1 - s y measured on the rounded
+// s = x y.  IEEE special cases: +-0 and +inf are returned as they are (the
+// seed gives inf and 0 there), x < 0 and NaN give NaN (the seed is NaN).
 DF double fsqrt(double x) {
+  EXACT_FP
   const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  double d = fma(-g, g, x);
-  g = fma(d, h, g);
-  d = fma(-g, g, x);
-  g = fma(d, h, g);
+  const double s = x * y;
+  const double e = fma(-s, y, 1.0);
+  const double g = fma(s * e, fma(e, 0.375, 0.5), s);
   // one class test: -0, +0, +inf
   return __builtin_amdgcn_class(x, (1 << 5) | (1 << 6) | (1 << 9)) ? x : g;
 }
 
-// 1/sqrt(x) for x > 0 from the hardware seed: two coupled Newton steps on
-// (sqrt x, 1/(2 sqrt x)); within 2 ulp of 1/sqrt(x) (checked on the GPU).
+// 1/sqrt(x) for x > 0, the same correction on the seed itself; within 2 ulp
+// (checked on the GPU).
 DF double rsq_acc(double x) {
+  EXACT_FP
   const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  double r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  r = fma(-g, h, 0.5);
-  h = fma(h, r, h);
-  return 2.0 * h;
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 // One Newton step on the hardware seeds (relative error 2^-24 on gfx950, so
 // about 2^-47 after the step: at most ~20 ulp, measured on the GPU), for the
 // face flux, whose every quotient and root enters the flux at O(1) weight.
 DF double rcp1(double x) {
+  EXACT_FP
   const double r = __builtin_amdgcn_rcp(x);
   return fma(r, fma(-x, r, 1.0), r);
 }
 DF double rsq1(double x) {
+  EXACT_FP
   const double y = __builtin_amdgcn_rsq(x);
   return fma(y * fma(-(x * y), y, 1.0), 0.5, y);
 }
 
 // van Leer with the division as a reciprocal (stage-kernel form)
 DF double vanleer_fast(double a, double b) {
+  EXACT_FP
   const double ab = a + b;
   const double safe = fabs(ab) > 1e-30 ? ab : 1.0;
   const double r = 2.0 * a * b * rcp(safe);
   return (a * b > 0.0) ? r : 0.0;
-}
-
-template <int LIM>
-DF double limit_fast(double a, double b) {
-  if constexpr (LIM == LIM_VANLEER) return vanleer_fast(a, b);
-  else return minmod_fast(a, b);
 }
 
 DF void cons_to_prim_fast(const double q[5], double g, double pv[5]) {
@@ -267,86 +266,132 @@ DF void cons_to_prim_fast(const double q[5], double g, double pv[5]) {
   pv[4] = (g - 1.0) * (q[4] - rho * ke);
 }
 
-// flux/roe.py:21-85 on left/right primitives (rho, u, v, w, p), unit normal n.
-DF void roe_flux_prim(const double pl[5], const double pr[5], const double n[3], double g, double F[5]) {
-  const double gm1 = g - 1.0;
-  const double rgm1 = rcp(gm1);
-  const double rhoL = max_floor(pl[0], 1e-300), rhoR = max_floor(pr[0], 1e-300);
-  const double uL = pl[1], vL = pl[2], wL = pl[3], pL = pl[4];
-  const double uR = pr[1], vR = pr[2], wR = pr[3], pR = pr[4];
-  const double EL = pL * rgm1 + rhoL * (0.5 * (uL * uL + vL * vL + wL * wL));
-  const double ER = pR * rgm1 + rhoR * (0.5 * (uR * uR + vR * vR + wR * wR));
-  // 1/sqrt(rho) gives sqrt(rho), 1/rho and, below, 1/sqrt(rhoL rhoR)
+// The gas constants the stage kernels use, computed once on the host and held
+// in scalar registers (no conversion of them is left in a kernel).
+struct StageGas {
+  double gm1;      // gamma - 1
+  double gm1h;     // (gamma - 1) / 2
+  double cg2;      // 2 gamma / (gamma - 1)
+  double R, rR;    // R and 1 / R
+  double Ts;
+  double cmu;      // (T0 + Ts) / T0^1.5 (times the block's mu0: Sutherland's factor of T^1.5 / (T + Ts))
+  double ckap;     // gamma R / ((gamma - 1) Pr): kappa / mu
+};
+
+// x is the same in every lane of a wave: held in scalar registers
+DF double uniform(double x) {
+  typedef int pair2 __attribute__((__vector_size__(8)));
+  pair2 u = __builtin_bit_cast(pair2, x);
+  u[0] = __builtin_amdgcn_readfirstlane(u[0]);
+  u[1] = __builtin_amdgcn_readfirstlane(u[1]);
+  return __builtin_bit_cast(double, u);
+}
+
+// Primitives (rho, u, v, w, p) and temperature of one cell
+// (physics/eos.py:12-17, rhs/viscous.py:36) from one reciprocal: 1/rho gives
+// the velocities and, with 1/R, the temperature; its floor
+// p / max(rho R, 1e-300) is p * 1e300 wherever rho R does not exceed 1e-300.
+DF void prim_and_temp(const double q[5], const StageGas& gas, double pv[6]) {
+  EXACT_FP
+  const double r = rcp(q[0]);
+  pv[0] = q[0];
+  pv[1] = q[1] * r;
+  pv[2] = q[2] * r;
+  pv[3] = q[3] * r;
+  const double m2 = fma(q[3], pv[3], fma(q[2], pv[2], q[1] * pv[1]));
+  pv[4] = gas.gm1 * fma(-0.5, m2, q[4]);
+  pv[5] = pv[4] * (q[0] * gas.R > 1e-300 ? r * gas.rR : 1e300);
+}
+
+// Twice the area-weighted Roe flux (flux/roe.py:21-85 times |n| + 1e-300,
+// rhs/invscd.py:53-97) between the reconstructed primitives pl and pr
+// (rho, u, v, w, p) of a face with area vector S (not normalised).  Twice,
+// because the factor 1/2 of the flux is cheaper in the cell's 1/vol.
+//
+// The reference builds the jumps of the conservative variables and recovers
+// from them, through the Roe average, quantities that the primitives give
+// directly.  With a hat for the Roe average these are identities for any
+// rho_L, rho_R > 0 (the floored densities included):
+//   (g-1) (dE - u^.dm + q^2/2 drho) = dp,   dm.n - u^n drho = rho^ du_n,
+//   (dm - u^ drho) / rho^ = du,             u^ = u_L + a du,  H^ = H_L + a dH,
+//   a = sqrt(rho_R) / (sqrt(rho_L) + sqrt(rho_R))
+// so neither the conservative states nor their jumps are formed (and the
+// cancellation in the sums on the left does not arise).  The momentum flux
+//   m_L u_L + m_R u_R - u^ sa - w du + S P  =  F0 u_L + (m_R - a sa - w) du + S P
+// (m mass fluxes, sa the summed wave strengths, w the shear weight, P all
+// terms along the normal) and the energy flux likewise take three fma per
+// component.  Working with S instead of the unit normal leaves one 1/|S| and
+// no final product with |S|.  Harten's fix |l| < eps: (l^2/eps + eps) / 2 is
+// |l| + (eps - |l|)^2 / (2 eps), zero extra where |l| >= eps.  About 130
+// instructions and six seeds, 205 and seven in the form with conservative
+// jumps.  The floors are min/max, which drop a NaN: a NaN primitive makes the
+// pressure NaN, and dp carries it into every component.
+DF void roe_flux2(const double pl[5], const double pr[5], const double S[3], const StageGas& gas, double F[5]) {
+  EXACT_FP
+  const double rhoL = fmax(pl[0], 1e-300), rhoR = fmax(pr[0], 1e-300);
   const double isL = rsq1(rhoL), isR = rsq1(rhoR);
-  const double HL = (EL + pL) * (isL * isL), HR = (ER + pR) * (isR * isR);
-
   const double sqL = rhoL * isL, sqR = rhoR * isR;
-  // max(sqL + sqR, 1e-150) is sqL + sqR itself: both roots are >= 1e-150
-  // after the 1e-300 floors (and NaN stays NaN), so the floor never acts
-  const double rs = rcp1(sqL + sqR);
-  const double uh = (sqL * uL + sqR * uR) * rs;
-  const double vh = (sqL * vL + sqR * vR) * rs;
-  const double wh = (sqL * wL + sqR * wR) * rs;
-  const double Hh = (sqL * HL + sqR * HR) * rs;
-  const double q2 = uh * uh + vh * vh + wh * wh;
-  const double c2 = max_floor(gm1 * (Hh - 0.5 * q2), 1e-30);
+  const double a = sqR * rcp1(sqL + sqR);
+  const double uL = pl[1], vL = pl[2], wL = pl[3], uR = pr[1], vR = pr[2], wR = pr[3];
+  // twice the total enthalpies: 2 g/(g-1) p/rho + |u|^2
+  const double kL = fma(wL, wL, fma(vL, vL, uL * uL)), kR = fma(wR, wR, fma(vR, vR, uR * uR));
+  const double HL = fma(gas.cg2, pl[4] * (isL * isL), kL), HR = fma(gas.cg2, pr[4] * (isR * isR), kR);
+  const double du = uR - uL, dv = vR - vL, dw = wR - wL, dH = HR - HL;
+  const double uh = fma(a, du, uL), vh = fma(a, dv, vL), wh = fma(a, dw, wL), Hh = fma(a, dH, HL);
+  const double hq = Hh - fma(wh, wh, fma(vh, vh, uh * uh));     // 2 H^ - q^2
+  const double c2 = fmax(gas.gm1h * hq, 1e-30);
   const double isc = rsq1(c2);
-  const double rc2 = isc * isc;
-  const double ch = c2 * isc;
-  const double unh = uh * n[0] + vh * n[1] + wh * n[2];
-  const double rhoh = sqL * sqR;
-
-  const double eps = 0.1 * (fabs(unh) + ch);
-  const double reps = rcp1(eps);
-  const double lam1 = unh - ch, lam5 = unh + ch;
-  const double al1 = fabs(lam1) >= eps ? fabs(lam1) : 0.5 * (lam1 * lam1 * reps + eps);
-  const double al5 = fabs(lam5) >= eps ? fabs(lam5) : 0.5 * (lam5 * lam5 * reps + eps);
-  const double al2 = fabs(unh);
-
-  const double d0 = rhoR - rhoL;
-  const double d1 = rhoR * uR - rhoL * uL, d2 = rhoR * vR - rhoL * vL, d3 = rhoR * wR - rhoL * wL;
-  const double d4 = ER - EL;
-  const double dp = gm1 * (d4 - uh * d1 - vh * d2 - wh * d3 + 0.5 * q2 * d0);
-  const double dun = (d1 * n[0] + d2 * n[1] + d3 * n[2]) - unh * d0;
-  const double rcd = rhoh * ch * dun;
-  const double a1 = (dp - rcd) * (0.5 * rc2);
-  const double a5 = (dp + rcd) * (0.5 * rc2);
-  const double a23 = d0 - dp * rc2;
-
-  const double rrh = isL * isR;
-  const double dut = (d1 - uh * d0) * rrh, dvt_ = (d2 - vh * d0) * rrh, dwt = (d3 - wh * d0) * rrh;
-  const double dunf = dut * n[0] + dvt_ * n[1] + dwt * n[2];
-  const double tx = dut - dunf * n[0], ty = dvt_ - dunf * n[1], tz = dwt - dunf * n[2];
-
-  const double unL = uL * n[0] + vL * n[1] + wL * n[2];
-  const double unR = uR * n[0] + vR * n[1] + wR * n[2];
-  const double w1 = al1 * a1, w5 = al5 * a5, w2 = al2 * a23, w2r = al2 * rhoh;
-  // F = 1/2 (FL + FR) - 1/2 (w1 R1 + w5 R5 + al2 (a23 R2 + dvt)), with the
-  // acoustic pair gathered: w1 (u - c n) + w5 (u + c n) = (w1 + w5) u + c (w5 - w1) n
-  const double mL = rhoL * unL, mR = rhoR * unR;        // mass fluxes
-  const double sw = w1 + w5, dw = ch * (w5 - w1), sa = sw + w2;
-  F[0] = 0.5 * ((mL + mR) - sa);
-  F[1] = 0.5 * (((mL * uL + pL * n[0]) + (mR * uR + pR * n[0])) - (uh * sa + n[0] * dw + w2r * tx));
-  F[2] = 0.5 * (((mL * vL + pL * n[1]) + (mR * vR + pR * n[1])) - (vh * sa + n[1] * dw + w2r * ty));
-  F[3] = 0.5 * (((mL * wL + pL * n[2]) + (mR * wR + pR * n[2])) - (wh * sa + n[2] * dw + w2r * tz));
-  F[4] = 0.5 * (((EL + pL) * unL + (ER + pR) * unR) -
-                (Hh * sw + unh * dw + w2 * (0.5 * q2) + w2r * (uh * tx + vh * ty + wh * tz)));
+  const double rc2 = isc * isc, c = c2 * isc;
+  // |S| and 1/|S|; a zero face keeps a harmless 1e-140
+  const double nn = fmax(fma(S[2], S[2], fma(S[1], S[1], S[0] * S[0])), 1e-280);
+  const double rA = rsq1(nn);
+  const double C = c * (nn * rA);
+  const double unL = fma(wL, S[2], fma(vL, S[1], uL * S[0])), unR = fma(wR, S[2], fma(vR, S[1], uR * S[0]));
+  const double dS = unR - unL;
+  const double un = fma(a, dS, unL);
+  const double base = fabs(un) + C;                              // eps = 0.1 base
+  const double h = rcp1(0.2 * base);                             // 1 / (2 eps)
+  const double l1 = un - C, l5 = un + C;
+  const double e1 = fmax(fma(0.1, base, -fabs(l1)), 0.0), e5 = fmax(fma(0.1, base, -fabs(l5)), 0.0);
+  const double al1 = fma(e1 * h, e1, fabs(l1)), al5 = fma(e5 * h, e5, fabs(l5));
+  const double dun = dS * rA;
+  const double dp = pr[4] - pl[4];
+  const double rcd = rhoL * rhoR * c * dun;                      // rho^ c (rho^ du_n)
+  const double hc = 0.5 * rc2;
+  const double w1 = al1 * ((dp - rcd) * hc), w5 = al5 * ((dp + rcd) * hc);
+  const double aun = fabs(un);
+  const double w2 = aun * fma(-dp, rc2, rhoR - rhoL), w = aun * (sqL * sqR);
+  const double sa = (w1 + w5) + w2;
+  const double Q = fma(w, dun, (w1 - w5) * c) * rA;
+  const double P = (pl[4] + pr[4]) + Q;
+  const double mL = rhoL * unL, mR = rhoR * unR;
+  const double k = fma(-a, sa, mR), kw = k - w;
+  F[0] = (mL + mR) - sa;
+  F[1] = fma(S[0], P, fma(kw, du, F[0] * uL));
+  F[2] = fma(S[1], P, fma(kw, dv, F[0] * vL));
+  F[3] = fma(S[2], P, fma(kw, dw, F[0] * wL));
+  const double ud = fma(wh, dw, fma(vh, dv, uh * du));
+  F[4] = fma(0.5, fma(w2, hq, fma(dH, k, F[0] * HL)), fma(un, Q, -(w * ud)));
 }
 
 // MUSCL-2 face states of one cell along one axis (physics/reconstruct/
 // muscl2.py:18-37) from the primitives of the cell (pv) and its neighbours
 // (pvm below, pvp above): with the limited slope s = lim(pv - pvm, pvp - pv),
 // the left state of the cell's high face is pv + s/2 and the right state of
-// its low face pv - s/2 -- the slope face_flux_prim evaluates once for each
-// of the two faces, here once.  The minmod form carries the NaN of the cell
-// two away from each face in, as face_flux_prim does.
+// its low face pv - s/2 -- the slope face_states evaluates once for each of
+// the two faces, here once.  The minmod form carries the NaN of the cell two
+// away from each face in, as face_states does.
 template <int LIM>
 DF void muscl_cell(const double pvm[5], const double pv[5], const double pvp[5], double pLhi[5], double pRlo[5]) {
+  EXACT_FP
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    const double s = limit_fast<LIM>(pv[v] - pvm[v], pvp[v] - pv[v]);
-    pLhi[v] = pv[v] + 0.5 * s;
-    pRlo[v] = pv[v] - 0.5 * s;
+    const double am = pv[v] - pvm[v], ap = pvp[v] - pv[v];
+    double s;
+    if constexpr (LIM == LIM_VANLEER) s = vanleer_fast(am, ap);
+    else s = minmod_fast(am, ap);
+    pLhi[v] = fma(0.5, s, pv[v]);
+    pRlo[v] = fma(-0.5, s, pv[v]);
   }
   if constexpr (LIM == LIM_MINMOD) {
     pLhi[4] = fma(0.0, pvm[4], pLhi[4]);
@@ -354,92 +399,101 @@ DF void muscl_cell(const double pvm[5], const double pv[5], const double pvp[5],
   }
 }
 
-// The reconstructed states enter the face flux as computed values: every
-// kernel form (faces reconstructed in place, or from states kept from the
-// previous plane) then compiles the same flux code -- the same contractions
-// of products into fused multiply-adds -- so all forms give the same bits.
-DF void face_state_fence(double x[5]) {
-#pragma unroll
-  for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(x[v]));
-}
-
-// Area-weighted Roe flux of one face from its reconstructed left/right
-// primitives and the face normal nf = (kxyz[d, :] at the two cells) / 2
-// (rhs/invscd.py:53-97).
-DF void face_flux_n(const double pL[5], const double pR[5], double nf0, double nf1, double nf2, double g,
-                    double Fa[5]) {
-  // |n| + 1e-300 and its reciprocal from one 1/sqrt (|n| = 0: 1e-300, 1e300)
-  const double nn = nf0 * nf0 + nf1 * nf1 + nf2 * nf2;
-  const double isn = rsq1(nn);
-  const bool pos = nn > 0.0;
-  const double nm = (pos ? nn * isn : 0.0) + 1e-300;
-  const double rn = pos ? isn : 1e300;
-  const double nu[3] = {nf0 * rn, nf1 * rn, nf2 * rn};
-  double F[5];
-  roe_flux_prim(pL, pR, nu, g, F);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) Fa[v] = F[v] * nm;
-}
-
-// ... from kxyz[d, :] at the cells either side
-DF void face_flux_lr(const double pL[5], const double pR[5], const double k0[3], const double k1[3], double g,
-                     double Fa[5]) {
-  face_flux_n(pL, pR, 0.5 * (k0[0] + k1[0]), 0.5 * (k0[1] + k1[1]), 0.5 * (k0[2] + k1[2]), g, Fa);
-}
-
-// ... from kxyz[d, :] / 2 at the cells either side: k0h + k1h is
-// 0.5 (k0 + k1) exactly (halving is exact and commutes with rounding), so
-// the same bits as face_flux_lr
-DF void face_flux_lr_h(const double pL[5], const double pR[5], const double k0h[3], const double k1h[3], double g,
-                       double Fa[5]) {
-  face_flux_n(pL, pR, k0h[0] + k1h[0], k0h[1] + k1h[1], k0h[2] + k1h[2], g, Fa);
-}
-
-
 // The reconstructed states of one face from the primitives of cells a-1, a,
-// a+1, a+2 (rhs/invscd.py:53-97), on the stage-kernel forms.
+// a+1, a+2 (rhs/invscd.py:53-97).
 template <int LIM>
-DF void face_states_prim(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
+DF void face_states_fast(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
                          double pL[5], double pR[5]) {
+  EXACT_FP
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    const double sL = limit_fast<LIM>(pv1[v] - pv0[v], pv2[v] - pv1[v]);
-    const double sR = limit_fast<LIM>(pv2[v] - pv1[v], pv3[v] - pv2[v]);
-    pL[v] = pv1[v] + 0.5 * sL;
-    pR[v] = pv2[v] - 0.5 * sR;
+    const double a = pv1[v] - pv0[v], b = pv2[v] - pv1[v], c = pv3[v] - pv2[v];
+    double sL, sR;
+    if constexpr (LIM == LIM_VANLEER) {
+      sL = vanleer_fast(a, b);
+      sR = vanleer_fast(b, c);
+    } else {
+      double lo, hi;
+      minmod_range(b, lo, hi);
+      sL = minmod_in(a, lo, hi);
+      sR = minmod_in(c, lo, hi);
+    }
+    pL[v] = fma(0.5, sL, pv1[v]);
+    pR[v] = fma(-0.5, sR, pv2[v]);
   }
   if constexpr (LIM == LIM_MINMOD) {
     // The reference's minmod is NaN when a slope is, which makes the face
     // flux NaN whenever any primitive of the four cells is NaN (a NaN in
     // pL or pR reaches every flux component through the pressure jump).
-    // minmod_fast drops NaN, so the NaN of the outer cells is carried in
+    // minmod_in drops NaN, so the NaN of the outer cells is carried in
     // here: a cell with any NaN primitive has a NaN pressure (p is computed
     // from all five conservative variables), and 0 * p is +-0 otherwise.
     // (van Leer selects 0 for a NaN slope in the reference as well.)
     pL[4] = fma(0.0, pv0[4], pL[4]);
     pR[4] = fma(0.0, pv3[4], pR[4]);
   }
-  face_state_fence(pL);
-  face_state_fence(pR);
 }
 
-// One face from the primitives of cells a-1 .. a+2 and kxyz[d, :] at cells a
-// and a+1.
+// Twice the flux of one face (roe_flux2) from the primitives of cells a-1 ..
+// a+2 and kxyz[d, :] / 2 at cells a and a+1: the area vector is their sum.
 template <int LIM>
-DF void face_flux_prim(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
-                       const double k0[3], const double k1[3], double g, double Fa[5]) {
+DF void face_flux2(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
+                   const double k0h[3], const double k1h[3], const StageGas& gas, double F[5]) {
+  EXACT_FP
   double pL[5], pR[5];
-  face_states_prim<LIM>(pv0, pv1, pv2, pv3, pL, pR);
-  face_flux_lr(pL, pR, k0, k1, g, Fa);
+  face_states_fast<LIM>(pv0, pv1, pv2, pv3, pL, pR);
+  const double S[3] = {k0h[0] + k1h[0], k0h[1] + k1h[1], k0h[2] + k1h[2]};
+  roe_flux2(pL, pR, S, gas, F);
 }
 
-// ... from kxyz[d, :] / 2 at cells a and a+1 (face_flux_lr_h: the same bits)
-template <int LIM>
-DF void face_flux_prim_h(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
-                         const double k0h[3], const double k1h[3], double g, double Fa[5]) {
-  double pL[5], pR[5];
-  face_states_prim<LIM>(pv0, pv1, pv2, pv3, pL, pR);
-  face_flux_lr_h(pL, pR, k0h, k1h, g, Fa);
+// Viscous flux tensor of one cell (rhs/viscous.py:30-108): velocity and
+// temperature (u, v, w, T) at the cell, the differences d[l][s] = s(+e_l) -
+// s(-e_l) of (u, v, w, T), kh = kxyz / 2 at the cell (the 1/2 of the central
+// differences, exact on the metrics), cmu = the block's Sutherland factor.
+DF void viscous_flux_fast(const double uvwT[4], const double d[3][4], const double kh[9], double cmu,
+                          const StageGas& gas, double G[9]) {
+  EXACT_FP
+  const double T = uvwT[3];
+  const double mu = cmu * (T * fsqrt(T)) * rcp(T + gas.Ts);
+  const double mu2 = mu + mu, kappa = gas.ckap * mu;
+  double gr[4][3];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) gr[s][m] = fma(d[2][s], kh[6 + m], fma(d[1][s], kh[3 + m], d[0][s] * kh[m]));
+  const double m3 = mu2 * ((gr[0][0] + gr[1][1] + gr[2][2]) * (1.0 / 3.0));
+  const double t00 = fma(mu2, gr[0][0], -m3), t11 = fma(mu2, gr[1][1], -m3), t22 = fma(mu2, gr[2][2], -m3);
+  const double t01 = mu * (gr[0][1] + gr[1][0]), t02 = mu * (gr[0][2] + gr[2][0]), t12 = mu * (gr[1][2] + gr[2][1]);
+  const double u = uvwT[0], v = uvwT[1], w = uvwT[2];
+  G[0] = t00; G[1] = t01; G[2] = t02; G[3] = t11; G[4] = t12; G[5] = t22;
+  G[6] = fma(w, t02, fma(v, t01, fma(u, t00, kappa * gr[3][0])));
+  G[7] = fma(w, t12, fma(v, t11, fma(u, t01, kappa * gr[3][1])));
+  G[8] = fma(w, t22, fma(v, t12, fma(u, t02, kappa * gr[3][2])));
+}
+
+// The viscous divergence (rhs/viscous.py:86-108), sum over l, j of kxyz[l, j]
+// (G_j(+e_l) - G_j(-e_l)) / 2 for each row, as one running sum per row in a
+// fixed order: first the lower i-neighbour's share (visc_div_im: known as
+// soon as the cell's metrics are, one plane before the rest), then the j and
+// k differences dj, dk, then the upper i-neighbour's.  kh = kxyz / 2.
+DF void visc_div_im(const double Gm[9], const double kh[9], double vis[4]);
+DF void visc_div_jk(const double dj[9], const double dk[9], const double kh[9], double vis[4]);
+DF void visc_div_ip(const double Gp[9], const double kh[9], double vis[4]);
+
+// The update of one cell: vis the viscous divergence, A twice the summed face
+// differences (j, then k, then i), rvh = 1 / (2 (vol + 1e-300)); Shu-Osher
+// (solver/step.py:45-53) as a q0 + b (qs + dt rhs).
+struct StageCoef {
+  double a, b, dt;
+};
+DF StageCoef stage_coef(int stage, double dt) {
+  const double a = stage == 1 ? 0.0 : (stage == 2 ? 0.75 : 1.0 / 3.0);
+  const double b = stage == 1 ? 1.0 : (stage == 2 ? 0.25 : 2.0 / 3.0);
+  return StageCoef{uniform(a), uniform(b), uniform(dt)};
+}
+DF double stage_update(const StageCoef& sc, double q0, double qs, double A, double rvh, double vis) {
+  EXACT_FP
+  return fma(sc.b, fma(sc.dt, fma(-A, rvh, vis), qs), sc.a * q0);
 }
 
 struct Gas {
@@ -473,30 +527,6 @@ FD void viscous_flux(const double pv[5], double T, const double d[3][4], const d
   G[8] = u * t02 + v * t12 + w * t22 - (-kappa * gr[3][2]);
 }
 
-// viscous_flux on the stage-kernel forms (reciprocals, x*sqrt(x) for x^1.5).
-DF void viscous_flux_fast(const double pv[5], double T, const double d[3][4], const double k[9], const Gas& gas,
-                          double G[9]) {
-  const double x = T * rcp(gas.T0);
-  const double mu = gas.mu0 * (x * fsqrt(x)) * (gas.T0 + gas.Ts) * rcp(T + gas.Ts);
-  const double kappa = gas.gamma * gas.R * rcp(gas.gamma - 1.0) * mu * rcp(gas.Pr_lam);
-  double gr[4][3];
-  for (int s = 0; s < 4; ++s)
-    for (int m = 0; m < 3; ++m)
-      gr[s][m] = d[0][s] * k[0 * 3 + m] + d[1][s] * k[1 * 3 + m] + d[2][s] * k[2 * 3 + m];
-  const double divu3 = (gr[0][0] + gr[1][1] + gr[2][2]) * (1.0 / 3.0);
-  const double t00 = 2 * mu * (gr[0][0] - divu3);
-  const double t01 = mu * (gr[0][1] + gr[1][0]);
-  const double t02 = mu * (gr[0][2] + gr[2][0]);
-  const double t11 = 2 * mu * (gr[1][1] - divu3);
-  const double t12 = mu * (gr[1][2] + gr[2][1]);
-  const double t22 = 2 * mu * (gr[2][2] - divu3);
-  const double u = pv[1], v = pv[2], w = pv[3];
-  G[0] = t00; G[1] = t01; G[2] = t02; G[3] = t11; G[4] = t12; G[5] = t22;
-  G[6] = u * t00 + v * t01 + w * t02 + kappa * gr[3][0];
-  G[7] = u * t01 + v * t11 + w * t12 + kappa * gr[3][1];
-  G[8] = u * t02 + v * t12 + w * t22 + kappa * gr[3][2];
-}
-
 DF double temperature_fast(const double pv[5], double R) { return pv[4] * rcp(max_floor(pv[0] * R, 1e-300)); }
 
 // T = p / max(rho R, 1e-300)  (rhs/viscous.py:36)
@@ -508,6 +538,30 @@ FD int gidx(int r, int j) {
   if (r == 3) return 6 + j;
   const int a = r < j ? r : j, b = r < j ? j : r;
   return a == 0 ? b : (a == 1 ? 2 + b : 5);
+}
+
+DF void visc_div_im(const double Gm[9], const double kh[9], double vis[4]) {
+  EXACT_FP
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    vis[r] = fma(-Gm[gidx(r, 2)], kh[2], fma(-Gm[gidx(r, 1)], kh[1], -Gm[gidx(r, 0)] * kh[0]));
+}
+DF void visc_div_jk(const double dj[9], const double dk[9], const double kh[9], double vis[4]) {
+  EXACT_FP
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const int c = gidx(r, m);
+      vis[r] = fma(dk[c], kh[6 + m], fma(dj[c], kh[3 + m], vis[r]));
+    }
+}
+DF void visc_div_ip(const double Gp[9], const double kh[9], double vis[4]) {
+  EXACT_FP
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) vis[r] = fma(Gp[gidx(r, m)], kh[m], vis[r]);
 }
 
 }  // namespace famrdp
