@@ -89,213 +89,141 @@ FD void limiter_vjp(int lim, double A, double B, double ls, double& lA, double& 
   else limiter_vjp_t<LIM_MINMOD>(A, B, ls, lA, lB);
 }
 
-// Forward Roe flux on primitives (identical arithmetic to roe_flux_prim) with
-// the reverse sweep: given lF (cotangent of F), accumulate into lpl, lpr.
+FD double rsq_hd(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return rsq_acc(x);
+#else
+  return 1.0 / sqrt(x);
+#endif
+}
+
+// Reverse of roe_flux2 (famrdp_math.h: twice the area-weighted Roe flux of a
+// face with area vector S, from the jumps of the primitives): f = cotangent
+// of its five components; the cotangents of the left and right primitives are
+// written to lpl, lpr.  The forward values are computed again, with the full
+// reciprocals and roots, and swept backwards; the same identities of the Roe
+// average that shorten the forward flux leave about 280 instructions where
+// the sweep through conservative jumps took 430, and far fewer values alive.
+// cg2 = 2 g / (g - 1), gm1h = (g - 1) / 2.
+FD void roe_flux2_vjp(const double pl[5], const double pr[5], const double S[3], double cg2, double gm1h,
+                      const double f[5], double lpl[5], double lpr[5]) {
+  const double rhoL = max_floor(pl[0], 1e-300), rhoR = max_floor(pr[0], 1e-300);
+  const double isL = rsq_hd(rhoL), isR = rsq_hd(rhoR);
+  const double sqL = rhoL * isL, sqR = rhoR * isR;
+  const double rs = rcp_hd(sqL + sqR);
+  const double a = sqR * rs;
+  const double irL = isL * isL, irR = isR * isR;
+  const double HL = cg2 * (pl[4] * irL) + (pl[1] * pl[1] + pl[2] * pl[2] + pl[3] * pl[3]);
+  const double HR = cg2 * (pr[4] * irR) + (pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3]);
+  double du[3], uh[3];
+  for (int m = 0; m < 3; ++m) {
+    du[m] = pr[1 + m] - pl[1 + m];
+    uh[m] = pl[1 + m] + a * du[m];
+  }
+  const double dH = HR - HL;
+  const double hq = (HL + a * dH) - (uh[0] * uh[0] + uh[1] * uh[1] + uh[2] * uh[2]);
+  const double c2raw = gm1h * hq;
+  const double c2 = max_floor(c2raw, 1e-30);
+  const double isc = rsq_hd(c2);
+  const double rc2 = isc * isc, c = c2 * isc;
+  const double nn0 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
+  const double nn = nn0 > 1e-280 ? nn0 : 1e-280;
+  const double rA = rsq_hd(nn);
+  const double A = nn * rA, C = c * A;
+  const double unL = pl[1] * S[0] + pl[2] * S[1] + pl[3] * S[2], unR = pr[1] * S[0] + pr[2] * S[1] + pr[3] * S[2];
+  const double dS = unR - unL, un = unL + a * dS;
+  const double aun = fabs(un), sun = dabs(un);
+  const double base = aun + C, h = rcp_hd(0.2 * base);
+  const double l1 = un - C, l5 = un + C;
+  const double x1 = 0.1 * base - fabs(l1), x5 = 0.1 * base - fabs(l5);
+  const double e1 = x1 > 0.0 ? x1 : 0.0, e5 = x5 > 0.0 ? x5 : 0.0;
+  const double eh1 = e1 * h, eh5 = e5 * h;
+  const double al1 = fabs(l1) + eh1 * e1, al5 = fabs(l5) + eh5 * e5;
+  const double dun = dS * rA, dp = pr[4] - pl[4], dr = rhoR - rhoL;
+  const double rr = rhoL * rhoR, rcd = rr * c * dun, hc = 0.5 * rc2;
+  const double a1 = (dp - rcd) * hc, a5 = (dp + rcd) * hc, a23 = dr - dp * rc2;
+  const double w1 = al1 * a1, w5 = al5 * a5, w2 = aun * a23, sLR = sqL * sqR, w = aun * sLR;
+  const double sa = (w1 + w5) + w2;
+  const double Q = (w * dun + (w1 - w5) * c) * rA;
+  const double mR = rhoR * unR;
+  const double F0 = (rhoL * unL + mR) - sa;
+  const double k = mR - a * sa, kw = k - w;
+  const double ud = uh[0] * du[0] + uh[1] * du[1] + uh[2] * du[2];
+
+  // ---- backwards: momentum and energy components
+  const double h4 = 0.5 * f[4];
+  const double b_F0 = f[0] + (f[1] * pl[1] + f[2] * pl[2] + f[3] * pl[3]) + h4 * HL;
+  const double b_kw = f[1] * du[0] + f[2] * du[1] + f[3] * du[2];
+  const double b_P = f[1] * S[0] + f[2] * S[1] + f[3] * S[2];
+  const double b_ud = -f[4] * w;
+  double b_HL = h4 * F0, b_dH = h4 * k, b_hq = h4 * w2;
+  const double b_k = h4 * dH + b_kw;
+  double b_un = f[4] * Q;
+  const double q = (f[4] * un + b_P) * rA;
+  const double b_w = q * dun - f[4] * ud - b_kw;
+  double b_dun = q * w;
+  const double b_sa = -b_F0 - b_k * a;
+  double b_a = -b_k * sa;
+  // ---- wave strengths
+  const double b_w1 = q * c + b_sa, b_w5 = b_sa - q * c, b_w2 = h4 * hq + b_sa;
+  double b_c = q * (w1 - w5);
+  const double b_aun = b_w2 * a23 + b_w * sLR, b_a23 = b_w2 * aun, b_sLR = b_w * aun;
+  const double b_al1 = b_w1 * a1, b_al5 = b_w5 * a5;
+  const double t1 = b_w1 * al1, t5 = b_w5 * al5;
+  const double b_rcd = (t5 - t1) * hc;
+  const double b_dp = (t1 + t5) * hc - b_a23 * rc2;
+  // rc2 enters through hc = rc2 / 2 (a1, a5 = (dp -+ rcd) hc) and a23
+  const double b_rc2 = 0.5 * (t1 * (dp - rcd) + t5 * (dp + rcd)) - b_a23 * dp;
+  b_c += b_rcd * (rr * dun);
+  b_dun += b_rcd * (rr * c);
+  const double b_rr = b_rcd * (c * dun);
+  // ---- Harten's fix: al = |l| + e^2 h, e = max(base / 10 - |l|, 0), h = 5 / base
+  const double g1 = b_al1 * (1.0 - 2.0 * eh1) * dabs(l1), g5 = b_al5 * (1.0 - 2.0 * eh5) * dabs(l5);
+  const double b_base = 0.2 * (b_al1 * (eh1 * (1.0 - eh1)) + b_al5 * (eh5 * (1.0 - eh5)));
+  b_un += (g1 + g5) + (b_base + b_aun) * sun;
+  b_c += (b_base + (g5 - g1)) * A;
+  // ---- normal velocities
+  b_a += b_un * dS;
+  const double b_dS = b_un * a + b_dun * rA;
+  const double b_mR = b_F0 + b_k;
+  const double b_unL = (b_un - b_dS) + b_F0 * rhoL, b_unR = b_dS + b_mR * rhoR;
+  // ---- sound speed, Roe average
+  const double b_c2 = rc2 * (0.5 * b_c * c - b_rc2 * rc2);
+  b_hq += gm1h * (b_c2 * dmax_floor(c2raw, 1e-30));
+  b_HL += b_hq;
+  b_dH += a * b_hq;
+  b_a += b_hq * dH;
+  b_HL -= b_dH;
+  double b_rhoL = b_F0 * unL + b_rr * rhoR - b_a23, b_rhoR = b_mR * unR + b_rr * rhoL + b_a23;
+  for (int m = 0; m < 3; ++m) {
+    const double b_uh = b_ud * du[m] - 2.0 * uh[m] * b_hq;
+    const double b_du = kw * f[1 + m] + b_ud * uh[m] + a * b_uh;
+    b_a += b_uh * du[m];
+    lpl[1 + m] = F0 * f[1 + m] + (b_uh - b_du) + b_unL * S[m] + 2.0 * b_HL * pl[1 + m];
+    lpr[1 + m] = b_du + b_unR * S[m] + 2.0 * b_dH * pr[1 + m];
+  }
+  const double cL = b_HL * cg2 * irL, cR = b_dH * cg2 * irR;
+  lpl[4] = b_P - b_dp + cL;
+  lpr[4] = b_P + b_dp + cR;
+  const double b_s = b_a * rs;                 // a = sqR / (sqL + sqR)
+  const double b_sL = b_sLR * sqR - b_s * a, b_sR = b_sLR * sqL + b_s * (1.0 - a);
+  b_rhoL += 0.5 * b_sL * isL - cL * (pl[4] * irL);
+  b_rhoR += 0.5 * b_sR * isR - cR * (pr[4] * irR);
+  lpl[0] = b_rhoL * dmax_floor(pl[0], 1e-300);
+  lpr[0] = b_rhoR * dmax_floor(pr[0], 1e-300);
+}
+
+// The same for the flux itself with a unit normal (flux/roe.py:21-85),
+// accumulating into lpl, lpr.
 FD void roe_flux_prim_vjp(const double pl[5], const double pr[5], const double n[3], double g, const double lF[5],
                           double lpl[5], double lpr[5]) {
-  // ---------------- forward (kept intermediates) ----------------
-  const double gm1 = g - 1.0;
-  const double rgm1 = rcp_hd(gm1);
-  const double rhoL = max_floor(pl[0], 1e-300), rhoR = max_floor(pr[0], 1e-300);
-  const double uL = pl[1], vL = pl[2], wL = pl[3], pL = pl[4];
-  const double uR = pr[1], vR = pr[2], wR = pr[3], pR = pr[4];
-  const double keL = 0.5 * (uL * uL + vL * vL + wL * wL);
-  const double keR = 0.5 * (uR * uR + vR * vR + wR * wR);
-  const double EL = pL * rgm1 + rhoL * keL, ER = pR * rgm1 + rhoR * keR;
-  const double irL = rcp_hd(rhoL), irR = rcp_hd(rhoR);
-  const double HL = (EL + pL) * irL, HR = (ER + pR) * irR;
-  const double sqL = sqrt_hd(rhoL), sqR = sqrt_hd(rhoR);
-  const double S = sqL + sqR;
-  const double Sf = max_floor(S, 1e-150);
-  const double rs = rcp_hd(Sf);
-  const double nuh = sqL * uL + sqR * uR, nvh = sqL * vL + sqR * vR, nwh = sqL * wL + sqR * wR;
-  const double nHh = sqL * HL + sqR * HR;
-  const double uh = nuh * rs, vh = nvh * rs, wh = nwh * rs, Hh = nHh * rs;
-  const double q2 = uh * uh + vh * vh + wh * wh;
-  const double c2raw = gm1 * (Hh - 0.5 * q2);
-  const double c2 = max_floor(c2raw, 1e-30);
-  const double rc2 = rcp_hd(c2);
-  const double ch = sqrt_hd(c2);
-  const double unh = uh * n[0] + vh * n[1] + wh * n[2];
-  const double rhoh = sqL * sqR;
-  const double eps = 0.1 * (fabs(unh) + ch);
-  const double reps = rcp_hd(eps);
-  const double lam1 = unh - ch, lam5 = unh + ch;
-  const bool br1 = fabs(lam1) >= eps, br5 = fabs(lam5) >= eps;
-  const double al1 = br1 ? fabs(lam1) : 0.5 * (lam1 * lam1 * reps + eps);
-  const double al5 = br5 ? fabs(lam5) : 0.5 * (lam5 * lam5 * reps + eps);
-  const double al2 = fabs(unh);
-  const double d0 = rhoR - rhoL;
-  const double d1 = rhoR * uR - rhoL * uL, d2 = rhoR * vR - rhoL * vL, d3 = rhoR * wR - rhoL * wL;
-  const double d4 = ER - EL;
-  const double dp = gm1 * (d4 - uh * d1 - vh * d2 - wh * d3 + 0.5 * q2 * d0);
-  const double dun = (d1 * n[0] + d2 * n[1] + d3 * n[2]) - unh * d0;
-  const double rcd = rhoh * ch * dun;
-  const double a1 = (dp - rcd) * (0.5 * rc2), a5 = (dp + rcd) * (0.5 * rc2);
-  const double a23 = d0 - dp * rc2;
-  const double rrh = rcp_hd(rhoh);
-  const double e1 = d1 - uh * d0, e2 = d2 - vh * d0, e3 = d3 - wh * d0;
-  const double dut = e1 * rrh, dvt = e2 * rrh, dwt = e3 * rrh;
-  const double dunf = dut * n[0] + dvt * n[1] + dwt * n[2];
-  const double tx = dut - dunf * n[0], ty = dvt - dunf * n[1], tz = dwt - dunf * n[2];
-  const double unL = uL * n[0] + vL * n[1] + wL * n[2], unR = uR * n[0] + vR * n[1] + wR * n[2];
-  const double w1 = al1 * a1, w5 = al5 * a5, w2 = al2 * a23, w2r = al2 * rhoh;
-  const double uht = uh * tx + vh * ty + wh * tz;
-
-  // ---------------- reverse ----------------
-  const double f0 = lF[0], f1 = lF[1], f2 = lF[2], f3 = lF[3], f4 = lF[4];
-  double b_rhoL = 0, b_rhoR = 0, b_uL = 0, b_vL = 0, b_wL = 0, b_pL = 0, b_uR = 0, b_vR = 0, b_wR = 0, b_pR = 0;
-  double b_unL = 0, b_unR = 0, b_EL = 0, b_ER = 0;
-  double b_w1 = 0, b_w5 = 0, b_w2 = 0, b_w2r = 0, b_uh = 0, b_vh = 0, b_wh = 0, b_Hh = 0, b_q2 = 0;
-  double b_ch = 0, b_unh = 0, b_tx = 0, b_ty = 0, b_tz = 0;
-  // F0
-  b_rhoL += 0.5 * f0 * unL; b_unL += 0.5 * f0 * rhoL; b_rhoR += 0.5 * f0 * unR; b_unR += 0.5 * f0 * rhoR;
-  b_w1 -= 0.5 * f0; b_w5 -= 0.5 * f0; b_w2 -= 0.5 * f0;
-  // F1..F3
-  const double fm[3] = {f1, f2, f3};
-  const double uLv[3] = {uL, vL, wL}, uRv[3] = {uR, vR, wR}, uhv[3] = {uh, vh, wh}, tv[3] = {tx, ty, tz};
-  double b_uLv[3] = {0, 0, 0}, b_uRv[3] = {0, 0, 0}, b_uhv[3] = {0, 0, 0}, b_tv[3] = {0, 0, 0};
-  for (int m = 0; m < 3; ++m) {
-    const double fv = fm[m];
-    const double cn = ch * n[m];
-    b_rhoL += 0.5 * fv * uLv[m] * unL; b_uLv[m] += 0.5 * fv * rhoL * unL; b_unL += 0.5 * fv * rhoL * uLv[m];
-    b_pL += 0.5 * fv * n[m];
-    b_rhoR += 0.5 * fv * uRv[m] * unR; b_uRv[m] += 0.5 * fv * rhoR * unR; b_unR += 0.5 * fv * rhoR * uRv[m];
-    b_pR += 0.5 * fv * n[m];
-    b_w1 -= 0.5 * fv * (uhv[m] - cn); b_w5 -= 0.5 * fv * (uhv[m] + cn); b_w2 -= 0.5 * fv * uhv[m];
-    b_w2r -= 0.5 * fv * tv[m];
-    b_uhv[m] -= 0.5 * fv * (w1 + w5 + w2);
-    b_ch -= 0.5 * fv * (w5 - w1) * n[m];          // through cn = ch n_m
-    b_tv[m] -= 0.5 * fv * w2r;
-  }
-  // F4
-  b_EL += 0.5 * f4 * unL; b_pL += 0.5 * f4 * unL; b_unL += 0.5 * f4 * (EL + pL);
-  b_ER += 0.5 * f4 * unR; b_pR += 0.5 * f4 * unR; b_unR += 0.5 * f4 * (ER + pR);
-  {
-    const double cun = ch * unh;
-    b_w1 -= 0.5 * f4 * (Hh - cun); b_w5 -= 0.5 * f4 * (Hh + cun);
-    b_w2 -= 0.5 * f4 * (0.5 * q2); b_w2r -= 0.5 * f4 * uht;
-    b_Hh -= 0.5 * f4 * (w1 + w5);
-    const double b_cun = -0.5 * f4 * (w5 - w1);
-    b_ch += b_cun * unh; b_unh += b_cun * ch;
-    b_q2 -= 0.5 * f4 * w2 * 0.5;
-    for (int m = 0; m < 3; ++m) {
-      b_uhv[m] -= 0.5 * f4 * w2r * tv[m];
-      b_tv[m] -= 0.5 * f4 * w2r * uhv[m];
-    }
-  }
-  b_uh += b_uhv[0]; b_vh += b_uhv[1]; b_wh += b_uhv[2];
-  b_tx += b_tv[0]; b_ty += b_tv[1]; b_tz += b_tv[2];
-  b_uL += b_uLv[0]; b_vL += b_uLv[1]; b_wL += b_uLv[2];
-  b_uR += b_uRv[0]; b_vR += b_uRv[1]; b_wR += b_uRv[2];
-  // w1 = al1 a1, w5 = al5 a5, w2 = al2 a23, w2r = al2 rhoh
-  double b_al1 = b_w1 * a1, b_a1 = b_w1 * al1, b_al5 = b_w5 * a5, b_a5 = b_w5 * al5;
-  double b_al2 = b_w2 * a23 + b_w2r * rhoh, b_a23 = b_w2 * al2, b_rhoh = b_w2r * al2;
-  // unL, unR
-  b_uL += b_unL * n[0]; b_vL += b_unL * n[1]; b_wL += b_unL * n[2];
-  b_uR += b_unR * n[0]; b_vR += b_unR * n[1]; b_wR += b_unR * n[2];
-  // t = dv - dunf n;  dunf = dv . n
-  const double b_dunf = -(b_tx * n[0] + b_ty * n[1] + b_tz * n[2]);
-  const double b_dut = b_tx + b_dunf * n[0], b_dvt = b_ty + b_dunf * n[1], b_dwt = b_tz + b_dunf * n[2];
-  // dut = (d1 - uh d0) rrh etc.
-  double b_d0 = 0, b_d1 = 0, b_d2 = 0, b_d3 = 0, b_d4 = 0;
-  b_d1 += b_dut * rrh; b_uh -= b_dut * d0 * rrh; b_d0 -= b_dut * uh * rrh;
-  b_d2 += b_dvt * rrh; b_vh -= b_dvt * d0 * rrh; b_d0 -= b_dvt * vh * rrh;
-  b_d3 += b_dwt * rrh; b_wh -= b_dwt * d0 * rrh; b_d0 -= b_dwt * wh * rrh;
-  const double b_rrh = b_dut * e1 + b_dvt * e2 + b_dwt * e3;
-  b_rhoh -= b_rrh * rrh * rrh;
-  // a23 = d0 - dp rc2 ; a1 = (dp - rcd) rc2/2 ; a5 = (dp + rcd) rc2/2
-  double b_dp = 0, b_rc2 = 0, b_rcd = 0;
-  b_d0 += b_a23; b_dp -= b_a23 * rc2; b_rc2 -= b_a23 * dp;
-  b_dp += b_a1 * 0.5 * rc2; b_rcd -= b_a1 * 0.5 * rc2; b_rc2 += b_a1 * 0.5 * (dp - rcd);
-  b_dp += b_a5 * 0.5 * rc2; b_rcd += b_a5 * 0.5 * rc2; b_rc2 += b_a5 * 0.5 * (dp + rcd);
-  // rcd = rhoh ch dun
-  b_rhoh += b_rcd * ch * dun; b_ch += b_rcd * rhoh * dun;
-  const double b_dun = b_rcd * rhoh * ch;
-  // dun = d.n - unh d0
-  b_d1 += b_dun * n[0]; b_d2 += b_dun * n[1]; b_d3 += b_dun * n[2]; b_unh -= b_dun * d0; b_d0 -= b_dun * unh;
-  // dp = gm1 (d4 - uh d1 - vh d2 - wh d3 + q2/2 d0)
-  {
-    const double e = gm1 * b_dp;
-    b_d4 += e; b_uh -= e * d1; b_d1 -= e * uh; b_vh -= e * d2; b_d2 -= e * vh; b_wh -= e * d3; b_d3 -= e * wh;
-    b_q2 += e * 0.5 * d0; b_d0 += e * 0.5 * q2;
-  }
-  // d0..d4
-  b_rhoR += b_d0; b_rhoL -= b_d0;
-  b_rhoR += b_d1 * uR + b_d2 * vR + b_d3 * wR;
-  b_rhoL -= b_d1 * uL + b_d2 * vL + b_d3 * wL;
-  b_uR += b_d1 * rhoR; b_vR += b_d2 * rhoR; b_wR += b_d3 * rhoR;
-  b_uL -= b_d1 * rhoL; b_vL -= b_d2 * rhoL; b_wL -= b_d3 * rhoL;
-  b_ER += b_d4; b_EL -= b_d4;
-  // al2 = |unh|
-  b_unh += b_al2 * dabs(unh);
-  // Harten-fixed al1, al5
-  double b_eps = 0.0, b_lam1 = 0.0, b_lam5 = 0.0;
-  if (br1) b_lam1 += b_al1 * dabs(lam1);
-  else { b_lam1 += b_al1 * lam1 * reps; b_eps += b_al1 * 0.5 * (1.0 - lam1 * lam1 * reps * reps); }
-  if (br5) b_lam5 += b_al5 * dabs(lam5);
-  else { b_lam5 += b_al5 * lam5 * reps; b_eps += b_al5 * 0.5 * (1.0 - lam5 * lam5 * reps * reps); }
-  b_unh += b_lam1 + b_lam5; b_ch += b_lam5 - b_lam1;
-  // eps = 0.1 (|unh| + ch)
-  b_unh += 0.1 * b_eps * dabs(unh); b_ch += 0.1 * b_eps;
-  // rhoh = sqL sqR
-  double b_sqL = b_rhoh * sqR, b_sqR = b_rhoh * sqL;
-  // unh = uh.n
-  b_uh += b_unh * n[0]; b_vh += b_unh * n[1]; b_wh += b_unh * n[2];
-  // ch = sqrt(c2), rc2 = 1/c2, c2 = max(c2raw, 1e-30)
-  double b_c2 = b_ch * 0.5 * (ch * rc2) - b_rc2 * rc2 * rc2;   // 1/ch = ch/c2
-  const double b_c2raw = b_c2 * dmax_floor(c2raw, 1e-30);
-  b_Hh += gm1 * b_c2raw; b_q2 -= 0.5 * gm1 * b_c2raw;
-  // q2 = |uh|^2
-  b_uh += 2.0 * uh * b_q2; b_vh += 2.0 * vh * b_q2; b_wh += 2.0 * wh * b_q2;
-  // uh = nuh rs, ... Hh = nHh rs
-  double b_rs = b_uh * nuh + b_vh * nvh + b_wh * nwh + b_Hh * nHh;
-  b_sqL += (b_uh * uL + b_vh * vL + b_wh * wL + b_Hh * HL) * rs;
-  b_sqR += (b_uh * uR + b_vh * vR + b_wh * wR + b_Hh * HR) * rs;
-  b_uL += b_uh * sqL * rs; b_vL += b_vh * sqL * rs; b_wL += b_wh * sqL * rs;
-  b_uR += b_uh * sqR * rs; b_vR += b_vh * sqR * rs; b_wR += b_wh * sqR * rs;
-  const double b_HL = b_Hh * sqL * rs, b_HR = b_Hh * sqR * rs;
-  // rs = 1/max(S, 1e-150)
-  const double b_S = -b_rs * rs * rs * dmax_floor(S, 1e-150);
-  b_sqL += b_S; b_sqR += b_S;
-  // sq = sqrt(rho)
-  b_rhoL += b_sqL * 0.5 * (sqL * irL); b_rhoR += b_sqR * 0.5 * (sqR * irR);   // 1/sqrt(rho) = sqrt(rho)/rho
-  // H = (E + p)/rho
-  b_EL += b_HL * irL; b_pL += b_HL * irL; b_rhoL -= b_HL * HL * irL;
-  b_ER += b_HR * irR; b_pR += b_HR * irR; b_rhoR -= b_HR * HR * irR;
-  // E = p/(g-1) + rho ke
-  b_pL += b_EL * rgm1; b_rhoL += b_EL * keL;
-  b_pR += b_ER * rgm1; b_rhoR += b_ER * keR;
-  const double b_keL = b_EL * rhoL, b_keR = b_ER * rhoR;
-  b_uL += b_keL * uL; b_vL += b_keL * vL; b_wL += b_keL * wL;
-  b_uR += b_keR * uR; b_vR += b_keR * vR; b_wR += b_keR * wR;
-  // rho = max(pv0, 1e-300)
-  lpl[0] += b_rhoL * dmax_floor(pl[0], 1e-300);
-  lpr[0] += b_rhoR * dmax_floor(pr[0], 1e-300);
-  lpl[1] += b_uL; lpl[2] += b_vL; lpl[3] += b_wL; lpl[4] += b_pL;
-  lpr[1] += b_uR; lpr[2] += b_vR; lpr[3] += b_wR; lpr[4] += b_pR;
-}
-
-// Reverse of one inviscid face (face_flux_prim): given lFa = cotangent of
-// F * |n| for the face between cells a and a+1 whose left/right states come
-// from cells a-1..a+2, return the cotangents of the reconstructed states and
-// of the two limited slopes:  pL = pv1 + s1/2, pR = pv2 - s2/2.
-template <int LIM>
-FD void face_states(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
-                    double pL[5], double pR[5]) {
+  double f[5], bl[5], br[5];
+  for (int v = 0; v < 5; ++v) f[v] = 0.5 * lF[v];
+  roe_flux2_vjp(pl, pr, n, 2.0 * g / (g - 1.0), 0.5 * (g - 1.0), f, bl, br);
   for (int v = 0; v < 5; ++v) {
-    const double sL = limit(LIM, pv1[v] - pv0[v], pv2[v] - pv1[v]);
-    const double sR = limit(LIM, pv2[v] - pv1[v], pv3[v] - pv2[v]);
-    pL[v] = pv1[v] + 0.5 * sL;
-    pR[v] = pv2[v] - 0.5 * sR;
+    lpl[v] += bl[v];
+    lpr[v] += br[v];
   }
-}
-
-FD void face_normal(const double k0[3], const double k1[3], double nu[3], double& nm) {
-  const double nf0 = 0.5 * (k0[0] + k1[0]), nf1 = 0.5 * (k0[1] + k1[1]), nf2 = 0.5 * (k0[2] + k1[2]);
-  nm = sqrt_hd(nf0 * nf0 + nf1 * nf1 + nf2 * nf2) + 1e-300;
-  const double rn = rcp_hd(nm);
-  nu[0] = nf0 * rn; nu[1] = nf1 * rn; nu[2] = nf2 * rn;
 }
 
 // Viscous flux tensor (rhs/viscous.py:30-108) reverse.  Inputs as

@@ -126,6 +126,10 @@ struct famrdp_plan {
   BlockDesc* d_blocks_adj = nullptr;         // same blocks with q -> qh (recompute buffer)
   std::vector<BlockDesc> h_blocks_adj;
   std::vector<double*> adj_bufs;
+  SweepTile* d_sweep_ik = nullptr;           // reverse sweeps along i (with k), along j and of the viscous part
+  SweepTile* d_sweep_j = nullptr;
+  SweepTile* d_sweep_v = nullptr;
+  int nsweep_ik = 0, nsweep_j = 0, nsweep_v = 0;
   HaloEntry* d_halo_sorted = nullptr;        // halo entries sorted by source cell
   HaloSrc* d_halo_src = nullptr;
   int nhalo_src = 0;
@@ -556,6 +560,9 @@ int famrdp_plan_destroy(famrdp_plan* p) {
   if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
   for (auto* x : p->adj_bufs) (void)hipFree(x);
   if (p->d_blocks_adj) (void)hipFree(p->d_blocks_adj);
+  if (p->d_sweep_ik) (void)hipFree(p->d_sweep_ik);
+  if (p->d_sweep_j) (void)hipFree(p->d_sweep_j);
+  if (p->d_sweep_v) (void)hipFree(p->d_sweep_v);
   if (p->d_halo_sorted) (void)hipFree(p->d_halo_sorted);
   if (p->d_halo_src) (void)hipFree(p->d_halo_src);
   if (p->d_halo_S) (void)hipFree(p->d_halo_S);
@@ -611,9 +618,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": each padded size must be >= 2*ghost"));
     if ((int64_t)d[0] * d[1] * d[2] > INT32_MAX)   // tile kernels index cells in 32 bits
       return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^31 or more cells"));
-    // the reverse kernels address cells with 32-bit byte offsets; an adjoint
-    // plan allocates 80 doubles per cell (stage and adjoint buffers), so such a
-    // block would need over 300 GB of them anyway
+    // the reverse kernels address cells with 32-bit byte offsets
     if ((plan_flags & FAMRDP_PLAN_ADJOINT) && (int64_t)d[0] * d[1] * d[2] >= (int64_t(1) << 29))
       return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^29 or more cells in an adjoint plan"));
     p->N.push_back((int64_t)d[0] * d[1] * d[2]);
@@ -649,7 +654,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       const int64_t n = p->N[b];
       // qh, la, lb, (l0: the caller's cotangent array, bound by each
       // famrdp_step_vjp), fs, vs
-      const int64_t sizes[6] = {5 * n, 5 * n, 5 * n, 0, 30 * n, 16 * n};
+      const int64_t sizes[6] = {5 * n, 5 * n, 5 * n, 0, 5 * n, 8 * n};
       double* bufs[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
       for (int i = 0; i < 6; ++i) {
         if (sizes[i] == 0) {
@@ -788,6 +793,30 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   }
   p->persistent_grid = std::min(p->ntiles, ncu * 8);
   p->ncu = ncu;
+  if (p->has_adjoint) {
+    SweepSet ik{{}, {}, SWEEP_IK}, jj{{}, {}, SWEEP_J}, vv{{}, {}, SWEEP_V};
+    for (int b = 0; b < nblocks; ++b) {
+      const int32_t* d = &dims[3 * b];
+      ik.along.push_back(d[0]);
+      ik.across.push_back(d[1] * d[2]);
+      vv.along.push_back(d[0]);
+      vv.across.push_back(d[1] * (d[2] + 4));
+      jj.along.push_back(d[1]);
+      jj.across.push_back(d[0] * d[2]);
+    }
+    const int64_t slots = SWEEP_WAVES * 4 * (int64_t)ncu;   // four SIMDs per CU
+    const int li = sweep_len({&ik, &vv}, slots), lj = sweep_len({&jj}, slots);
+    const std::vector<SweepTile> tabs[3] = {sweep_tiles(ik, li), sweep_tiles(jj, lj), sweep_tiles(vv, li)};
+    SweepTile** dst[3] = {&p->d_sweep_ik, &p->d_sweep_j, &p->d_sweep_v};
+    int* cnt[3] = {&p->nsweep_ik, &p->nsweep_j, &p->nsweep_v};
+    for (int t = 0; t < 3; ++t) {
+      *cnt[t] = (int)tabs[t].size();
+      const size_t bytes = sizeof(SweepTile) * tabs[t].size();
+      if (hipMalloc(dst[t], bytes) != hipSuccess ||
+          hipMemcpy(*dst[t], tabs[t].data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
+        return cleanup(fail(FAMRDP_E_HIP, "plan_create: sweep table upload failed"));
+    }
+  }
   if (hipMalloc(&p->d_monitor, sizeof(double) * p->persistent_grid) != hipSuccess)
     return cleanup(fail(FAMRDP_E_HIP, "plan_create: monitor buffer allocation failed"));
   *out = p;
@@ -936,7 +965,8 @@ int step_vjp_impl(famrdp_plan* p, double* const* q_start, const double* const* q
   }
   // ---- reverse the three stages
   for (int stage = 3; stage >= 1; --stage) {
-    launch_stage_vjp(p->d_blocks_adj, p->d_tiles, p->ntiles, stage, p->gas, dt, p->limiter, st);
+    launch_stage_vjp(p->d_blocks_adj, p->d_sweep_v, p->nsweep_v, p->d_sweep_ik, p->nsweep_ik, p->d_sweep_j, p->nsweep_j,
+                     stage, p->gas, dt, p->limiter, st);
     LAUNCH_CHECK();
   }
   // ---- BCs reversed (Face order backwards), then the halo copy

@@ -28,8 +28,8 @@ struct BlockDesc {
   double* la;           // stage cotangents, ping (5, N)
   double* lb;           // stage cotangents, pong (5, N)
   double* l0;           // cotangent of the post-halo/BC state (5, N): the caller's cotangent array
-  double* fs;           // inviscid face reverse scratch (3 axes x 10, N)
-  double* vs;           // viscous reverse scratch (16, N)
+  double* fs;           // cotangent of the primitives from the i and k axes (5, N)
+  double* vs;           // viscous reverse: (u, v, w, T), then the j differences (8, N)
 };
 
 // One ghost cell written by the halo exchange: the final writer (dict order)

@@ -378,9 +378,9 @@ DF void roe_flux2(const double pl[5], const double pr[5], const double S[3], con
 // muscl2.py:18-37) from the primitives of the cell (pv) and its neighbours
 // (pvm below, pvp above): with the limited slope s = lim(pv - pvm, pvp - pv),
 // the left state of the cell's high face is pv + s/2 and the right state of
-// its low face pv - s/2 -- the slope face_states evaluates once for each of
+// its low face pv - s/2 -- the slope face_states_fast evaluates once for each of
 // the two faces, here once.  The minmod form carries the NaN of the cell two
-// away from each face in, as face_states does.
+// away from each face in, as face_states_fast does.
 template <int LIM>
 DF void muscl_cell(const double pvm[5], const double pv[5], const double pvp[5], double pLhi[5], double pRlo[5]) {
   EXACT_FP

@@ -1,23 +1,37 @@
 // Reverse-mode stage kernels of the TVD-RK3 step.
 //
-// One RK stage  q_out = a q0 + b (q_s + dt L(q_s))  is reversed by two
-// gather-form kernels (no atomics, deterministic):
-//   k_vjp_faces_visc
-//                 every cell x: cotangent of the viscous flux tensor G(x)
-//                 from the divergence at its six neighbours, reverse sweep of
-//                 G into d/d(u, v, w, T) and d/d(central differences); then
-//                 every inviscid face whose left cell is x: cotangent of
-//                 F*|n| from the two cells that difference it, Roe + Harten
-//                 reverse sweep, stored as (d/d pL, d/d pR) at x;
-//   k_vjp_cell    every cell y: gathers the face states, the MUSCL slopes of
-//                 y-1, y, y+1 (limiter reverse), the central differences of
-//                 its neighbours and T, maps the primitive cotangent to
-//                 conservative variables and applies the RK coefficients.
+// One RK stage  q_out = a q0 + b (q_s + dt L(q_s))  is reversed by two kernels
+// (no atomics, deterministic).  Every cell's reverse needs, along each axis,
+// the cotangents of four faces and of three limited slopes; instead of passing
+// them through memory, each axis is swept so that they stay with the wave.  A
+// wave never waits for another one: no barriers, LDS only as the threads' own
+// store.  Thirteen doubles per cell go from the first kernel to the second:
+//   k_vjp_i   two independent sweeps along i, k-neighbours in the wave's lanes:
+//             sweep_visc  the cotangent of the viscous flux tensor G from the
+//                         divergence at the six neighbours, the reverse of G
+//                         into d/d(u, v, w, T) and d/d(central differences),
+//                         and of the latter the i and k ones; the j ones are
+//                         passed on;
+//             sweep_ik    the inviscid i and k axes;
+//   k_vjp_j   the j axis: a wave holds 64 columns (i, k) and marches along j; a
+//             cell's axes complete, it adds the viscous part, maps the
+//             primitive cotangent to conservative variables and applies the RK
+//             coefficients.
 // Functions cite the forward code they reverse in famrdp_jax (rhs/invscd.py,
 // rhs/viscous.py, solver/step.py).  This file is its own translation unit,
 // compiled with the default machine scheduler (the rest of the library uses
-// the max-ilp one): these two kernels measured 2.5 % and 6.5 % faster with it,
-// the marching stage kernel 2.4 % slower.
+// the max-ilp one, with which the two inviscid sweeps spill or come close).
+//
+// One stage of 10^6 cells (curvilinear 96^3) takes 133 + 87 us; two gather
+// kernels that passed 46 doubles per cell (three faces' state cotangents, the
+// viscous ones) took 223 + 184 us.  What bounds them now: k_vjp_j moves 42
+// doubles a cell that no other access could save (68 us at the 4.9 TB/s of a
+// large copy); k_vjp_i 48 (78 us), at two waves per SIMD whose loads and FP64
+// chains overlap only with each other's.  Its two sweeps as launches of their
+// own: 73 + 75 us.  Measured and not kept: the next step's loads issued a step
+// ahead (the face's reverse alone takes 156 registers: spills, 101 us for
+// sweep_ik); sweep_visc at three waves per SIMD (164 registers with its carried
+// values in LDS: 74 us, and longer waits for small blocks).
 #include "famrdp_kernels.h"
 #include "famrdp_adjoint.h"
 #include "famrdp_reverse.h"
@@ -25,9 +39,8 @@
 namespace famrdp {
 
 // Cells are addressed with 32-bit element indices (an adjoint plan's blocks
-// hold fewer than 2^29 cells: famrdp_plan_create refuses larger ones, whose 80
-// doubles per cell of stage and adjoint buffers would exceed 300 GB), loads and stores through a 32-bit byte offset from
-// a base that is the same for the whole workgroup -- the base stays in scalar
+// hold fewer than 2^29 cells: famrdp_plan_create refuses larger ones), loads
+// and stores through a 32-bit byte offset from a base that is the same for the whole wave -- the base stays in scalar
 // registers and a cell costs one 32-bit offset, however many arrays it reads
 // (global loads and stores: the pointers come from the device block table).
 __device__ __forceinline__ double rd(const double* __restrict__ a, unsigned i) {
@@ -45,227 +58,259 @@ __device__ __forceinline__ void rd_prim(const double* __restrict__ q, int64_t N,
 }
 
 // ---------------------------------------------------------------------------
-// inviscid faces (rhs/invscd.py:53-131 reversed)
+// one axis of the inviscid part, swept (rhs/invscd.py:53-131 reversed)
 // ---------------------------------------------------------------------------
+
+// What a sweep along an axis carries when it processes cell s, s increasing.
+// The registers of the face's reverse decide how much a wave can hold besides,
+// so only what the face needs as it is stays in registers: the primitives of
+// cell s and the left state of the face (s-1 | s).  The rest lies in the
+// thread's own LDS column: primitives, scaled cotangent and axis metrics of
+// cell s-1, the difference p(s-1) - p(s-2), the cotangent of the right state
+// of face (s-2 | s-1), what cell s-1 already holds (the slope of s-2 reaching
+// up, and what the caller adds) and the incomplete sum of cell s-2.
+struct AxisSweep {
+  double pc[5], pLn[5];
+  double* rest;
+};
+enum : int { SW_PM = 0, SW_DA = 5, SW_LPR = 10, SW_CARRY = 15, SW_ACC = 20, SW_MR = 25, SW_KD = 30, SW_N = 33 };
+constexpr int SWEEP_NT = 256;
+__device__ __forceinline__ double& sw(const AxisSweep& st, int i) { return st.rest[i * SWEEP_NT]; }
+// x is computed by here (not later, from operands that would stay alive)
+__device__ __forceinline__ void pin(double (&x)[5]) {
+#pragma unroll
+  for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(x[v]));
+}
+
+// What one step of a sweep reads: the state of the cell after (s+1), the
+// cotangent, volume and metrics of cell s.
+template <int NK>
+struct SweepLoads {
+  double q[5], l[5], vol, k[NK];
+};
+// k rows from row k0, and (NK = 6) from row 6
+template <int NK>
+__device__ __forceinline__ void sweep_load(SweepLoads<NK>& x, const BlockDesc& b, const double* __restrict__ qs,
+                                           const double* __restrict__ lin, unsigned c, unsigned cn, int k0) {
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    x.l[v] = rd(lin + v * b.N, c);
+    x.q[v] = rd(qs + v * b.N, cn);
+  }
+  x.vol = rd(b.vol, c);
+#pragma unroll
+  for (int m = 0; m < 3; ++m) x.k[m] = rd(b.kxyz + (k0 + m) * b.N, c);
+  if constexpr (NK == 6) {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) x.k[3 + m] = rd(b.kxyz + (6 + m) * b.N, c);
+  }
+}
+
+// The cotangent of a cell's flux difference, per unit of twice the flux:
+// c_mu lin / (2 (vol + 1e-300)); a face takes it from the cell on its right
+// and, negated, from the cell on its left, where those cells difference it.
+//
+// One step: cell s with primitives st.pc, pn = p(s+1), mr and kd of cell s.
+// vl, vr: cells s-1 and s difference their faces (2 .. n-3); face: the face
+// (s-1 | s) exists (left cell in 1 .. n-3); in: cell s-1 has a slope (1 ..
+// n-2); kp: added to what cell s holds.  Completes cell s-2 into out; st then
+// stands at s+1.
 template <int LIM>
-__device__ __forceinline__ void cell_vjp_faces(const BlockDesc& b, const double* __restrict__ qs,
-                                               const double* __restrict__ lin, double c_mu, unsigned a, double g,
-                                               const double pva[5], const double kka[9]) {
-  const int ni = b.ni, nj = b.nj, nk = b.nk;
-  const int64_t N = b.N;
-  const unsigned njk = (unsigned)nj * (unsigned)nk;
-  const int k = (int)(a % (unsigned)nk), j = (int)((a / (unsigned)nk) % (unsigned)nj), i = (int)(a / njk);
-  // the cell's own 1/vol and scaled cotangent, shared by its three faces
-  double lma[5];
-  const double rva = rcp_hd(rd(b.vol, a) + 1e-300);
+__device__ __forceinline__ void axis_step(AxisSweep& st, const double pn[5], const double mr[5], const double kd[3],
+                                          bool vl, bool vr, bool face, bool in, double cg2, double gm1h,
+                                          const double kp[5], double out[5]) {
+  double pLs[5], lpl[5] = {0, 0, 0, 0, 0}, lpr[5] = {0, 0, 0, 0, 0};
+  {
+    double pm[5], pRs[5];
 #pragma unroll
-  for (int v = 0; v < 5; ++v) lma[v] = c_mu * rd(lin + v * N, a);
-  // axes k, j, i: the viscous part that runs first in the same thread ends
-  // with the k-neighbours, so the k faces find them in cache; each axis writes
-  // only its own face slots, so the order leaves every result unchanged
+    for (int v = 0; v < 5; ++v) pm[v] = sw(st, SW_PM + v);
+    muscl_cell<LIM>(pm, st.pc, pn, pLs, pRs);
+    if (face) {
+      double f[5], S[3];
 #pragma unroll
-  for (int d = 2; d >= 0; --d) {
-    const int ad = d == 0 ? i : (d == 1 ? j : k);
-    const int nd = d == 0 ? ni : (d == 1 ? nj : nk);
-    const unsigned sd = d == 0 ? njk : (d == 1 ? (unsigned)nk : 1u);
-    double lpl[5] = {0, 0, 0, 0, 0}, lpr[5] = {0, 0, 0, 0, 0};
-    const bool va = ad >= 2 && ad <= nd - 3, vb = ad + 1 >= 2 && ad + 1 <= nd - 3;
-    if (ad >= 1 && ad <= nd - 3 && (va || vb)) {
-      const unsigned a1 = a + sd;
-      double lFa[5];
-      const double ra = va ? rva : 0.0, rb = vb ? rcp_hd(rd(b.vol, a1) + 1e-300) : 0.0;
+      for (int m = 0; m < 3; ++m) S[m] = 0.5 * (sw(st, SW_KD + m) + kd[m]);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double ma = va ? lma[v] : 0.0, mb = vb ? c_mu * rd(lin + v * N, a1) : 0.0;
-        lFa[v] = -ra * ma + rb * mb;
-      }
-      double pv[4][5];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        if (s == 1) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) pv[1][v] = pva[v];
-          continue;
-        }
-        double qq[5];
-        const unsigned cc = a + (unsigned)(s - 1) * sd;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) qq[v] = rd(qs + v * N, cc);
-        cons_to_prim_fast(qq, g, pv[s]);
-      }
-      double pL[5], pR[5];
-      face_states<LIM>(pv[0], pv[1], pv[2], pv[3], pL, pR);
-      double k0[3], k1[3];
-#pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        k0[m] = kka[d * 3 + m];
-        k1[m] = rd(b.kxyz + (d * 3 + m) * N, a1);
-      }
-      double nu[3], nm;
-      face_normal(k0, k1, nu, nm);
-      double lF[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) lF[v] = lFa[v] * nm;
-      roe_flux_prim_vjp(pL, pR, nu, g, lF, lpl, lpr);
+      for (int v = 0; v < 5; ++v) f[v] = (vr ? mr[v] : 0.0) - (vl ? sw(st, SW_MR + v) : 0.0);
+      roe_flux2_vjp(st.pLn, pRs, S, cg2, gm1h, f, lpl, lpr);
     }
+  }
+  pin(lpl);
+  pin(lpr);
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    const double B = st.pc[v] - sw(st, SW_PM + v), lp = sw(st, SW_LPR + v);
+    double lA = 0.0, lB = 0.0;
+    if (in) limiter_vjp_t<LIM>(sw(st, SW_DA + v), B, 0.5 * (lpl[v] - lp), lA, lB);
+    out[v] = sw(st, SW_ACC + v) - lA;
+    sw(st, SW_ACC + v) = ((lp + lpl[v]) + (lA - lB)) + sw(st, SW_CARRY + v);
+    sw(st, SW_CARRY + v) = lB + kp[v];
+    sw(st, SW_DA + v) = B;
+    sw(st, SW_LPR + v) = lpr[v];
+    sw(st, SW_PM + v) = st.pc[v];
+    sw(st, SW_MR + v) = mr[v];
+    st.pc[v] = pn[v];
+    st.pLn[v] = pLs[v];
+  }
+#pragma unroll
+  for (int m = 0; m < 3; ++m) sw(st, SW_KD + m) = kd[m];
+}
+
+// Start of a sweep whose first step processes cell s: c3, c2, c1 the cells
+// s-2, s-1 and s.
+template <int LIM>
+__device__ __forceinline__ void sweep_begin(AxisSweep& st, const BlockDesc& b, const double* __restrict__ qs,
+                                            const double* __restrict__ lin, unsigned c3, unsigned c2, unsigned c1,
+                                            int k0, double g, double hcm) {
+  double p0[5], pm[5], pr[5];
+  rd_prim(qs, b.N, c3, g, p0);
+  rd_prim(qs, b.N, c2, g, pm);
+  rd_prim(qs, b.N, c1, g, st.pc);
+  muscl_cell<LIM>(p0, pm, st.pc, st.pLn, pr);
+  const double r = hcm * rcp_hd(rd(b.vol, c2) + 1e-300);
+#pragma unroll
+  for (int v = 0; v < SW_N; ++v) sw(st, v) = 0.0;
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    sw(st, SW_PM + v) = pm[v];
+    sw(st, SW_MR + v) = r * rd(lin + v * b.N, c2);
+  }
+#pragma unroll
+  for (int m = 0; m < 3; ++m) sw(st, SW_KD + m) = rd(b.kxyz + (k0 + m) * b.N, c2);
+}
+
+// x of the lane below / above (the end lane of the wave keeps its own): a
+// wave-wide DPP shift, two moves for a double and no LDS
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double x) {
+  typedef int pair2 __attribute__((__vector_size__(8)));
+  pair2 u = __builtin_bit_cast(pair2, x);
+  u[0] = __builtin_amdgcn_update_dpp(u[0], u[0], CTRL, 0xf, 0xf, false);
+  u[1] = __builtin_amdgcn_update_dpp(u[1], u[1], CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, u);
+}
+__device__ __forceinline__ double lane_below(double x) { return lane_shift<0x138>(x); }   // wave_shr:1
+__device__ __forceinline__ double lane_above(double x) { return lane_shift<0x130>(x); }   // wave_shl:1
+
+// The k axis of the 64 consecutive cells of one plane a wave holds: each lane
+// its cell's low face, the rest from the lanes beside it.  A lane's result
+// needs three lanes either side, so lanes 3 .. 60 are complete.  Rows end
+// inside a wave: faces and slopes exist by the cell's own k, and what a lane
+// takes from the next row is a face or slope that does not exist there (zero).
+template <int LIM>
+__device__ __forceinline__ void lanes_k(const double pv[5], const double mr[5], const double kd[3], int k, int nk,
+                                        double cg2, double gm1h, double out[5]) {
+  double pL[5], pR[5], dA[5], dB[5], f[5], lpl[5] = {0, 0, 0, 0, 0}, lpr[5] = {0, 0, 0, 0, 0};
+  double S[3];
+  {
+    double pb[5], pa[5], ph[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-      at(b.fs + (d * 10 + v) * N, a) = lpl[v];
-      at(b.fs + (d * 10 + 5 + v) * N, a) = lpr[v];
+      pb[v] = lane_below(pv[v]);
+      pa[v] = lane_above(pv[v]);
+      dA[v] = pv[v] - pb[v];
+      dB[v] = pa[v] - pv[v];
     }
+    muscl_cell<LIM>(pb, pv, pa, ph, pR);
+    const bool vl = k - 1 >= 2 && k - 1 <= nk - 3, vr = k >= 2 && k <= nk - 3;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      pL[v] = lane_below(ph[v]);
+      const double mb = lane_below(mr[v]);
+      f[v] = (vr ? mr[v] : 0.0) - (vl ? mb : 0.0);
+    }
+#pragma unroll
+    for (int m = 0; m < 3; ++m) S[m] = 0.5 * (lane_below(kd[m]) + kd[m]);
+  }
+  if (k >= 2 && k <= nk - 2) roe_flux2_vjp(pL, pR, S, cg2, gm1h, f, lpl, lpr);
+  const bool in = k >= 1 && k <= nk - 2;
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    const double lh = lane_above(lpl[v]);      // left state of the cell's high face
+    double lA = 0.0, lB = 0.0;
+    if (in) limiter_vjp_t<LIM>(dA[v], dB[v], 0.5 * (lh - lpr[v]), lA, lB);
+    out[v] = ((lpr[v] + lh) + (lA - lB)) + (lane_below(lB) - lane_above(lA));
   }
 }
 
 // ---------------------------------------------------------------------------
-// viscous flux tensor (rhs/viscous.py:86-108 and 30-84 reversed)
+// viscous part (rhs/viscous.py:86-108 and 30-84 reversed)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void cell_vjp_visc(const BlockDesc& b, const double* __restrict__ qs,
-                                              const double* __restrict__ lin, double c_mu, unsigned x,
-                                              const Gas& gas, const double pv[5], const double kk[9]) {
-  const int ni = b.ni, nj = b.nj, nk = b.nk;
-  const int64_t N = b.N;
-  const unsigned sj = (unsigned)nk, si = (unsigned)nj * (unsigned)nk;
-  const int k = (int)(x % sj), j = (int)((x / sj) % (unsigned)nj), i = (int)(x / si);
-  const unsigned cm[3] = {x + (unsigned)(wrap_m(i, ni) - i) * si, x + (unsigned)(wrap_m(j, nj) - j) * sj,
-                          x + (unsigned)(wrap_m(k, nk) - k)};
-  const unsigned cp[3] = {x + (unsigned)(wrap_p(i, ni) - i) * si, x + (unsigned)(wrap_p(j, nj) - j) * sj,
-                          x + (unsigned)(wrap_p(k, nk) - k)};
-  // cotangent of G(x): the divergence at x - e_l uses +G(x)/2, at x + e_l uses -G(x)/2
-  double lG[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+
+// What the viscous reverse needs of a cell besides its place: u, v, w, T and
+// the momentum and energy cotangents (unscaled: every result is linear in
+// them and takes c_mu at the end).
+struct ViscCell {
+  double w[4], m[4];
+};
+__device__ __forceinline__ void load_visc(const double* __restrict__ qs, const double* __restrict__ lin, int64_t N,
+                                          unsigned c, const Gas& gas, ViscCell& x) {
+  double pv[5];
+  rd_prim(qs, N, c, gas.gamma, pv);
+  x.w[0] = pv[1];
+  x.w[1] = pv[2];
+  x.w[2] = pv[3];
+  x.w[3] = temperature_fast(pv, gas.R);
 #pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    const unsigned ym = cm[l], yp = cp[l];
+  for (int r = 0; r < 4; ++r) x.m[r] = rd(lin + (r + 1) * N, c);
+}
+
+// lG += sgn / 2 x (kxyz[l, :] times the cotangents of a neighbour): the
+// divergence at x - e_l holds +G(x) / 2, at x + e_l it holds -G(x) / 2.
+// kh = kxyz[l, :] / 2 of the neighbour.
+__device__ __forceinline__ void add_lG(double lG[9], const double m[4], const double kh[3], double sgn) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double mm = c_mu * rd(lin + (r + 1) * N, ym), mp = c_mu * rd(lin + (r + 1) * N, yp);
+  for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int jj = 0; jj < 3; ++jj)
-        lG[gidx(r, jj)] += 0.5 * (rd(b.kxyz + (l * 3 + jj) * N, ym) * mm - rd(b.kxyz + (l * 3 + jj) * N, yp) * mp);
-    }
-  }
-  double d[3][4];
-  const double T = temperature_fast(pv, gas.R);
-#pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    double pp[5], pm[5];
-    rd_prim(qs, N, cp[l], gas.gamma, pp);
-    rd_prim(qs, N, cm[l], gas.gamma, pm);
-    d[l][0] = 0.5 * (pp[1] - pm[1]);
-    d[l][1] = 0.5 * (pp[2] - pm[2]);
-    d[l][2] = 0.5 * (pp[3] - pm[3]);
-    d[l][3] = 0.5 * (temperature_fast(pp, gas.R) - temperature_fast(pm, gas.R));
-  }
-  double lu = 0, lv = 0, lw = 0, lT = 0, ld[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-  viscous_flux_vjp(pv, T, d, kk, gas.gamma, gas.R, b.mu0, gas.T0, gas.Ts, gas.Pr_lam, lG, lu, lv, lw, lT, ld);
-  at(b.vs, x) = lu;
-  at(b.vs + N, x) = lv;
-  at(b.vs + 2 * N, x) = lw;
-  at(b.vs + 3 * N, x) = lT;
-#pragma unroll
-  for (int l = 0; l < 3; ++l)
-#pragma unroll
-    for (int s = 0; s < 4; ++s) at(b.vs + (4 + 4 * l + s) * N, x) = ld[l][s];
+    for (int jj = 0; jj < 3; ++jj) lG[gidx(r, jj)] += (sgn * kh[jj]) * m[r];
 }
 
 // ---------------------------------------------------------------------------
-// per-cell gather, primitive -> conservative, RK coefficients
-//   mode 0: l0 = c0 lin,  lout = c_next lin + g     (stage 3; lin is l0, each
-//           cell's value read before it is written)
-//   mode 1: l0 += c0 lin, lout = c_next lin + g     (stage 2)
-//   mode 2: l0 += lin + g                           (stage 1)
+// a cell whose axes are summed (lpv, cotangent of its primitives): viscous
+// gather, primitive -> conservative, RK coefficients
+//   stage 3: lout = 2/3 lin + g                      (its share of l0, lin / 3,
+//            waits: lin is l0 itself, still read by other waves)
+//   stage 2: l0 = l0 / 3 + 3/4 lin, lout = 1/4 lin + g
+//   stage 1: l0 += lin + g
 // ---------------------------------------------------------------------------
-template <int LIM>
-__device__ __forceinline__ void cell_vjp_gather(const BlockDesc& b, const double* __restrict__ qs,
-                                                const double* lin, double* lout, unsigned y, const Gas& gas,
-                                                double c_next, double c0, int mode) {
-  const int ni = b.ni, nj = b.nj, nk = b.nk;
+__device__ __forceinline__ void cell_vjp_finish(const BlockDesc& b, const double* __restrict__ qs, const double* lin,
+                                                double* lout, int j, unsigned y, const Gas& gas, int stage,
+                                                double lpv[5]) {
   const int64_t N = b.N;
-  const unsigned sj = (unsigned)nk, si = (unsigned)nj * (unsigned)nk;
-  const int k = (int)(y % sj), j = (int)((y / sj) % (unsigned)nj), i = (int)(y / si);
-  // the cell's own state and primitives, converted once for the three axes
-  double qy[5], pvy[5];
+  double q[5], pv[5], ls4[4];
 #pragma unroll
-  for (int v = 0; v < 5; ++v) qy[v] = rd(qs + v * N, y);
-  cons_to_prim_fast(qy, gas.gamma, pvy);
-  double lpv[5] = {0, 0, 0, 0, 0};
-  // ---- inviscid: face states and MUSCL slopes along each axis
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double* fsd = b.fs + (int64_t)(d * 10) * N;
-    const int yd = d == 0 ? i : (d == 1 ? j : k);
-    const int nd = d == 0 ? ni : (d == 1 ? nj : nk);
-    const unsigned sd = d == 0 ? si : (d == 1 ? sj : 1u);
-    double fl[5], fr[5];   // cotangents of the left state of face (y, y+1), right state of (y-1, y)
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      fl[v] = rd(fsd + v * N, y);
-      fr[v] = yd >= 1 ? rd(fsd + (5 + v) * N, y - sd) : 0.0;
-      lpv[v] += fl[v];
-      if (yd >= 1) lpv[v] += fr[v];
-    }
-    // slopes s(x) = lim(pv(x)-pv(x-1), pv(x+1)-pv(x)) for x = y-1, y, y+1
-    double pv[5][5];
-#pragma unroll
-    for (int s = 0; s < 5; ++s) {
-      const int xd = yd + s - 2;
-      if (s == 2)
-#pragma unroll
-        for (int v = 0; v < 5; ++v) pv[2][v] = pvy[v];
-      else if (xd >= 0 && xd < nd) rd_prim(qs, N, y + (unsigned)(s - 2) * sd, gas.gamma, pv[s]);
-      else
-#pragma unroll
-        for (int v = 0; v < 5; ++v) pv[s][v] = 0.0;
-    }
-#pragma unroll
-    for (int o = -1; o <= 1; ++o) {
-      const int xd = yd + o;
-      if (xd < 1 || xd > nd - 2) continue;
-      const unsigned xc = y + (unsigned)o * sd;
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        const double ls = o == 0 ? 0.5 * fl[v] - 0.5 * fr[v]
-                                 : 0.5 * rd(fsd + v * N, xc) - 0.5 * rd(fsd + (5 + v) * N, xc - sd);
-        const double A = pv[o + 2][v] - pv[o + 1][v], B = pv[o + 3][v] - pv[o + 2][v];
-        double lA, lB;
-        limiter_vjp_t<LIM>(A, B, ls, lA, lB);
-        if (o == 0) lpv[v] += lA - lB;
-        else if (o == 1) lpv[v] -= lA;
-        else lpv[v] += lB;
-      }
-    }
+  for (int v = 0; v < 5; ++v) {
+    q[v] = rd(qs + v * N, y);
+    lpv[v] += rd(b.fs + v * N, y);
   }
-  // ---- viscous: own uses plus the central differences of the neighbours
-  const unsigned cm[3] = {y + (unsigned)(wrap_m(i, ni) - i) * si, y + (unsigned)(wrap_m(j, nj) - j) * sj,
-                          y + (unsigned)(wrap_m(k, nk) - k)};
-  const unsigned cp[3] = {y + (unsigned)(wrap_p(i, ni) - i) * si, y + (unsigned)(wrap_p(j, nj) - j) * sj,
-                          y + (unsigned)(wrap_p(k, nk) - k)};
-  double ls4[4] = {rd(b.vs, y), rd(b.vs + N, y), rd(b.vs + 2 * N, y), rd(b.vs + 3 * N, y)};
+  cons_to_prim_fast(q, gas.gamma, pv);
+  // viscous: vs holds what k_vjp_visc summed (u, v, w, T) and the cotangents
+  // of the cell's central differences along j
+  const unsigned jm = y + (unsigned)((wrap_m(j, b.nj) - j) * b.nk), jp = y + (unsigned)((wrap_p(j, b.nj) - j) * b.nk);
 #pragma unroll
-  for (int l = 0; l < 3; ++l)
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      ls4[s] += 0.5 * rd(b.vs + (4 + 4 * l + s) * N, cm[l]) - 0.5 * rd(b.vs + (4 + 4 * l + s) * N, cp[l]);
+  for (int s = 0; s < 4; ++s)
+    ls4[s] = rd(b.vs + s * N, y) + 0.5 * (rd(b.vs + (4 + s) * N, jm) - rd(b.vs + (4 + s) * N, jp));
   lpv[1] += ls4[0]; lpv[2] += ls4[1]; lpv[3] += ls4[2];
-  temperature_vjp(pvy, gas.R, ls4[3], lpv[0], lpv[4]);
+  temperature_vjp(pv, gas.R, ls4[3], lpv[0], lpv[4]);
   double gq[5] = {0, 0, 0, 0, 0};
-  cons_to_prim_vjp(qy, gas.gamma, lpv, gq);
+  cons_to_prim_vjp(q, gas.gamma, lpv, gq);
   // ---- RK coefficients (solver/step.py:45-53 reversed)
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
     const double li = rd(lin + v * N, y);
     gmem_double& l0 = at(b.l0 + v * N, y);
-    if (mode == 2) {
-      l0 += li + gq[v];
+    if (stage == 3) {
+      at(lout + v * N, y) = (2.0 / 3.0) * li + gq[v];
+    } else if (stage == 2) {
+      l0 = (1.0 / 3.0) * l0 + 0.75 * li;
+      at(lout + v * N, y) = 0.25 * li + gq[v];
     } else {
-      l0 = (mode == 0 ? 0.0 : l0) + c0 * li;
-      at(lout + v * N, y) = c_next * li + gq[v];
+      l0 += li + gq[v];
     }
   }
 }
 
 // Stage selector for the reverse sweep: which buffers a stage reads/writes.
-//   stage 3: qs = q2, lin = l0 (the cotangent of q_new, which the gather
-//            replaces cell by cell with its q0 share: l0 = lin / 3), lout = lb
+//   stage 3: qs = q2, lin = l0 (the cotangent of q_new), lout = lb
 //   stage 2: qs = q1, lin = lb, lout = la
 //   stage 1: qs = qh, lin = la
 __device__ __forceinline__ void vjp_bufs(const BlockDesc& b, int stage, const double*& qs, const double*& lin,
@@ -279,59 +324,244 @@ __device__ __forceinline__ double stage_cmu(int stage, double dt) {
   return stage == 3 ? (2.0 / 3.0) * dt : (stage == 2 ? 0.25 * dt : dt);
 }
 
-// The viscous part first: the face part reuses the neighbours' state and
-// metrics it loaded (from registers or cache).  The scheduling barrier keeps
-// the two parts' instructions apart (two waves per SIMD, as the face part
-// alone needs: 207 registers with the default scheduler, no spills).
-template <int LIM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_vjp_faces_visc(const BlockDesc* __restrict__ blocks, const Tile* __restrict__ tiles, int stage, Gas gas, double dt) {
-  const Tile tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];   // neighbouring tiles on one XCD (shared L2)
-  const BlockDesc& b = blocks[tl.block];
-  const int64_t c = (int64_t)tl.start + threadIdx.x;
-  if (c >= b.N) return;
+// The viscous part: a wave marches along i over 64 cells of a plane, lanes
+// 2 .. 61 complete (a cell takes the difference cotangents of its neighbours,
+// which take the state of theirs).  The rows of a plane are laid out with two
+// cells of periodic image at either end (nk + 4 lanes a row), so the lanes
+// beside a lane are its k-neighbours in the roll's sense too; planes and rows
+// wrap in their index.  Step s reverses G at plane s -- i-neighbours carried,
+// k-neighbours from the lanes, j-neighbours loaded -- and completes plane s-1.
+__device__ __forceinline__ void sweep_visc(const BlockDesc& b, const SweepTile& tl, int stage, const Gas& gas,
+                                           double dt) {
+  const int lane = threadIdx.x & 63, ni = b.ni, nj = b.nj, nk = b.nk, ne = nj * (nk + 4);
+  const int64_t N = b.N;
+  const unsigned njk = (unsigned)nj * (unsigned)nk;
   const double *qs, *lin;
   double* lout;
   vjp_bufs(b, stage, qs, lin, lout);
   const double cmu = stage_cmu(stage, dt * b.dt_scale);
-  // the cell's primitives, converted once for both parts (and rounded once:
-  // the same values reach every use), and its metrics, loaded once for both
-  double pv[5], kk[9];
-  rd_prim(qs, b.N, (unsigned)c, gas.gamma, pv);
+  const int e0 = tl.base - 2 + lane, e = e0 < 0 ? 0 : (e0 >= ne ? ne - 1 : e0);
+  const int j = e / (nk + 4), ke = e % (nk + 4) - 2;
+  const int k = ke < 0 ? ke + nk : (ke >= nk ? ke - nk : ke);
+  const bool own = lane >= 2 && lane <= 61 && e0 < ne && ke >= 0 && ke < nk;
+  const unsigned cp = (unsigned)(j * nk + k);
+  const unsigned ojm = (unsigned)((wrap_m(j, nj) - j) * nk), ojp = (unsigned)((wrap_p(j, nj) - j) * nk);
+  auto cell = [&](int s) -> unsigned { return (unsigned)(s < 0 ? s + ni : (s >= ni ? s - ni : s)) * njk + cp; };
+
+  // planes s-1 and s: state, cotangents, kxyz[0, :] / 2
+  ViscCell xm, xc;
+  double km[3], kc[3];
+  load_visc(qs, lin, N, cell(tl.p0 - 2), gas, xm);
+  load_visc(qs, lin, N, cell(tl.p0 - 1), gas, xc);
 #pragma unroll
-  for (int m = 0; m < 9; ++m) kk[m] = rd(b.kxyz + m * b.N, (unsigned)c);
-  cell_vjp_visc(b, qs, lin, cmu, (unsigned)c, gas, pv, kk);
-  __builtin_amdgcn_sched_barrier(0);
-  cell_vjp_faces<LIM>(b, qs, lin, cmu, (unsigned)c, gas.gamma, pv, kk);
+  for (int m = 0; m < 3; ++m) {
+    km[m] = 0.5 * rd(b.kxyz + m * N, cell(tl.p0 - 2));
+    kc[m] = 0.5 * rd(b.kxyz + m * N, cell(tl.p0 - 1));
+  }
+  double acc[4] = {0, 0, 0, 0};    // plane s-1 without the share of plane s
+  double ldi[4] = {0, 0, 0, 0};    // cotangents of the i differences of plane s-1, halved
+  for (int s = tl.p0 - 1; s <= tl.p1; ++s) {
+    const unsigned c = cell(s), cn = cell(s + 1);
+    ViscCell xn, xj;
+    double kn[3], kk[9], lG[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, d[3][4], kj[3];
+    load_visc(qs, lin, N, cn, gas, xn);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kn[m] = 0.5 * rd(b.kxyz + m * N, cn);
+#pragma unroll
+    for (int m = 3; m < 9; ++m) kk[m] = rd(b.kxyz + m * N, c);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kk[m] = 2.0 * kc[m];
+    // j-neighbours
+    load_visc(qs, lin, N, c + ojm, gas, xj);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kj[m] = 0.5 * rd(b.kxyz + (3 + m) * N, c + ojm);
+    add_lG(lG, xj.m, kj, 1.0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[1][q] = -xj.w[q];
+    load_visc(qs, lin, N, c + ojp, gas, xj);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kj[m] = 0.5 * rd(b.kxyz + (3 + m) * N, c + ojp);
+    add_lG(lG, xj.m, kj, -1.0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[1][q] = 0.5 * (d[1][q] + xj.w[q]);
+    // k-neighbours
+    {
+      double mb[4], ma[4], kb[3], ka[3];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        mb[q] = lane_below(xc.m[q]);
+        ma[q] = lane_above(xc.m[q]);
+        d[2][q] = 0.5 * (lane_above(xc.w[q]) - lane_below(xc.w[q]));
+      }
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        const double h = 0.5 * kk[6 + m];
+        kb[m] = lane_below(h);
+        ka[m] = lane_above(h);
+      }
+      add_lG(lG, mb, kb, 1.0);
+      add_lG(lG, ma, ka, -1.0);
+    }
+    // i-neighbours
+    add_lG(lG, xm.m, km, 1.0);
+    add_lG(lG, xn.m, kn, -1.0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[0][q] = 0.5 * (xn.w[q] - xm.w[q]);
+    double l4[4] = {0, 0, 0, 0}, ld[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    const double pv[5] = {0.0, xc.w[0], xc.w[1], xc.w[2], 0.0};
+    viscous_flux_vjp(pv, xc.w[3], d, kk, gas.gamma, gas.R, b.mu0, gas.T0, gas.Ts, gas.Pr_lam, lG, l4[0], l4[1], l4[2],
+                     l4[3], ld);
+    const bool out1 = s > tl.p0 && own, out0 = s >= tl.p0 && s < tl.p1 && own;
+    const unsigned cm = cell(s - 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (out1) at(b.vs + q * N, cm) = cmu * (acc[q] - 0.5 * ld[0][q]);
+      if (out0) at(b.vs + (4 + q) * N, c) = cmu * ld[1][q];
+      acc[q] = (l4[q] + ldi[q]) + 0.5 * (lane_below(ld[2][q]) - lane_above(ld[2][q]));
+      ldi[q] = 0.5 * ld[0][q];
+    }
+    xm = xc;
+    xc = xn;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      km[m] = kc[m];
+      kc[m] = kn[m];
+    }
+  }
 }
 
-// at most 128 VGPRs: this memory-bound gather wants four waves per SIMD
+// The i and k axes: lanes 3 .. 60 hold the plane cells from base on, planes p0
+// .. p1-1.  The wave starts three planes early and ends two late (the slopes
+// and faces around its first and last plane).  Writes the sum of both axes
+// (the cotangent of the five primitives) to fs.
 template <int LIM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_vjp_cell(const BlockDesc* __restrict__ blocks, const Tile* __restrict__ tiles,
-                                                  int stage, Gas gas) {
-  const Tile tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];   // neighbouring tiles on one XCD (shared L2)
-  const BlockDesc& b = blocks[tl.block];
-  const int64_t c = (int64_t)tl.start + threadIdx.x;
-  if (c >= b.N) return;
+__device__ __forceinline__ void sweep_ik(double* rest, const BlockDesc& b, const SweepTile& tl, int stage,
+                                         const Gas& gas, double dt) {
+  const int lane = threadIdx.x & 63, ni = b.ni, nk = b.nk;
+  const int64_t N = b.N;
+  const unsigned njk = (unsigned)b.nj * (unsigned)nk;
   const double *qs, *lin;
   double* lout;
   vjp_bufs(b, stage, qs, lin, lout);
-  const double c_next = stage == 3 ? 2.0 / 3.0 : 0.25;
-  const double c0 = stage == 3 ? 1.0 / 3.0 : 0.75;
-  cell_vjp_gather<LIM>(b, qs, lin, lout, (unsigned)c, gas, c_next, c0, stage == 3 ? 0 : (stage == 2 ? 1 : 2));
+  const double hcm = uniform(0.5 * stage_cmu(stage, dt * b.dt_scale));
+  const double g = gas.gamma, cg2 = uniform(2.0 * g / (g - 1.0)), gm1h = uniform(0.5 * (g - 1.0));
+  // the lane's plane cell (the nearest one where it lies outside the plane)
+  const int cl = tl.base - 3 + lane;
+  const unsigned cp = cl < 0 ? 0u : (cl >= (int)njk ? njk - 1u : (unsigned)cl);
+  const int k = (int)(cp % (unsigned)nk);
+  const bool own = lane >= 3 && lane <= 60 && cl < (int)njk;
+  auto cell = [&](int s) -> unsigned { return (unsigned)(s < 0 ? 0 : (s >= ni ? ni - 1 : s)) * njk + cp; };
+
+  AxisSweep st;
+  st.rest = rest + threadIdx.x;
+  sweep_begin<LIM>(st, b, qs, lin, cell(tl.p0 - 3), cell(tl.p0 - 2), cell(tl.p0 - 1), 0, g, hcm);
+  SweepLoads<6> x;
+  for (int s = tl.p0 - 1; s <= tl.p1 + 1; ++s) {
+    double pn[5], mr[5], kd[3], out[5], kp[5] = {0, 0, 0, 0, 0};
+    sweep_load(x, b, qs, lin, cell(s), cell(s + 1), 0);
+    const double r = hcm * rcp_hd(x.vol + 1e-300);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) mr[v] = r * x.l[v];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kd[m] = x.k[m];
+    if (s >= tl.p0 && s < tl.p1) {
+      lanes_k<LIM>(st.pc, mr, x.k + 3, k, nk, cg2, gm1h, kp);
+      pin(kp);
+    }
+    cons_to_prim_fast(x.q, g, pn);
+    axis_step<LIM>(st, pn, mr, kd, s - 1 >= 2 && s - 1 <= ni - 3, s >= 2 && s <= ni - 3, s >= 2 && s <= ni - 2,
+                   s >= 2 && s <= ni - 1, cg2, gm1h, kp, out);
+    if (s >= tl.p0 + 2 && own) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) at(b.fs + v * N, cell(s - 2)) = out[v];
+    }
+  }
+}
+
+// Both sweeps that march along i, one launch: neither needs the other, and
+// waves of the one (loads, few chains) and of the other (FP64 chains) fill
+// each other's waits on a SIMD.  Each wave its own tile of its sweep's table,
+// no barrier; workgroups alternate between the sweeps in groups of eight (one
+// to each XCD), so both spread over every XCD, each in its table's order.
+template <int LIM>
+__global__ void __launch_bounds__(SWEEP_NT) __attribute__((amdgpu_waves_per_eu(2)))
+k_vjp_i(const BlockDesc* __restrict__ blocks, const SweepTile* __restrict__ sv, int nv,
+        const SweepTile* __restrict__ sik, int nik, int stage, Gas gas, double dt) {
+  __shared__ double rest[SW_N * SWEEP_NT];
+  const int gv = (nv + 3) / 4, gik = (nik + 3) / 4, wg = (int)blockIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int paired = 8 * ((gv < gik ? gv : gik) / 8);   // workgroups of each sweep that alternate
+  const bool visc = wg < 2 * paired ? (wg >> 3) & 1 : wg - paired < gv;
+  int idx;
+  if (wg < 2 * paired) idx = (wg >> 4) * 8 + (wg & 7);
+  else idx = visc ? wg - paired : wg - gv;
+  if (visc) {
+    const int t = xcd_remap(idx, gv) * 4 + w;
+    if (t < nv) sweep_visc(blocks[sv[t].block], sv[t], stage, gas, dt);
+  } else {
+    const int t = xcd_remap(idx, gik) * 4 + w;
+    if (t < nik) sweep_ik<LIM>(rest, blocks[sik[t].block], sik[t], stage, gas, dt);
+  }
+}
+
+// The j axis, and what is left to do for a cell: lanes are 64 columns (i, k)
+// from base on (k fastest), rows p0 .. p1-1.
+template <int LIM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_vjp_j(const BlockDesc* __restrict__ blocks, const SweepTile* __restrict__ tiles, int ntiles, int stage, Gas gas,
+        double dt) {
+  const int w = xcd_remap(blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w >= ntiles) return;
+  const SweepTile tl = tiles[w];
+  const BlockDesc& b = blocks[tl.block];
+  const int lane = threadIdx.x & 63, nj = b.nj, nk = b.nk;
+  const int64_t N = b.N;
+  const unsigned njk = (unsigned)nj * (unsigned)nk, nik = (unsigned)b.ni * (unsigned)nk;
+  const double *qs, *lin;
+  double* lout;
+  vjp_bufs(b, stage, qs, lin, lout);
+  const double hcm = uniform(0.5 * stage_cmu(stage, dt * b.dt_scale));
+  const double g = gas.gamma, cg2 = uniform(2.0 * g / (g - 1.0)), gm1h = uniform(0.5 * (g - 1.0));
+  const unsigned cl = (unsigned)(tl.base + lane);
+  const bool own = cl < nik;
+  const unsigned cc = own ? cl : nik - 1u;
+  const int i = (int)(cc / (unsigned)nk), k = (int)(cc % (unsigned)nk);
+  const unsigned col = (unsigned)i * njk + (unsigned)k;
+  auto cell = [&](int s) -> unsigned { return col + (unsigned)(s < 0 ? 0 : (s >= nj ? nj - 1 : s)) * (unsigned)nk; };
+
+  __shared__ double rest[SW_N * SWEEP_NT];
+  AxisSweep st;
+  st.rest = rest + threadIdx.x;
+  sweep_begin<LIM>(st, b, qs, lin, cell(tl.p0 - 3), cell(tl.p0 - 2), cell(tl.p0 - 1), 3, g, hcm);
+  SweepLoads<3> x;
+  for (int s = tl.p0 - 1; s <= tl.p1 + 1; ++s) {
+    double pn[5], mr[5], kd[3], out[5], kp[5] = {0, 0, 0, 0, 0};
+    sweep_load(x, b, qs, lin, cell(s), cell(s + 1), 3);
+    const double r = hcm * rcp_hd(x.vol + 1e-300);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) mr[v] = r * x.l[v];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) kd[m] = x.k[m];
+    cons_to_prim_fast(x.q, g, pn);
+    axis_step<LIM>(st, pn, mr, kd, s - 1 >= 2 && s - 1 <= nj - 3, s >= 2 && s <= nj - 3, s >= 2 && s <= nj - 2,
+                   s >= 2 && s <= nj - 1, cg2, gm1h, kp, out);
+    if (s >= tl.p0 + 2 && own) {
+      cell_vjp_finish(b, qs, lin, lout, s - 2, cell(s - 2), gas, stage, out);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
 // host launcher
 // ---------------------------------------------------------------------------
-void launch_stage_vjp(const BlockDesc* blocks, const Tile* tiles, int ntiles, int stage, const Gas& gas, double dt,
-                      int lim, hipStream_t st) {
+void launch_stage_vjp(const BlockDesc* blocks, const SweepTile* sv, int nv, const SweepTile* sik, int nik,
+                      const SweepTile* sj, int nsj, int stage, const Gas& gas, double dt, int lim, hipStream_t st) {
+  const unsigned wi = (unsigned)((nv + 3) / 4 + (nik + 3) / 4), wj = (unsigned)((nsj + 3) / 4);
   if (lim == LIM_VANLEER) {
-    k_vjp_faces_visc<LIM_VANLEER><<<ntiles, 256, 0, st>>>(blocks, tiles, stage, gas, dt);
-    k_vjp_cell<LIM_VANLEER><<<ntiles, 256, 0, st>>>(blocks, tiles, stage, gas);
+    k_vjp_i<LIM_VANLEER><<<wi, SWEEP_NT, 0, st>>>(blocks, sv, nv, sik, nik, stage, gas, dt);
+    k_vjp_j<LIM_VANLEER><<<wj, SWEEP_NT, 0, st>>>(blocks, sj, nsj, stage, gas, dt);
   } else {
-    k_vjp_faces_visc<LIM_MINMOD><<<ntiles, 256, 0, st>>>(blocks, tiles, stage, gas, dt);
-    k_vjp_cell<LIM_MINMOD><<<ntiles, 256, 0, st>>>(blocks, tiles, stage, gas);
+    k_vjp_i<LIM_MINMOD><<<wi, SWEEP_NT, 0, st>>>(blocks, sv, nv, sik, nik, stage, gas, dt);
+    k_vjp_j<LIM_MINMOD><<<wj, SWEEP_NT, 0, st>>>(blocks, sj, nsj, stage, gas, dt);
   }
 }
 
