@@ -9,31 +9,10 @@ namespace famrdp {
 
 // ---------------------------------------------------------------------------
 // BC faces reversed (physics/bc/*.py): the ghost cotangent moves to the inner
-// cell it was built from (or to q_inf for farfield) and is cleared.
+// cell it was built from (or to q_inf for farfield) and is cleared.  An
+// isothermal face is linearised at the inner layers that the forward ghost
+// pass recorded (famrdp_ghost.h, GhostSnap).
 // ---------------------------------------------------------------------------
-
-// Copy of the inner layers of isothermal faces just before the face is
-// applied (the reverse sweep linearises at those values).
-__global__ void k_bc_snapshot(const BlockDesc* __restrict__ blocks, const BcEntry* __restrict__ entries, int ghost,
-                              double* __restrict__ snap, int64_t maxcells) {
-  const BcEntry e = entries[blockIdx.y];
-  if (e.kind != BC_WALL_ISOTHERMAL) return;
-  const BlockDesc b = blocks[e.block];
-  const int ax = e.face / 2;
-  const bool lo = (e.face % 2) == 0;
-  const int n[3] = {b.ni, b.nj, b.nk};
-  const int64_t st[3] = {(int64_t)b.nj * b.nk, b.nk, 1};
-  const int t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
-  const int64_t ncell = (int64_t)n[t1] * n[t2];
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= ncell) return;
-  const int64_t base = (t / n[t2]) * st[t1] + (t % n[t2]) * st[t2];
-  for (int gl = 0; gl < ghost; ++gl) {
-    const int inner = lo ? 2 * ghost - 1 - gl : n[ax] - 2 * ghost + gl;
-    const int64_t ci = base + inner * st[ax];
-    for (int v = 0; v < 5; ++v) snap[(((int64_t)blockIdx.y * ghost + gl) * 5 + v) * maxcells + t] = b.qh[v * b.N + ci];
-  }
-}
 
 __global__ void k_bc_face_vjp(const BlockDesc* __restrict__ blocks, const BcEntry* __restrict__ entries, int ghost,
                               double gamma, double R, const double* __restrict__ snap, double* __restrict__ part,

@@ -80,12 +80,49 @@ int cfl_scratch(double** ptr) {
 
 }  // namespace
 
+// The small device arrays of a plan, gathered so that one allocation and one
+// copy make them all: an allocation or a synchronous copy costs 10-30 us
+// whatever its size, and a plan has about forty such arrays.
+class TableSet {
+ public:
+  template <class T>
+  void table(T** dst, const std::vector<T>& src) {   // a device copy of src (none of an empty one)
+    if (src.empty()) return;
+    const size_t at = (bytes_.size() + ALIGN - 1) / ALIGN * ALIGN;
+    bytes_.resize(at + sizeof(T) * src.size());
+    std::memcpy(bytes_.data() + at, src.data(), sizeof(T) * src.size());
+    slots_.push_back({reinterpret_cast<void**>(dst), at, false});
+  }
+  template <class T>
+  void scratch(T** dst, size_t count) {              // not initialised
+    if (count == 0) return;
+    slots_.push_back({reinterpret_cast<void**>(dst), scratch_, true});
+    scratch_ += (sizeof(T) * count + ALIGN - 1) / ALIGN * ALIGN;
+  }
+  bool make(char** mem) {
+    const size_t tables = (bytes_.size() + ALIGN - 1) / ALIGN * ALIGN;
+    if (tables + scratch_ == 0) return true;
+    if (hipMalloc(mem, tables + scratch_) != hipSuccess) return false;
+    if (!bytes_.empty() && hipMemcpy(*mem, bytes_.data(), bytes_.size(), hipMemcpyHostToDevice) != hipSuccess)
+      return false;
+    for (const Slot& s : slots_) *s.dst = *mem + (s.scratch ? tables : 0) + s.at;
+    return true;
+  }
+
+ private:
+  static constexpr size_t ALIGN = 256;
+  struct Slot { void** dst; size_t at; bool scratch; };
+  std::vector<char> bytes_;
+  std::vector<Slot> slots_;
+  size_t scratch_ = 0;
+};
+
 struct famrdp_plan {
   int nblocks = 0, ghost = 2, limiter = 0;
   Gas gas{};
   std::vector<int32_t> dims;             // 3 per block
   std::vector<int64_t> N;
-  // device tables
+  char* d_tables = nullptr;              // holds every d_ array below
   BlockDesc* d_blocks = nullptr;
   // staging ring for block-table uploads: a slot is reused only after the
   // copy that last read it has completed (its event), so uploads do not
@@ -100,6 +137,13 @@ struct famrdp_plan {
   HaloEntry* d_halo = nullptr;
   int nhalo = 0;
   double* d_halo_stage = nullptr;
+  // ghost cells of a step (famrdp_ghost.h)
+  GhostEntry* d_ghost = nullptr;
+  GhostChain* d_chains = nullptr;
+  BcEntry* d_ops = nullptr;
+  GhostSnap* d_snaps = nullptr;
+  double* d_ghost_stage = nullptr;
+  int nghost_direct = 0, nghost_staged = 0, nghost_late = 0, nsnaps = 0;
   BcEntry* d_bc[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   int nbc[6] = {0, 0, 0, 0, 0, 0};
   int64_t bc_maxcells[6] = {0, 0, 0, 0, 0, 0};
@@ -150,11 +194,9 @@ namespace {
 inline int face_axis(int f) { return f / 2; }
 inline bool face_lo(int f) { return f % 2 == 0; }
 
-int build_halo_table(famrdp_plan* p, int ncut, const famrdp_cut* cuts, std::vector<HaloEntry>& out) {
+// The copies of the exchange, in the order given (a later one wins).
+int add_cuts(const famrdp_plan* p, int ncut, const famrdp_cut* cuts, GhostTable& table) {
   const int g = p->ghost;
-  // final writer per target cell: slot[b][cell] = index into `src` (or -1)
-  std::vector<std::vector<int64_t>> slot(p->nblocks);
-  std::vector<std::pair<int32_t, int32_t>> src;
   for (int c = 0; c < ncut; ++c) {
     const famrdp_cut& ct = cuts[c];
     if (ct.tgt_block < 0 || ct.tgt_block >= p->nblocks || ct.src_block < 0 || ct.src_block >= p->nblocks ||
@@ -173,24 +215,12 @@ int build_halo_table(famrdp_plan* p, int ncut, const famrdp_cut* cuts, std::vect
     ext_s[as] = g;
     if (ext_t[0] != ext_s[0] || ext_t[1] != ext_s[1] || ext_t[2] != ext_s[2])
       return fail(FAMRDP_E_INVALID, "cut " + std::to_string(c) + ": ghost slab and source slab shapes differ");
-    auto& sl = slot[ct.tgt_block];
-    if (sl.empty()) sl.assign((size_t)p->N[ct.tgt_block], -1);
     for (int a = 0; a < ext_t[0]; ++a)
       for (int b = 0; b < ext_t[1]; ++b)
         for (int k = 0; k < ext_t[2]; ++k) {
-          const int64_t tc = ((int64_t)(lo_t[0] + a) * dt[1] + (lo_t[1] + b)) * dt[2] + (lo_t[2] + k);
           const int64_t sc = ((int64_t)(lo_s[0] + a) * ds[1] + (lo_s[1] + b)) * ds[2] + (lo_s[2] + k);
-          sl[(size_t)tc] = (int64_t)src.size();
-          src.emplace_back(ct.src_block, (int32_t)sc);
+          table.copy(ct.tgt_block, lo_t[0] + a, lo_t[1] + b, lo_t[2] + k, ct.src_block, (int32_t)sc);
         }
-  }
-  for (int b = 0; b < p->nblocks; ++b) {
-    if (slot[b].empty()) continue;
-    for (int64_t tc = 0; tc < p->N[b]; ++tc) {
-      const int64_t s = slot[b][(size_t)tc];
-      if (s < 0) continue;
-      out.push_back(HaloEntry{b, (int32_t)tc, src[(size_t)s].first, src[(size_t)s].second});
-    }
   }
   return FAMRDP_OK;
 }
@@ -270,9 +300,10 @@ int copy_blocks(famrdp_plan* p, hipStream_t st, Dst dst_of, Src src_of) {
   return FAMRDP_OK;
 }
 
-int launch_halo(famrdp_plan* p, hipStream_t st, const BlockDesc* table = nullptr) {
+// The halo exchange on its own.
+int launch_halo(famrdp_plan* p, hipStream_t st) {
   if (p->nhalo == 0) return FAMRDP_OK;
-  const BlockDesc* tb = table ? table : p->d_blocks;
+  const BlockDesc* tb = p->d_blocks;
   k_halo_gather<<<nblk(p->nhalo), 256, 0, st>>>(tb, p->d_halo, p->nhalo, p->d_halo_stage);
   LAUNCH_CHECK();
   k_halo_scatter<<<nblk(p->nhalo), 256, 0, st>>>(tb, p->d_halo, p->nhalo, p->d_halo_stage);
@@ -280,18 +311,33 @@ int launch_halo(famrdp_plan* p, hipStream_t st, const BlockDesc* table = nullptr
   return FAMRDP_OK;
 }
 
-// BC faces in Face order; with `snapshot`, the inner layers of isothermal
-// faces are saved just before each face is applied (for the reverse sweep).
-int launch_bc(famrdp_plan* p, hipStream_t st, const BlockDesc* table = nullptr, bool snapshot = false) {
-  const BlockDesc* tb = table ? table : p->d_blocks;
+// The BC faces in Face order, on their own.
+int launch_bc(famrdp_plan* p, hipStream_t st) {
   for (int f = 0; f < 6; ++f) {
     if (p->nbc[f] == 0) continue;
     dim3 grid(nblk(p->bc_maxcells[f]), (unsigned)p->nbc[f]);
-    if (snapshot) {
-      k_bc_snapshot<<<grid, 256, 0, st>>>(tb, p->d_bc[f], p->ghost, p->d_bc_snap[f], p->bc_maxcells[f]);
-      LAUNCH_CHECK();
-    }
-    k_bc_face<<<grid, 256, 0, st>>>(tb, p->d_bc[f], p->ghost, p->gas.gamma, p->gas.R);
+    k_bc_face<<<grid, 256, 0, st>>>(p->d_blocks, p->d_bc[f], p->ghost, p->gas.gamma, p->gas.R);
+    LAUNCH_CHECK();
+  }
+  return FAMRDP_OK;
+}
+
+// Halo exchange and BCs of a step (workspace plans); with `snapshot`, the
+// inner layers of isothermal faces are recorded as each face finds them (for
+// the reverse sweep).
+int launch_ghosts(famrdp_plan* p, hipStream_t st, const BlockDesc* tb, bool snapshot = false) {
+  const int nsnap = snapshot ? p->nsnaps : 0;
+  const int n1 = p->nghost_direct + p->nghost_staged + nsnap, n2 = p->nghost_staged + p->nghost_late;
+  SnapPtrs snap{};
+  for (int f = 0; f < 6; ++f) snap.face[f] = p->d_bc_snap[f];
+  if (n1 > 0) {
+    k_ghost_first<<<nblk(n1), 256, 0, st>>>(tb, p->d_ghost, p->nghost_direct, p->nghost_staged, p->d_chains, p->d_ops,
+                                            p->gas.gamma, p->gas.R, p->d_ghost_stage, p->d_snaps, nsnap, snap);
+    LAUNCH_CHECK();
+  }
+  if (n2 > 0) {
+    k_ghost_second<<<nblk(n2), 256, 0, st>>>(tb, p->d_ghost + p->nghost_direct, p->nghost_staged, p->nghost_late,
+                                             p->d_chains, p->d_ops, p->gas.gamma, p->gas.R, p->d_ghost_stage);
     LAUNCH_CHECK();
   }
   return FAMRDP_OK;
@@ -364,9 +410,7 @@ int launch_stages(famrdp_plan* p, double dt, int flags, hipStream_t st, bool adj
 }
 
 int run_step(famrdp_plan* p, double dt, int flags, hipStream_t st) {
-  int rc = launch_halo(p, st);
-  if (rc) return rc;
-  rc = launch_bc(p, st);
+  const int rc = launch_ghosts(p, st, p->d_blocks);
   if (rc) return rc;
   return launch_stages(p, dt, flags, st);
 }
@@ -559,35 +603,17 @@ int famrdp_plan_destroy(famrdp_plan* p) {
   if (p->graph) (void)hipGraphDestroy(p->graph);
   if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
   for (auto* x : p->adj_bufs) (void)hipFree(x);
-  if (p->d_blocks_adj) (void)hipFree(p->d_blocks_adj);
-  if (p->d_sweep_ik) (void)hipFree(p->d_sweep_ik);
-  if (p->d_sweep_j) (void)hipFree(p->d_sweep_j);
-  if (p->d_sweep_v) (void)hipFree(p->d_sweep_v);
-  if (p->d_halo_sorted) (void)hipFree(p->d_halo_sorted);
-  if (p->d_halo_src) (void)hipFree(p->d_halo_src);
-  if (p->d_halo_S) (void)hipFree(p->d_halo_S);
-  for (int f = 0; f < 6; ++f) {
-    if (p->d_bc_snap[f]) (void)hipFree(p->d_bc_snap[f]);
-    if (p->d_bc_part[f]) (void)hipFree(p->d_bc_part[f]);
-    if (p->d_bc_red[f]) (void)hipFree(p->d_bc_red[f]);
-  }
   for (auto* x : p->q1) (void)hipFree(x);
   for (auto* x : p->q2) (void)hipFree(x);
   for (auto* x : p->G) (void)hipFree(x);
-  for (int f = 0; f < 6; ++f) if (p->d_bc[f]) (void)hipFree(p->d_bc[f]);
-  if (p->d_halo) (void)hipFree(p->d_halo);
-  if (p->d_halo_stage) (void)hipFree(p->d_halo_stage);
-  if (p->d_tiles) (void)hipFree(p->d_tiles);
-  if (p->d_monitor) (void)hipFree(p->d_monitor);
-  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) if (p->d_tiles3[v]) (void)hipFree(p->d_tiles3[v]);
-  if (p->d_blocks) (void)hipFree(p->d_blocks);
+  if (p->d_tables) (void)hipFree(p->d_tables);
   for (int s = 0; s < famrdp_plan::NSTAGE; ++s) {
     if (p->stage_ev[s]) {
       if (p->stage_used[s]) (void)hipEventSynchronize(p->stage_ev[s]);
       (void)hipEventDestroy(p->stage_ev[s]);
     }
-    if (p->h_stage[s]) (void)hipHostFree(p->h_stage[s]);
   }
+  if (p->h_stage[0]) (void)hipHostFree(p->h_stage[0]);   // one allocation for the ring
   delete p;
   return FAMRDP_OK;
 }
@@ -623,6 +649,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^29 or more cells in an adjoint plan"));
     p->N.push_back((int64_t)d[0] * d[1] * d[2]);
   }
+  TableSet tables;
   // workspace and block table
   p->h_blocks.resize(nblocks);
   for (int b = 0; b < nblocks; ++b) {
@@ -673,27 +700,25 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       p->h_blocks[b].qh = a.qh; p->h_blocks[b].la = a.la; p->h_blocks[b].lb = a.lb;
       p->h_blocks[b].l0 = a.l0; p->h_blocks[b].fs = a.fs; p->h_blocks[b].vs = a.vs;
     }
-    if (hipMalloc(&p->d_blocks_adj, sizeof(BlockDesc) * nblocks) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: adjoint block table allocation failed"));
+    tables.scratch(&p->d_blocks_adj, nblocks);
   }
-  if (hipMalloc(&p->d_blocks, sizeof(BlockDesc) * nblocks) != hipSuccess)
-    return cleanup(fail(FAMRDP_E_HIP, "plan_create: block table allocation failed"));
-  for (int s = 0; s < famrdp_plan::NSTAGE; ++s)
-    if (hipHostMalloc(&p->h_stage[s], sizeof(BlockDesc) * nblocks) != hipSuccess ||
-        hipEventCreateWithFlags(&p->stage_ev[s], hipEventDisableTiming) != hipSuccess)
+  tables.scratch(&p->d_blocks, nblocks);
+  if (hipHostMalloc(&p->h_stage[0], sizeof(BlockDesc) * nblocks * famrdp_plan::NSTAGE) != hipSuccess)
+    return cleanup(fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed"));
+  for (int s = 0; s < famrdp_plan::NSTAGE; ++s) {
+    p->h_stage[s] = p->h_stage[0] + (size_t)s * nblocks;
+    if (hipEventCreateWithFlags(&p->stage_ev[s], hipEventDisableTiming) != hipSuccess)
       return cleanup(fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed"));
-  // halo gather table
-  std::vector<HaloEntry> halo;
-  rc = build_halo_table(p, ncut, cuts, halo);
-  if (rc) return cleanup(rc);
-  p->nhalo = (int)halo.size();
-  if (p->nhalo > 0) {
-    if (hipMalloc(&p->d_halo, sizeof(HaloEntry) * halo.size()) != hipSuccess ||
-        hipMalloc(&p->d_halo_stage, sizeof(double) * 5 * halo.size()) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: halo table allocation failed"));
-    if (hipMemcpy(p->d_halo, halo.data(), sizeof(HaloEntry) * halo.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: halo table upload failed"));
   }
+  // halo gather table
+  GhostTable ghosts(ghost, nblocks, dims);
+  rc = add_cuts(p, ncut, cuts, ghosts);
+  if (rc) return cleanup(rc);
+  std::vector<HaloEntry> halo;
+  ghosts.halo(halo);
+  p->nhalo = (int)halo.size();
+  tables.table(&p->d_halo, halo);
+  tables.scratch(&p->d_halo_stage, 5 * halo.size());
   // BC tables grouped by face (Face order, dispatch.py:15)
   std::vector<BcEntry> byface[6];
   for (int i = 0; i < nbc; ++i) {
@@ -718,10 +743,21 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       if (!replaced) uniq.push_back(e);
     }
     p->nbc[f] = (int)uniq.size();
-    if (uniq.empty()) continue;
-    if (hipMalloc(&p->d_bc[f], sizeof(BcEntry) * uniq.size()) != hipSuccess ||
-        hipMemcpy(p->d_bc[f], uniq.data(), sizeof(BcEntry) * uniq.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: bc table upload failed"));
+    byface[f] = uniq;
+    tables.table(&p->d_bc[f], uniq);
+  }
+  if (p->has_workspace) {   // exchange and BCs of a step in one table
+    ghosts.boundary(byface, p->bc_maxcells, p->has_adjoint);
+    ghosts.finish();
+    p->nghost_direct = ghosts.ndirect;
+    p->nghost_staged = ghosts.nstaged;
+    p->nghost_late = ghosts.nlate;
+    p->nsnaps = (int)ghosts.snaps.size();
+    tables.table(&p->d_ghost, ghosts.entries);
+    tables.table(&p->d_chains, ghosts.chains);
+    tables.table(&p->d_ops, ghosts.ops);
+    tables.table(&p->d_snaps, ghosts.snaps);
+    tables.scratch(&p->d_ghost_stage, 5 * (size_t)ghosts.nstaged);
   }
   if (p->has_adjoint) {
     if (p->nhalo > 0) {
@@ -736,21 +772,16 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
         us.back().count++;
       }
       p->nhalo_src = (int)us.size();
-      if (hipMalloc(&p->d_halo_sorted, sizeof(HaloEntry) * sorted.size()) != hipSuccess ||
-          hipMalloc(&p->d_halo_src, sizeof(HaloSrc) * us.size()) != hipSuccess ||
-          hipMalloc(&p->d_halo_S, sizeof(double) * 5 * us.size()) != hipSuccess ||
-          hipMemcpy(p->d_halo_sorted, sorted.data(), sizeof(HaloEntry) * sorted.size(), hipMemcpyHostToDevice) !=
-              hipSuccess ||
-          hipMemcpy(p->d_halo_src, us.data(), sizeof(HaloSrc) * us.size(), hipMemcpyHostToDevice) != hipSuccess)
-        return cleanup(fail(FAMRDP_E_HIP, "plan_create: adjoint halo table failed"));
+      tables.table(&p->d_halo_sorted, sorted);
+      tables.table(&p->d_halo_src, us);
+      tables.scratch(&p->d_halo_S, 5 * us.size());
     }
     for (int f = 0; f < 6; ++f) {
       if (p->nbc[f] == 0) continue;
       const size_t n = (size_t)p->nbc[f] * 5 * (size_t)p->bc_maxcells[f];
-      if (hipMalloc(&p->d_bc_snap[f], sizeof(double) * n * p->ghost) != hipSuccess ||
-          hipMalloc(&p->d_bc_part[f], sizeof(double) * n) != hipSuccess ||
-          hipMalloc(&p->d_bc_red[f], sizeof(double) * p->nbc[f] * 5 * BC_RED_PARTS) != hipSuccess)
-        return cleanup(fail(FAMRDP_E_HIP, "plan_create: adjoint BC buffers failed"));
+      tables.scratch(&p->d_bc_snap[f], n * p->ghost);
+      tables.scratch(&p->d_bc_part[f], n);
+      tables.scratch(&p->d_bc_red[f], (size_t)p->nbc[f] * 5 * BC_RED_PARTS);
     }
   }
   // tile table for the batched launches
@@ -758,9 +789,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   for (int b = 0; b < nblocks; ++b)
     for (int64_t s = 0; s < p->N[b]; s += 256) tiles.push_back(Tile{b, (int32_t)s});
   p->ntiles = (int)tiles.size();
-  if (hipMalloc(&p->d_tiles, sizeof(Tile) * tiles.size()) != hipSuccess ||
-      hipMemcpy(p->d_tiles, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice) != hipSuccess)
-    return cleanup(fail(FAMRDP_E_HIP, "plan_create: tile table upload failed"));
+  tables.table(&p->d_tiles, tiles);
   for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
     int TI, TJ, TK;
     tile_dims(v, TI, TJ, TK);
@@ -782,15 +811,12 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
           for (int k = 0; k < d[2]; k += TK) tiles3.push_back(Tile3{b, i, j, k});
     }
     p->ntiles3[v] = (int)tiles3.size();
-    if (hipMalloc(&p->d_tiles3[v], sizeof(Tile3) * tiles3.size()) != hipSuccess ||
-        hipMemcpy(p->d_tiles3[v], tiles3.data(), sizeof(Tile3) * tiles3.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: tile table upload failed"));
+    tables.table(&p->d_tiles3[v], tiles3);
   }
   int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) == hipSuccess) ncu = prop.multiProcessorCount;
-  }
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    ncu = 256;
   p->persistent_grid = std::min(p->ntiles, ncu * 8);
   p->ncu = ncu;
   if (p->has_adjoint) {
@@ -811,14 +837,11 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
     int* cnt[3] = {&p->nsweep_ik, &p->nsweep_j, &p->nsweep_v};
     for (int t = 0; t < 3; ++t) {
       *cnt[t] = (int)tabs[t].size();
-      const size_t bytes = sizeof(SweepTile) * tabs[t].size();
-      if (hipMalloc(dst[t], bytes) != hipSuccess ||
-          hipMemcpy(*dst[t], tabs[t].data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
-        return cleanup(fail(FAMRDP_E_HIP, "plan_create: sweep table upload failed"));
+      tables.table(dst[t], tabs[t]);
     }
   }
-  if (hipMalloc(&p->d_monitor, sizeof(double) * p->persistent_grid) != hipSuccess)
-    return cleanup(fail(FAMRDP_E_HIP, "plan_create: monitor buffer allocation failed"));
+  tables.scratch(&p->d_monitor, p->persistent_grid);
+  if (!tables.make(&p->d_tables)) return cleanup(fail(FAMRDP_E_HIP, "plan_create: table upload failed"));
   *out = p;
   return FAMRDP_OK;
 }
@@ -955,9 +978,7 @@ int step_vjp_impl(famrdp_plan* p, double* const* q_start, const double* const* q
     rc = copy_blocks(p, st, [&](int b) { return p->h_blocks_adj[b].qh; }, [&](int b) { return q_start[b]; });
     if (rc) return rc;
   }
-  rc = launch_halo(p, st, p->d_blocks_adj);
-  if (rc) return rc;
-  rc = launch_bc(p, st, p->d_blocks_adj, true);
+  rc = launch_ghosts(p, st, p->d_blocks_adj, true);
   if (rc) return rc;
   if (!q1s) {
     rc = launch_stages(p, dt, flags & ~FAMRDP_VJP_CONSUME_START, st, true, 2);

@@ -53,6 +53,11 @@ struct BcEntry {
   double q_inf[5];
 };
 
+// Where the reverse sweep's recorded boundary values of each face go.
+struct SnapPtrs {
+  double* face[6];
+};
+
 // Work tile of the batched (multi-block) launches: `len` consecutive cells of
 // block `block` starting at flat cell index `start`.
 struct Tile {

@@ -8,6 +8,7 @@
 //   * halo gather/scatter (pre-exchange semantics) and ghost-cell BC faces;
 //   * grid metrics and the CFL / positivity reduction.
 #include "famrdp_kernels.h"
+#include "famrdp_ghost.h"
 #include "famrdp_tiles.h"
 
 namespace famrdp {
@@ -344,8 +345,9 @@ __global__ void k_halo_scatter(const BlockDesc* __restrict__ blocks, const HaloE
 }
 
 // ---------------------------------------------------------------------------
-// Ghost-cell BCs (physics/bc/*.py).  One launch per face index (Face order),
-// covering that face of every block that has a BC there; blockIdx.y = entry.
+// Ghost-cell BCs on their own (physics/bc/*.py).  One launch per face index
+// (Face order), covering that face of every block that has a BC there;
+// blockIdx.y = entry.
 // ---------------------------------------------------------------------------
 
 __global__ void k_bc_face(const BlockDesc* __restrict__ blocks, const BcEntry* __restrict__ entries, int ghost,
@@ -353,51 +355,98 @@ __global__ void k_bc_face(const BlockDesc* __restrict__ blocks, const BcEntry* _
   const BcEntry e = entries[blockIdx.y];
   const BlockDesc b = blocks[e.block];
   const int ax = e.face / 2;            // 0: i, 1: j, 2: k
-  const bool lo = (e.face % 2) == 0;
-  const int n[3] = {b.ni, b.nj, b.nk};
-  const int64_t st[3] = {(int64_t)b.nj * b.nk, b.nk, 1};
-  const int t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
-  const int64_t ncell = (int64_t)n[t1] * n[t2];
+  const int na = ax == 0 ? b.ni : (ax == 1 ? b.nj : b.nk);
+  const int64_t sj = b.nk, si = (int64_t)b.nj * b.nk;
+  const int64_t sa = ax == 0 ? si : (ax == 1 ? sj : (int64_t)1);
+  const int n1 = ax == 0 ? b.nj : b.ni, n2 = ax == 2 ? b.nj : b.nk;
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= ncell) return;
-  const int a = (int)(t / n[t2]), c2 = (int)(t % n[t2]);
-  const int64_t base = a * st[t1] + c2 * st[t2];
-  const int na = n[ax];
+  if (t >= (int64_t)n1 * n2) return;
+  const int64_t base = (t / n2) * (ax == 0 ? sj : si) + (t % n2) * (ax == 2 ? sj : (int64_t)1);
   for (int gl = 0; gl < ghost; ++gl) {
-    // bc/base.py:21-33 mirror pairs; extrapolation reads the first interior layer
-    const int outer = lo ? gl : na - 1 - gl;
-    int inner = lo ? 2 * ghost - 1 - gl : na - 2 * ghost + gl;
-    if (e.kind == BC_EXTRAPOLATE) inner = lo ? ghost : na - 1 - ghost;
-    const int64_t co = base + outer * st[ax], ci = base + inner * st[ax];
-    double qi[5], qo[5];
-    for (int v = 0; v < 5; ++v) qi[v] = b.q[v * b.N + ci];
-    switch (e.kind) {
-      case BC_WALL_ADIABATIC:
-        qo[0] = qi[0]; qo[1] = -qi[1]; qo[2] = -qi[2]; qo[3] = -qi[3]; qo[4] = qi[4];
-        break;
-      case BC_WALL_ISOTHERMAL: {   // bc/wall.py:35-58
-        const double rho_i = qi[0];
-        const double ke_i = 0.5 * (qi[1] * qi[1] + qi[2] * qi[2] + qi[3] * qi[3]) / rho_i;
-        const double p_g = (gamma - 1.0) * (qi[4] - ke_i);
-        const double rho_g = p_g / (R * e.T_wall);
-        const double scale = rho_g / rho_i;
-        const double mu = -qi[1] * scale, mv = -qi[2] * scale, mw = -qi[3] * scale;
-        const double ke_g = 0.5 * (mu * mu + mv * mv + mw * mw) / rho_g;
-        qo[0] = rho_g; qo[1] = mu; qo[2] = mv; qo[3] = mw; qo[4] = p_g / (gamma - 1.0) + ke_g;
-        break;
-      }
-      case BC_MIRROR_NORMAL:
-        for (int v = 0; v < 5; ++v) qo[v] = (v == ax + 1) ? qi[v] * -1.0 : qi[v] * 1.0;
-        break;
-      case BC_FARFIELD:
-        for (int v = 0; v < 5; ++v) qo[v] = e.q_inf[v] * 1.0;
-        break;
-      default:  // BC_EXTRAPOLATE
-        for (int v = 0; v < 5; ++v) qo[v] = qi[v];
-        break;
-    }
-    for (int v = 0; v < 5; ++v) b.q[v * b.N + co] = qo[v];
+    int outer, inner;
+    bc_pair(e, ghost, na, gl, outer, inner);
+    const int64_t co = base + outer * sa, ci = base + inner * sa;
+    double q[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = b.q[v * b.N + ci];
+    bc_apply(e, gamma, R, q);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) b.q[v * b.N + co] = q[v];
   }
+}
+
+// ---------------------------------------------------------------------------
+// Ghost cells of a step (famrdp_ghost.h): 20 bytes of table and 80 of state an
+// entry, in one launch or two, where the exchange and the faces one after the
+// other were up to eight (55 x 55 x 15 free stream all around: 36 us, now 4).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void ghost_value(const BlockDesc* __restrict__ blocks, const GhostChain* __restrict__ chains,
+                                            const BcEntry* __restrict__ ops, int sb, int sc, int chain, double gamma,
+                                            double R, double q[5]) {
+  if (sb >= 0) {
+    const BlockDesc& s = blocks[sb];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = s.q[v * s.N + sc];
+  } else {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = 0.0;   // replaced by the chain's free stream
+  }
+  if (chain > 0) {
+    const GhostChain& c = chains[chain];
+    for (int i = 0; i < c.n; ++i) bc_apply(ops[c.op[i]], gamma, R, q);
+  }
+}
+
+// Direct entries, then the staged ones into the staging buffer, then the
+// recorded values.
+__global__ void __launch_bounds__(256) k_ghost_first(const BlockDesc* __restrict__ blocks,
+                                                     const GhostEntry* __restrict__ e, int ndirect, int nstaged,
+                                                     const GhostChain* __restrict__ chains,
+                                                     const BcEntry* __restrict__ ops, double gamma, double R,
+                                                     double* __restrict__ stage, const GhostSnap* __restrict__ snaps,
+                                                     int nsnap, SnapPtrs snap) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  double q[5];
+  if (t < ndirect + nstaged) {
+    const GhostEntry h = e[t];
+    ghost_value(blocks, chains, ops, h.sb, h.sc, h.chain, gamma, R, q);
+    if (t < ndirect) {
+      const BlockDesc& b = blocks[h.tb];
+#pragma unroll
+      for (int v = 0; v < 5; ++v) b.q[v * b.N + h.tc] = q[v];
+    } else {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) stage[(int64_t)v * nstaged + (t - ndirect)] = q[v];
+    }
+  } else if (t < ndirect + nstaged + nsnap) {
+    const GhostSnap h = snaps[t - ndirect - nstaged];
+    ghost_value(blocks, chains, ops, h.sb, h.sc, h.chain, gamma, R, q);
+    double* dst = snap.face[h.face] + h.off;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) dst[v * h.stride] = q[v];
+  }
+}
+
+// The staged entries from the staging buffer, and the direct ones whose target
+// a staged entry or a record had to read first.
+__global__ void __launch_bounds__(256) k_ghost_second(const BlockDesc* __restrict__ blocks,
+                                                      const GhostEntry* __restrict__ e, int nstaged, int nlate,
+                                                      const GhostChain* __restrict__ chains,
+                                                      const BcEntry* __restrict__ ops, double gamma, double R,
+                                                      const double* __restrict__ stage) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nstaged + nlate) return;
+  const GhostEntry h = e[t];
+  double q[5];
+  if (t < nstaged) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = stage[(int64_t)v * nstaged + t];
+  } else {
+    ghost_value(blocks, chains, ops, h.sb, h.sc, h.chain, gamma, R, q);
+  }
+  const BlockDesc& b = blocks[h.tb];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) b.q[v * b.N + h.tc] = q[v];
 }
 
 // ---------------------------------------------------------------------------
