@@ -243,10 +243,12 @@ int upload_table(famrdp_plan* p, BlockDesc* dst, const std::vector<BlockDesc>& s
 // when a pointer changed.
 // q1t / q2t: where the step's stage-1/2 results go (caller arrays), or NULL
 // for the plan's workspace.
-int bind(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol, hipStream_t st,
-         bool need_q = true, double* const* q1t = nullptr, double* const* q2t = nullptr) {
+// Puts the caller's arrays into the host copy of the block table and says
+// whether the plan's table and the reverse sweep's have changed by it.
+int bind_host(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol, bool need_q,
+              double* const* q1t, double* const* q2t, bool& changed, bool& changed_adj) {
   if (need_q && !q) return fail(FAMRDP_E_INVALID, "q pointer array is NULL");
-  bool changed = !p->blocks_uploaded, changed_adj = !p->blocks_uploaded;
+  changed = changed_adj = !p->blocks_uploaded;
   for (int b = 0; b < p->nblocks; ++b) {
     BlockDesc& d = p->h_blocks[b];
     if (q && !q[b]) return fail(FAMRDP_E_INVALID, "q[" + std::to_string(b) + "] is NULL");
@@ -262,17 +264,29 @@ int bind(famrdp_plan* p, double* const* q, const double* const* kxyz, const doub
     d.q1 = s1;
     d.q2 = s2;
   }
+  return FAMRDP_OK;
+}
+
+int upload_adj(famrdp_plan* p, hipStream_t st) {
+  for (int b = 0; b < p->nblocks; ++b) {
+    BlockDesc a = p->h_blocks[b];
+    a.q = p->h_blocks_adj[b].qh;
+    p->h_blocks_adj[b] = a;
+  }
+  return upload_table(p, p->d_blocks_adj, p->h_blocks_adj, st);
+}
+
+int bind(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol, hipStream_t st,
+         bool need_q = true, double* const* q1t = nullptr, double* const* q2t = nullptr) {
+  bool changed, changed_adj;
+  int rc = bind_host(p, q, kxyz, vol, need_q, q1t, q2t, changed, changed_adj);
+  if (rc) return rc;
   if (changed) {
-    int rc = upload_table(p, p->d_blocks, p->h_blocks, st);
+    rc = upload_table(p, p->d_blocks, p->h_blocks, st);
     if (rc) return rc;
   }
   if (p->has_adjoint && changed_adj) {
-    for (int b = 0; b < p->nblocks; ++b) {
-      BlockDesc a = p->h_blocks[b];
-      a.q = p->h_blocks_adj[b].qh;
-      p->h_blocks_adj[b] = a;
-    }
-    int rc = upload_table(p, p->d_blocks_adj, p->h_blocks_adj, st);
+    rc = upload_adj(p, st);
     if (rc) return rc;
   }
   p->blocks_uploaded = true;
@@ -1094,6 +1108,37 @@ int famrdp_step(famrdp_plan* p, double* const* q, const double* const* kxyz, con
   return run_step(p, dt, flags, S(stream));
 }
 
+int famrdp_step_from(famrdp_plan* p, const double* const* q_in, double* const* q, const double* const* kxyz,
+                     const double* const* vol, double dt, int32_t flags, void* stream) {
+  if (!p || !q_in || !kxyz || !vol) return fail(FAMRDP_E_INVALID, "step_from: NULL plan or pointer arrays");
+  if (!p->has_workspace) return fail(FAMRDP_E_INVALID, "step_from: plan was created without stage workspace");
+  for (int b = 0; b < p->nblocks; ++b)
+    if (!q_in[b] || !kxyz[b] || !vol[b] || (q && q_in[b] == q[b]))
+      return fail(FAMRDP_E_INVALID, "step_from: NULL q_in/kxyz/vol or q_in the same array as q for block " +
+                                        std::to_string(b));
+  hipStream_t st = S(stream);
+  bool changed, changed_adj;
+  int rc = bind_host(p, q, kxyz, vol, true, nullptr, nullptr, changed, changed_adj);
+  if (rc) return rc;
+  p->blocks_uploaded = false;
+  if (p->has_adjoint && changed_adj && (rc = upload_adj(p, st))) return rc;
+  for (int b0 = 0; b0 < p->nblocks; b0 += STEP_START_BLOCKS) {
+    const int n = std::min(STEP_START_BLOCKS, p->nblocks - b0);
+    StepStart ss{};
+    int64_t most = 0;
+    for (int b = 0; b < n; ++b) {
+      ss.block[b] = p->h_blocks[b0 + b];
+      ss.src[b] = q_in[b0 + b];
+      most = std::max(most, p->N[b0 + b]);
+    }
+    // four 16-byte accesses per thread, until the chip is full
+    const int gx = (int)std::min<int64_t>((5 * most + 2047) / 2048, 4096);
+    k_step_start<<<dim3(gx, n), 256, 0, st>>>(ss, p->d_blocks + b0);
+    LAUNCH_CHECK();
+  }
+  p->blocks_uploaded = true;
+  return run_step(p, dt, flags, st);
+}
 int famrdp_step_stages(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol,
                        double dt, int32_t flags, double* const* q1_out, double* const* q2_out, void* stream) {
   if (!p || !kxyz || !vol || !q1_out || !q2_out) return fail(FAMRDP_E_INVALID, "step_stages: NULL plan or pointer arrays");

@@ -65,6 +65,8 @@ SIGNATURES = {
                             ctypes.POINTER(Bc), ctypes.POINTER(Gas), i32, i32, i32], i32),
     "famrdp_plan_destroy": ([vp], i32),
     "famrdp_step": ([vp, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp), f64, i32, vp], i32),
+    "famrdp_step_from": ([vp, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp), f64, i32,
+                          vp], i32),
     "famrdp_step_graph": ([vp, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp), f64, i32, i32, vp], i32),
     "famrdp_step_stages": ([vp, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(vp), f64, i32, ctypes.POINTER(vp),
                             ctypes.POINTER(vp), vp], i32),
@@ -147,6 +149,9 @@ def require_gpu():
 def device_f64(x):
     """Contiguous float64 tensor on the current GPU (copies host data in)."""
     torch = _torch()
+    if isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.float64 and x.is_contiguous() and \
+            x.device.index == torch.cuda.current_device():
+        return x            # what the conversions below return for it, without their 2 us
     require_gpu()
     if isinstance(x, torch.Tensor):
         if x.dtype != torch.float64:

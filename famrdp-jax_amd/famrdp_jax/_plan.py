@@ -9,10 +9,16 @@ from . import _lib as L
 from .core.constants import BCType, Face
 
 BC_WALL_ADIABATIC, BC_WALL_ISOTHERMAL, BC_MIRROR_NORMAL, BC_FARFIELD, BC_EXTRAPOLATE = range(5)
+_FACES = tuple(Face)                           # plain tuples and ints: looking an enum member up costs 0.1-0.3 us,
+_CUT1TO1, _WALL, _SYMMETRY, _FARFIELD, _OUTFLOW = (  # and a functional step asks for every face of every block
+    int(t) for t in (BCType.CUT1TO1, BCType.WALL, BCType.SYMMETRY, BCType.FARFIELD, BCType.OUTFLOW))
 DEFAULT_Q_INF = (1.0, 0.0, 0.0, 0.0, 2.5)      # physics/bc/dispatch.py:30
 
 
 def _bct(topo, face):
+    v = topo.bc_type.get(face)      # Face members and plain ints are the same key
+    if v is not None:
+        return int(v)
     for k, v in topo.bc_type.items():
         if int(k) == int(face):
             return int(v)
@@ -20,6 +26,9 @@ def _bct(topo, face):
 
 
 def _params(bc_params, face):
+    v = bc_params.get(face)
+    if v is not None:
+        return v
     for k, v in bc_params.items():
         if int(k) == int(face):
             return v
@@ -30,6 +39,8 @@ def _floats(x):
     try:
         import torch
         if isinstance(x, torch.Tensor):
+            if x.dim() == 1 and x.dtype == torch.float64:
+                return tuple(x.tolist())
             return tuple(float(v) for v in x.detach().cpu().reshape(-1).tolist())
     except ImportError:  # pragma: no cover
         pass
@@ -44,7 +55,7 @@ def cuts_from_topology(topos):
     cuts = []
     for i, topo in enumerate(topos):
         for face, info in topo.neighbors.items():
-            if info is None or _bct(topo, face) != int(BCType.CUT1TO1):
+            if info is None or _bct(topo, face) != _CUT1TO1:
                 continue
             nb_id, src_face, orient = info
             cuts.append((i, int(face), id_to_idx[nb_id], int(src_face), int(orient)))
@@ -57,21 +68,21 @@ def bcs_from_config(topos, bc_params, ghost_unused=None):
     ``{"extrapolate": True}`` selects the extrapolation extension."""
     out = []
     for b, topo in enumerate(topos):
-        for face in Face:
+        for face in _FACES:
             bct = _bct(topo, face)
-            if bct is None or bct == int(BCType.CUT1TO1):
+            if bct is None or bct == _CUT1TO1:
                 continue
             p = _params(bc_params, face)
-            if bct == int(BCType.WALL):
+            if bct == _WALL:
                 if p.get("wall_type", "adiabatic") == "isothermal":
                     out.append((b, int(face), BC_WALL_ISOTHERMAL, float(p.get("T_wall", 300.0)), DEFAULT_Q_INF))
                 else:
                     out.append((b, int(face), BC_WALL_ADIABATIC, 0.0, DEFAULT_Q_INF))
-            elif bct == int(BCType.SYMMETRY):
+            elif bct == _SYMMETRY:
                 out.append((b, int(face), BC_MIRROR_NORMAL, 0.0, DEFAULT_Q_INF))
-            elif bct == int(BCType.FARFIELD):
+            elif bct == _FARFIELD:
                 out.append((b, int(face), BC_FARFIELD, 0.0, _floats(p.get("q_inf", DEFAULT_Q_INF))))
-            elif bct == int(BCType.OUTFLOW) and p.get("extrapolate", False):
+            elif bct == _OUTFLOW and p.get("extrapolate", False):
                 out.append((b, int(face), BC_EXTRAPOLATE, 0.0, DEFAULT_Q_INF))
     return out
 
@@ -125,6 +136,11 @@ class Plan:
         else:
             L.check(self._lib.famrdp_step(self._h, self._ptrs(qs), self._ptrs(kxyzs), self._ptrs(vols), float(dt),
                                           flags, L.stream()))
+
+    def step_from(self, srcs, qs, kxyzs, vols, dt, *, batched=False):
+        """One step from the device tensors ``srcs`` (unchanged) into ``qs``."""
+        L.check(self._lib.famrdp_step_from(self._h, self._ptrs(srcs), self._ptrs(qs), self._ptrs(kxyzs),
+                                           self._ptrs(vols), float(dt), 1 if batched else 0, L.stream()))
 
     def autotune(self, qs, kxyzs, vols, dt, *, batched=False, reps=3):
         """Time every stage-kernel variant (tile shapes of the fused kernel and
@@ -182,16 +198,18 @@ class Plan:
         L.check(self._lib.famrdp_plan_set_block_params(self._h, arr(mu0), arr(dt_scale)))
 
     def check_state(self, qs, out):
-        """Enqueue the state monitor: out (device tensor, >= 1 double) gets the
-        number of bad interior cells over all blocks."""
+        """Enqueue the state monitor: out (device or pinned tensor, >= 1 double)
+        gets the number of bad interior cells over all blocks."""
         L.check(self._lib.famrdp_plan_check_state(self._h, self._ptrs(qs), L.ptr(out), L.stream()))
 
     def raise_if_bad(self, qs):
         """Config.nan_check: monitor the state and raise FloatingPointError if
         any interior cell is non-finite or has rho <= 0 or p <= 0."""
+        # the count lands in pinned host memory: no copy to wait for behind the kernel
         torch = L._torch()
-        out = torch.empty(1, dtype=torch.float64, device="cuda")
+        out = torch.empty(1, dtype=torch.float64, pin_memory=True)
         self.check_state(qs, out)
+        torch.cuda.current_stream().synchronize()
         nbad = int(out.item())
         if nbad:
             raise FloatingPointError(f"nan_check: {nbad} interior cells are non-finite or have rho <= 0 or p <= 0")

@@ -137,6 +137,11 @@ int famrdp_plan_destroy(famrdp_plan* plan);
  * in place on q[b].  Pointer arrays have nblocks entries (host memory). */
 int famrdp_step(famrdp_plan* plan, double* const* q, const double* const* kxyz, const double* const* vol, double dt,
                 int32_t flags, void* stream);
+/* famrdp_step from q_in[b] (left as it is) into q[b] (another array of the
+ * same size): the functional form, which copies every block and binds the
+ * pointers in one launch.  Same bits as a copy and famrdp_step. */
+int famrdp_step_from(famrdp_plan* plan, const double* const* q_in, double* const* q, const double* const* kxyz,
+                     const double* const* vol, double dt, int32_t flags, void* stream);
 /* nsteps steps replayed from a hipGraph captured for these pointers, dt and
  * flags (captured on first use, re-captured when any of them changes). */
 int famrdp_step_graph(famrdp_plan* plan, double* const* q, const double* const* kxyz, const double* const* vol,
