@@ -6,8 +6,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -85,25 +87,35 @@ int cfl_scratch(double** ptr) {
 // whatever its size, and a plan has about forty such arrays.
 class TableSet {
  public:
+  TableSet() = default;
+  TableSet(const TableSet&) = delete;
+  TableSet& operator=(const TableSet&) = delete;
+  ~TableSet() { std::free(bytes_); }
   template <class T>
   void table(T** dst, const std::vector<T>& src) {   // a device copy of src (none of an empty one)
     if (src.empty()) return;
-    const size_t at = (bytes_.size() + ALIGN - 1) / ALIGN * ALIGN;
-    bytes_.resize(at + sizeof(T) * src.size());
-    std::memcpy(bytes_.data() + at, src.data(), sizeof(T) * src.size());
+    const size_t at = up(len_), end = at + sizeof(T) * src.size();
+    if (end > cap_) {                                // (realloc moves large buffers without a copy)
+      cap_ = std::max(end, 2 * cap_);
+      char* p = static_cast<char*>(std::realloc(bytes_, cap_));
+      if (!p) throw std::bad_alloc();
+      bytes_ = p;
+    }
+    std::memcpy(bytes_ + at, src.data(), sizeof(T) * src.size());
+    len_ = end;
     slots_.push_back({reinterpret_cast<void**>(dst), at, false});
   }
   template <class T>
   void scratch(T** dst, size_t count) {              // not initialised
     if (count == 0) return;
     slots_.push_back({reinterpret_cast<void**>(dst), scratch_, true});
-    scratch_ += (sizeof(T) * count + ALIGN - 1) / ALIGN * ALIGN;
+    scratch_ += up(sizeof(T) * count);
   }
   bool make(char** mem) {
-    const size_t tables = (bytes_.size() + ALIGN - 1) / ALIGN * ALIGN;
+    const size_t tables = up(len_);
     if (tables + scratch_ == 0) return true;
     if (hipMalloc(mem, tables + scratch_) != hipSuccess) return false;
-    if (!bytes_.empty() && hipMemcpy(*mem, bytes_.data(), bytes_.size(), hipMemcpyHostToDevice) != hipSuccess)
+    if (len_ > 0 && hipMemcpy(*mem, bytes_, len_, hipMemcpyHostToDevice) != hipSuccess)
       return false;
     for (const Slot& s : slots_) *s.dst = *mem + (s.scratch ? tables : 0) + s.at;
     return true;
@@ -112,9 +124,10 @@ class TableSet {
  private:
   static constexpr size_t ALIGN = 256;
   struct Slot { void** dst; size_t at; bool scratch; };
-  std::vector<char> bytes_;
+  static size_t up(size_t n) { return (n + ALIGN - 1) / ALIGN * ALIGN; }
+  char* bytes_ = nullptr;
+  size_t len_ = 0, cap_ = 0, scratch_ = 0;
   std::vector<Slot> slots_;
-  size_t scratch_ = 0;
 };
 
 struct famrdp_plan {
@@ -152,7 +165,9 @@ struct famrdp_plan {
   double* d_monitor = nullptr;    // per-workgroup partial counts of the state monitor (persistent_grid)
   Tile3* d_tiles3[NUM_TILE_VARIANTS] = {};
   int ntiles3[NUM_TILE_VARIANTS] = {};
-  int tile_variant = 0;
+  int tile_variant = -1;          // -1: by the blocks' sizes (default_variant)
+  int auto_all = 0;               // then: the variant of launches over all blocks
+  std::vector<int> auto_block;    // and of a block's own launches
   int persistent_grid = 0;
   int ncu = 256;                  // compute units of the device the plan was made on
   // workspace
@@ -366,22 +381,25 @@ hipEvent_t next_event(famrdp_plan* p) {
   return p->ev_pool[p->ev_used++];
 }
 
-// the i-marching variants address a block's arrays with 32-bit byte offsets
+// the i-marching and wide variants address a block's arrays with 32-bit byte offsets
 bool variant_fits(const famrdp_plan* p, int v) {
-  if (!is_march_variant(v)) return true;
+  if (!is_march_variant(v) && !is_wide_variant(v)) return true;
   for (int b = 0; b < p->nblocks; ++b)
     if (!march_fits(p->N[b])) return false;
   return true;
 }
 
+int batched_variant(const famrdp_plan* p) { return p->tile_variant < 0 ? p->auto_all : p->tile_variant; }
+
 int launch_stages(famrdp_plan* p, double dt, int flags, hipStream_t st, bool adj = false, int nstages = 3) {
   const bool direct = (flags & FAMRDP_STEP_DIRECT) != 0;
   const BlockDesc* dtab = adj ? p->d_blocks_adj : p->d_blocks;
   const std::vector<BlockDesc>& htab = adj ? p->h_blocks_adj : p->h_blocks;
+  const int vb = batched_variant(p);
   if (flags & FAMRDP_STEP_BATCHED) {
     // every batched launch indexes a device tile table: refuse to launch without one
     if (!p->d_blocks || (direct ? (!p->d_tiles || p->ntiles < 1)
-                                : (!p->d_tiles3[p->tile_variant] || p->ntiles3[p->tile_variant] < 1)))
+                                : (!p->d_tiles3[vb] || p->ntiles3[vb] < 1)))
       return fail(FAMRDP_E_INVALID, "batched step: tile table missing");
   }
   for (int stage = 1; stage <= nstages; ++stage) {
@@ -390,12 +408,11 @@ int launch_stages(famrdp_plan* p, double dt, int flags, hipStream_t st, bool adj
     if (tm && (!e0 || !e1)) return fail(FAMRDP_E_HIP, "hipEventCreate failed");
     if (tm) HIP_TRY(hipEventRecord(e0, st));
     if (!direct && (flags & FAMRDP_STEP_BATCHED)) {
-      const int v = p->tile_variant;
-      launch_fused_batched(v, dtab, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt, p->ncu, st);
+      launch_fused_batched(vb, dtab, p->d_tiles3[vb], p->ntiles3[vb], stage, p->gas, p->limiter, dt, p->ncu, st);
       LAUNCH_CHECK();
     } else if (!direct) {
       for (int b = 0; b < p->nblocks; ++b) {
-        launch_fused(p->tile_variant, htab[b], stage, p->gas, p->limiter, dt, p->ncu, st);
+        launch_fused(p->tile_variant < 0 ? p->auto_block[b] : p->tile_variant, htab[b], stage, p->gas, p->limiter, dt, p->ncu, st);
         LAUNCH_CHECK();
       }
     } else if (flags & FAMRDP_STEP_BATCHED) {
@@ -833,6 +850,9 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
     ncu = 256;
   p->persistent_grid = std::min(p->ntiles, ncu * 8);
   p->ncu = ncu;
+  p->auto_all = default_variant(nblocks, dims, ncu, variant_fits(p, 18));
+  for (int b = 0; b < nblocks; ++b)
+    p->auto_block.push_back(default_variant(1, &dims[3 * b], ncu, march_fits(p->N[b])));
   if (p->has_adjoint) {
     SweepSet ik{{}, {}, SWEEP_IK}, jj{{}, {}, SWEEP_J}, vv{{}, {}, SWEEP_V};
     for (int b = 0; b < nblocks; ++b) {
@@ -873,8 +893,8 @@ int famrdp_plan_set_tile(famrdp_plan* p, int32_t variant) {
 
 int famrdp_plan_get_tile(const famrdp_plan* p, int32_t* variant, int32_t* dims3) {
   if (!p) return fail(FAMRDP_E_INVALID, "get_tile: plan is NULL");
-  if (variant) *variant = p->tile_variant;
-  if (dims3) tile_dims(p->tile_variant, dims3[0], dims3[1], dims3[2]);
+  if (variant) *variant = batched_variant(p);
+  if (dims3) tile_dims(batched_variant(p), dims3[0], dims3[1], dims3[2]);
   return FAMRDP_OK;
 }
 
@@ -888,21 +908,16 @@ int famrdp_plan_autotune(famrdp_plan* p, double* const* q, const double* const* 
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
-  int best = 0;
-  float best_ms = 1e30f;
-  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
-    if (!variant_fits(p, v)) {
-      if (ms_out) ms_out[v] = 1e30;
-      continue;
-    }
-    // stages 1 and 2 read q (and q1) and write the q1, q2 workspace only: the
-    // state is untouched; stage 2 also reads q0, as stage 3 does
-    for (int r = 0; r <= reps; ++r) {
-      if (r == 1) HIP_TRY(hipEventRecord(e0, st));
+  // ms of one pair of stages 1 and 2 of variant v, over n pairs after `warm`
+  // untimed ones.  They read q (and q1) and
+  // write the q1, q2 workspace only: the state is untouched; stage 2 also
+  // reads q0, as stage 3 does.
+  auto time_pairs = [&](int v, int warm, int n, float& ms) -> int {
+    for (int r = -warm; r < n; ++r) {
+      if (r == 0) HIP_TRY(hipEventRecord(e0, st));
       for (int stage = 1; stage <= 2; ++stage) {
         if (flags & FAMRDP_STEP_BATCHED) {
-          launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt, p->ncu,
-                               st);
+          launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt, p->ncu, st);
         } else {
           for (int b = 0; b < p->nblocks; ++b)
             launch_fused(v, p->h_blocks[b], stage, p->gas, p->limiter, dt, p->ncu, st);
@@ -912,13 +927,34 @@ int famrdp_plan_autotune(famrdp_plan* p, double* const* q, const double* const* 
     }
     HIP_TRY(hipEventRecord(e1, st));
     HIP_TRY(hipEventSynchronize(e1));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-    ms /= reps;
-    if (ms_out) ms_out[v] = ms;
+    float t = 0.f;
+    HIP_TRY(hipEventElapsedTime(&t, e0, e1));
+    ms = t / n;
+    return FAMRDP_OK;
+  };
+  // one timed pair each (after an untimed one), then the rest of the pairs for
+  // those within 1.5 of the best
+  float ms[NUM_TILE_VARIANTS], first = 1e30f;
+  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
+    ms[v] = 1e30f;
+    if (!variant_fits(p, v)) continue;
+    rc = time_pairs(v, 1, 1, ms[v]);
+    if (rc) return rc;
+    first = std::min(first, ms[v]);
+  }
+  int best = 0;
+  float best_ms = 1e30f;
+  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
+    if (reps > 1 && ms[v] <= 1.5f * first) {
+      float rest = 0.f;
+      rc = time_pairs(v, 0, reps - 1, rest);
+      if (rc) return rc;
+      ms[v] = (ms[v] + rest * (reps - 1)) / reps;
+    }
+    if (ms_out) ms_out[v] = variant_fits(p, v) ? ms[v] : 1e30;
     // ties (within 1.5 %: stages 1 and 2 rank variants that close only to
     // about that) keep the earlier variant
-    if (ms < best_ms * 0.985f) { best_ms = ms; best = v; }
+    if (ms[v] < best_ms * 0.985f) { best_ms = ms[v]; best = v; }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

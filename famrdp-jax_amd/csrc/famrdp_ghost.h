@@ -18,8 +18,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <map>
-#include <utility>
 #include <vector>
 
 #include "famrdp_kernels.h"
@@ -116,9 +114,11 @@ struct GhostShell {
     for (int i = 0; i < n[0]; ++i)
       for (int j = 0; j < n[1]; ++j) {
         const bool whole = layer(i, n[0], g) >= 0 || layer(j, n[1], g) >= 0;
+        const int32_t row = (int32_t)(((int64_t)i * n[1] + j) * n[2]);
+        int64_t s = index(i, j, 0);           // numbers run along a row
         for (int k = 0; k < n[2]; ++k) {
           if (!whole && k == g && n[2] > 2 * g) k = n[2] - g;
-          f((int32_t)(((int64_t)i * n[1] + j) * n[2] + k), index(i, j, k));
+          f(row + k, s++);
         }
       }
   }
@@ -130,6 +130,7 @@ struct GhostShell {
 struct GhostTable {
   struct Val {
     int32_t sb, sc, chain;   // chain -1: untouched
+    int32_t ss;              // the source's number in its block's shell, -1 for an interior cell
   };
   int ghost;
   std::vector<GhostShell> shell;
@@ -139,23 +140,28 @@ struct GhostTable {
   std::vector<GhostEntry> entries;         // [direct | staged | late direct]
   int ndirect = 0, nstaged = 0, nlate = 0;
   std::vector<GhostSnap> snaps;
+  std::vector<int32_t> snap_ss;            // Val::ss of the recorded values
 
   GhostTable(int ghost_, int nblocks, const int32_t* dims) : ghost(ghost_) {
     chains.push_back(GhostChain{0, {0, 0, 0, 0, 0, 0}});
     for (int b = 0; b < nblocks; ++b) {
       shell.emplace_back(ghost, dims + 3 * b);
-      val.emplace_back((size_t)shell[b].size, Val{0, 0, -1});
+      val.emplace_back((size_t)shell[b].size, Val{0, 0, -1, -1});
     }
   }
 
   // the exchange's copy of cell sc of block sb to the ghost cell (i, j, k) of
   // block tb; a later copy wins
   void copy(int tb, int i, int j, int k, int sb, int32_t sc) {
-    val[tb][(size_t)shell[tb].index(i, j, k)] = Val{sb, sc, 0};
+    val[tb][(size_t)shell[tb].index(i, j, k)] = Val{sb, sc, 0, (int32_t)shell[sb].index_of(sc)};
   }
 
   // The exchange's final copies, ordered by target.
   void halo(std::vector<HaloEntry>& out) const {
+    size_t n = 0;
+    for (const auto& vals : val)
+      for (const Val& v : vals) n += v.chain >= 0;
+    out.reserve(n);
     for (int b = 0; b < (int)shell.size(); ++b)
       shell[b].each([&](int32_t c, int64_t s) {
         const Val& v = val[b][(size_t)s];
@@ -166,13 +172,20 @@ struct GhostTable {
   // The boundary conditions, in order; with `snap`, the inner layers of
   // isothermal faces as they are when the face is applied.
   void boundary(const std::vector<BcEntry> (&bc)[6], const int64_t (&maxcells)[6], bool snap) {
-    std::map<std::pair<int32_t, int32_t>, int32_t> longer;   // (chain, op) -> chain
+    size_t nsnap = 0;
+    for (int f = 0; f < 6; ++f)
+      for (const BcEntry& op : bc[f])
+        if (snap && op.kind == BC_WALL_ISOTHERMAL) nsnap += (size_t)(ghost * maxcells[f]);
+    snaps.reserve(nsnap);
+    snap_ss.reserve(nsnap);
+    std::vector<int32_t> longer;   // chain -> that chain and the operation at hand, -1: not made yet
     for (int f = 0; f < 6; ++f) {
       const int ax = f / 2, t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
       for (size_t e = 0; e < bc[f].size(); ++e) {
         const BcEntry& op = bc[f][e];
         const int32_t iop = (int32_t)ops.size();
         ops.push_back(op);
+        longer.assign(chains.size(), -1);
         const GhostShell& sh = shell[op.block];
         auto& vals = val[op.block];
         int x[3];
@@ -184,21 +197,24 @@ struct GhostTable {
               x[ax] = inner;
               const int32_t ci = (int32_t)(((int64_t)x[0] * sh.n[1] + x[1]) * sh.n[2] + x[2]);
               const int64_t si = sh.index(x[0], x[1], x[2]);
-              Val v = si >= 0 && vals[(size_t)si].chain >= 0 ? vals[(size_t)si] : Val{op.block, ci, 0};
-              if (snap && op.kind == BC_WALL_ISOTHERMAL)
+              Val v = si >= 0 && vals[(size_t)si].chain >= 0 ? vals[(size_t)si] : Val{op.block, ci, 0, (int32_t)si};
+              if (snap && op.kind == BC_WALL_ISOTHERMAL) {
+                snap_ss.push_back(v.ss);
                 snaps.push_back(GhostSnap{v.sb, v.sc, v.chain, f,
                                           ((int64_t)e * ghost + gl) * 5 * maxcells[f] + (int64_t)x[t1] * sh.n[t2] + x[t2],
                                           maxcells[f]});
-              if (op.kind == BC_FARFIELD) v = Val{-1, 0, 0};
+              }
+              if (op.kind == BC_FARFIELD) v = Val{-1, 0, 0, -1};
               if (op.kind != BC_EXTRAPOLATE) {
-                auto it = longer.find({v.chain, iop});
-                if (it == longer.end()) {
+                // (a cell read here is never one this operation has written: longer covers its chain)
+                int32_t& next = longer[(size_t)v.chain];
+                if (next < 0) {
                   GhostChain c = chains[(size_t)v.chain];
                   c.op[c.n++] = iop;
-                  it = longer.emplace(std::make_pair(v.chain, iop), (int32_t)chains.size()).first;
+                  next = (int32_t)chains.size();
                   chains.push_back(c);
                 }
-                v.chain = it->second;
+                v.chain = next;
               }
               x[ax] = outer;
               vals[(size_t)sh.index(x[0], x[1], x[2])] = v;
@@ -209,41 +225,37 @@ struct GhostTable {
 
   // Entries in launch order.
   void finish() {
-    std::vector<std::vector<bool>> awaited(shell.size());   // targets whose old value a staged entry or snapshot reads
-    for (size_t b = 0; b < shell.size(); ++b) awaited[b].assign((size_t)shell[b].size, false);
-    auto written = [&](int32_t sb, int32_t sc) -> int64_t {
-      if (sb < 0) return -1;
-      const int64_t s = shell[(size_t)sb].index_of(sc);
-      return s >= 0 && val[(size_t)sb][(size_t)s].chain >= 0 ? s : -1;
-    };
-    std::vector<GhostEntry> direct, staged, late;
-    for (const GhostSnap& s : snaps) {
-      const int64_t w = written(s.sb, s.sc);
-      if (w >= 0) awaited[(size_t)s.sb][(size_t)w] = true;
-    }
+    // per target: 1 a staged entry or a snapshot reads its old value, 2 it is staged itself
+    std::vector<std::vector<char>> flag(shell.size());
+    for (size_t b = 0; b < shell.size(); ++b) flag[b].assign((size_t)shell[b].size, 0);
+    auto waits = [&](int32_t sb, int32_t ss) { return sb >= 0 && ss >= 0 && val[(size_t)sb][(size_t)ss].chain >= 0; };
+    for (size_t i = 0; i < snaps.size(); ++i)
+      if (waits(snaps[i].sb, snap_ss[i])) flag[(size_t)snaps[i].sb][(size_t)snap_ss[i]] |= 1;
+    int64_t total = 0;
+    nstaged = nlate = 0;
+    for (size_t b = 0; b < val.size(); ++b)
+      for (size_t s = 0; s < val[b].size(); ++s) {
+        const Val& v = val[b][s];
+        if (v.chain < 0) continue;
+        ++total;
+        if (!waits(v.sb, v.ss)) continue;
+        flag[(size_t)v.sb][(size_t)v.ss] |= 1;
+        flag[b][s] |= 2;
+        ++nstaged;
+      }
+    for (size_t b = 0; b < val.size(); ++b)
+      for (size_t s = 0; s < val[b].size(); ++s) nlate += flag[b][s] == 1 && val[b][s].chain >= 0;
+    ndirect = (int)(total - nstaged - nlate);
+    entries.resize((size_t)total);
+    GhostEntry *direct = entries.data(), *staged = direct + ndirect, *late = staged + nstaged;
     for (int b = 0; b < (int)shell.size(); ++b)
       shell[b].each([&](int32_t c, int64_t s) {
         const Val& v = val[b][(size_t)s];
         if (v.chain < 0) return;
-        const GhostEntry e{b, c, v.sb, v.sc, v.chain};
-        const int64_t w = written(v.sb, v.sc);
-        if (w >= 0) {
-          awaited[(size_t)v.sb][(size_t)w] = true;
-          staged.push_back(e);
-        } else {
-          direct.push_back(e);
-        }
+        const int f = flag[b][(size_t)s];
+        GhostEntry*& to = f >= 2 ? staged : (f == 1 ? late : direct);
+        *to++ = GhostEntry{b, c, v.sb, v.sc, v.chain};
       });
-    entries.clear();
-    for (const GhostEntry& e : direct) {
-      if (awaited[(size_t)e.tb][(size_t)shell[(size_t)e.tb].index_of(e.tc)]) late.push_back(e);
-      else entries.push_back(e);
-    }
-    ndirect = (int)entries.size();
-    nstaged = (int)staged.size();
-    nlate = (int)late.size();
-    entries.insert(entries.end(), staged.begin(), staged.end());
-    entries.insert(entries.end(), late.begin(), late.end());
   }
 };
 

@@ -1301,6 +1301,7 @@ __global__ void __launch_bounds__(NTH) k_stage_split_batched(const BlockDesc* __
 }  // namespace famrdp
 
 #include "famrdp_march.h"
+#include "famrdp_wide.h"
 
 namespace famrdp {
 
@@ -1335,7 +1336,11 @@ namespace famrdp {
   X(16, 8, 32, 32, 2)            \
   X(17, 8, 32, 52, 2)            \
   X(18, 8, 32, 10, 2)
-constexpr int NUM_TILE_VARIANTS = 19;
+// Wide kernel (famrdp_wide.h): (id, TI, TJ, TK).
+#define FAMRDP_WIDE_VARIANTS(X) \
+  X(19, 3, 4, 4)                \
+  X(20, 4, 4, 8)
+constexpr int NUM_TILE_VARIANTS = 21;
 
 inline bool is_march_variant(int v) {
   switch (v) {
@@ -1346,19 +1351,67 @@ inline bool is_march_variant(int v) {
   }
 }
 
+inline bool is_wide_variant(int v) {
+  switch (v) {
+#define FAMRDP_IW(id, a, b, c) case id: return true;
+    FAMRDP_WIDE_VARIANTS(FAMRDP_IW)
+#undef FAMRDP_IW
+    default: return false;
+  }
+}
+
 inline void tile_dims(int v, int& ti, int& tj, int& tk) {
   switch (v) {
 #define FAMRDP_TD5(id, a, b, c, n) case id: ti = a; tj = b; tk = c; return;
 #define FAMRDP_TD6(id, a, b, c, rs, w) case id: ti = a; tj = b; tk = c; return;
 #define FAMRDP_TDM(id, b, c, l, w) case id: ti = l; tj = b; tk = c; return;
+#define FAMRDP_TDW(id, a, b, c) case id: ti = a; tj = b; tk = c; return;
     FAMRDP_TILE_VARIANTS(FAMRDP_TD6)
     FAMRDP_SPLIT_VARIANTS(FAMRDP_TD5)
     FAMRDP_MARCH_VARIANTS(FAMRDP_TDM)
+    FAMRDP_WIDE_VARIANTS(FAMRDP_TDW)
+#undef FAMRDP_TDW
 #undef FAMRDP_TD5
 #undef FAMRDP_TD6
 #undef FAMRDP_TDM
     default: ti = 4; tj = 4; tk = 16;
   }
+}
+
+// Workgroups of a stage of one block with variant v.
+inline int64_t stage_tiles(int v, int ni, int nj, int nk) {
+  int TI, TJ, TK;
+  tile_dims(v, TI, TJ, TK);
+  if (is_march_variant(v)) return (int64_t)march_nseg(ni, TI) * march_tiling(TJ, TK, nj, nk).count();
+  return (int64_t)((ni + TI - 1) / TI) * ((nj + TJ - 1) / TJ) * ((nk + TK - 1) / TK);
+}
+
+// The variant of blocks that were not tuned: of the five below the one whose
+// stage should be shortest.  A stage lasts as its workgroups per compute unit
+// (n, rounded up) take; measured (minmod; van Leer is 10-17 % longer for all
+// alike), in us, for cubes of 12^3 to 124^3 cells, flat and long blocks and
+// lattices of small ones, the lines hold within 10 %:
+//   19 wide 3x4x4    3.5 + 1.75 n   (20^3 5.3, 36^3 9.8, 72^3 56.6)
+//   20 wide 4x4x8    1.5 + 5.6 n    (32^3 7.4, 44^3 17.7)
+//    1 fused 4x8x16  15.3 n         (44^3 15.6, 60^3 31.1, 72^3 58.3)
+//   12 re-staging    5 + 6.5 n      (52^3 24.3, 80^3 59.7, 104^3 126.6)
+//   18 marching      45 n, 65 at least (80^3 68, 96^3 87.7, 124^3 171)
+// The fused kernel of 8x4x8 cells that every untuned block took before:
+// 12.1 at 20^3, 27.5 at 52^3, 65.8 at 80^3, 109 at 96^3, 258 at 124^3.
+inline int default_variant(int nblocks, const int32_t* dims, int ncu, bool fits32) {
+  struct Line { int v; double base, per, least; };
+  constexpr Line lines[] = {
+      {19, 3.5, 1.75, 0}, {20, 1.5, 5.6, 0}, {1, 0, 15.3, 0}, {12, 5, 6.5, 0}, {18, 0, 45, 65}};
+  int best = 12;
+  double best_t = 1e300;
+  for (const Line& l : lines) {
+    if (!fits32 && (is_march_variant(l.v) || is_wide_variant(l.v))) continue;
+    int64_t n = 0;
+    for (int b = 0; b < nblocks; ++b) n += stage_tiles(l.v, dims[3 * b], dims[3 * b + 1], dims[3 * b + 2]);
+    const double t = std::max(l.least, l.base + l.per * (double)((n + ncu - 1) / ncu));
+    if (t < best_t) { best_t = t; best = l.v; }
+  }
+  return best;
 }
 
 // One stage of one block (plain launch) with variant v; the limiter is a
@@ -1389,6 +1442,10 @@ inline void launch_stage_lim(int v, const BlockDesc& d, int stage, const StageGa
     return;
     FAMRDP_MARCH_VARIANTS(FAMRDP_ML)
 #undef FAMRDP_ML
+#define FAMRDP_WL(id, a, b, c) \
+  case id: k_stage_wide<a, b, c, LIM><<<nt, WideGeom<a, b, c>::NTH, 0, st>>>(d, stage, gas, dt, ntj, ntk); return;
+    FAMRDP_WIDE_VARIANTS(FAMRDP_WL)
+#undef FAMRDP_WL
   }
 }
 
@@ -1430,6 +1487,12 @@ inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3
     return;
     FAMRDP_MARCH_VARIANTS(FAMRDP_MB)
 #undef FAMRDP_MB
+#define FAMRDP_WB(id, a, b, c)                                                                                      \
+  case id:                                                                                                          \
+    k_stage_wide_batched<a, b, c, LIM><<<ntiles, WideGeom<a, b, c>::NTH, 0, st>>>(blocks, tiles, stage, gas, dt);   \
+    return;
+    FAMRDP_WIDE_VARIANTS(FAMRDP_WB)
+#undef FAMRDP_WB
   }
 }
 

@@ -1,4 +1,4 @@
-// Tile geometry of the fused and split stage kernels: the periodic wrap of
+// Tile geometry of the fused, split and wide stage kernels: the periodic wrap of
 // tile coordinates into a block and the cell index (three wrap modes), and
 // the LDS slot maps of a fused tile.  Host-callable, so the index arithmetic
 // can be checked on the CPU.
@@ -107,6 +107,102 @@ struct FusedGeom {
     if (h < 2 * TI * TK) return Loc3{(h / TK) % TI, h / (TI * TK) ? TJ : -1, h % TK};
     h -= 2 * TI * TK;
     return Loc3{(h / TJ) % TI, h % TJ, h / (TI * TJ) ? TK : -1};
+  }
+};
+
+// The wide kernel's tile: FusedGeom's slots of staged cells and tensors, a
+// slot per face of every axis, and threads for all of them.
+template <int TI, int TJ, int TK>
+struct WideGeom {
+  using T = FusedGeom<TI, TJ, TK>;
+  static constexpr int NGW = (T::NG + 63) / 64 * 64;     // threads of the tensors, whole waves
+  static constexpr int F_J = 0, F_K = T::F1, F_I = T::F1 + T::F2, NF = T::F0 + T::F1 + T::F2;   // face slots
+  static constexpr int NTH = NGW + (NF + 63) / 64 * 64;
+  static constexpr int NLDS = 6 * T::NPV + 9 * T::NG + 5 * NF;
+  static constexpr int NIT = (T::NPV + NTH - 1) / NTH;
+
+  // n / D for 0 <= n < 1024 and D <= 64 (n e < 2^16 with e < D the excess of
+  // the rounded-up reciprocal): a full-rate multiply in place of the
+  // quarter-rate ones of a 32-bit division; other n give some number
+  template <int D>
+  __host__ __device__ static constexpr int div(int n) {
+    static_assert(D <= 64, "divisor");
+    if constexpr ((D & (D - 1)) == 0) return n / D;
+    return (int)(((unsigned)(n & 0xffff) * (unsigned)((65536 + D - 1) / D)) >> 16);
+  }
+  // face slot h: its axis and its right cell; along the axis the right cell's
+  // coordinate runs over 0 .. extent (face f lies between cells f-1 and f)
+  // (selects only, as the maps below: a wave holds faces of two axes)
+  __host__ __device__ static constexpr int face_axis_of(int h) { return h < F_K ? 1 : (h < F_I ? 2 : 0); }
+  __host__ __device__ static constexpr Loc3 face_cell(int h) {
+    const bool j = h < F_K, k = !j && h < F_I;
+    const int u = h - F_K, v = h - F_I;
+    const int xj = div<(TJ + 1) * TK>(h), xk = div<TJ * (TK + 1)>(u), xi = div<TJ * TK>(v);
+    const int rj = h - xj * ((TJ + 1) * TK), rk = u - xk * (TJ * (TK + 1)), ri = v - xi * (TJ * TK);
+    const int yj = div<TK>(rj), yk = div<TK + 1>(rk), yi = div<TK>(ri);
+    const int zj = rj - yj * TK, zk = rk - yk * (TK + 1), zi = ri - yi * TK;
+    return Loc3{j ? xj : (k ? xk : xi), j ? yj : (k ? yk : yi), j ? zj : (k ? zk : zi)};
+  }
+  // T::pv_cell and T::g_cell
+  __host__ __device__ static constexpr Loc3 pv_cell(int h) {
+    const bool r0 = h < T::NR0, r1 = h < T::NR0 + T::NR1, r2 = h < T::NR0 + T::NR1 + T::NR2;
+    const int b0 = div<T::B0J * T::B0K>(h), p0 = h - b0 * (T::B0J * T::B0K), r = div<T::B0K>(p0);
+    const int x0 = b0 - 1, y0 = r - 1, z0 = p0 - r * T::B0K - 1;
+    const Loc3 o = outer(h - T::NR0, h - T::NR0 - T::NR1, h - T::NR0 - T::NR1 - T::NR2, r1, r2, 2);
+    return Loc3{r0 ? x0 : o.x, r0 ? y0 : o.y, r0 ? z0 : o.z};
+  }
+  __host__ __device__ static constexpr Loc3 g_cell(int h) {
+    const bool r0 = h < T::NT, r1 = h < T::NT + 2 * TJ * TK, r2 = h < T::NT + 2 * TJ * TK + 2 * TI * TK;
+    const int x0 = div<TJ * TK>(h), p0 = h - x0 * (TJ * TK), y0 = div<TK>(p0), z0 = p0 - y0 * TK;
+    const Loc3 o = outer(h - T::NT, h - T::NT - 2 * TJ * TK, h - T::NT - 2 * TJ * TK - 2 * TI * TK, r1, r2, 1);
+    return Loc3{r0 ? x0 : o.x, r0 ? y0 : o.y, r0 ? z0 : o.z};
+  }
+  // a cell `far` before the tile or as far past it: along i from index u of
+  // its layer pair if in_i, else along j from v if in_j, else along k from w
+  __host__ __device__ static constexpr Loc3 outer(int u, int v, int w, bool in_i, bool in_j, int far) {
+    const int n = in_i ? TJ * TK : (in_j ? TI * TK : TI * TJ), h = in_i ? u : (in_j ? v : w);
+    const bool up = h >= n;
+    const int r = up ? h - n : h;
+    const int qk = div<TK>(r), qj = div<TJ>(r);
+    const int a = in_i || in_j ? qk : qj, b = in_i || in_j ? r - qk * TK : r - qj * TJ;
+    const int e = up ? (in_i ? TI : (in_j ? TJ : TK)) + far - 1 : -far;
+    return Loc3{in_i ? e : a, in_i ? a : (in_j ? e : b), in_i || in_j ? b : e};
+  }
+  // a if !c, b if c, without a branch
+  __host__ __device__ static constexpr int pick(bool c, int a, int b) { return a ^ ((a ^ b) & -(int)c); }
+  // T::pv_slot of the cell s steps along axis e (0, 1, 2) from cell l, whose
+  // other two coordinates lie in the box
+  __host__ __device__ static constexpr int pv_step(const Loc3& l, int e, int s) {
+    const int stride = pick(e == 0, pick(e == 1, 1, T::B0K), T::B0J * T::B0K);
+    const int ext = pick(e == 0, pick(e == 1, TK, TJ), TI), c = pick(e == 0, pick(e == 1, l.z, l.y), l.x) + s;
+    const int box = ((l.x + 1) * T::B0J + l.y + 1) * T::B0K + l.z + 1 + s * stride;
+    const int lay = pick(e == 0, pick(e == 1, TI * TJ, TI * TK), TJ * TK);
+    const int a = pick(e == 0, l.x, l.y), b = pick(e == 2, l.z, l.y);   // the two coordinates across e
+    const int out = pick(e == 0, pick(e == 1, T::NR0 + T::NR1 + T::NR2, T::NR0 + T::NR1), T::NR0) +
+                    pick(c > 0, 0, lay) + a * pick(e == 2, TK, TJ) + b;
+    return pick((unsigned)(c + 1) > (unsigned)(ext + 1), box, out);
+  }
+  // T::g_slot of the cell s = +-1 steps along axis e from tile cell l
+  __host__ __device__ static constexpr int g_step(const Loc3& l, int e, int s) {
+    const int stride = pick(e == 0, pick(e == 1, 1, TK), TJ * TK);
+    const int ext = pick(e == 0, pick(e == 1, TK, TJ), TI), c = pick(e == 0, pick(e == 1, l.z, l.y), l.x) + s;
+    const int in = (l.x * TJ + l.y) * TK + l.z + s * stride;
+    const int lay = pick(e == 0, pick(e == 1, TI * TJ, TI * TK), TJ * TK);
+    const int a = pick(e == 0, l.x, l.y), b = pick(e == 2, l.z, l.y);
+    const int out = T::NT + pick(e == 0, pick(e == 1, 2 * TJ * TK + 2 * TI * TK, 2 * TJ * TK), 0) +
+                    pick(c > 0, 0, lay) + a * pick(e == 2, TK, TJ) + b;
+    return pick((unsigned)c >= (unsigned)ext, in, out);
+  }
+  // slot of the low face of tile cell (x, y, z) along D; the high face is
+  // high_face further on
+  template <int D>
+  __host__ __device__ static constexpr int low_face(int x, int y, int z) {
+    return D == 1 ? F_J + (x * (TJ + 1) + y) * TK + z
+                  : (D == 2 ? F_K + (x * TJ + y) * (TK + 1) + z : F_I + (x * TJ + y) * TK + z);
+  }
+  template <int D>
+  __host__ __device__ static constexpr int high_face() {
+    return D == 1 ? TK : (D == 2 ? 1 : TJ * TK);
   }
 };
 
