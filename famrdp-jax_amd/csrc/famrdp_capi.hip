@@ -538,8 +538,15 @@ int famrdp_invscd_rhs(const double* q, const double* kxyz, const double* vol, do
                       int32_t nk, double gamma, int32_t limiter, void* stream) {
   if (bad_lim(limiter)) return fail(FAMRDP_E_KEY, "unknown limiter code " + std::to_string(limiter));
   if (ni < 1 || nj < 1 || nk < 1 || !q || !kxyz || !vol || !rhs) return fail(FAMRDP_E_INVALID, "invscd_rhs: bad arguments");
-  const int64_t N = (int64_t)ni * nj * nk;
-  k_invscd_rhs<<<nblk(N), 256, 0, S(stream)>>>(q, kxyz, vol, rhs, ni, nj, nk, gamma, limiter);
+  Gas g{};
+  g.gamma = gamma;
+  g.R = g.Pr_lam = g.T0 = 1.0;
+  const unsigned grid = rhs_grid<4, 4, 4>(ni, nj, nk);
+  constexpr int nth = CrossGeom<4, 4, 4>::NTH;
+  if (limiter == LIM_VANLEER)
+    k_invscd_rhs<4, 4, 4, LIM_VANLEER><<<grid, nth, 0, S(stream)>>>(q, kxyz, vol, rhs, ni, nj, nk, stage_gas(g), gamma);
+  else
+    k_invscd_rhs<4, 4, 4, LIM_MINMOD><<<grid, nth, 0, S(stream)>>>(q, kxyz, vol, rhs, ni, nj, nk, stage_gas(g), gamma);
   LAUNCH_CHECK();
   return FAMRDP_OK;
 }
@@ -548,10 +555,9 @@ int famrdp_viscous_rhs(const double* q, const double* kxyz, double* rhs, int32_t
                        const famrdp_gas* gas, double* work, void* stream) {
   if (ni < 1 || nj < 1 || nk < 1 || !q || !kxyz || !rhs || !gas || !work)
     return fail(FAMRDP_E_INVALID, "viscous_rhs: bad arguments");
-  const int64_t N = (int64_t)ni * nj * nk;
-  k_viscous_flux<<<nblk(N), 256, 0, S(stream)>>>(q, kxyz, work, ni, nj, nk, to_gas(gas));
-  LAUNCH_CHECK();
-  k_viscous_div<<<nblk(N), 256, 0, S(stream)>>>(work, kxyz, rhs, ni, nj, nk);
+  const Gas g = to_gas(gas);
+  k_viscous_rhs<4, 8, 8><<<rhs_grid<4, 8, 8>(ni, nj, nk), WideGeom<4, 8, 8>::NGW, 0, S(stream)>>>(q, kxyz, rhs, ni, nj, nk,
+                                                                                    stage_gas(g), g.mu0, g.gamma);
   LAUNCH_CHECK();
   return FAMRDP_OK;
 }

@@ -250,31 +250,6 @@ __global__ void __launch_bounds__(256) k_stage(const double* __restrict__ qin, c
   if (c < N) cell_stage(qin, q0, qout, kxyz, vol, G, ni, nj, nk, N, c, g, lim, dt, stage);
 }
 
-// RHS only (the unit entry points compute_invscd_rhs / compute_viscous_rhs)
-__global__ void __launch_bounds__(256) k_invscd_rhs(const double* __restrict__ q, const double* __restrict__ kxyz,
-                                                    const double* __restrict__ vol, double* __restrict__ rhs, int ni,
-                                                    int nj, int nk, double g, int lim) {
-  const int64_t N = (int64_t)ni * nj * nk;
-  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double inv[5];
-  cell_invscd(q, kxyz, vol, ni, nj, nk, N, c, g, lim, inv);
-  for (int v = 0; v < 5; ++v) rhs[v * N + c] = inv[v];
-}
-
-__global__ void __launch_bounds__(256) k_viscous_div(const double* __restrict__ G, const double* __restrict__ kxyz,
-                                                     double* __restrict__ rhs, int ni, int nj, int nk) {
-  const int64_t N = (int64_t)ni * nj * nk;
-  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double vis[4];
-  cell_viscous_div(G, kxyz, ni, nj, nk, N, c, vis);
-  rhs[c] = 0.0;
-  for (int v = 0; v < 4; ++v) rhs[(v + 1) * N + c] = vis[v];
-}
-
-// Generic RK combination for rk3_step(q, L, dt): out = a*x + b*(y + c*z), or
-// y + c*z when mode == 1 (time/rk.py:17-19).
 __global__ void k_axpby(double* __restrict__ out, double a, const double* __restrict__ x, double b,
                         const double* __restrict__ y, double c, const double* __restrict__ z, int64_t n, int mode) {
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1302,6 +1277,7 @@ __global__ void __launch_bounds__(NTH) k_stage_split_batched(const BlockDesc* __
 
 #include "famrdp_march.h"
 #include "famrdp_wide.h"
+#include "famrdp_rhs.h"
 
 namespace famrdp {
 

@@ -326,12 +326,15 @@ DF void prim_and_temp(const double q[5], const StageGas& gas, double pv[6]) {
 // instructions and six seeds, 205 and seven in the form with conservative
 // jumps.  The floors are min/max, which drop a NaN: a NaN primitive makes the
 // pressure NaN, and dp carries it into every component.
+template <bool FULL = false>
 DF void roe_flux2(const double pl[5], const double pr[5], const double S[3], const StageGas& gas, double F[5]) {
   EXACT_FP
+  auto recip = [](double x) { return FULL ? rcp(x) : rcp1(x); };
+  auto root = [](double x) { return FULL ? rsq_acc(x) : rsq1(x); };
   const double rhoL = fmax(pl[0], 1e-300), rhoR = fmax(pr[0], 1e-300);
-  const double isL = rsq1(rhoL), isR = rsq1(rhoR);
+  const double isL = root(rhoL), isR = root(rhoR);
   const double sqL = rhoL * isL, sqR = rhoR * isR;
-  const double a = sqR * rcp1(sqL + sqR);
+  const double a = sqR * recip(sqL + sqR);
   const double uL = pl[1], vL = pl[2], wL = pl[3], uR = pr[1], vR = pr[2], wR = pr[3];
   // twice the total enthalpies: 2 g/(g-1) p/rho + |u|^2
   const double kL = fma(wL, wL, fma(vL, vL, uL * uL)), kR = fma(wR, wR, fma(vR, vR, uR * uR));
@@ -340,17 +343,17 @@ DF void roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   const double uh = fma(a, du, uL), vh = fma(a, dv, vL), wh = fma(a, dw, wL), Hh = fma(a, dH, HL);
   const double hq = Hh - fma(wh, wh, fma(vh, vh, uh * uh));     // 2 H^ - q^2
   const double c2 = fmax(gas.gm1h * hq, 1e-30);
-  const double isc = rsq1(c2);
+  const double isc = root(c2);
   const double rc2 = isc * isc, c = c2 * isc;
   // |S| and 1/|S|; a zero face keeps a harmless 1e-140
   const double nn = fmax(fma(S[2], S[2], fma(S[1], S[1], S[0] * S[0])), 1e-280);
-  const double rA = rsq1(nn);
+  const double rA = root(nn);
   const double C = c * (nn * rA);
   const double unL = fma(wL, S[2], fma(vL, S[1], uL * S[0])), unR = fma(wR, S[2], fma(vR, S[1], uR * S[0]));
   const double dS = unR - unL;
   const double un = fma(a, dS, unL);
   const double base = fabs(un) + C;                              // eps = 0.1 base
-  const double h = rcp1(0.2 * base);                             // 1 / (2 eps)
+  const double h = recip(0.2 * base);                             // 1 / (2 eps)
   const double l1 = un - C, l5 = un + C;
   const double e1 = fmax(fma(0.1, base, -fabs(l1)), 0.0), e5 = fmax(fma(0.1, base, -fabs(l5)), 0.0);
   const double al1 = fma(e1 * h, e1, fabs(l1)), al5 = fma(e5 * h, e5, fabs(l5));
@@ -436,14 +439,14 @@ DF void face_states_fast(const double pv0[5], const double pv1[5], const double 
 
 // Twice the flux of one face (roe_flux2) from the primitives of cells a-1 ..
 // a+2 and kxyz[d, :] / 2 at cells a and a+1: the area vector is their sum.
-template <int LIM>
+template <int LIM, bool FULL = false>
 DF void face_flux2(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
                    const double k0h[3], const double k1h[3], const StageGas& gas, double F[5]) {
   EXACT_FP
   double pL[5], pR[5];
   face_states_fast<LIM>(pv0, pv1, pv2, pv3, pL, pR);
   const double S[3] = {k0h[0] + k1h[0], k0h[1] + k1h[1], k0h[2] + k1h[2]};
-  roe_flux2(pL, pR, S, gas, F);
+  roe_flux2<FULL>(pL, pR, S, gas, F);
 }
 
 // Viscous flux tensor of one cell (rhs/viscous.py:30-108): velocity and

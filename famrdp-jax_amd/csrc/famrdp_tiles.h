@@ -1,4 +1,4 @@
-// Tile geometry of the fused, split and wide stage kernels: the periodic wrap of
+// Tile geometry of the fused, split and wide stage kernels and the RHS kernels: the periodic wrap of
 // tile coordinates into a block and the cell index (three wrap modes), and
 // the LDS slot maps of a fused tile.  Host-callable, so the index arithmetic
 // can be checked on the CPU.
@@ -121,12 +121,12 @@ struct WideGeom {
   static constexpr int NLDS = 6 * T::NPV + 9 * T::NG + 5 * NF;
   static constexpr int NIT = (T::NPV + NTH - 1) / NTH;
 
-  // n / D for 0 <= n < 1024 and D <= 64 (n e < 2^16 with e < D the excess of
-  // the rounded-up reciprocal): a full-rate multiply in place of the
+  // n / D for 0 <= n < 1024 (exact while n e < 2^16, e the excess of D times the
+  // rounded-up reciprocal 2^16 / D): a full-rate multiply in place of the
   // quarter-rate ones of a 32-bit division; other n give some number
   template <int D>
   __host__ __device__ static constexpr int div(int n) {
-    static_assert(D <= 64, "divisor");
+    static_assert(1023 * ((65536 + D - 1) / D * D - 65536) < 65536, "divisor");
     if constexpr ((D & (D - 1)) == 0) return n / D;
     return (int)(((unsigned)(n & 0xffff) * (unsigned)((65536 + D - 1) / D)) >> 16);
   }
@@ -203,6 +203,40 @@ struct WideGeom {
   template <int D>
   __host__ __device__ static constexpr int high_face() {
     return D == 1 ? TK : (D == 2 ? 1 : TJ * TK);
+  }
+};
+
+// A TI x TJ x TK tile of the inviscid term: the cells two deep along each axis,
+// and a slot per face (WideGeom's).
+template <int TI, int TJ, int TK>
+struct CrossGeom {
+  using W = WideGeom<TI, TJ, TK>;
+  static constexpr int NT = TI * TJ * TK;
+  static constexpr int AI = TJ * TK, AJ = TI * TK, AK = TI * TJ;      // a layer across i, j, k
+  static constexpr int NC = NT + 4 * (AI + AJ + AK), NF = W::NF;
+  static constexpr int NTH = (NF + 63) / 64 * 64;
+
+  // local coordinates of slot h: the tile, then the layers -2, -1, T, T + 1 of
+  // each axis
+  __host__ __device__ static constexpr Loc3 cell(int h) {
+    const bool r0 = h < NT, r1 = h < NT + 4 * AI, r2 = h < NT + 4 * (AI + AJ);
+    const int u = r0 ? h : (r1 ? h - NT : (r2 ? h - NT - 4 * AI : h - NT - 4 * (AI + AJ)));
+    const int area = r0 || r1 ? AI : (r2 ? AJ : AK), row = r0 || r1 || r2 ? TK : TJ;
+    const int l = u / area, p = u % area, a = p / row, b = p % row;
+    const int ext = r1 ? TI : (r2 ? TJ : TK), e = l < 2 ? l - 2 : ext + l - 2;
+    return r0 ? Loc3{l, a, b} : (r1 ? Loc3{e, a, b} : (r2 ? Loc3{a, e, b} : Loc3{a, b, e}));
+  }
+  // slot of the cell s steps along axis e from cell l, whose other two
+  // coordinates lie in the tile
+  __host__ __device__ static constexpr int step(const Loc3& l, int e, int s) {
+    const int ext = W::pick(e == 0, W::pick(e == 1, TK, TJ), TI);
+    const int c = W::pick(e == 0, W::pick(e == 1, l.z, l.y), l.x) + s;
+    const int in = (l.x * TJ + l.y) * TK + l.z + s * W::pick(e == 0, W::pick(e == 1, 1, TK), TJ * TK);
+    const int area = W::pick(e == 0, W::pick(e == 1, AK, AJ), AI);
+    const int base = NT + W::pick(e == 0, W::pick(e == 1, 4 * (AI + AJ), 4 * AI), 0);
+    const int a = W::pick(e == 0, l.x, l.y), b = W::pick(e == 2, l.z, l.y);
+    const int layer = W::pick(c < 0, c - ext + 2, c + 2);
+    return W::pick((unsigned)c >= (unsigned)ext, in, base + layer * area + a * W::pick(e == 2, TK, TJ) + b);
   }
 };
 

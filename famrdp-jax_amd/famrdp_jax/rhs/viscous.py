@@ -14,8 +14,8 @@ def compute_viscous_rhs(q, metrics, *, gas, ghost: int):
     kx = L.device_f64(metrics.kxyz)
     _, ni, nj, nk = qd.shape
     rhs = torch.empty_like(qd)
-    work = torch.empty((9, ni, nj, nk), dtype=torch.float64, device=qd.device)
     g = L.gas_struct(gas)
-    L.check(L.lib().famrdp_viscous_rhs(L.ptr(qd), L.ptr(kx), L.ptr(rhs), ni, nj, nk, ctypes.byref(g), L.ptr(work),
+    # (the scratch argument must not be NULL but is no longer written)
+    L.check(L.lib().famrdp_viscous_rhs(L.ptr(qd), L.ptr(kx), L.ptr(rhs), ni, nj, nk, ctypes.byref(g), L.ptr(rhs),
                                        L.stream()))
     return L.like_input(rhs, q)

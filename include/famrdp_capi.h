@@ -89,7 +89,8 @@ int famrdp_roe_flux(const double* UL, const double* UR, const double* nxyz, doub
 /* famrdp_jax/rhs/invscd.py:18-133 (reconstruct/flux names are unused there). */
 int famrdp_invscd_rhs(const double* q, const double* kxyz, const double* vol, double* rhs, int32_t ni, int32_t nj,
                       int32_t nk, double gamma, int32_t limiter, void* stream);
-/* famrdp_jax/rhs/viscous.py:19-119.  work: caller scratch of 9*ni*nj*nk doubles. */
+/* famrdp_jax/rhs/viscous.py:19-119.  work: not written any more (once scratch of
+ * 9*ni*nj*nk doubles); must not be NULL. */
 int famrdp_viscous_rhs(const double* q, const double* kxyz, double* rhs, int32_t ni, int32_t nj, int32_t nk,
                        const famrdp_gas* gas, double* work, void* stream);
 /* famrdp_jax/time/rk.py:17-19 combination: out = a*x + b*(y + c*z), or

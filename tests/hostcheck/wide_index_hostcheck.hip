@@ -14,7 +14,8 @@ namespace {
 bool same(Loc3 a, Loc3 b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
 Loc3 step(Loc3 l, int e, int s) { return Loc3{l.x + (e == 0 ? s : 0), l.y + (e == 1 ? s : 0), l.z + (e == 2 ? s : 0)}; }
 
-template <int TI, int TJ, int TK>
+// FACES: the kernel has a thread per face as well
+template <int TI, int TJ, int TK, bool FACES = true>
 int64_t check() {
   using T = FusedGeom<TI, TJ, TK>;
   using W = WideGeom<TI, TJ, TK>;
@@ -59,7 +60,7 @@ int64_t check() {
       if (W::face_axis_of(lo[e] + up[e]) != e || !same(W::face_cell(lo[e] + up[e]), step(l, e, 1))) ++bad;
     }
   }
-  if (W::NGW < T::NG || W::NTH - W::NGW < W::NF || W::NGW % 64 != 0 || W::NTH > 1024) ++bad;
+  if (W::NGW < T::NG || W::NTH - W::NGW < W::NF || W::NGW % 64 != 0 || (FACES ? W::NTH : W::NGW) > 1024) ++bad;
   return bad;
 }
 
@@ -68,6 +69,7 @@ int64_t check() {
 extern "C" int64_t wide_bad(int ti, int tj, int tk) {
   if (ti == 3 && tj == 4 && tk == 4) return check<3, 4, 4>();
   if (ti == 4 && tj == 4 && tk == 8) return check<4, 4, 8>();
+  if (ti == 4 && tj == 8 && tk == 8) return check<4, 8, 8, false>();   // the viscous RHS kernel's
   if (ti == 3 && tj == 4 && tk == 5) return check<3, 4, 5>();   // no two extents alike
   return -1;
 }

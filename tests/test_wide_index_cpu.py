@@ -26,6 +26,6 @@ def hc(tmp_path_factory):
     return lib
 
 
-@pytest.mark.parametrize("shape", [(3, 4, 4), (4, 4, 8), (3, 4, 5)])
+@pytest.mark.parametrize("shape", [(3, 4, 4), (4, 4, 8), (4, 8, 8), (3, 4, 5)])
 def test_wide_slot_maps(hc, shape):
     assert hc.wide_bad(*shape) == 0
