@@ -156,7 +156,7 @@ struct famrdp_plan {
   BcEntry* d_ops = nullptr;
   GhostSnap* d_snaps = nullptr;
   double* d_ghost_stage = nullptr;
-  int nghost_direct = 0, nghost_staged = 0, nghost_late = 0, nsnaps = 0;
+  int nghost_direct = 0, nghost_staged = 0, nghost_late = 0, nghost_kept = 0, nsnaps = 0;
   BcEntry* d_bc[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   int nbc[6] = {0, 0, 0, 0, 0, 0};
   int64_t bc_maxcells[6] = {0, 0, 0, 0, 0, 0};
@@ -789,6 +789,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
     p->nghost_direct = ghosts.ndirect;
     p->nghost_staged = ghosts.nstaged;
     p->nghost_late = ghosts.nlate;
+    p->nghost_kept = ghosts.nkept;
     p->nsnaps = (int)ghosts.snaps.size();
     tables.table(&p->d_ghost, ghosts.entries);
     tables.table(&p->d_chains, ghosts.chains);
@@ -1164,6 +1165,19 @@ int famrdp_step_from(famrdp_plan* p, const double* const* q_in, double* const* q
   if (rc) return rc;
   p->blocks_uploaded = false;
   if (p->has_adjoint && changed_adj && (rc = upload_adj(p, st))) return rc;
+  if (p->nblocks <= STEP_START_BLOCKS) {
+    StepStart ss{};
+    for (int b = 0; b < p->nblocks; ++b) {
+      ss.block[b] = p->h_blocks[b];
+      ss.src[b] = q_in[b];
+    }
+    const int n = p->nghost_direct + p->nghost_staged + p->nghost_late + p->nghost_kept;
+    k_step_start<<<p->ntiles + nblk(n), 256, 0, st>>>(ss, p->d_blocks, p->nblocks, p->d_tiles, p->ntiles, p->ghost,
+                                                      p->d_ghost, n, p->d_chains, p->d_ops, p->gas.gamma, p->gas.R);
+    LAUNCH_CHECK();
+    p->blocks_uploaded = true;
+    return launch_stages(p, dt, flags, st);
+  }
   for (int b0 = 0; b0 < p->nblocks; b0 += STEP_START_BLOCKS) {
     const int n = std::min(STEP_START_BLOCKS, p->nblocks - b0);
     StepStart ss{};
@@ -1175,7 +1189,7 @@ int famrdp_step_from(famrdp_plan* p, const double* const* q_in, double* const* q
     }
     // four 16-byte accesses per thread, until the chip is full
     const int gx = (int)std::min<int64_t>((5 * most + 2047) / 2048, 4096);
-    k_step_start<<<dim3(gx, n), 256, 0, st>>>(ss, p->d_blocks + b0);
+    k_step_copy<<<dim3(gx, n), 256, 0, st>>>(ss, p->d_blocks + b0);
     LAUNCH_CHECK();
   }
   p->blocks_uploaded = true;

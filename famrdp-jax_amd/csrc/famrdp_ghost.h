@@ -137,8 +137,10 @@ struct GhostTable {
   std::vector<std::vector<Val>> val;       // per block and ghost cell
   std::vector<BcEntry> ops;
   std::vector<GhostChain> chains;          // 0: the value itself
-  std::vector<GhostEntry> entries;         // [direct | staged | late direct]
-  int ndirect = 0, nstaged = 0, nlate = 0;
+  // [direct | staged | late direct | kept]: kept are the ghost cells that
+  // nothing writes, as copies of themselves, for a step into other arrays
+  std::vector<GhostEntry> entries;
+  int ndirect = 0, nstaged = 0, nlate = 0, nkept = 0;
   std::vector<GhostSnap> snaps;
   std::vector<int32_t> snap_ss;            // Val::ss of the recorded values
 
@@ -232,11 +234,11 @@ struct GhostTable {
     for (size_t i = 0; i < snaps.size(); ++i)
       if (waits(snaps[i].sb, snap_ss[i])) flag[(size_t)snaps[i].sb][(size_t)snap_ss[i]] |= 1;
     int64_t total = 0;
-    nstaged = nlate = 0;
+    nstaged = nlate = nkept = 0;
     for (size_t b = 0; b < val.size(); ++b)
       for (size_t s = 0; s < val[b].size(); ++s) {
         const Val& v = val[b][s];
-        if (v.chain < 0) continue;
+        if (v.chain < 0) { ++nkept; continue; }
         ++total;
         if (!waits(v.sb, v.ss)) continue;
         flag[(size_t)v.sb][(size_t)v.ss] |= 1;
@@ -246,12 +248,12 @@ struct GhostTable {
     for (size_t b = 0; b < val.size(); ++b)
       for (size_t s = 0; s < val[b].size(); ++s) nlate += flag[b][s] == 1 && val[b][s].chain >= 0;
     ndirect = (int)(total - nstaged - nlate);
-    entries.resize((size_t)total);
-    GhostEntry *direct = entries.data(), *staged = direct + ndirect, *late = staged + nstaged;
+    entries.resize((size_t)total + nkept);
+    GhostEntry *direct = entries.data(), *staged = direct + ndirect, *late = staged + nstaged, *kept = late + nlate;
     for (int b = 0; b < (int)shell.size(); ++b)
       shell[b].each([&](int32_t c, int64_t s) {
         const Val& v = val[b][(size_t)s];
-        if (v.chain < 0) return;
+        if (v.chain < 0) { *kept++ = GhostEntry{b, c, b, c, 0}; return; }
         const int f = flag[b][(size_t)s];
         GhostEntry*& to = f >= 2 ? staged : (f == 1 ? late : direct);
         *to++ = GhostEntry{b, c, v.sb, v.sc, v.chain};

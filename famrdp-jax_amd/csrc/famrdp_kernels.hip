@@ -355,6 +355,14 @@ __global__ void k_bc_face(const BlockDesc* __restrict__ blocks, const BcEntry* _
 // entry, in one launch or two, where the exchange and the faces one after the
 // other were up to eight (55 x 55 x 15 free stream all around: 36 us, now 4).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void ghost_chain(const GhostChain* __restrict__ chains, const BcEntry* __restrict__ ops,
+                                            int chain, double gamma, double R, double q[5]) {
+  if (chain > 0) {
+    const GhostChain& c = chains[chain];
+    for (int i = 0; i < c.n; ++i) bc_apply(ops[c.op[i]], gamma, R, q);
+  }
+}
+
 __device__ __forceinline__ void ghost_value(const BlockDesc* __restrict__ blocks, const GhostChain* __restrict__ chains,
                                             const BcEntry* __restrict__ ops, int sb, int sc, int chain, double gamma,
                                             double R, double q[5]) {
@@ -366,10 +374,7 @@ __device__ __forceinline__ void ghost_value(const BlockDesc* __restrict__ blocks
 #pragma unroll
     for (int v = 0; v < 5; ++v) q[v] = 0.0;   // replaced by the chain's free stream
   }
-  if (chain > 0) {
-    const GhostChain& c = chains[chain];
-    for (int i = 0; i < c.n; ++i) bc_apply(ops[c.op[i]], gamma, R, q);
-  }
+  ghost_chain(chains, ops, chain, gamma, R, q);
 }
 
 // Direct entries, then the staged ones into the staging buffer, then the
@@ -547,12 +552,10 @@ __global__ void __launch_bounds__(256) k_cfl_final(const double* __restrict__ pa
 }
 
 // ---------------------------------------------------------------------------
-// Start of a step that leaves its input alone: the state of up to
-// STEP_START_BLOCKS blocks copied into the arrays the step works in, and their
-// descriptors put into the plan's block table, both from the launch's
-// arguments.  One launch of 3 us in place of a copy per block (2.5 us each,
-// and a launch on the host) and a table upload of 5-7 us from pinned memory.
-// Bound by HBM (80 bytes per cell); 16-byte accesses where both arrays allow.
+// Start of a step that leaves its input alone: the states of up to
+// STEP_START_BLOCKS blocks go into the arrays the step works in, and their
+// descriptors into the plan's block table, both from the launch's arguments.
+// Bound by HBM (80 bytes per cell); on a small block by the launch.
 // ---------------------------------------------------------------------------
 constexpr int STEP_START_BLOCKS = 16;
 struct StepStart {
@@ -561,8 +564,52 @@ struct StepStart {
 };
 static_assert(sizeof(StepStart) <= 3072, "launch arguments");
 
-// grid: (chunks, blocks of this launch); blocks + first is its part of the table
-__global__ void __launch_bounds__(256) k_step_start(const StepStart s, BlockDesc* __restrict__ blocks) {
+// A plan of no more blocks: the interior by the plan's tiles of 256 cells, a
+// cell per thread, then the ghost cells by the ghost table's entries.  The
+// entries' sources are values of before the exchange, which the input arrays
+// keep, so what takes two launches in place (k_ghost_first, k_ghost_second)
+// is part of this one: 20^3 cells 4.0 us, with the copy apart 9.6 in three.
+__global__ void __launch_bounds__(256) k_step_start(const StepStart s, BlockDesc* __restrict__ blocks, int nblocks,
+                                                    const Tile* __restrict__ tiles, int ntiles, int ghost,
+                                                    const GhostEntry* __restrict__ e, int nentries,
+                                                    const GhostChain* __restrict__ chains,
+                                                    const BcEntry* __restrict__ ops, double gamma, double R) {
+  if (blockIdx.x == 0 && (int)threadIdx.x < nblocks) blocks[threadIdx.x] = s.block[threadIdx.x];
+  double q[5];
+  if ((int)blockIdx.x < ntiles) {
+    const Tile tl = tiles[blockIdx.x];
+    const BlockDesc& d = s.block[tl.block];
+    const int64_t c = (int64_t)tl.start + threadIdx.x;
+    if (c >= d.N) return;
+    const int r = (int)c / d.nk, k = (int)c - r * d.nk, i = r / d.nj, j = r - i * d.nj;   // (c < 2^31 in a plan)
+    if (i < ghost || j < ghost || k < ghost || i >= d.ni - ghost || j >= d.nj - ghost || k >= d.nk - ghost) return;
+    const double* src = s.src[tl.block];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = src[v * d.N + c];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) d.q[v * d.N + c] = q[v];
+    return;
+  }
+  const int t = ((int)blockIdx.x - ntiles) * 256 + (int)threadIdx.x;
+  if (t >= nentries) return;
+  const GhostEntry h = e[t];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) q[v] = 0.0;   // a chain without a source starts with a free stream
+  if (h.sb >= 0) {
+    const int64_t N = s.block[h.sb].N;
+    const double* src = s.src[h.sb];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = src[v * N + h.sc];
+  }
+  ghost_chain(chains, ops, h.chain, gamma, R, q);
+  const BlockDesc& d = s.block[h.tb];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) d.q[v * d.N + h.tc] = q[v];
+}
+
+// A share of the blocks of a larger plan, whole arrays (16-byte accesses where
+// both allow); the exchange follows in place.  Grid: (chunks, blocks).
+__global__ void __launch_bounds__(256) k_step_copy(const StepStart s, BlockDesc* __restrict__ blocks) {
   const BlockDesc& d = s.block[blockIdx.y];
   const double* __restrict__ src = s.src[blockIdx.y];
   double* __restrict__ dst = d.q;
