@@ -574,8 +574,13 @@ int famrdp_axpby(double* out, double a, const double* x, double b, const double*
 int famrdp_compute_metrics(const double* xyz, double* jac, double* kxyz, double* vol, int32_t ni, int32_t nj,
                            int32_t nk, void* stream) {
   if (ni < 1 || nj < 1 || nk < 1 || !xyz || !jac || !kxyz || !vol) return fail(FAMRDP_E_INVALID, "compute_metrics: bad arguments");
-  const int64_t N = (int64_t)ni * nj * nk;
-  k_metrics<<<nblk(N), 256, 0, S(stream)>>>(xyz, jac, kxyz, vol, ni, nj, nk);
+  // segments as long as leaves four workgroups per CU, 8 planes at most (a
+  // segment starts with four planes that it does not work on): 20^3 takes 7.1
+  // us with 1 plane and 17.2 with 8, 204^3 403 with 1, 308 with 8, 315 with 16
+  const int64_t tiles = (int64_t)((nj + METRIC_TJ - 1) / METRIC_TJ) * ((nk + METRIC_TK - 1) / METRIC_TK);
+  const int len = (int)std::clamp<int64_t>((ni * tiles + 1023) / 1024, 1, 8);
+  k_metrics<<<(unsigned)(tiles * ((ni + len - 1) / len)), METRIC_TJ * METRIC_TK, 0, S(stream)>>>(xyz, jac, kxyz, vol,
+                                                                                                ni, nj, nk, len);
   LAUNCH_CHECK();
   return FAMRDP_OK;
 }

@@ -432,43 +432,104 @@ __global__ void __launch_bounds__(256) k_ghost_second(const BlockDesc* __restric
 // ---------------------------------------------------------------------------
 // Grid metrics (mesh/metric.py:18-70): 4th-order central differences with
 // roll wrap, J[m][l] = dx_m/dxi_l, jac = det J, kxyz = inv(J) as [l][m].
+// The floor is HBM (112 bytes a cell); what held it up were the 36 loads a
+// cell, every wave's at 16 cycles of a CU's address unit.  So a workgroup
+// holds TJ x TK columns (a thread each) and walks planes along i: the five
+// planes of the i difference stay in registers, a plane with two cells around
+// it lies in LDS for the other two, and a cell takes three loads and its share
+// of the halo's.  The next plane's loads are issued before a plane is worked
+// on; two LDS planes in turn leave one barrier a plane.  164 x 132 x 148 cells
+// 100 us (127 with a thread per cell), 204^3 318 (363), 264^3 613 (755): what
+// is left are the eleven streams it writes.
 // ---------------------------------------------------------------------------
 
-__global__ void k_metrics(const double* __restrict__ xyz, double* __restrict__ jac, double* __restrict__ kxyz,
-                          double* __restrict__ vol, int ni, int nj, int nk) {
-  const int64_t N = (int64_t)ni * nj * nk;
-  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  const int k = (int)(c % nk), j = (int)((c / nk) % nj), i = (int)(c / ((int64_t)nk * nj));
-  const int idx[3] = {i, j, k};
-  const int n[3] = {ni, nj, nk};
-  const int64_t st[3] = {(int64_t)nj * nk, nk, 1};
-  double J[3][3];
-  for (int l = 0; l < 3; ++l) {
-    int64_t o[4];
-    const int sh[4] = {2, 1, -1, -2};
-    for (int s = 0; s < 4; ++s) {
-      int ii = idx[l] + sh[s];
-      ii = ((ii % n[l]) + n[l]) % n[l];
-      o[s] = c + (int64_t)(ii - idx[l]) * st[l];
-    }
-    for (int m = 0; m < 3; ++m) {
-      const double* f = xyz + m * N;
-      J[m][l] = (-f[o[0]] + 8.0 * f[o[1]] - 8.0 * f[o[2]] + f[o[3]]) / 12.0;
-    }
+__device__ __forceinline__ int roll(int i, int n) {
+  const int r = i % n;
+  return r < 0 ? r + n : r;
+}
+
+constexpr int METRIC_TJ = 8, METRIC_TK = 32;
+
+// Workgroups: (segment of len planes, tile), the tile index fastest.
+__global__ void __launch_bounds__(METRIC_TJ * METRIC_TK) __attribute__((amdgpu_waves_per_eu(4))) k_metrics(const double* __restrict__ xyz,
+                                                                   double* __restrict__ jac, double* __restrict__ kxyz,
+                                                                   double* __restrict__ vol, int ni, int nj, int nk,
+                                                                   int len) {
+  constexpr int TJ = METRIC_TJ, TK = METRIC_TK, W = TK + 4, P = (TJ + 4) * W, HJ = 4 * TK, H = HJ + 4 * TJ;
+  static_assert(H <= TJ * TK, "a thread per halo cell");
+  __shared__ double lds[2][3][P];
+  const int t = threadIdx.x, tj = t / TK, tk = t % TK;
+  const int ntk = (nk + TK - 1) / TK, ntj = (nj + TJ - 1) / TJ;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), tile = wg % (ntj * ntk), seg = wg / (ntj * ntk);
+  const int j0 = tile / ntk * TJ, k0 = tile % ntk * TK;
+  const int iA = seg * len, iB = min(iA + len, ni);
+  const int64_t N = (int64_t)ni * nj * nk, si = (int64_t)nj * nk;
+  const bool own = j0 + tj < nj && k0 + tk < nk;
+  const int64_t col = (int64_t)roll(j0 + tj, nj) * nk + roll(k0 + tk, nk);
+  const int slot = (tj + 2) * W + tk + 2;
+  // the thread's halo cell: rows -2, -1, TJ, TJ + 1, then columns likewise
+  int hj = 0, hk = 0;
+  if (t < HJ) {
+    const int e = t / TK;
+    hj = e < 2 ? e - 2 : TJ + e - 2;
+    hk = t % TK;
+  } else if (t < H) {
+    const int e = (t - HJ) / TJ;
+    hj = (t - HJ) % TJ;
+    hk = e < 2 ? e - 2 : TK + e - 2;
   }
-  const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-  const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-  const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-  const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
-  const double inv[3][3] = {
-      {c00 / det, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det, (J[0][1] * J[1][2] - J[0][2] * J[1][1]) / det},
-      {c01 / det, (J[0][0] * J[2][2] - J[0][2] * J[2][0]) / det, (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det},
-      {c02 / det, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det, (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det}};
-  jac[c] = det;
-  vol[c] = fabs(det);
-  for (int l = 0; l < 3; ++l)
-    for (int m = 0; m < 3; ++m) kxyz[(l * 3 + m) * N + c] = inv[l][m];
+  const int64_t hcol = (int64_t)roll(j0 + hj, nj) * nk + roll(k0 + hk, nk);
+  const int hslot = (hj + 2) * W + hk + 2;
+  double f[3][5], h[3];                  // planes i-2 .. i+2 of the column; the halo cell on plane i
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) f[m][p + 1] = xyz[m * N + roll(iA + p - 2, ni) * si + col];
+    h[m] = xyz[m * N + iA * si + hcol];
+  }
+  double nf[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) nf[m] = xyz[m * N + roll(iA + 2, ni) * si + col];
+  for (int i = iA; i < iB; ++i) {
+    double (*s)[P] = lds[(i - iA) & 1];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) f[m][p] = f[m][p + 1];
+      f[m][4] = nf[m];
+      s[m][slot] = f[m][2];
+      if (t < H) s[m][hslot] = h[m];
+    }
+    __syncthreads();
+    const int64_t pn = roll(i + 3, ni) * si, ph = roll(i + 1, ni) * si;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      nf[m] = xyz[m * N + pn + col];
+      h[m] = xyz[m * N + ph + hcol];
+    }
+    double J[3][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const double* c = s[m] + slot;
+      J[m][0] = (-f[m][4] + 8.0 * f[m][3] - 8.0 * f[m][1] + f[m][0]) / 12.0;
+      J[m][1] = (-c[2 * W] + 8.0 * c[W] - 8.0 * c[-W] + c[-2 * W]) / 12.0;
+      J[m][2] = (-c[2] + 8.0 * c[1] - 8.0 * c[-1] + c[-2]) / 12.0;
+    }
+    if (!own) continue;
+    const int64_t c = i * si + col;
+    const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+    const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+    const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+    const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
+    const double inv[3][3] = {
+        {c00 / det, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det, (J[0][1] * J[1][2] - J[0][2] * J[1][1]) / det},
+        {c01 / det, (J[0][0] * J[2][2] - J[0][2] * J[2][0]) / det, (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det},
+        {c02 / det, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det, (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det}};
+    jac[c] = det;
+    vol[c] = fabs(det);
+    for (int l = 0; l < 3; ++l)
+      for (int m = 0; m < 3; ++m) kxyz[(l * 3 + m) * N + c] = inv[l][m];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -476,6 +537,23 @@ __global__ void k_metrics(const double* __restrict__ xyz, double* __restrict__ j
 // atomics): per-workgroup max spectral radius and bad-cell count, then one
 // workgroup reduces them.
 // ---------------------------------------------------------------------------
+
+// coordinates of cell c of an (., nj, nk) block; 32-bit divisions where c has
+// no more (the same for a whole launch: N decides).  k_cfl_partial reads 120
+// bytes a cell; on 164 x 132 x 148 cells 64-bit divisions held it at 90 us, 79
+// without.
+__device__ __forceinline__ void cell_coords(int64_t c, int64_t N, int nj, int nk, int& i, int& j, int& k) {
+  if (N <= INT32_MAX) {
+    const unsigned u = (unsigned)c, r = u / (unsigned)nk, p = r / (unsigned)nj;
+    k = (int)(u - r * (unsigned)nk);
+    j = (int)(r - p * (unsigned)nj);
+    i = (int)p;
+  } else {
+    k = (int)(c % nk);
+    j = (int)((c / nk) % nj);
+    i = (int)(c / ((int64_t)nk * nj));
+  }
+}
 
 __global__ void __launch_bounds__(256) k_cfl_partial(const double* __restrict__ q, const double* __restrict__ kxyz,
                                                      const double* __restrict__ vol, int ni, int nj, int nk, int ghost,
@@ -488,7 +566,9 @@ __global__ void __launch_bounds__(256) k_cfl_partial(const double* __restrict__ 
   const int64_t nint = (int64_t)ii * jj * kk;
   double lam = 0.0, bad = 0.0;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < nint; t += (int64_t)gridDim.x * blockDim.x) {
-    const int k = (int)(t % kk) + ghost, j = (int)((t / kk) % jj) + ghost, i = (int)(t / ((int64_t)kk * jj)) + ghost;
+    int i, j, k;
+    cell_coords(t, nint, jj, kk, i, j, k);
+    i += ghost; j += ghost; k += ghost;
     const int64_t c = ((int64_t)i * nj + j) * nk + k;
     double pv[5];
     load_prim(q, N, c, gas.gamma, pv);
