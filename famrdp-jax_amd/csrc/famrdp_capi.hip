@@ -165,6 +165,7 @@ struct famrdp_plan {
   double* d_monitor = nullptr;    // per-workgroup partial counts of the state monitor (persistent_grid)
   Tile3* d_tiles3[NUM_TILE_VARIANTS] = {};
   int ntiles3[NUM_TILE_VARIANTS] = {};
+  int len3[NUM_TILE_VARIANTS] = {};   // variant_len of all blocks
   int tile_variant = -1;          // -1: by the blocks' sizes (default_variant)
   int auto_all = 0;               // then: the variant of launches over all blocks
   std::vector<int> auto_block;    // and of a block's own launches
@@ -408,7 +409,7 @@ int launch_stages(famrdp_plan* p, double dt, int flags, hipStream_t st, bool adj
     if (tm && (!e0 || !e1)) return fail(FAMRDP_E_HIP, "hipEventCreate failed");
     if (tm) HIP_TRY(hipEventRecord(e0, st));
     if (!direct && (flags & FAMRDP_STEP_BATCHED)) {
-      launch_fused_batched(vb, dtab, p->d_tiles3[vb], p->ntiles3[vb], stage, p->gas, p->limiter, dt, p->ncu, st);
+      launch_fused_batched(vb, dtab, p->d_tiles3[vb], p->ntiles3[vb], stage, p->gas, p->limiter, dt, p->len3[vb], st);
       LAUNCH_CHECK();
     } else if (!direct) {
       for (int b = 0; b < p->nblocks; ++b) {
@@ -452,7 +453,7 @@ extern "C" {
 
 const char* famrdp_last_error(void) { return g_last_error.c_str(); }
 
-const char* famrdp_version(void) { return "famrdp-mi355x 0.16 (gfx950, fp64, fused, split and i-marching stage kernels, autotuned)"; }
+const char* famrdp_version(void) { return "famrdp-mi355x 0.17 (gfx950, fp64, fused, split, i-marching and wide stage kernels, chosen by size or autotuned)"; }
 
 int famrdp_cons_to_prim(const double* q, double* pv, int64_t n, double gamma, void* stream) {
   if (n < 0 || (n > 0 && (!q || !pv))) return fail(FAMRDP_E_INVALID, "cons_to_prim: bad arguments");
@@ -827,6 +828,10 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       tables.scratch(&p->d_bc_red[f], (size_t)p->nbc[f] * 5 * BC_RED_PARTS);
     }
   }
+  int dev = 0, ncu = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    ncu = 256;
   // tile table for the batched launches
   std::vector<Tile> tiles;
   for (int b = 0; b < nblocks; ++b)
@@ -836,12 +841,13 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
     int TI, TJ, TK;
     tile_dims(v, TI, TJ, TK);
+    p->len3[v] = variant_len(v, nblocks, dims, ncu);
     std::vector<Tile3> tiles3;
     for (int b = 0; b < nblocks; ++b) {
       const int32_t* d = &dims[3 * b];
       if (is_march_variant(v)) {   // i0 = 2 x segment index + strip bit
         const MarchTiling mt = march_tiling(TJ, TK, d[1], d[2]);
-        for (int sg = 0; sg < march_nseg(d[0], TI); ++sg)
+        for (int sg = 0; sg < march_nseg(d[0], p->len3[v]); ++sg)
           for (int t = 0; t < mt.count(); ++t) {
             int j0, k0, tr;
             march_tile_of(mt, TJ, TK, t, j0, k0, tr);
@@ -856,10 +862,6 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
     p->ntiles3[v] = (int)tiles3.size();
     tables.table(&p->d_tiles3[v], tiles3);
   }
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    ncu = 256;
   p->persistent_grid = std::min(p->ntiles, ncu * 8);
   p->ncu = ncu;
   p->auto_all = default_variant(nblocks, dims, ncu, variant_fits(p, 18));
@@ -906,7 +908,10 @@ int famrdp_plan_set_tile(famrdp_plan* p, int32_t variant) {
 int famrdp_plan_get_tile(const famrdp_plan* p, int32_t* variant, int32_t* dims3) {
   if (!p) return fail(FAMRDP_E_INVALID, "get_tile: plan is NULL");
   if (variant) *variant = batched_variant(p);
-  if (dims3) tile_dims(batched_variant(p), dims3[0], dims3[1], dims3[2]);
+  if (dims3) {
+    tile_dims(batched_variant(p), dims3[0], dims3[1], dims3[2]);
+    dims3[0] = p->len3[batched_variant(p)];
+  }
   return FAMRDP_OK;
 }
 
@@ -929,7 +934,8 @@ int famrdp_plan_autotune(famrdp_plan* p, double* const* q, const double* const* 
       if (r == 0) HIP_TRY(hipEventRecord(e0, st));
       for (int stage = 1; stage <= 2; ++stage) {
         if (flags & FAMRDP_STEP_BATCHED) {
-          launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt, p->ncu, st);
+          launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt,
+                               p->len3[v], st);
         } else {
           for (int b = 0; b < p->nblocks; ++b)
             launch_fused(v, p->h_blocks[b], stage, p->gas, p->limiter, dt, p->ncu, st);

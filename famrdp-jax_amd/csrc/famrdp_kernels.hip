@@ -1429,8 +1429,8 @@ namespace famrdp {
   X(7, 8, 8, 8, 512)              \
   X(8, 2, 8, 16, 256)             \
   X(9, 4, 8, 8, 320)
-// i-marching kernel: (id, TJ, TK, segment length L, waves per SIMD); its
-// tile table holds (2 x segment index + strip bit, j0, k0) per march_tiling.
+// i-marching kernel: (id, TJ, TK, segment length L about which march_len
+// chooses, waves per SIMD); its tile table holds (2 x segment index + strip bit, j0, k0) per march_tiling.
 // The 10-plane segments of 18 are for blocks of about 100^3 cells, which the
 // longer segments leave with fewer workgroups than the GPU holds at once.
 #define FAMRDP_MARCH_VARIANTS(X) \
@@ -1481,11 +1481,18 @@ inline void tile_dims(int v, int& ti, int& tj, int& tk) {
   }
 }
 
-// Workgroups of a stage of one block with variant v.
+// Planes a workgroup of variant v takes along i when these blocks are launched
+// together: a tile's, or at most a segment's.
+inline int variant_len(int v, int nblocks, const int32_t* dims, int ncu) {
+  int TI, TJ, TK;
+  tile_dims(v, TI, TJ, TK);
+  return is_march_variant(v) ? march_len(TJ, TK, TI, nblocks, dims, 2 * ncu) : TI;
+}
+
+// Tiles of one block with variant v (not a marching one).
 inline int64_t stage_tiles(int v, int ni, int nj, int nk) {
   int TI, TJ, TK;
   tile_dims(v, TI, TJ, TK);
-  if (is_march_variant(v)) return (int64_t)march_nseg(ni, TI) * march_tiling(TJ, TK, nj, nk).count();
   return (int64_t)((ni + TI - 1) / TI) * ((nj + TJ - 1) / TJ) * ((nk + TK - 1) / TK);
 }
 
@@ -1498,20 +1505,29 @@ inline int64_t stage_tiles(int v, int ni, int nj, int nk) {
 //   20 wide 4x4x8    1.5 + 5.6 n    (32^3 7.4, 44^3 17.7)
 //    1 fused 4x8x16  15.3 n         (44^3 15.6, 60^3 31.1, 72^3 58.3)
 //   12 re-staging    5 + 6.5 n      (52^3 24.3, 80^3 59.7, 104^3 126.6)
-//   18 marching      45 n, 65 at least (80^3 68, 96^3 87.7, 124^3 171)
+//   18 marching      6.9 per plane of march_len's count, 4.7 with no more than
+//                    a workgroup per CU (72^3 49.6, 96^3 65.4, 112^3 107, 124^3 147)
 // The fused kernel of 8x4x8 cells that every untuned block took before:
 // 12.1 at 20^3, 27.5 at 52^3, 65.8 at 80^3, 109 at 96^3, 258 at 124^3.
 inline int default_variant(int nblocks, const int32_t* dims, int ncu, bool fits32) {
-  struct Line { int v; double base, per, least; };
-  constexpr Line lines[] = {
-      {19, 3.5, 1.75, 0}, {20, 1.5, 5.6, 0}, {1, 0, 15.3, 0}, {12, 5, 6.5, 0}, {18, 0, 45, 65}};
+  struct Line { int v; double base, per; };
+  constexpr Line lines[] = {{19, 3.5, 1.75}, {20, 1.5, 5.6}, {1, 0, 15.3}, {12, 5, 6.5}, {18, 0, 6.9}};
   int best = 12;
   double best_t = 1e300;
   for (const Line& l : lines) {
     if (!fits32 && (is_march_variant(l.v) || is_wide_variant(l.v))) continue;
-    int64_t n = 0;
-    for (int b = 0; b < nblocks; ++b) n += stage_tiles(l.v, dims[3 * b], dims[3 * b + 1], dims[3 * b + 2]);
-    const double t = std::max(l.least, l.base + l.per * (double)((n + ncu - 1) / ncu));
+    double t;
+    if (is_march_variant(l.v)) {
+      int TI, TJ, TK;
+      int64_t n = 0;
+      tile_dims(l.v, TI, TJ, TK);
+      march_len(TJ, TK, TI, nblocks, dims, 2 * ncu, &t, &n);
+      t *= n <= ncu ? 4.7 : l.per;
+    } else {
+      int64_t n = 0;
+      for (int b = 0; b < nblocks; ++b) n += stage_tiles(l.v, dims[3 * b], dims[3 * b + 1], dims[3 * b + 2]);
+      t = l.base + l.per * (double)((n + ncu - 1) / ncu);
+    }
     if (t < best_t) { best_t = t; best = l.v; }
   }
   return best;
@@ -1538,11 +1554,14 @@ inline void launch_stage_lim(int v, const BlockDesc& d, int stage, const StageGa
     return;
     FAMRDP_SPLIT_VARIANTS(FAMRDP_SL)
 #undef FAMRDP_SL
-#define FAMRDP_ML(id, b, c, l, w)                                                                \
-  case id:                                                                                       \
-    k_stage_march<b, c, l, LIM, w><<<nti * march_tiling(b, c, d.nj, d.nk).count(), b * c, 0, st>>>( \
-        d, stage, gas, dt);                                                                      \
-    return;
+#define FAMRDP_ML(id, b, c, l, w)                                                                          \
+  case id: {                                                                                               \
+    const int32_t dims[3] = {d.ni, d.nj, d.nk};                                                            \
+    const int len = variant_len(v, 1, dims, ncu);                                                          \
+    const int nwg = march_nseg(d.ni, len) * march_tiling(b, c, d.nj, d.nk).count();                        \
+    k_stage_march<b, c, LIM, w><<<nwg, b * c, 0, st>>>(d, stage, gas, dt, len);                            \
+    return;                                                                                                \
+  }
     FAMRDP_MARCH_VARIANTS(FAMRDP_ML)
 #undef FAMRDP_ML
 #define FAMRDP_WL(id, a, b, c) \
@@ -1566,10 +1585,10 @@ inline void launch_fused(int v, const BlockDesc& d, int stage, const Gas& gas, i
 }
 
 // One stage of every block in one launch (two for the split pair) over a tile
-// table built for v.
+// table built for v (len: variant_len of all of them).
 template <int LIM>
 inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3* tiles, int ntiles, int stage,
-                                     const StageGas& gas, double dt, int ncu, hipStream_t st) {
+                                     const StageGas& gas, double dt, int len, hipStream_t st) {
   switch (v) {
 #define FAMRDP_TB(id, a, b, c, rs, w)                                                                       \
   case id:                                                                                                   \
@@ -1584,9 +1603,9 @@ inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3
     return;
     FAMRDP_SPLIT_VARIANTS(FAMRDP_SB)
 #undef FAMRDP_SB
-#define FAMRDP_MB(id, b, c, l, w)                                                                      \
-  case id:                                                                                              \
-    k_stage_march_batched<b, c, l, LIM, w><<<ntiles, b * c, 0, st>>>(blocks, tiles, stage, gas, dt);    \
+#define FAMRDP_MB(id, b, c, l, w)                                                                        \
+  case id:                                                                                                \
+    k_stage_march_batched<b, c, LIM, w><<<ntiles, b * c, 0, st>>>(blocks, tiles, stage, gas, dt, len);    \
     return;
     FAMRDP_MARCH_VARIANTS(FAMRDP_MB)
 #undef FAMRDP_MB
@@ -1600,10 +1619,10 @@ inline void launch_stage_batched_lim(int v, const BlockDesc* blocks, const Tile3
 }
 
 inline void launch_fused_batched(int v, const BlockDesc* blocks, const Tile3* tiles, int ntiles, int stage,
-                                 const Gas& gas, int lim, double dt, int ncu, hipStream_t st) {
+                                 const Gas& gas, int lim, double dt, int len, hipStream_t st) {
   const StageGas sg = stage_gas(gas);
-  if (lim == LIM_VANLEER) launch_stage_batched_lim<LIM_VANLEER>(v, blocks, tiles, ntiles, stage, sg, dt, ncu, st);
-  else launch_stage_batched_lim<LIM_MINMOD>(v, blocks, tiles, ntiles, stage, sg, dt, ncu, st);
+  if (lim == LIM_VANLEER) launch_stage_batched_lim<LIM_VANLEER>(v, blocks, tiles, ntiles, stage, sg, dt, len, st);
+  else launch_stage_batched_lim<LIM_MINMOD>(v, blocks, tiles, ntiles, stage, sg, dt, len, st);
 }
 
 }  // namespace famrdp

@@ -460,9 +460,9 @@ __device__ __forceinline__ void march_tile(double* lds, const BlockDesc& b, int 
 
 // Plain launch: grid = segments x march_tiling(...).count(), XCD-remapped.
 // Segments split the block's planes evenly (lengths differ by at most one).
-template <int TJ, int TK, int L, int LIM, int WPE>
+template <int TJ, int TK, int LIM, int WPE>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_stage_march(BlockDesc b, int stage, StageGas gas, double dt) {
+k_stage_march(BlockDesc b, int stage, StageGas gas, double dt, int len) {
   __shared__ double lds[MarchGeom<TJ, TK>::NLDS];
   const int w = xcd_remap(blockIdx.x, gridDim.x);
   const MarchTiling mt = march_tiling(TJ, TK, b.nj, b.nk);
@@ -470,22 +470,22 @@ k_stage_march(BlockDesc b, int stage, StageGas gas, double dt) {
   int j0, k0, tr;
   march_tile_of(mt, TJ, TK, w - seg * nt, j0, k0, tr);
   int pA, pB;
-  march_segment_bounds(seg, march_nseg(b.ni, L), b.ni, pA, pB);
+  march_segment_bounds(seg, march_nseg(b.ni, len), b.ni, pA, pB);
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
   double* qout = stage == 1 ? b.q1 : (stage == 2 ? b.q2 : b.q);
   march_tile<TJ, TK, LIM>(lds, b, tr, j0, k0, pA, pB, qin, qout, stage, gas, dt);
 }
 
 // Batched launch over a tile table whose i0 is 2 x segment index + strip bit.
-template <int TJ, int TK, int L, int LIM, int WPE>
+template <int TJ, int TK, int LIM, int WPE>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_stage_march_batched(const BlockDesc* __restrict__ blocks, const Tile3* __restrict__ tiles, int stage, StageGas gas,
-                      double dt) {
+                      double dt, int len) {
   __shared__ double lds[MarchGeom<TJ, TK>::NLDS];
   const Tile3 tl = tiles[xcd_remap(blockIdx.x, gridDim.x)];
   const BlockDesc& b = blocks[tl.block];
   int pA, pB;
-  march_segment_bounds(tl.i0 >> 1, march_nseg(b.ni, L), b.ni, pA, pB);
+  march_segment_bounds(tl.i0 >> 1, march_nseg(b.ni, len), b.ni, pA, pB);
   const double* qin = stage == 1 ? b.q : (stage == 2 ? b.q1 : b.q2);
   double* qout = stage == 1 ? b.q1 : (stage == 2 ? b.q2 : b.q);
   march_tile<TJ, TK, LIM>(lds, b, tl.i0 & 1, tl.j0, tl.k0, pA, pB, qin, qout, stage, gas, dt);

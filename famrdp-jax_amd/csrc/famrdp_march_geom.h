@@ -91,6 +91,39 @@ __host__ __device__ inline void march_tile_of(const MarchTiling& m, int TJ, int 
   }
 }
 
+// Planes per segment (at most) for blocks marched in one launch: near L, so
+// that the workgroups fill whole rounds of the `slots` the GPU holds at once.
+// A launch takes its rounds times a segment's planes and about 3.5 more (the
+// planes it starts and ends with): of the lengths from 0.7 to 1.4 L the one
+// for which that is least (units: that many planes).  A stage near L = 10
+// against 10 planes always, us: 60^3 43.6 and 59.5, 88^3 76.5 and 99.7, 96^3
+// 65.4 and 87.2, 112^3 107 and 139, 124^3 147 and 170, 204 x 104 x 54 111 and
+// 138; near 20 against 20: 124^3 137 and 148, 140^3 236 and 281.
+inline int march_len(int TJ, int TK, int L, int nblocks, const int32_t* dims, int slots, double* units = nullptr,
+                     int64_t* workgroups = nullptr) {
+  int best = L;
+  double best_t = 0.0;
+  for (int len = (7 * L + 9) / 10; len <= 14 * L / 10; ++len) {
+    int64_t wgs = 0;
+    int longest = 1;
+    for (int b = 0; b < nblocks; ++b) {
+      const int32_t* d = dims + 3 * b;
+      const int n = march_nseg(d[0], len);
+      wgs += (int64_t)n * march_tiling(TJ, TK, d[1], d[2]).count();
+      longest = longest > (d[0] + n - 1) / n ? longest : (d[0] + n - 1) / n;
+    }
+    const double t = (double)((wgs + slots - 1) / slots) * (longest + 3.5);
+    const bool nearer = (len < L ? L - len : len - L) < (best < L ? L - best : best - L);
+    if (best_t == 0.0 || t < best_t || (t == best_t && nearer)) {
+      best_t = t;
+      best = len;
+      if (units) *units = t;
+      if (workgroups) *workgroups = wgs;
+    }
+  }
+  return best;
+}
+
 template <int TJ, int TK>
 struct MarchGeom {
   static constexpr int NT = TJ * TK;                        // threads: one per tile column

@@ -159,7 +159,7 @@ int famrdp_step_stages(famrdp_plan* plan, double* const* q, const double* const*
  * and 10-13 are tile shapes of the fused stage kernel (4 and 10-13 stage the
  * primitives twice to need less LDS), 5-9 tile shapes of the split pair
  * (viscous tensor kernel + stage kernel), 14-18 shapes of the i-marching
- * kernel (a TJ x TK column walks a segment of TI planes along i), 19-20 tiles
+ * kernel (TJ x TK columns walk segments of about TI planes along i), 19-20 tiles
  * of the wide kernel (small blocks: a thread per viscous tensor and per face).
  * 14-20: same bits as the fused kernel; blocks under 59,652,323 cells, else
  * set_tile returns FAMRDP_E_INVALID and the autotuner reports 1e30 ms and skips
