@@ -399,13 +399,13 @@ FD void roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   const double Q = fma(w, dun, (w1 - w5) * c) * rA;
   const double P = (pl[4] + pr[4]) + Q;
   const double mL = rhoL * unL, mR = rhoR * unR;
-  const double iL = fma(-b, sa, mL) + w, iR = fma(-a, sa, mR) - w;
+  const double eL = fma(-b, sw, mL), eR = fma(-a, sw, mR);
+  const double iL = fma(-b, w2, eL) + w, iR = fma(-a, w2, eR) - w;
   F[0] = (mL + mR) - sa;
   F[1] = fma(S[0], P, fma(iR, uR, iL * uL));
   F[2] = fma(S[1], P, fma(iR, vR, iL * vL));
   F[3] = fma(S[2], P, fma(iR, wR, iL * wL));
   const double ud = fma(wh, wR - wL, fma(vh, vR - vL, uh * (uR - uL)));
-  const double eL = fma(-b, sw, mL), eR = fma(-a, sw, mR);
   F[4] = fma(0.5, fma(-w2, q2, fma(HR, eR, eL * HL)), fma(un, Q, -(w * ud)));
 }
 
