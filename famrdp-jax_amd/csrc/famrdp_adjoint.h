@@ -104,25 +104,26 @@ FD double rsq_hd(double x) {
 // reciprocals and roots, and swept backwards; the same identities of the Roe
 // average that shorten the forward flux leave about 280 instructions where
 // the sweep through conservative jumps took 430, and far fewer values alive.
-// cg2 = 2 g / (g - 1), gm1h = (g - 1) / 2.
+// Both weights a and b = 1 - a as there; b_a is the cotangent of a with b
+// following it.  cg2 = 2 g / (g - 1), gm1h = (g - 1) / 2.
 FD void roe_flux2_vjp(const double pl[5], const double pr[5], const double S[3], double cg2, double gm1h,
                       const double f[5], double lpl[5], double lpr[5]) {
   const double rhoL = max_floor(pl[0], 1e-300), rhoR = max_floor(pr[0], 1e-300);
   const double isL = rsq_hd(rhoL), isR = rsq_hd(rhoR);
   const double sqL = rhoL * isL, sqR = rhoR * isR;
   const double rs = rcp_hd(sqL + sqR);
-  const double a = sqR * rs;
+  const double a = sqR * rs, b = sqL * rs;
   const double irL = isL * isL, irR = isR * isR;
   const double HL = cg2 * (pl[4] * irL) + (pl[1] * pl[1] + pl[2] * pl[2] + pl[3] * pl[3]);
   const double HR = cg2 * (pr[4] * irR) + (pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3]);
   double du[3], uh[3];
   for (int m = 0; m < 3; ++m) {
     du[m] = pr[1 + m] - pl[1 + m];
-    uh[m] = pl[1 + m] + a * du[m];
+    uh[m] = a * pr[1 + m] + b * pl[1 + m];
   }
-  const double dH = HR - HL;
-  const double hq = (HL + a * dH) - (uh[0] * uh[0] + uh[1] * uh[1] + uh[2] * uh[2]);
-  const double c2raw = gm1h * hq;
+  const double Hh = a * HR + b * HL;
+  const double q2 = uh[0] * uh[0] + uh[1] * uh[1] + uh[2] * uh[2];
+  const double c2raw = gm1h * (Hh - q2);
   const double c2 = max_floor(c2raw, 1e-30);
   const double isc = rsq_hd(c2);
   const double rc2 = isc * isc, c = c2 * isc;
@@ -131,7 +132,7 @@ FD void roe_flux2_vjp(const double pl[5], const double pr[5], const double S[3],
   const double rA = rsq_hd(nn);
   const double A = nn * rA, C = c * A;
   const double unL = pl[1] * S[0] + pl[2] * S[1] + pl[3] * S[2], unR = pr[1] * S[0] + pr[2] * S[1] + pr[3] * S[2];
-  const double dS = unR - unL, un = unL + a * dS;
+  const double dS = unR - unL, un = a * unR + b * unL;
   const double aun = fabs(un), sun = dabs(un);
   const double base = aun + C, h = rcp_hd(0.2 * base);
   const double l1 = un - C, l5 = un + C;
@@ -143,29 +144,30 @@ FD void roe_flux2_vjp(const double pl[5], const double pr[5], const double S[3],
   const double rr = rhoL * rhoR, rcd = rr * c * dun, hc = 0.5 * rc2;
   const double a1 = (dp - rcd) * hc, a5 = (dp + rcd) * hc, a23 = dr - dp * rc2;
   const double w1 = al1 * a1, w5 = al5 * a5, w2 = aun * a23, sLR = sqL * sqR, w = aun * sLR;
-  const double sa = (w1 + w5) + w2;
+  const double sw = w1 + w5, sa = sw + w2;
   const double Q = (w * dun + (w1 - w5) * c) * rA;
-  const double mR = rhoR * unR;
-  const double F0 = (rhoL * unL + mR) - sa;
-  const double k = mR - a * sa, kw = k - w;
+  const double eL = rhoL * unL - b * sw, eR = rhoR * unR - a * sw;
+  const double iL = (eL - b * w2) + w, iR = (eR - a * w2) - w;
   const double ud = uh[0] * du[0] + uh[1] * du[1] + uh[2] * du[2];
 
   // ---- backwards: momentum and energy components
   const double h4 = 0.5 * f[4];
-  const double b_F0 = f[0] + (f[1] * pl[1] + f[2] * pl[2] + f[3] * pl[3]) + h4 * HL;
-  const double b_kw = f[1] * du[0] + f[2] * du[1] + f[3] * du[2];
+  const double fu = f[1] * du[0] + f[2] * du[1] + f[3] * du[2];
+  const double b_mL = f[0] + (f[1] * pl[1] + f[2] * pl[2] + f[3] * pl[3]) + h4 * HL;
+  const double b_mR = f[0] + (f[1] * pr[1] + f[2] * pr[2] + f[3] * pr[3]) + h4 * HR;
   const double b_P = f[1] * S[0] + f[2] * S[1] + f[3] * S[2];
   const double b_ud = -f[4] * w;
-  double b_HL = h4 * F0, b_dH = h4 * k, b_hq = h4 * w2;
-  const double b_k = h4 * dH + b_kw;
+  const double b_HL0 = h4 * eL, b_HR0 = h4 * eR;
   double b_un = f[4] * Q;
   const double q = (f[4] * un + b_P) * rA;
-  const double b_w = q * dun - f[4] * ud - b_kw;
+  const double b_w = q * dun - f[4] * ud - fu;
   double b_dun = q * w;
-  const double b_sa = -b_F0 - b_k * a;
-  double b_a = -b_k * sa;
+  const double b_sa = -(f[0] + (f[1] * uh[0] + f[2] * uh[1] + f[3] * uh[2]));
+  const double dH = HR - HL;
+  double b_a = -sa * fu - h4 * (sw * dH);
   // ---- wave strengths
-  const double b_w1 = q * c + b_sa, b_w5 = b_sa - q * c, b_w2 = h4 * hq + b_sa;
+  const double b_sw = b_sa - h4 * Hh;
+  const double b_w1 = b_sw + q * c, b_w5 = b_sw - q * c, b_w2 = b_sa - h4 * q2;
   double b_c = q * (w1 - w5);
   const double b_aun = b_w2 * a23 + b_w * sLR, b_a23 = b_w2 * aun, b_sLR = b_w * aun;
   const double b_al1 = b_w1 * a1, b_al5 = b_w5 * a5;
@@ -184,29 +186,26 @@ FD void roe_flux2_vjp(const double pl[5], const double pr[5], const double S[3],
   b_c += (b_base + (g5 - g1)) * A;
   // ---- normal velocities
   b_a += b_un * dS;
-  const double b_dS = b_un * a + b_dun * rA;
-  const double b_mR = b_F0 + b_k;
-  const double b_unL = (b_un - b_dS) + b_F0 * rhoL, b_unR = b_dS + b_mR * rhoR;
+  const double b_dS = b_dun * rA;
+  const double b_unL = (b * b_un - b_dS) + b_mL * rhoL, b_unR = (a * b_un + b_dS) + b_mR * rhoR;
   // ---- sound speed, Roe average
   const double b_c2 = rc2 * (0.5 * b_c * c - b_rc2 * rc2);
-  b_hq += gm1h * (b_c2 * dmax_floor(c2raw, 1e-30));
-  b_HL += b_hq;
-  b_dH += a * b_hq;
+  const double b_hq = gm1h * (b_c2 * dmax_floor(c2raw, 1e-30));
+  const double b_HL = b_HL0 + b * b_hq, b_HR = b_HR0 + a * b_hq;
+  const double b_q2 = -2.0 * (h4 * w2 + b_hq);
   b_a += b_hq * dH;
-  b_HL -= b_dH;
-  double b_rhoL = b_F0 * unL + b_rr * rhoR - b_a23, b_rhoR = b_mR * unR + b_rr * rhoL + b_a23;
+  double b_rhoL = b_mL * unL + b_rr * rhoR - b_a23, b_rhoR = b_mR * unR + b_rr * rhoL + b_a23;
   for (int m = 0; m < 3; ++m) {
-    const double b_uh = b_ud * du[m] - 2.0 * uh[m] * b_hq;
-    const double b_du = kw * f[1 + m] + b_ud * uh[m] + a * b_uh;
+    const double b_uh = b_ud * du[m] + b_q2 * uh[m], b_du = b_ud * uh[m];
     b_a += b_uh * du[m];
-    lpl[1 + m] = F0 * f[1 + m] + (b_uh - b_du) + b_unL * S[m] + 2.0 * b_HL * pl[1 + m];
-    lpr[1 + m] = b_du + b_unR * S[m] + 2.0 * b_dH * pr[1 + m];
+    lpl[1 + m] = iL * f[1 + m] + (b * b_uh - b_du) + b_unL * S[m] + 2.0 * b_HL * pl[1 + m];
+    lpr[1 + m] = iR * f[1 + m] + (a * b_uh + b_du) + b_unR * S[m] + 2.0 * b_HR * pr[1 + m];
   }
-  const double cL = b_HL * cg2 * irL, cR = b_dH * cg2 * irR;
+  const double cL = b_HL * cg2 * irL, cR = b_HR * cg2 * irR;
   lpl[4] = b_P - b_dp + cL;
   lpr[4] = b_P + b_dp + cR;
   const double b_s = b_a * rs;                 // a = sqR / (sqL + sqR)
-  const double b_sL = b_sLR * sqR - b_s * a, b_sR = b_sLR * sqL + b_s * (1.0 - a);
+  const double b_sL = b_sLR * sqR - b_s * a, b_sR = b_sLR * sqL + b_s * b;
   b_rhoL += 0.5 * b_sL * isL - cL * (pl[4] * irL);
   b_rhoR += 0.5 * b_sR * isR - cR * (pr[4] * irR);
   lpl[0] = b_rhoL * dmax_floor(pl[0], 1e-300);

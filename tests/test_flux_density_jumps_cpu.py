@@ -4,7 +4,10 @@ the lighter one, against flux/roe.py:21-85 in extended precision.
 
 Tolerance: the flux is about 140 operations none of which cancels terms much
 larger than the largest flux component, so its error is a few tens of roundings
-of that component: 64 of 2^-53."""
+of that component: 64 of 2^-53.  The reverse is held to
+the same number of roundings of what its result depends on: of the largest of
+its ten components and of what relative changes of the ten inputs would move it
+by (a light side's density cotangent can cancel to far less than its terms)."""
 import ctypes
 import os
 import shutil
@@ -57,5 +60,68 @@ def test_flux_between_light_and_heavy(hc, ratio, full):
     A = np.sqrt((x(S) ** 2).sum(axis=0))
     ref = (2 * A * ON.roe_flux(ON.prim_to_cons(x(pl), g), ON.prim_to_cons(x(pr), g), x(S) / A, gamma=g)).T
     err = np.abs(F - ref).max(axis=1) / np.abs(ref).max(axis=1)
+    print(f"ratio {ratio:g}: max {float(err.max()):.2e}")
+    assert float(err.max()) <= TOL
+
+
+def _vjp_reference(pl, pr, S, f):
+    """Cotangents of flux/roe.py:21-85 times 2 |S|, in extended precision: the complex step through the formulas."""
+    g, eps = np.longdouble(G), np.longdouble(1e-30)
+    mag = lambda z: np.where(z.real >= 0, z, -z)  # noqa: E731
+    out = np.zeros((len(pl), 10), dtype=np.longdouble)
+    A = np.sqrt((S.astype(np.longdouble) ** 2).sum(axis=1))
+    n = (S / A[:, None]).T
+    for k in range(10):
+        x = np.concatenate([pl, pr], axis=1).astype(np.clongdouble)
+        x[:, k] += 1j * eps
+        def conserved(p):
+            ke = 0.5 * (p[1] ** 2 + p[2] ** 2 + p[3] ** 2)
+            return np.stack([p[0], p[0] * p[1], p[0] * p[2], p[0] * p[3], p[4] / (g - 1) + p[0] * ke])
+        L, R = x[:, :5].T, x[:, 5:].T
+        UL, UR = conserved(L), conserved(R)
+        H = lambda U, p: (U[4] + p[4]) / U[0]  # noqa: E731
+        sL, sR = np.sqrt(L[0]), np.sqrt(R[0])
+        uh = (sL * L[1:4] + sR * R[1:4]) / (sL + sR)
+        Hh = (sL * H(UL, L) + sR * H(UR, R)) / (sL + sR)
+        q2 = (uh ** 2).sum(axis=0)
+        c2 = (g - 1) * (Hh - 0.5 * q2)
+        c, un, rho = np.sqrt(c2), (uh * n).sum(axis=0), sL * sR
+        e = np.longdouble("0.1") * (mag(un) + c)
+        fix = lambda l: np.where(mag(l).real >= e.real, mag(l), 0.5 * (l * l / e + e))  # noqa: E731
+        d = UR - UL
+        dp = (g - 1) * (d[4] - (uh * d[1:4]).sum(axis=0) + 0.5 * q2 * d[0])
+        dn = (d[1:4] * n).sum(axis=0) - un * d[0]
+        a1, a5, a2 = (dp - rho * c * dn) / (2 * c2), (dp + rho * c * dn) / (2 * c2), d[0] - dp / c2
+        t = (d[1:4] - uh * d[0]) / rho
+        t = t - (t * n).sum(axis=0) * n
+        one = np.ones_like(un)
+        wave = lambda s: np.stack([one, *(uh + s * c * n), Hh + s * c * un])  # noqa: E731
+        shear = np.stack([0 * one, *(rho * t), rho * (uh * t).sum(axis=0)])
+        diss = fix(un - c) * a1 * wave(-1) + fix(un + c) * a5 * wave(1) + \
+            mag(un) * (a2 * np.stack([one, *uh, 0.5 * q2]) + shear)
+        def physical(U, p):
+            v = (p[1:4] * n).sum(axis=0)
+            return np.stack([U[0] * v, *(U[1:4] * v + p[4] * n), (U[4] + p[4]) * v])
+        F = A * (physical(UL, L) + physical(UR, R) - diss)
+        out[:, k] = (f.T * F).sum(axis=0).imag / eps
+    return out
+
+
+@pytest.mark.parametrize("ratio", RATIOS)
+def test_reverse_between_light_and_heavy(hc, ratio):
+    n = 400
+    pl, pr, S = faces(ratio, n, 57)
+    f = np.random.default_rng(58).uniform(-1, 1, (n, 5))
+    lp = np.zeros((2, n, 5))
+    P = lambda a: np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    hc.hc_roe_flux2_vjp(n, P(pl), P(pr), P(S), ctypes.c_double(G), P(f), lp[0].ctypes.data_as(ctypes.c_void_p),
+                        lp[1].ctypes.data_as(ctypes.c_void_p))
+    ref = _vjp_reference(pl, pr, S, f)
+    move = np.zeros(n, dtype=np.longdouble)
+    for k in range(10):
+        x = np.concatenate([pl, pr], axis=1)
+        x[:, k] *= 1 + 1e-6
+        move += np.abs(_vjp_reference(x[:, :5], x[:, 5:], S, f) - ref).max(axis=1) / 1e-6
+    err = np.abs(np.concatenate([lp[0], lp[1]], axis=1) - ref).max(axis=1) / (np.abs(ref).max(axis=1) + move)
     print(f"ratio {ratio:g}: max {float(err.max()):.2e}")
     assert float(err.max()) <= TOL
