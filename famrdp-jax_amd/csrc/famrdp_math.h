@@ -216,17 +216,20 @@ FD double rcp(double x) {
 #endif
 }
 
-// sqrt(x) from the hardware reciprocal square-root seed and one cubic
-// correction s (1 + e/2 + 3 e^2 / 8), e = 1 - s y measured on the rounded
-// s = x y.  IEEE special cases: +-0 and +inf are returned as they are (the
-// seed gives inf and 0 there), x < 0 and NaN give NaN (the seed is NaN).
+// sqrt(x) from the hardware reciprocal square-root seed: one cubic correction
+// s (1 + e/2 + 3 e^2 / 8), e = 1 - s y measured on the rounded s = x y, then
+// the residual x - g^2 of the result, which leaves little but the last rounding
+// (without it 0.75 ulp and 0.32 rms instead of 0.50 and 0.29).  IEEE special
+// cases: +-0 and +inf are returned as they are (the seed gives inf and 0
+// there), x < 0 and NaN give NaN (the seed is NaN).
 FD double fsqrt(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   EXACT_FP
   const double y = __builtin_amdgcn_rsq(x);
   const double s = x * y;
   const double e = fma(-s, y, 1.0);
-  const double g = fma(s * e, fma(e, 0.375, 0.5), s);
+  const double g0 = fma(s * e, fma(e, 0.375, 0.5), s);
+  const double g = fma(fma(-g0, g0, x), 0.5 * y, g0);
   // one class test: -0, +0, +inf
   return __builtin_amdgcn_class(x, (1 << 5) | (1 << 6) | (1 << 9)) ? x : g;
 #else
