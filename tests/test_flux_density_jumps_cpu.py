@@ -15,6 +15,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import numerics as ON
 
@@ -125,3 +126,26 @@ def test_reverse_between_light_and_heavy(hc, ratio):
     err = np.abs(np.concatenate([lp[0], lp[1]], axis=1) - ref).max(axis=1) / (np.abs(ref).max(axis=1) + move)
     print(f"ratio {ratio:g}: max {float(err.max()):.2e}")
     assert float(err.max()) <= TOL
+
+
+@pytest.mark.parametrize("jump", [1.0, 1e-3])
+def test_reverse_is_as_exact_as_autograd_in_64_bits(hc, jump):
+    """At equal densities, states apart or nearly equal: rms error no larger than autograd's through flux/roe.py."""
+    n = 2000
+    pl, pr, S = faces(1.0, n, 71)
+    pr = pl + jump * (pr - pl)
+    f = np.random.default_rng(72).uniform(-1, 1, (n, 5))
+    lp = np.zeros((2, n, 5))
+    P = lambda a: np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    hc.hc_roe_flux2_vjp(n, P(pl), P(pr), P(S), ctypes.c_double(G), P(f), lp[0].ctypes.data_as(ctypes.c_void_p),
+                        lp[1].ctypes.data_as(ctypes.c_void_p))
+    tl, tr, ts = torch.tensor(pl.T, requires_grad=True), torch.tensor(pr.T, requires_grad=True), torch.tensor(S.T)
+    A = torch.sqrt((ts ** 2).sum(dim=0))
+    F = 2.0 * A * ON.roe_flux(ON.prim_to_cons(tl, G), ON.prim_to_cons(tr, G), ts / A, gamma=G)
+    (F * torch.tensor(f.T)).sum().backward()
+    ref = _vjp_reference(pl, pr, S, f)
+    rms = lambda x: float(np.sqrt((((x - ref) / np.abs(ref).max(axis=1)[:, None]) ** 2).mean()))  # noqa: E731
+    ours = rms(np.concatenate([lp[0], lp[1]], axis=1))
+    theirs = rms(np.concatenate([tl.grad.numpy().T, tr.grad.numpy().T], axis=1))
+    print(f"jump {jump:g}: {ours:.2e}, autograd {theirs:.2e}")
+    assert ours <= theirs
