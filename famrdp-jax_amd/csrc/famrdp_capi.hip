@@ -556,9 +556,8 @@ int famrdp_viscous_rhs(const double* q, const double* kxyz, double* rhs, int32_t
                        const famrdp_gas* gas, double* work, void* stream) {
   if (ni < 1 || nj < 1 || nk < 1 || !q || !kxyz || !rhs || !gas || !work)
     return fail(FAMRDP_E_INVALID, "viscous_rhs: bad arguments");
-  const Gas g = to_gas(gas);
   k_viscous_rhs<4, 8, 8><<<rhs_grid<4, 8, 8>(ni, nj, nk), WideGeom<4, 8, 8>::NGW, 0, S(stream)>>>(q, kxyz, rhs, ni, nj, nk,
-                                                                                    stage_gas(g), g.mu0, g.gamma);
+                                                                                    to_gas(gas));
   LAUNCH_CHECK();
   return FAMRDP_OK;
 }

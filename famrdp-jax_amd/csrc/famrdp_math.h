@@ -272,12 +272,16 @@ FD double rsq1(double x) {
 #endif
 }
 
-// van Leer with the division as a reciprocal (stage-kernel form)
+// van Leer with the division as a reciprocal (stage-kernel form); FULL corrects
+// the quotient by its residual: rounded once, like a division
+template <bool FULL = false>
 FD double vanleer_fast(double a, double b) {
   EXACT_FP
   const double ab = a + b;
   const double safe = fabs(ab) > 1e-30 ? ab : 1.0;
-  const double r = 2.0 * a * b * rcp(safe);
+  const double n = 2.0 * a * b, ri = rcp(safe);
+  double r = n * ri;
+  if constexpr (FULL) r = fma(fma(-safe, r, n), ri, r);
   return (a * b > 0.0) ? r : 0.0;
 }
 
@@ -361,29 +365,45 @@ DF void prim_and_temp(const double q[5], const StageGas& gas, double pv[6]) {
 // with one-step seeds 7e-15 and 1.5e-14, as with conservative jumps.  The floors
 // are min/max, which drop a NaN: a NaN primitive makes the pressure NaN, and
 // dp carries it into every component.
+// FULL: every root and reciprocal rounded once (ten seeds instead of six), which
+// makes the flux as exact as the reference's formulas in IEEE arithmetic or more
+// (rms 1.5e-16 to their 2.5e-16 on those faces, 7.3e-16 to 8.8e-16 at twice the
+// speed of sound; with reciprocal roots and their squares 9.5e-16 there).
 template <bool FULL = false>
 FD void roe_flux2(const double pl[5], const double pr[5], const double S[3], const StageGas& gas, double F[5]) {
   EXACT_FP
   auto recip = [](double x) { return FULL ? rcp(x) : rcp1(x); };
-  auto root = [](double x) { return FULL ? rsq_acc(x) : rsq1(x); };
   const double rhoL = fmax(pl[0], 1e-300), rhoR = fmax(pr[0], 1e-300);
-  const double isL = root(rhoL), isR = root(rhoR);
-  const double sqL = rhoL * isL, sqR = rhoR * isR;
+  double sqL, sqR, irL, irR;                                      // sqrt(rho), 1 / rho
+  if constexpr (FULL) {
+    sqL = fsqrt(rhoL), sqR = fsqrt(rhoR);
+    irL = rcp(rhoL), irR = rcp(rhoR);
+  } else {
+    const double isL = rsq1(rhoL), isR = rsq1(rhoR);
+    sqL = rhoL * isL, sqR = rhoR * isR;
+    irL = isL * isL, irR = isR * isR;
+  }
   const double rs = recip(sqL + sqR);
   const double a = sqR * rs, b = sqL * rs;
   const double uL = pl[1], vL = pl[2], wL = pl[3], uR = pr[1], vR = pr[2], wR = pr[3];
   // twice the total enthalpies: 2 g/(g-1) p/rho + |u|^2
   const double kL = fma(wL, wL, fma(vL, vL, uL * uL)), kR = fma(wR, wR, fma(vR, vR, uR * uR));
-  const double HL = fma(gas.cg2, pl[4] * (isL * isL), kL), HR = fma(gas.cg2, pr[4] * (isR * isR), kR);
+  const double HL = fma(gas.cg2, pl[4] * irL, kL), HR = fma(gas.cg2, pr[4] * irR, kR);
   const double uh = fma(a, uR, b * uL), vh = fma(a, vR, b * vL), wh = fma(a, wR, b * wL), Hh = fma(a, HR, b * HL);
   const double q2 = fma(wh, wh, fma(vh, vh, uh * uh));
   const double c2 = fmax(gas.gm1h * (Hh - q2), 1e-30);
-  const double isc = root(c2);
-  const double rc2 = isc * isc, c = c2 * isc;
   // |S| and 1/|S|; a zero face keeps a harmless 1e-140
   const double nn = fmax(fma(S[2], S[2], fma(S[1], S[1], S[0] * S[0])), 1e-280);
-  const double rA = root(nn);
-  const double C = c * (nn * rA);
+  double c, rc2, A, rA;                                           // rc2 = 1 / c^2
+  if constexpr (FULL) {
+    c = fsqrt(c2), rc2 = rcp(c2);
+    A = fsqrt(nn), rA = rcp(A);
+  } else {
+    const double isc = rsq1(c2);
+    rc2 = isc * isc, c = c2 * isc;
+    rA = rsq1(nn), A = nn * rA;
+  }
+  const double C = c * A;
   const double unL = fma(wL, S[2], fma(vL, S[1], uL * S[0])), unR = fma(wR, S[2], fma(vR, S[1], uR * S[0]));
   const double un = fma(a, unR, b * unL);
   const double base = fabs(un) + C;                              // eps = 0.1 base
@@ -439,7 +459,7 @@ FD void muscl_cell(const double pvm[5], const double pv[5], const double pvp[5],
 
 // The reconstructed states of one face from the primitives of cells a-1, a,
 // a+1, a+2 (rhs/invscd.py:53-97).
-template <int LIM>
+template <int LIM, bool FULL = false>
 FD void face_states_fast(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
                          double pL[5], double pR[5]) {
   EXACT_FP
@@ -448,8 +468,8 @@ FD void face_states_fast(const double pv0[5], const double pv1[5], const double 
     const double a = pv1[v] - pv0[v], b = pv2[v] - pv1[v], c = pv3[v] - pv2[v];
     double sL, sR;
     if constexpr (LIM == LIM_VANLEER) {
-      sL = vanleer_fast(a, b);
-      sR = vanleer_fast(b, c);
+      sL = vanleer_fast<FULL>(a, b);
+      sR = vanleer_fast<FULL>(b, c);
     } else {
       double lo, hi;
       minmod_range(b, lo, hi);
@@ -479,7 +499,7 @@ FD void face_flux2(const double pv0[5], const double pv1[5], const double pv2[5]
                    const double k0h[3], const double k1h[3], const StageGas& gas, double F[5]) {
   EXACT_FP
   double pL[5], pR[5];
-  face_states_fast<LIM>(pv0, pv1, pv2, pv3, pL, pR);
+  face_states_fast<LIM, FULL>(pv0, pv1, pv2, pv3, pL, pR);
   const double S[3] = {k0h[0] + k1h[0], k0h[1] + k1h[1], k0h[2] + k1h[2]};
   roe_flux2<FULL>(pL, pR, S, gas, F);
 }

@@ -5,13 +5,19 @@
 // cell's viscous tensor are evaluated once: a thread per cell evaluated every
 // flux twice and 15 cells' primitives for it, and the tensors went through a
 // work array.  Indices are 64-bit and blocks of any size are taken.  The
-// fluxes are the stage kernels' with every reciprocal and root corrected to
-// full precision; primitives, temperature and the division by the volume are
-// IEEE quotients as before.  Error against 80-bit arithmetic, rms over largest
-// value, over random fields: inviscid 1.48e-14 on unit metrics and 8.8e-16 on
-// curvilinear ones (a face twice with IEEE quotients: 1.36e-14 and 1.00e-15;
-// IEEE quotients in this flux: 1.52e-14 and 8.8e-16), viscous 2.4e-15 and
-// 2.6e-15 (the same before).
+// inviscid fluxes are the stage kernels' with every root, reciprocal and van
+// Leer quotient rounded once; primitives, temperature, viscous tensors and the
+// division by the volume are IEEE quotients, and the divergence takes the
+// difference of two tensors before it takes the metrics, all as a thread per
+// cell did.  Error against 80-bit arithmetic, rms over the largest value, 24 x
+// 21 x 28 random cells (in brackets a thread per cell with IEEE quotients):
+//   5 % noise    unit metrics  3.3e-16 (3.4e-16), viscous 3.6e-16 (3.6e-16)
+//                curvilinear   1.2e-16 (1.3e-16), viscous 3.2e-16 (3.2e-16)
+//   jumps of e^2 unit metrics  1.7e-17 (1.7e-17), viscous 1.2e-17 (1.2e-17)
+//                curvilinear   1.4e-17 (1.3e-17), viscous 1.2e-17 (1.2e-17)
+// With reciprocal roots and their squares the inviscid ones at jumps are
+// 2.1e-17 and 1.6e-17; with the stage kernels' tensor and running divergence
+// the viscous ones 1.3e-17.
 #pragma once
 
 namespace famrdp {
@@ -19,9 +25,10 @@ namespace famrdp {
 // -(F(c+1/2) - F(c-1/2)) / (vol + 1e-300) summed over the axes along which
 // 2 <= c <= n-3, zero elsewhere.  A workgroup per tile, up to a limit of the
 // grid beyond which they take several.  A thread per face of the tile, then a thread per
-// variable and cell.  Bound by FP64 issue: 68 x 52 x 84 cells 28.6 us (83.6 as
-// a thread per cell), 132^3 207.  Tiles 4x4x8 took 29.7 and 224, 3x4x4 31.4 and
-// 247, 2x4x8 29.4 and 225; six waves per SIMD (spills) 28.0 and 225.
+// variable and cell.  Bound by FP64 issue: 68 x 52 x 84 cells 29.0 us (83.6 as
+// a thread per cell), 132^3 217.  (With six seeds a flux 28.6 and 207; the other
+// tiles then 4x4x8 29.7 and 224, 3x4x4 31.4 and 247, 2x4x8 29.4 and 225; six
+// waves per SIMD, spills, 28.0 and 225.)
 template <int TI, int TJ, int TK, int LIM>
 __global__ void __launch_bounds__((CrossGeom<TI, TJ, TK>::NTH)) __attribute__((amdgpu_waves_per_eu(5)))
 k_invscd_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, const double* __restrict__ vol,
@@ -106,13 +113,14 @@ k_invscd_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, cons
 
 // (0, viscous divergence) with the reference's periodic roll at the padded
 // edges.  Tiles as above; staged cells and tensors as in the fused stage kernel.
-// Bound by latency (two workgroups a CU): 68 x 52 x 84 cells 25.5 us (tensors
-// through memory 17.5 + 15.7), 132^3 171.  Tiles 4x4x8 took 26.8 and 189, 4x4x4
-// 26.9 and 200, 8x8x8 29.6 and 202.
+// Bound by latency (two workgroups a CU): 68 x 52 x 84 cells 26.9 us (tensors
+// through memory 17.5 + 15.7), 132^3 179.  (With the stage kernels' tensor 25.5
+// and 171; the other tiles then 4x4x8 26.8 and 189, 4x4x4 26.9 and 200, 8x8x8
+// 29.6 and 202.)
 template <int TI, int TJ, int TK>
 __global__ void __launch_bounds__((WideGeom<TI, TJ, TK>::NGW)) __attribute__((amdgpu_waves_per_eu(4)))
 k_viscous_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, double* __restrict__ rhs, int ni, int nj,
-              int nk, StageGas gas, double mu0, double gamma) {
+              int nk, Gas gas) {
   EXACT_FP
   using T = FusedGeom<TI, TJ, TK>;
   using W = WideGeom<TI, TJ, TK>;
@@ -123,7 +131,6 @@ k_viscous_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, dou
   const int ntj = (nj + TJ - 1) / TJ, ntk = (nk + TK - 1) / TK;
   const int64_t ntile = (int64_t)((ni + TI - 1) / TI) * ntj * ntk;
   const bool small = ni < WRAP_ONCE_MIN || nj < WRAP_ONCE_MIN || nk < WRAP_ONCE_MIN;
-  const double cmu = gas.cmu * mu0;
   for (int64_t tile = xcd_remap(blockIdx.x, gridDim.x); tile < ntile; tile += gridDim.x) {
     const int tk = (int)(tile % ntk), tj = (int)(tile / ntk % ntj), ti = (int)(tile / ntk / ntj);
     const int i0 = ti * TI, j0 = tj * TJ, k0 = tk * TK;
@@ -144,7 +151,7 @@ k_viscous_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, dou
       const int h = h0 + t;
       const int64_t c = cell(W::pv_cell(h < T::NPV ? h : T::NPV - 1));
       double pv[5];
-      load_prim(q, N, c, gamma, pv);
+      load_prim(q, N, c, gas.gamma, pv);
       if (h < T::NPV) {
         s_u[h] = pv[1];
         s_u[T::NPV + h] = pv[2];
@@ -153,47 +160,42 @@ k_viscous_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, dou
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int m = 0; m < 9; ++m) kh[m] = 0.5 * kh[m];
     if (t < T::NG) {
-      double d[3][4], uvwT[4], g9[9];
+      double d[3][4], uvw[5], g9[9];
       const int s0 = ((l.x + 1) * T::B0J + l.y + 1) * T::B0K + l.z + 1;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) uvwT[s] = s_u[s * T::NPV + s0];
+      for (int s = 0; s < 3; ++s) uvw[s + 1] = s_u[s * T::NPV + s0];
 #pragma unroll
       for (int e = 0; e < 3; ++e) {
         const int sp = W::pv_step(l, e, 1), sm = W::pv_step(l, e, -1);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) d[e][s] = s_u[s * T::NPV + sp] - s_u[s * T::NPV + sm];
+        for (int s = 0; s < 4; ++s) d[e][s] = 0.5 * (s_u[s * T::NPV + sp] - s_u[s * T::NPV + sm]);
       }
-      viscous_flux_fast(uvwT, d, kh, cmu, gas, g9);
+      viscous_flux(uvw, s_u[3 * T::NPV + s0], d, kh, gas, g9);
 #pragma unroll
       for (int m = 0; m < 9; ++m) s_g[m * T::NG + t] = g9[m];
     }
     __syncthreads();
     const int i = i0 + l.x, j = j0 + l.y, k = k0 + l.z;
     if (t < T::NT && i < ni && j < nj && k < nk) {
-      double vis[4] = {0.0, 0.0, 0.0, 0.0};
-      double gi[9], dj[9], dk[9];
-      int sm = W::g_step(l, 0, -1);
+      int sp[3], sm[3];
 #pragma unroll
-      for (int m = 0; m < 9; ++m) gi[m] = s_g[m * T::NG + sm];
-      visc_div_im(gi, kh, vis);
-      march_pin(vis);
-      int sp = W::g_step(l, 1, 1);
-      sm = W::g_step(l, 1, -1);
+      for (int e = 0; e < 3; ++e) {
+        sp[e] = W::g_step(l, e, 1);
+        sm[e] = W::g_step(l, e, -1);
+      }
+      double vis[4];
 #pragma unroll
-      for (int m = 0; m < 9; ++m) dj[m] = s_g[m * T::NG + sp] - s_g[m * T::NG + sm];
-      sp = W::g_step(l, 2, 1);
-      sm = W::g_step(l, 2, -1);
+      for (int r = 0; r < 4; ++r) {
+        vis[r] = 0.0;
 #pragma unroll
-      for (int m = 0; m < 9; ++m) dk[m] = s_g[m * T::NG + sp] - s_g[m * T::NG + sm];
-      visc_div_jk(dj, dk, kh, vis);
-      march_pin(vis);
-      sp = W::g_step(l, 0, 1);
-#pragma unroll
-      for (int m = 0; m < 9; ++m) gi[m] = s_g[m * T::NG + sp];
-      visc_div_ip(gi, kh, vis);
+        for (int m = 0; m < 3; ++m) {
+          const double* Gc = s_g + gidx(r, m) * T::NG;
+          const double di = 0.5 * (Gc[sp[0]] - Gc[sm[0]]), dj = 0.5 * (Gc[sp[1]] - Gc[sm[1]]),
+                       dk = 0.5 * (Gc[sp[2]] - Gc[sm[2]]);
+          vis[r] = vis[r] + fma(dk, kh[6 + m], fma(dj, kh[3 + m], di * kh[m]));
+        }
+      }
       const int64_t c = (int64_t)i * si + (int64_t)j * nk + k;
       rhs[c] = 0.0;
 #pragma unroll

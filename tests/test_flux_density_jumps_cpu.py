@@ -65,6 +65,29 @@ def test_flux_between_light_and_heavy(hc, ratio, full):
     assert float(err.max()) <= TOL
 
 
+@pytest.mark.parametrize("mach", [0.4, 2.0])
+def test_rhs_flux_is_as_exact_as_the_formulas_in_64_bits(hc, mach):
+    """The RHS entry point's form at equal densities: rms error no larger than that of flux/roe.py in IEEE arithmetic."""
+    n = 20000
+    pl, pr, S = faces(1.0, n, 91)
+    for p in (pl, pr):
+        p[:, 1:4] *= 2 * mach * np.sqrt(G * p[:, 4:] / p[:, :1])
+    F = np.zeros((n, 5))
+    P = lambda a: np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    hc.hc_roe_flux2(n, 1, P(pl), P(pr), P(S), ctypes.c_double(G), P(F))
+
+    def plain(T):
+        x = lambda a: a.T.astype(T)  # noqa: E731
+        A, g = np.sqrt((x(S) ** 2).sum(axis=0)), T(G)
+        return (2 * A * ON.roe_flux(ON.prim_to_cons(x(pl), g), ON.prim_to_cons(x(pr), g), x(S) / A, gamma=g)).T
+
+    ref = plain(np.longdouble)
+    rms = lambda x: np.sqrt((((x - ref) / np.abs(ref).max(axis=1)[:, None]) ** 2).mean(axis=0)).astype(float)  # noqa: E731
+    ours, theirs = rms(F), rms(plain(np.float64))
+    print(f"mach {mach:g}: {ours}, plain {theirs}")
+    assert (ours <= theirs).all()
+
+
 def _vjp_reference(pl, pr, S, f):
     """Cotangents of flux/roe.py:21-85 times 2 |S|, in extended precision: the complex step through the formulas."""
     g, eps = np.longdouble(G), np.longdouble(1e-30)
