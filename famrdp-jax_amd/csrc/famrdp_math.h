@@ -105,61 +105,89 @@ FD void physical_flux(const double U[5], const double n[3], double g, double F[5
 }
 
 // flux/roe.py:21-85: Roe flux for a unit normal n, Harten fix on lambda1/5.
+// fence(x, ...) marks values as computed by then; a kernel that is short of
+// registers passes one that holds the compiler to it.
+struct NoFence {
+  template <class... T>
+  FD void operator()(T&...) const {}
+};
+template <class Fence = NoFence>
 FD void roe_flux(const double UL[5], const double UR[5], const double n[3], double g,
-                 double eps_entropy, double F[5]) {
+                 double eps_entropy, double F[5], Fence fence = Fence{}) {
   const double rhoL = max_floor(UL[0], 1e-300), rhoR = max_floor(UR[0], 1e-300);
-  const double uL = UL[1] / rhoL, vL = UL[2] / rhoL, wL = UL[3] / rhoL;
-  const double uR = UR[1] / rhoR, vR = UR[2] / rhoR, wR = UR[3] / rhoR;
+  double uL = UL[1] / rhoL, vL = UL[2] / rhoL, wL = UL[3] / rhoL;
+  fence(uL, vL, wL);
+  double uR = UR[1] / rhoR, vR = UR[2] / rhoR, wR = UR[3] / rhoR;
+  fence(uR, vR, wR);
   const double keL = 0.5 * (uL * uL + vL * vL + wL * wL);
   const double keR = 0.5 * (uR * uR + vR * vR + wR * wR);
   const double pL = (g - 1.0) * (UL[4] - rhoL * keL);
   const double pR = (g - 1.0) * (UR[4] - rhoR * keR);
-  const double HL = (UL[4] + pL) / rhoL, HR = (UR[4] + pR) / rhoR;
+  double HL = (UL[4] + pL) / rhoL;
+  fence(HL);
+  double HR = (UR[4] + pR) / rhoR;
+  fence(HR);
 
   const double sqL = sqrt(rhoL), sqR = sqrt(rhoR);
   const double ss = max_floor(sqL + sqR, 1e-150);
-  const double uh = (sqL * uL + sqR * uR) / ss;
-  const double vh = (sqL * vL + sqR * vR) / ss;
-  const double wh = (sqL * wL + sqR * wR) / ss;
-  const double Hh = (sqL * HL + sqR * HR) / ss;
+  double uh = (sqL * uL + sqR * uR) / ss;
+  fence(uh);
+  double vh = (sqL * vL + sqR * vR) / ss;
+  fence(vh);
+  double wh = (sqL * wL + sqR * wR) / ss;
+  fence(wh);
+  double Hh = (sqL * HL + sqR * HR) / ss;
+  fence(Hh);
   const double q2 = uh * uh + vh * vh + wh * wh;
-  const double c2 = max_floor((g - 1.0) * (Hh - 0.5 * q2), 1e-30);
-  const double ch = sqrt(c2);
-  const double unh = uh * n[0] + vh * n[1] + wh * n[2];
-  const double rhoh = sqL * sqR;
+  double c2 = max_floor((g - 1.0) * (Hh - 0.5 * q2), 1e-30);
+  double ch = sqrt(c2);
+  double unh = uh * n[0] + vh * n[1] + wh * n[2];
+  double rhoh = sqL * sqR;
+  fence(c2, ch, unh, rhoh);
 
   const double eps = eps_entropy * (fabs(unh) + ch);
   const double lam1 = unh - ch, lam5 = unh + ch;
-  const double al1 = fabs(lam1) >= eps ? fabs(lam1) : 0.5 * (lam1 * lam1 / eps + eps);
-  const double al5 = fabs(lam5) >= eps ? fabs(lam5) : 0.5 * (lam5 * lam5 / eps + eps);
+  double al1 = fabs(lam1) >= eps ? fabs(lam1) : 0.5 * (lam1 * lam1 / eps + eps);
+  fence(al1);
+  double al5 = fabs(lam5) >= eps ? fabs(lam5) : 0.5 * (lam5 * lam5 / eps + eps);
+  fence(al5);
   const double al2 = fabs(unh);
 
   double dU[5];
   for (int v = 0; v < 5; ++v) dU[v] = UR[v] - UL[v];
   const double dp = (g - 1.0) * (dU[4] - uh * dU[1] - vh * dU[2] - wh * dU[3] + 0.5 * q2 * dU[0]);
   const double dun = (dU[1] * n[0] + dU[2] * n[1] + dU[3] * n[2]) - unh * dU[0];
-  const double a1 = (dp - rhoh * ch * dun) / (2.0 * c2);
-  const double a5 = (dp + rhoh * ch * dun) / (2.0 * c2);
-  const double a23 = dU[0] - dp / c2;
+  double a1 = (dp - rhoh * ch * dun) / (2.0 * c2);
+  fence(a1);
+  double a5 = (dp + rhoh * ch * dun) / (2.0 * c2);
+  fence(a5);
+  double a23 = dU[0] - dp / c2;
+  fence(a23);
 
   const double R1[5] = {1.0, uh - ch * n[0], vh - ch * n[1], wh - ch * n[2], Hh - ch * unh};
   const double R5[5] = {1.0, uh + ch * n[0], vh + ch * n[1], wh + ch * n[2], Hh + ch * unh};
   const double R2[5] = {1.0, uh, vh, wh, 0.5 * q2};
 
-  const double dut = dU[1] / rhoh - uh * dU[0] / rhoh;
-  const double dvt_ = dU[2] / rhoh - vh * dU[0] / rhoh;
-  const double dwt = dU[3] / rhoh - wh * dU[0] / rhoh;
+  double dut = dU[1] / rhoh - uh * dU[0] / rhoh;
+  fence(dut);
+  double dvt_ = dU[2] / rhoh - vh * dU[0] / rhoh;
+  fence(dvt_);
+  double dwt = dU[3] / rhoh - wh * dU[0] / rhoh;
+  fence(dwt);
   const double dunf = dut * n[0] + dvt_ * n[1] + dwt * n[2];
   const double tx = dut - dunf * n[0], ty = dvt_ - dunf * n[1], tz = dwt - dunf * n[2];
-  const double dvt[5] = {0.0, rhoh * tx, rhoh * ty, rhoh * tz, rhoh * (uh * tx + vh * ty + wh * tz)};
+  double dvt[5] = {0.0, rhoh * tx, rhoh * ty, rhoh * tz, rhoh * (uh * tx + vh * ty + wh * tz)};
+  fence(dvt[1], dvt[2], dvt[3], dvt[4]);
 
-  double FL[5], FR[5];
-  physical_flux(UL, n, g, FL);
-  physical_flux(UR, n, g, FR);
-  for (int v = 0; v < 5; ++v) {
-    const double absA = al1 * a1 * R1[v] + al5 * a5 * R5[v] + al2 * (a23 * R2[v] + dvt[v]);
-    F[v] = 0.5 * (FL[v] + FR[v]) - 0.5 * absA;
-  }
+  double FL[5], FR[5], absA[5];
+  for (int v = 0; v < 5; ++v) absA[v] = al1 * a1 * R1[v] + al5 * a5 * R5[v] + al2 * (a23 * R2[v] + dvt[v]);
+  fence(absA[0], absA[1], absA[2], absA[3], absA[4]);
+  double VL[5] = {UL[0], UL[1], UL[2], UL[3], UL[4]}, VR[5] = {UR[0], UR[1], UR[2], UR[3], UR[4]};
+  fence(VL[0], VL[1], VL[2], VL[3], VL[4]);
+  physical_flux(VL, n, g, FL);
+  fence(FL[0], FL[1], FL[2], FL[3], FL[4], VR[0], VR[1], VR[2], VR[3], VR[4]);
+  physical_flux(VR, n, g, FR);
+  for (int v = 0; v < 5; ++v) F[v] = 0.5 * (FL[v] + FR[v]) - 0.5 * absA[v];
 }
 
 // One face of rhs/invscd.py:53-97 (the MUSCL-2 slopes of the two cells either
@@ -369,8 +397,11 @@ DF void prim_and_temp(const double q[5], const StageGas& gas, double pv[6]) {
 // makes the flux as exact as the reference's formulas in IEEE arithmetic or more
 // (rms 1.5e-16 to their 2.5e-16 on those faces, 7.3e-16 to 8.8e-16 at twice the
 // speed of sound; with reciprocal roots and their squares 9.5e-16 there).
+//
+// Says whether no floor acted: where one does, the conservative states that the
+// reference forms and these identities part company.
 template <bool FULL = false>
-FD void roe_flux2(const double pl[5], const double pr[5], const double S[3], const StageGas& gas, double F[5]) {
+FD bool roe_flux2(const double pl[5], const double pr[5], const double S[3], const StageGas& gas, double F[5]) {
   EXACT_FP
   auto recip = [](double x) { return FULL ? rcp(x) : rcp1(x); };
   const double rhoL = fmax(pl[0], 1e-300), rhoR = fmax(pr[0], 1e-300);
@@ -391,9 +422,9 @@ FD void roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   const double HL = fma(gas.cg2, pl[4] * irL, kL), HR = fma(gas.cg2, pr[4] * irR, kR);
   const double uh = fma(a, uR, b * uL), vh = fma(a, vR, b * vL), wh = fma(a, wR, b * wL), Hh = fma(a, HR, b * HL);
   const double q2 = fma(wh, wh, fma(vh, vh, uh * uh));
-  const double c2 = fmax(gas.gm1h * (Hh - q2), 1e-30);
+  const double c2raw = gas.gm1h * (Hh - q2), c2 = fmax(c2raw, 1e-30);
   // |S| and 1/|S|; a zero face keeps a harmless 1e-140
-  const double nn = fmax(fma(S[2], S[2], fma(S[1], S[1], S[0] * S[0])), 1e-280);
+  const double nnraw = fma(S[2], S[2], fma(S[1], S[1], S[0] * S[0])), nn = fmax(nnraw, 1e-280);
   double c, rc2, A, rA;                                           // rc2 = 1 / c^2
   if constexpr (FULL) {
     c = fsqrt(c2), rc2 = rcp(c2);
@@ -430,6 +461,7 @@ FD void roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   F[3] = fma(S[2], P, fma(iR, wR, iL * wL));
   const double ud = fma(wh, wR - wL, fma(vh, vR - vL, uh * (uR - uL)));
   F[4] = fma(0.5, fma(-w2, q2, fma(HR, eR, eL * HL)), fma(un, Q, -(w * ud)));
+  return pl[0] > 1e-300 && pr[0] > 1e-300 && c2raw > 1e-30 && nnraw > 1e-280;
 }
 
 // MUSCL-2 face states of one cell along one axis (physics/reconstruct/
@@ -495,13 +527,13 @@ FD void face_states_fast(const double pv0[5], const double pv1[5], const double 
 // Twice the flux of one face (roe_flux2) from the primitives of cells a-1 ..
 // a+2 and kxyz[d, :] / 2 at cells a and a+1: the area vector is their sum.
 template <int LIM, bool FULL = false>
-FD void face_flux2(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
+FD bool face_flux2(const double pv0[5], const double pv1[5], const double pv2[5], const double pv3[5],
                    const double k0h[3], const double k1h[3], const StageGas& gas, double F[5]) {
   EXACT_FP
   double pL[5], pR[5];
   face_states_fast<LIM, FULL>(pv0, pv1, pv2, pv3, pL, pR);
   const double S[3] = {k0h[0] + k1h[0], k0h[1] + k1h[1], k0h[2] + k1h[2]};
-  roe_flux2<FULL>(pL, pR, S, gas, F);
+  return roe_flux2<FULL>(pL, pR, S, gas, F);
 }
 
 // Viscous flux tensor of one cell (rhs/viscous.py:30-108): velocity and
