@@ -283,6 +283,26 @@ int bind_host(famrdp_plan* p, double* const* q, const double* const* kxyz, const
   return FAMRDP_OK;
 }
 
+// Whether an array of `in` and one of `out` (one per block, 5 N doubles each)
+// share memory: q_in and q of a step from one into the other.
+bool states_overlap(const famrdp_plan* p, const double* const* in, double* const* out) {
+  struct Range { uintptr_t lo, hi; bool out; };
+  std::vector<Range> v;
+  v.reserve(2 * (size_t)p->nblocks);
+  for (int b = 0; b < p->nblocks; ++b) {
+    const uintptr_t n = sizeof(double) * 5 * (uintptr_t)p->N[b], i = (uintptr_t)in[b], o = (uintptr_t)out[b];
+    v.push_back({i, i + n, false});
+    v.push_back({o, o + n, true});
+  }
+  std::sort(v.begin(), v.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
+  uintptr_t end[2] = {0, 0};               // how far the arrays so far reach, of in and of out
+  for (const Range& x : v) {
+    if (x.lo < end[x.out ? 0 : 1]) return true;
+    end[x.out] = std::max(end[x.out], x.hi);
+  }
+  return false;
+}
+
 int upload_adj(famrdp_plan* p, hipStream_t st) {
   for (int b = 0; b < p->nblocks; ++b) {
     BlockDesc a = p->h_blocks[b];
@@ -1166,9 +1186,10 @@ int famrdp_step_from(famrdp_plan* p, const double* const* q_in, double* const* q
   if (!p || !q_in || !kxyz || !vol) return fail(FAMRDP_E_INVALID, "step_from: NULL plan or pointer arrays");
   if (!p->has_workspace) return fail(FAMRDP_E_INVALID, "step_from: plan was created without stage workspace");
   for (int b = 0; b < p->nblocks; ++b)
-    if (!q_in[b] || !kxyz[b] || !vol[b] || (q && q_in[b] == q[b]))
-      return fail(FAMRDP_E_INVALID, "step_from: NULL q_in/kxyz/vol or q_in the same array as q for block " +
-                                        std::to_string(b));
+    if (!q_in[b] || !kxyz[b] || !vol[b])
+      return fail(FAMRDP_E_INVALID, "step_from: NULL q_in/kxyz/vol for block " + std::to_string(b));
+  // the launch that copies fills ghost cells from other blocks' q_in meanwhile
+  if (q && states_overlap(p, q_in, q)) return fail(FAMRDP_E_INVALID, "step_from: an array of q_in shares memory with one of q");
   hipStream_t st = S(stream);
   bool changed, changed_adj;
   int rc = bind_host(p, q, kxyz, vol, true, nullptr, nullptr, changed, changed_adj);

@@ -140,7 +140,8 @@ int famrdp_step(famrdp_plan* plan, double* const* q, const double* const* kxyz, 
                 int32_t flags, void* stream);
 /* famrdp_step from q_in[b] (left as it is) into q[b] (another array of the
  * same size): the functional form, which copies every block and binds the
- * pointers in one launch.  Same bits as a copy and famrdp_step. */
+ * pointers in one launch.  Same bits as a copy and famrdp_step.  No array of
+ * q_in may share memory with one of q, of whatever block (FAMRDP_E_INVALID). */
 int famrdp_step_from(famrdp_plan* plan, const double* const* q_in, double* const* q, const double* const* kxyz,
                      const double* const* vol, double dt, int32_t flags, void* stream);
 /* nsteps steps replayed from a hipGraph captured for these pointers, dt and
