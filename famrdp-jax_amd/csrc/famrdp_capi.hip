@@ -253,21 +253,20 @@ int upload_table(famrdp_plan* p, BlockDesc* dst, const std::vector<BlockDesc>& s
   return FAMRDP_OK;
 }
 
-// Point the block tables at the caller's arrays.  q == nullptr leaves the
-// state pointers as they are (the reverse sweep reads its own copy, qh);
-// kxyz / vol == nullptr keep the bound metrics.  Tables are re-uploaded only
-// when a pointer changed.
-// q1t / q2t: where the step's stage-1/2 results go (caller arrays), or NULL
-// for the plan's workspace.
 // Puts the caller's arrays into the host copy of the block table and says
-// whether the plan's table and the reverse sweep's have changed by it.
+// whether the plan's table and the reverse sweep's have changed by it.  q ==
+// nullptr leaves the state pointers as they are (the reverse sweep reads its own
+// copy, qh); kxyz / vol == nullptr keep the bound metrics.  q1t / q2t: where the
+// step's stage-1/2 results go (caller arrays), or NULL for the plan's workspace.
+// Arguments that are refused leave the table as it is.
 int bind_host(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol, bool need_q,
               double* const* q1t, double* const* q2t, bool& changed, bool& changed_adj) {
   if (need_q && !q) return fail(FAMRDP_E_INVALID, "q pointer array is NULL");
+  for (int b = 0; q && b < p->nblocks; ++b)
+    if (!q[b]) return fail(FAMRDP_E_INVALID, "q[" + std::to_string(b) + "] is NULL");
   changed = changed_adj = !p->blocks_uploaded;
   for (int b = 0; b < p->nblocks; ++b) {
     BlockDesc& d = p->h_blocks[b];
-    if (q && !q[b]) return fail(FAMRDP_E_INVALID, "q[" + std::to_string(b) + "] is NULL");
     const double* kx = kxyz ? kxyz[b] : d.kxyz;
     const double* vo = vol ? vol[b] : d.vol;
     double* s1 = q1t ? q1t[b] : p->q1[b];
@@ -312,11 +311,13 @@ int upload_adj(famrdp_plan* p, hipStream_t st) {
   return upload_table(p, p->d_blocks_adj, p->h_blocks_adj, st);
 }
 
+// bind_host, and the tables uploaded where a pointer changed.
 int bind(famrdp_plan* p, double* const* q, const double* const* kxyz, const double* const* vol, hipStream_t st,
          bool need_q = true, double* const* q1t = nullptr, double* const* q2t = nullptr) {
   bool changed, changed_adj;
   int rc = bind_host(p, q, kxyz, vol, need_q, q1t, q2t, changed, changed_adj);
   if (rc) return rc;
+  p->blocks_uploaded = false;   // until all of it is
   if (changed) {
     rc = upload_table(p, p->d_blocks, p->h_blocks, st);
     if (rc) return rc;

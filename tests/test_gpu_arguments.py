@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from famrdp_jax import _lib as L
 from famrdp_jax import cases
 from famrdp_jax._plan import plan_for
 from _util import to_dev
@@ -32,4 +33,25 @@ def test_step_from_refuses_arrays_that_share_memory():
             plan.step_from(src, bad, kx, vo, 1e-3)
     plan.step_from(src, into, kx, vo, 1e-3)
     for q, w in zip(into, want):
+        assert torch.equal(q, w)
+
+
+def test_a_refused_call_leaves_the_plan_bound_as_it_was():
+    """A call with a NULL state after a valid one, then a valid one with the other pointers of the refused call."""
+    print("case: NULL state pointer between two steps", flush=True)
+    plan, src, kx, vo = _two_blocks()
+    first, second = [q.clone() for q in src], [q.clone() for q in src]
+    plan.step(first, kx, vo, 1e-3, batched=True)
+    second[1:] = first[1:]                       # the second call differs in block 0 alone
+    rest = [q.clone() for q in second]
+    ptrs = plan._ptrs(second)
+    ptrs[len(src) - 1] = None
+    rc = plan._lib.famrdp_step(plan._h, ptrs, plan._ptrs(kx), plan._ptrs(vo), 1e-3, 1, L.stream())
+    with pytest.raises(ValueError, match="is NULL"):
+        L.check(rc)
+    keep = first[0].clone()
+    plan.step(second, kx, vo, 1e-3, batched=True)
+    plan.step(rest, kx, vo, 1e-3, batched=True)
+    assert torch.equal(first[0], keep)
+    for q, w in zip(second, rest):
         assert torch.equal(q, w)
