@@ -16,6 +16,7 @@
 #include "famrdp_kernels.hip"
 #include "famrdp_adjoint.hip"
 #include "famrdp_reverse.h"
+#include "famrdp_tune.h"
 #include "../../include/famrdp_capi.h"
 
 using namespace famrdp;
@@ -942,60 +943,56 @@ int famrdp_plan_autotune(famrdp_plan* p, double* const* q, const double* const* 
   int rc = bind(p, q, kxyz, vol, S(stream));
   if (rc) return rc;
   hipStream_t st = S(stream);
-  hipEvent_t e0, e1;
-  HIP_TRY(hipEventCreate(&e0));
-  HIP_TRY(hipEventCreate(&e1));
-  // ms of one pair of stages 1 and 2 of variant v, over n pairs after `warm`
-  // untimed ones.  They read q (and q1) and
-  // write the q1, q2 workspace only: the state is untouched; stage 2 also
-  // reads q0, as stage 3 does.
-  auto time_pairs = [&](int v, int warm, int n, float& ms) -> int {
-    for (int r = -warm; r < n; ++r) {
-      if (r == 0) HIP_TRY(hipEventRecord(e0, st));
-      for (int stage = 1; stage <= 2; ++stage) {
-        if (flags & FAMRDP_STEP_BATCHED) {
-          launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], stage, p->gas, p->limiter, dt,
-                               p->len3[v], st);
-        } else {
-          for (int b = 0; b < p->nblocks; ++b)
-            launch_fused(v, p->h_blocks[b], stage, p->gas, p->limiter, dt, p->ncu, st);
-        }
-        LAUNCH_CHECK();
-      }
+  struct Events {   // given back however the tuning ends
+    hipEvent_t e[3] = {nullptr, nullptr, nullptr};
+    ~Events() {
+      for (hipEvent_t x : e)
+        if (x) (void)hipEventDestroy(x);
     }
-    HIP_TRY(hipEventRecord(e1, st));
-    HIP_TRY(hipEventSynchronize(e1));
-    float t = 0.f;
-    HIP_TRY(hipEventElapsedTime(&t, e0, e1));
-    ms = t / n;
+  } ev;
+  for (hipEvent_t& e : ev.e) HIP_TRY(hipEventCreate(&e));
+  // stages 1 and 2 of variant v n times.  They read q (and q1) and write the
+  // q1, q2 workspace only: the state is untouched; stage 2 also reads q0, as
+  // stage 3 does.
+  auto pairs = [&](int v, int n) -> int {
+    for (int stage = 0; stage < 2 * n; ++stage) {
+      if (flags & FAMRDP_STEP_BATCHED) {
+        launch_fused_batched(v, p->d_blocks, p->d_tiles3[v], p->ntiles3[v], 1 + stage % 2, p->gas, p->limiter, dt,
+                             p->len3[v], st);
+      } else {
+        for (int b = 0; b < p->nblocks; ++b)
+          launch_fused(v, p->h_blocks[b], 1 + stage % 2, p->gas, p->limiter, dt, p->ncu, st);
+      }
+      LAUNCH_CHECK();
+    }
     return FAMRDP_OK;
   };
-  // one timed pair each (after an untimed one), then the rest of the pairs for
-  // those within 1.5 of the best
-  float ms[NUM_TILE_VARIANTS], first = 1e30f;
-  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
-    ms[v] = 1e30f;
-    if (!variant_fits(p, v)) continue;
-    rc = time_pairs(v, 1, 1, ms[v]);
-    if (rc) return rc;
-    first = std::min(first, ms[v]);
-  }
-  int best = 0;
-  float best_ms = 1e30f;
-  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) {
-    if (reps > 1 && ms[v] <= 1.5f * first) {
-      float rest = 0.f;
-      rc = time_pairs(v, 0, reps - 1, rest);
-      if (rc) return rc;
-      ms[v] = (ms[v] + rest * (reps - 1)) / reps;
+  auto first = [&](int v, float& cold, float& warm) -> int {
+    for (int i = 0; i < 3; ++i) {
+      HIP_TRY(hipEventRecord(ev.e[i], st));
+      if (i < 2 && (rc = pairs(v, 1))) return rc;
     }
-    if (ms_out) ms_out[v] = variant_fits(p, v) ? ms[v] : 1e30;
-    // ties (within 1.5 %: stages 1 and 2 rank variants that close only to
-    // about that) keep the earlier variant
-    if (ms[v] < best_ms * 0.985f) { best_ms = ms[v]; best = v; }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+    HIP_TRY(hipEventSynchronize(ev.e[2]));
+    HIP_TRY(hipEventElapsedTime(&cold, ev.e[0], ev.e[1]));
+    HIP_TRY(hipEventElapsedTime(&warm, ev.e[1], ev.e[2]));
+    return FAMRDP_OK;
+  };
+  auto rest = [&](int v, int n, float& t) -> int {
+    HIP_TRY(hipEventRecord(ev.e[0], st));
+    if ((rc = pairs(v, n))) return rc;
+    HIP_TRY(hipEventRecord(ev.e[1], st));
+    HIP_TRY(hipEventSynchronize(ev.e[1]));
+    HIP_TRY(hipEventElapsedTime(&t, ev.e[0], ev.e[1]));
+    t /= n;
+    return FAMRDP_OK;
+  };
+  bool fits[NUM_TILE_VARIANTS];
+  float ms[NUM_TILE_VARIANTS];
+  for (int v = 0; v < NUM_TILE_VARIANTS; ++v) fits[v] = variant_fits(p, v);
+  int best = 0;
+  rc = tune_variants(NUM_TILE_VARIANTS, fits, reps, first, rest, ms, best);
+  if (rc) return rc;
+  for (int v = 0; ms_out && v < NUM_TILE_VARIANTS; ++v) ms_out[v] = fits[v] ? ms[v] : 1e30;
   return famrdp_plan_set_tile(p, best);
 }
 

@@ -167,8 +167,8 @@ int famrdp_step_stages(famrdp_plan* plan, double* const* q, const double* const*
  * them.  famrdp_plan_autotune times `reps`
  * stage-1 + stage-2 launch pairs of every variant for these arrays (both write
  * only the plan's workspace, so the state is not modified; stage 2 also reads
- * q0 like stage 3; one pair only of variants that take 1.5 times the best's or
- * more), writes the per-variant ms of one pair to ms_out (may be
+ * q0 like stage 3; of variants that take 1.5 times the best's or more in both of
+ * two first pairs, the better of those), writes the per-variant ms of one pair to ms_out (may be
  * NULL; FAMRDP_NUM_TILE_VARIANTS entries) and keeps the fastest; a variant
  * within 1.5 % of an earlier one counts as a tie and the earlier one stays.
  * Until either is called a plan takes the variant its blocks' sizes suggest
