@@ -596,6 +596,11 @@ int famrdp_axpby(double* out, double a, const double* x, double b, const double*
 int famrdp_compute_metrics(const double* xyz, double* jac, double* kxyz, double* vol, int32_t ni, int32_t nj,
                            int32_t nk, void* stream) {
   if (ni < 1 || nj < 1 || nk < 1 || !xyz || !jac || !kxyz || !vol) return fail(FAMRDP_E_INVALID, "compute_metrics: bad arguments");
+  if (!metrics_marched(ni, nj, nk)) {
+    k_metrics_cell<<<nblk((int64_t)ni * nj * nk), 256, 0, S(stream)>>>(xyz, jac, kxyz, vol, ni, nj, nk);
+    LAUNCH_CHECK();
+    return FAMRDP_OK;
+  }
   // segments as long as leaves four workgroups per CU, 8 planes at most (a
   // segment starts with four planes that it does not work on): 20^3 takes 7.1
   // us with 1 plane and 17.2 with 8, 204^3 403 with 1, 308 with 8, 315 with 16

@@ -437,7 +437,8 @@ __global__ void __launch_bounds__(256) k_ghost_second(const BlockDesc* __restric
 // holds TJ x TK columns (a thread each) and walks planes along i: the five
 // planes of the i difference stay in registers, a plane with two cells around
 // it lies in LDS for the other two, and a cell takes three loads and its share
-// of the halo's.  The next plane's loads are issued before a plane is worked
+// of the halo's (small and thin grids are left to a thread per cell:
+// metrics_marched).  The next plane's loads are issued before a plane is worked
 // on; two LDS planes in turn leave one barrier a plane.  164 x 132 x 148 cells
 // 100 us (127 with a thread per cell), 204^3 318 (363), 264^3 613 (755): what
 // is left are the eleven streams it writes.
@@ -449,6 +450,60 @@ __device__ __forceinline__ int roll(int i, int n) {
 }
 
 constexpr int METRIC_TJ = 8, METRIC_TK = 32;
+
+// jac, vol and kxyz of cell c from its Jacobian
+__device__ __forceinline__ void metrics_of(const double J[3][3], int64_t c, int64_t N, double* __restrict__ jac,
+                                           double* __restrict__ kxyz, double* __restrict__ vol) {
+  const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+  const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+  const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+  const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
+  const double inv[3][3] = {
+      {c00 / det, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det, (J[0][1] * J[1][2] - J[0][2] * J[1][1]) / det},
+      {c01 / det, (J[0][0] * J[2][2] - J[0][2] * J[2][0]) / det, (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det},
+      {c02 / det, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det, (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det}};
+  jac[c] = det;
+  vol[c] = fabs(det);
+  for (int l = 0; l < 3; ++l)
+    for (int m = 0; m < 3; ++m) kxyz[(l * 3 + m) * N + c] = inv[l][m];
+}
+
+// Whether a grid is marched in tiles: where there are cells enough (below, the
+// segments' first planes cost more than the loads they save: 36^3 cells 6.2 us
+// marched, 5.0 a thread per cell; 60^3 9.8 and 11.0; 120,000 of 33 along k 9.3
+// and 7.1, 400,000 of 24 13.7 and 16) and the tiles' columns are not too many for
+// the block's (columns past it take their share of the time: at 10^6 cells of 18
+// along k, 1.8 times the columns, 30 us both; of 16, twice, 33 and 28.5; of 9,
+// 3.6 times, 49 and 31; of 1, 32 times, 359 and 29).  Large grids, bound by
+// memory, bear more: 8 * 10^6 cells of 16 262 and 306, of 14, 2.3 times, 309 both.
+inline bool metrics_marched(int ni, int nj, int nk) {
+  const int64_t N = (int64_t)ni * nj * nk;
+  const double columns = (double)((nj + METRIC_TJ - 1) / METRIC_TJ * METRIC_TJ) *
+                         (double)((nk + METRIC_TK - 1) / METRIC_TK * METRIC_TK) / ((double)nj * nk);
+  return N >= (1 << 17) && columns <= (N < (1 << 18) ? 1.2 : (N < (1 << 22) ? 1.9 : 2.3));
+}
+
+// The others: a thread per cell.
+__global__ void __launch_bounds__(256) k_metrics_cell(const double* __restrict__ xyz, double* __restrict__ jac,
+                                                      double* __restrict__ kxyz, double* __restrict__ vol, int ni, int nj,
+                                                      int nk) {
+  const int64_t N = (int64_t)ni * nj * nk;
+  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (c >= N) return;
+  const int k = (int)(c % nk), j = (int)((c / nk) % nj), i = (int)(c / ((int64_t)nk * nj));
+  const int idx[3] = {i, j, k}, n[3] = {ni, nj, nk};
+  const int64_t st[3] = {(int64_t)nj * nk, nk, 1};
+  double J[3][3];
+  for (int l = 0; l < 3; ++l) {
+    int64_t o[5];
+    for (int s = -2; s <= 2; ++s) o[s + 2] = c + (int64_t)(roll(idx[l] + s, n[l]) - idx[l]) * st[l];
+    for (int m = 0; m < 3; ++m) {
+      const double* f = xyz + m * N;
+      J[m][l] = (-f[o[4]] + 8.0 * f[o[3]] - 8.0 * f[o[1]] + f[o[0]]) / 12.0;
+    }
+  }
+  metrics_of(J, c, N, jac, kxyz, vol);
+}
 
 // Workgroups: (segment of len planes, tile), the tile index fastest.
 __global__ void __launch_bounds__(METRIC_TJ * METRIC_TK) __attribute__((amdgpu_waves_per_eu(4))) k_metrics(const double* __restrict__ xyz,
@@ -515,20 +570,7 @@ __global__ void __launch_bounds__(METRIC_TJ * METRIC_TK) __attribute__((amdgpu_w
       J[m][1] = (-c[2 * W] + 8.0 * c[W] - 8.0 * c[-W] + c[-2 * W]) / 12.0;
       J[m][2] = (-c[2] + 8.0 * c[1] - 8.0 * c[-1] + c[-2]) / 12.0;
     }
-    if (!own) continue;
-    const int64_t c = i * si + col;
-    const double c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-    const double c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-    const double c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-    const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
-    const double inv[3][3] = {
-        {c00 / det, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det, (J[0][1] * J[1][2] - J[0][2] * J[1][1]) / det},
-        {c01 / det, (J[0][0] * J[2][2] - J[0][2] * J[2][0]) / det, (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det},
-        {c02 / det, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det, (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / det}};
-    jac[c] = det;
-    vol[c] = fabs(det);
-    for (int l = 0; l < 3; ++l)
-      for (int m = 0; m < 3; ++m) kxyz[(l * 3 + m) * N + c] = inv[l][m];
+    if (own) metrics_of(J, i * si + col, N, jac, kxyz, vol);
   }
 }
 
