@@ -148,6 +148,7 @@ struct famrdp_plan {
   int stage_next = 0;
   std::vector<BlockDesc> h_blocks;
   bool blocks_uploaded = false;
+  bool table_in_graph = false;    // a captured launch writes the device table whenever its graph is replayed
   HaloEntry* d_halo = nullptr;
   int nhalo = 0;
   double* d_halo_stage = nullptr;
@@ -265,7 +266,7 @@ int bind_host(famrdp_plan* p, double* const* q, const double* const* kxyz, const
   if (need_q && !q) return fail(FAMRDP_E_INVALID, "q pointer array is NULL");
   for (int b = 0; q && b < p->nblocks; ++b)
     if (!q[b]) return fail(FAMRDP_E_INVALID, "q[" + std::to_string(b) + "] is NULL");
-  changed = changed_adj = !p->blocks_uploaded;
+  changed = changed_adj = !p->blocks_uploaded || p->table_in_graph;
   for (int b = 0; b < p->nblocks; ++b) {
     BlockDesc& d = p->h_blocks[b];
     const double* kx = kxyz ? kxyz[b] : d.kxyz;
@@ -1194,6 +1195,9 @@ int famrdp_step_from(famrdp_plan* p, const double* const* q_in, double* const* q
   // the launch that copies fills ghost cells from other blocks' q_in meanwhile
   if (q && states_overlap(p, q_in, q)) return fail(FAMRDP_E_INVALID, "step_from: an array of q_in shares memory with one of q");
   hipStream_t st = S(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capture) != hipSuccess) (void)hipGetLastError();   // (the launch will say)
+  p->table_in_graph |= capture != hipStreamCaptureStatusNone;
   bool changed, changed_adj;
   int rc = bind_host(p, q, kxyz, vol, true, nullptr, nullptr, changed, changed_adj);
   if (rc) return rc;

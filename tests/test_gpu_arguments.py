@@ -55,3 +55,36 @@ def test_a_refused_call_leaves_the_plan_bound_as_it_was():
     assert torch.equal(first[0], keep)
     for q, w in zip(second, rest):
         assert torch.equal(q, w)
+
+
+def test_replays_of_a_captured_step_between_in_place_ones():
+    """A functional step in a graph and a resident stepper of one configuration share a plan: each replay writes the
+    plan's block table, and the stepper's next step must not run on it."""
+    from famrdp_jax.solver.step import step
+    from famrdp_jax.solver.stepper import Stepper
+    print("case: captured functional step and in-place steps in turn", flush=True)
+    state, cfg = cases.case_c3(nb_axis=2, lo=9, hi=14)[:2]
+    state, dt = to_dev(state), 1e-3
+    ref = Stepper(state, cfg)
+    ref.advance(dt, 4, batched=True)
+    want, once = [q.clone() for q in ref.qs], [b.q for b in step(state, cfg, dt).blocks]
+    st = Stepper(state, cfg)
+    st.advance(dt, 1, batched=True)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(state, cfg, dt)
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = step(state, cfg, dt)
+    for _ in range(3):
+        st.advance(dt, 1, batched=True)
+        for b in out.blocks:
+            b.q.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        for b, w in zip(out.blocks, once):
+            assert torch.equal(b.q, w)
+    for q, w in zip(st.qs, want):
+        assert torch.equal(q, w)
