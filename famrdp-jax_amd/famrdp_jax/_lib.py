@@ -175,6 +175,11 @@ def like_input(t, ref):
     return t.detach().cpu().numpy()
 
 
+def forward_ad() -> bool:
+    """Whether a forward-mode level is open (its tensors carry tangents without requires_grad)."""
+    return _torch().autograd.forward_ad._current_level >= 0
+
+
 def ptr(t) -> int:
     return t.data_ptr() if t is not None else 0
 

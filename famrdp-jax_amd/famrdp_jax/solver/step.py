@@ -21,7 +21,7 @@ def step(state: State, cfg: Config, dt: float) -> State:
     # several blocks: one launch per stage over all of them instead of one per
     # block (the same bits; 8 blocks of 13^3-44^3 cells, a stage: 112 -> 33 us)
     many = len(src) > 1
-    if any(q.requires_grad for q in src):     # autograd sees the copy
+    if any(q.requires_grad for q in src) or L.forward_ad():     # autograd, reverse or forward, sees the copy
         qs = [q.clone() for q in src]
         plan.step(qs, kx, vo, dt, batched=many)
     else:

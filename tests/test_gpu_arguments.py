@@ -88,3 +88,20 @@ def test_replays_of_a_captured_step_between_in_place_ones():
             assert torch.equal(b.q, w)
     for q, w in zip(st.qs, want):
         assert torch.equal(q, w)
+
+
+def test_forward_mode_sees_the_copy_as_reverse_mode_does():
+    from famrdp_jax.core.types import Block, State
+    from famrdp_jax.solver.step import step
+    from torch.autograd import forward_ad as fwd
+    print("case: functional step of dual tensors", flush=True)
+    state, cfg = cases.case_c3(nb_axis=2, lo=9, hi=14)[:2]
+    state = to_dev(state)
+    plain = [b.q for b in step(state, cfg, 1e-3).blocks]
+    tangents = [torch.rand_like(b.q) for b in state.blocks]
+    with fwd.dual_level():
+        dual = State(blocks=tuple(Block(q=fwd.make_dual(b.q.clone(), t), xyz=b.xyz)
+                                  for b, t in zip(state.blocks, tangents)), metrics=state.metrics)
+        for b, t, q in zip(step(dual, cfg, 1e-3).blocks, tangents, plain):
+            primal, tangent = fwd.unpack_dual(b.q)
+            assert torch.equal(primal, q) and torch.equal(tangent, t)
