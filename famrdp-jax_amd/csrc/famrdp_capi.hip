@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
 #include <string>
@@ -688,18 +689,27 @@ int famrdp_plan_destroy(famrdp_plan* p) {
   return FAMRDP_OK;
 }
 
-int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, int32_t ncut, const famrdp_cut* cuts,
-                       int32_t nbc, const famrdp_bc* bcs, const famrdp_gas* gas, int32_t limiter, int32_t ghost,
-                       int32_t plan_flags) {
-  if (!out) return fail(FAMRDP_E_INVALID, "plan_create: out is NULL");
-  *out = nullptr;
+}  // extern "C"
+
+namespace {
+
+// A plan in the making, destroyed unless it is given away.
+struct PlanOwner {
+  famrdp_plan* p;
+  ~PlanOwner() { (void)famrdp_plan_destroy(p); }
+};
+
+int plan_create_impl(famrdp_plan** out, int32_t nblocks, const int32_t* dims, int32_t ncut, const famrdp_cut* cuts,
+                     int32_t nbc, const famrdp_bc* bcs, const famrdp_gas* gas, int32_t limiter, int32_t ghost,
+                     int32_t plan_flags) {
   if (nblocks < 1 || !dims || !gas || ncut < 0 || nbc < 0 || (ncut > 0 && !cuts) || (nbc > 0 && !bcs))
     return fail(FAMRDP_E_INVALID, "plan_create: bad arguments");
   if (bad_lim(limiter)) return fail(FAMRDP_E_KEY, "unknown limiter code " + std::to_string(limiter));
   if (ghost < 1) return fail(FAMRDP_E_INVALID, "ghost must be >= 1");
   if (ghost != 2 && !(plan_flags & FAMRDP_PLAN_NO_WORKSPACE))
     return fail(FAMRDP_E_UNSUPPORTED, "the step needs ghost=2 (the MUSCL-2 stencil width)");
-  famrdp_plan* p = new famrdp_plan();
+  PlanOwner owner{new famrdp_plan()};
+  famrdp_plan* p = owner.p;
   p->nblocks = nblocks;
   p->ghost = ghost;
   p->limiter = limiter;
@@ -707,16 +717,15 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   p->dims.assign(dims, dims + 3 * nblocks);
   p->has_workspace = !(plan_flags & FAMRDP_PLAN_NO_WORKSPACE);
   int rc = FAMRDP_OK;
-  auto cleanup = [&](int code) { famrdp_plan_destroy(p); return code; };
   for (int b = 0; b < nblocks; ++b) {
     const int32_t* d = &dims[3 * b];
     if (d[0] < 2 * ghost || d[1] < 2 * ghost || d[2] < 2 * ghost)
-      return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": each padded size must be >= 2*ghost"));
+      return fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": each padded size must be >= 2*ghost");
     if ((int64_t)d[0] * d[1] * d[2] > INT32_MAX)   // tile kernels index cells in 32 bits
-      return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^31 or more cells"));
+      return fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^31 or more cells");
     // the reverse kernels address cells with 32-bit byte offsets
     if ((plan_flags & FAMRDP_PLAN_ADJOINT) && (int64_t)d[0] * d[1] * d[2] >= (int64_t(1) << 29))
-      return cleanup(fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^29 or more cells in an adjoint plan"));
+      return fail(FAMRDP_E_INVALID, "block " + std::to_string(b) + ": 2^29 or more cells in an adjoint plan");
     p->N.push_back((int64_t)d[0] * d[1] * d[2]);
   }
   TableSet tables;
@@ -730,7 +739,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
       if (q1) (void)hipFree(q1);
       if (q2) (void)hipFree(q2);
       if (G) (void)hipFree(G);
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: workspace allocation failed"));
+      return fail(FAMRDP_E_HIP, "plan_create: workspace allocation failed");
     }
     p->q1.push_back(q1);
     p->q2.push_back(q2);
@@ -759,10 +768,10 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
           continue;
         }
         if (hipMalloc(&bufs[i], sizeof(double) * sizes[i]) != hipSuccess)
-          return cleanup(fail(FAMRDP_E_HIP, "plan_create: adjoint workspace allocation failed"));
+          return fail(FAMRDP_E_HIP, "plan_create: adjoint workspace allocation failed");
         p->adj_bufs.push_back(bufs[i]);
         if (hipMemset(bufs[i], 0, sizeof(double) * sizes[i]) != hipSuccess)
-          return cleanup(fail(FAMRDP_E_HIP, "plan_create: adjoint workspace clear failed"));
+          return fail(FAMRDP_E_HIP, "plan_create: adjoint workspace clear failed");
       }
       BlockDesc& a = p->h_blocks_adj[b];
       a.qh = bufs[0]; a.la = bufs[1]; a.lb = bufs[2]; a.l0 = bufs[3]; a.fs = bufs[4]; a.vs = bufs[5];
@@ -774,16 +783,16 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   }
   tables.scratch(&p->d_blocks, nblocks);
   if (hipHostMalloc(&p->h_stage[0], sizeof(BlockDesc) * nblocks * famrdp_plan::NSTAGE) != hipSuccess)
-    return cleanup(fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed"));
+    return fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed");
   for (int s = 0; s < famrdp_plan::NSTAGE; ++s) {
     p->h_stage[s] = p->h_stage[0] + (size_t)s * nblocks;
     if (hipEventCreateWithFlags(&p->stage_ev[s], hipEventDisableTiming) != hipSuccess)
-      return cleanup(fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed"));
+      return fail(FAMRDP_E_HIP, "plan_create: block table staging allocation failed");
   }
   // halo gather table
   GhostTable ghosts(ghost, nblocks, dims);
   rc = add_cuts(p, ncut, cuts, ghosts);
-  if (rc) return cleanup(rc);
+  if (rc) return rc;
   std::vector<HaloEntry> halo;
   ghosts.halo(halo);
   p->nhalo = (int)halo.size();
@@ -794,7 +803,7 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
   for (int i = 0; i < nbc; ++i) {
     const famrdp_bc& c = bcs[i];
     if (c.block < 0 || c.block >= nblocks || c.face < 0 || c.face > 5 || c.kind < 0 || c.kind > 4)
-      return cleanup(fail(FAMRDP_E_INVALID, "bc " + std::to_string(i) + ": block, face or kind out of range"));
+      return fail(FAMRDP_E_INVALID, "bc " + std::to_string(i) + ": block, face or kind out of range");
     BcEntry e{};
     e.block = c.block; e.face = c.face; e.kind = c.kind; e.T_wall = c.T_wall;
     for (int v = 0; v < 5; ++v) e.q_inf[v] = c.q_inf[v];
@@ -916,9 +925,26 @@ int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, 
     }
   }
   tables.scratch(&p->d_monitor, p->persistent_grid);
-  if (!tables.make(&p->d_tables)) return cleanup(fail(FAMRDP_E_HIP, "plan_create: table upload failed"));
+  if (!tables.make(&p->d_tables)) return fail(FAMRDP_E_HIP, "plan_create: table upload failed");
   *out = p;
+  owner.p = nullptr;
   return FAMRDP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int famrdp_plan_create(famrdp_plan** out, int32_t nblocks, const int32_t* dims, int32_t ncut, const famrdp_cut* cuts,
+                       int32_t nbc, const famrdp_bc* bcs, const famrdp_gas* gas, int32_t limiter, int32_t ghost,
+                       int32_t plan_flags) {
+  if (!out) return fail(FAMRDP_E_INVALID, "plan_create: out is NULL");
+  *out = nullptr;
+  try {   // its tables grow with the blocks: nothing may leave a C entry
+    return plan_create_impl(out, nblocks, dims, ncut, cuts, nbc, bcs, gas, limiter, ghost, plan_flags);
+  } catch (const std::exception&) {
+    return fail(FAMRDP_E_HIP, "plan_create: out of host memory for the plan's tables");
+  }
 }
 
 int famrdp_plan_set_tile(famrdp_plan* p, int32_t variant) {
