@@ -207,7 +207,7 @@ class Plan:
         any interior cell is non-finite or has rho <= 0 or p <= 0."""
         # the count lands in pinned host memory: no copy to wait for behind the kernel
         torch = L._torch()
-        out = torch.empty(1, dtype=torch.float64, pin_memory=True)
+        out = torch.empty(1, dtype=torch.float64, device="cpu", pin_memory=True)   # whatever the default device is
         self.check_state(qs, out)
         torch.cuda.current_stream().synchronize()
         nbad = int(out.item())

@@ -105,3 +105,20 @@ def test_forward_mode_sees_the_copy_as_reverse_mode_does():
         for b, t, q in zip(step(dual, cfg, 1e-3).blocks, tangents, plain):
             primal, tangent = fwd.unpack_dual(b.q)
             assert torch.equal(primal, q) and torch.equal(tangent, t)
+
+
+def test_state_check_under_another_default_device():
+    from dataclasses import replace
+    from famrdp_jax.solver.step import step
+    from famrdp_jax.solver.stepper import Stepper
+    print("case: nan_check with torch's default device set to the GPU", flush=True)
+    state, cfg = cases.case_c1(9)[:2]
+    state, cfg = to_dev(state), replace(cfg, nan_check=True)
+    torch.set_default_device("cuda")
+    try:
+        out = step(state, cfg, 1e-3)
+        st = Stepper(state, cfg)
+        st.advance(1e-3, 1)
+    finally:
+        torch.set_default_device(None)
+    assert torch.equal(out.blocks[0].q, st.qs[0])
