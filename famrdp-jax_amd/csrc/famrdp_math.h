@@ -379,23 +379,26 @@ DF void prim_and_temp(const double q[5], const StageGas& gas, double pv[6]) {
 //   m_L u_L + m_R u_R - u^ sa - w du + S P
 //     = (m_L - b sa + w) u_L + (m_R - a sa - w) u_R + S P
 // (m mass fluxes, sa the summed wave strengths, w the shear weight, P all
-// terms along the normal) takes three fma per component, and the energy flux
-// likewise, in which the contact wave w2 keeps its own q^2 / 2 (with the
-// acoustic waves' H^ and w2 (H^ - q^2 / 2) taken off again it would cancel at
-// large density jumps).  Working with S instead of the unit normal leaves one
+// terms along the normal) takes three fma per component.  The energy flux is
+// that of the two sides, (E + p) u_n, which no root or reciprocal enters, less
+// the waves; the contact wave w2 keeps its own q^2 / 2 (with the acoustic
+// waves' H^ and w2 (H^ - q^2 / 2) taken off again it would cancel at large
+// density jumps).  Working with S instead of the unit normal leaves one
 // 1/|S| and no final product with |S|.  Harten's fix |l| < eps: (l^2/eps + eps)
 // / 2 is |l| + (eps - |l|)^2 / (2 eps), zero extra where |l| >= eps.  About 140
 // instructions and six seeds, 205 and seven in the form with conservative
 // jumps.  Error against 113-bit arithmetic over the largest component, random
-// faces with p ~ 1, |u| < 0.5, exact seeds, rms: 1.9e-16 at equal densities and
-// 3e-16 at a ratio of 1e6 either way (conservative jumps 2.6e-16 and 3.3e-15;
+// faces with p ~ 1, |u| < 0.5, exact seeds, rms: 1.5e-16 at equal densities and
+// 3e-16 at a ratio of 1e6 either way (conservative jumps 2.7e-16 and 3.2e-15;
 // gathered about the left state 1.9e-16, and 4.4e-11 with that one lighter);
-// with one-step seeds 7e-15 and 1.5e-14, as with conservative jumps.  The floors
+// with one-step seeds 4e-15 and 1.5e-14 (7e-15 and 1.5e-14), and 1.0e-16 between
+// states a thousandth apart (6.6e-15; with the energy flux gathered by side, as
+// H times a mass flux, 4.5e-15 and with exact seeds 1.3e-16).  The floors
 // are min/max, which drop a NaN: a NaN primitive makes the pressure NaN, and
 // dp carries it into every component.
 // FULL: every root and reciprocal rounded once (ten seeds instead of six), which
 // makes the flux as exact as the reference's formulas in IEEE arithmetic or more
-// (rms 1.5e-16 to their 2.5e-16 on those faces, 7.3e-16 to 8.8e-16 at twice the
+// (rms 1.4e-16 to their 2.5e-16 on those faces, 7.3e-16 to 8.8e-16 at twice the
 // speed of sound; with reciprocal roots and their squares 9.5e-16 there).
 //
 // Says whether no floor acted: where one does, the conservative states that the
@@ -417,9 +420,10 @@ FD bool roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   const double rs = recip(sqL + sqR);
   const double a = sqR * rs, b = sqL * rs;
   const double uL = pl[1], vL = pl[2], wL = pl[3], uR = pr[1], vR = pr[2], wR = pr[3];
-  // twice the total enthalpies: 2 g/(g-1) p/rho + |u|^2
+  // twice E + p, 2 g/(g-1) p + rho |u|^2, and twice the total enthalpies
   const double kL = fma(wL, wL, fma(vL, vL, uL * uL)), kR = fma(wR, wR, fma(vR, vR, uR * uR));
-  const double HL = fma(gas.cg2, pl[4] * irL, kL), HR = fma(gas.cg2, pr[4] * irR, kR);
+  const double hL = fma(rhoL, kL, gas.cg2 * pl[4]), hR = fma(rhoR, kR, gas.cg2 * pr[4]);
+  const double HL = hL * irL, HR = hR * irR;
   const double uh = fma(a, uR, b * uL), vh = fma(a, vR, b * vL), wh = fma(a, wR, b * wL), Hh = fma(a, HR, b * HL);
   const double q2 = fma(wh, wh, fma(vh, vh, uh * uh));
   const double c2raw = gas.gm1h * (Hh - q2), c2 = fmax(c2raw, 1e-30);
@@ -453,14 +457,13 @@ FD bool roe_flux2(const double pl[5], const double pr[5], const double S[3], con
   const double Q = fma(w, dun, (w1 - w5) * c) * rA;
   const double P = (pl[4] + pr[4]) + Q;
   const double mL = rhoL * unL, mR = rhoR * unR;
-  const double eL = fma(-b, sw, mL), eR = fma(-a, sw, mR);
-  const double iL = fma(-b, w2, eL) + w, iR = fma(-a, w2, eR) - w;
+  const double iL = fma(-b, sa, mL) + w, iR = fma(-a, sa, mR) - w;
   F[0] = (mL + mR) - sa;
   F[1] = fma(S[0], P, fma(iR, uR, iL * uL));
   F[2] = fma(S[1], P, fma(iR, vR, iL * vL));
   F[3] = fma(S[2], P, fma(iR, wR, iL * wL));
   const double ud = fma(wh, wR - wL, fma(vh, vR - vL, uh * (uR - uL)));
-  F[4] = fma(0.5, fma(-w2, q2, fma(HR, eR, eL * HL)), fma(un, Q, -(w * ud)));
+  F[4] = fma(0.5, fma(-w2, q2, fma(-sw, Hh, fma(hR, unR, hL * unL))), fma(un, Q, -(w * ud)));
   return pl[0] > 1e-300 && pr[0] > 1e-300 && c2raw > 1e-30 && nnraw > 1e-280;
 }
 

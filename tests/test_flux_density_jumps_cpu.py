@@ -65,6 +65,29 @@ def test_flux_between_light_and_heavy(hc, ratio, full):
     assert float(err.max()) <= TOL
 
 
+@pytest.mark.parametrize("full", [0, 1])
+@pytest.mark.parametrize("speed", [0.1, 0.5, 2.4])
+def test_energy_flux_of_equal_states_is_as_exact_as_in_64_bits(hc, speed, full):
+    """No waves there: twice (E + p) u.S, rms error no larger than that product's in IEEE arithmetic."""
+    n = 20000
+    pl, _, S = faces(1.0, n, 91)
+    pl[:, 1:4] *= 2 * speed
+    F = np.zeros((n, 5))
+    P = lambda a: np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    hc.hc_roe_flux2(n, full, P(pl), P(pl), P(S), ctypes.c_double(G), P(F))
+
+    def plain(T):
+        rho, u, v, w, p = pl.T.astype(T)
+        s, g = S.T.astype(T), T(G)
+        E = p / (g - 1) + rho * (T(0.5) * (u * u + v * v + w * w))
+        return 2 * ((E + p) * (u * s[0] + v * s[1] + w * s[2]))
+
+    ref = plain(np.longdouble)
+    rms = lambda x: float(np.sqrt(((x - ref) ** 2).mean()))  # noqa: E731
+    print(f"speed {speed:g}: {rms(F[:, 4]):.2e}, plain {rms(plain(np.float64)):.2e}")
+    assert rms(F[:, 4]) <= rms(plain(np.float64))
+
+
 @pytest.mark.parametrize("mach", [0.4, 2.0])
 def test_rhs_flux_is_as_exact_as_the_formulas_in_64_bits(hc, mach):
     """The RHS entry point's form at equal densities: rms error no larger than that of flux/roe.py in IEEE arithmetic."""
