@@ -10,8 +10,8 @@ famrdp_jax/_lib/libfamrdp_hip.so:
   instruction-level parallelism (max-ilp): the stage kernels are issue-bound
   FP64 code at two workgroups per CU, and this schedule measured 2 % faster on
   the fused kernel and 2.4 % faster on the marching kernel than the default;
-* csrc/famrdp_reverse.hip (the two reverse stage kernels) with the default
-  scheduler, which measured 2.5 % (faces) and 6.5 % (gather) faster on them.
+* csrc/famrdp_reverse.hip (the reverse stage's sweeps) with the default
+  scheduler: with max-ilp the two inviscid sweeps spill or come close.
 
 Packed FP32 instructions are disabled in both (the kernels are FP64; this keeps
 the compiler from forming them in any FP32 helper code).

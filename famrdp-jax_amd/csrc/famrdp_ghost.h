@@ -124,9 +124,10 @@ struct GhostShell {
   }
 };
 
-// The ghost table of a plan.  `cuts(b, f)` reports the copies of the exchange
-// through copy(); bc[f] holds the boundary conditions of face f (at most one
-// per block), in the order of the blocks' application.
+// The ghost table of a plan: copy() takes the copies of the exchange, then
+// boundary() the boundary conditions -- bc[f] those of face f (at most one per
+// block), in the order of the blocks' application -- and finish() orders the
+// entries.
 struct GhostTable {
   struct Val {
     int32_t sb, sc, chain;   // chain -1: untouched

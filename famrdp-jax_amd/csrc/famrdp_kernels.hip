@@ -1543,12 +1543,12 @@ inline int64_t stage_tiles(int v, int ni, int nj, int nk) {
 // (n, rounded up) take; measured (minmod; van Leer is 10-17 % longer for all
 // alike), in us, for cubes of 12^3 to 124^3 cells, flat and long blocks and
 // lattices of small ones, the lines hold within 10 %:
-//   19 wide 3x4x4    3.5 + 1.75 n   (20^3 5.3, 36^3 9.8, 72^3 56.6)
-//   20 wide 4x4x8    1.5 + 5.6 n    (32^3 7.4, 44^3 17.7)
-//    1 fused 4x8x16  15.3 n         (44^3 15.6, 60^3 31.1, 72^3 58.3)
-//   12 re-staging    5 + 6.5 n      (52^3 24.3, 80^3 59.7, 104^3 126.6)
+//   19 wide 3x4x4    3.5 + 1.75 n   (20^3 5.4, 36^3 9.9, 72^3 54.8)
+//   20 wide 4x4x8    1.5 + 5.6 n    (32^3 7.6, 44^3 17.2)
+//    1 fused 4x8x16  15.3 n         (44^3 15.8, 60^3 30.7, 72^3 58.6)
+//   12 re-staging    5 + 6.5 n      (52^3 24.2, 84^3 75.2, 104^3 125.2)
 //   18 marching      6.9 per plane of march_len's count, 4.7 with no more than
-//                    a workgroup per CU (72^3 49.6, 96^3 65.4, 112^3 107, 124^3 147)
+//                    a workgroup per CU (72^3 50.5, 96^3 66.2, 112^3 111, 124^3 151)
 // The fused kernel of 8x4x8 cells that every untuned block took before:
 // 12.1 at 20^3, 27.5 at 52^3, 65.8 at 80^3, 109 at 96^3, 258 at 124^3.
 inline int default_variant(int nblocks, const int32_t* dims, int ncu, bool fits32) {

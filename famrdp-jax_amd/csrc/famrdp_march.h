@@ -37,10 +37,12 @@
 //
 // What bounds it (260^3 padded, stage 2, random smooth state): neither FP64
 // issue nor HBM alone.  The same launch with every load an L2 hit takes
-// 1.09 ms, its VALU instructions alone 0.64 ms, its bytes past L2 (6 GB, 1.8
+// 1.09 ms, its VALU instructions alone 0.66 ms, its bytes past L2 (6 GB, 1.8
 // times the compulsory 3.5 GB: halos, the re-read of the plane being updated)
-// 1.2 ms at the 4.9 TB/s of a large copy; at two waves per SIMD (255
-// registers, 77.7 KB of LDS) the three overlap to 1.40 ms (132^3: 209 us).
+// 1.2 ms at the 4.9 TB/s of a large copy; at two waves per SIMD (256
+// registers, 77.7 KB of LDS) the three overlap to 1.40 ms (132^3: 212 us; with
+// the Roe flux gathered about its left state and no residual on the square
+// root, 1,229 instead of 1,268 instructions per 64 cells, 1.37 and 211).
 // With three barriers per plane, conservative jumps in the Roe flux and the
 // far-end faces' loads inside their round: 1.51 ms (231 us).
 //

@@ -22,7 +22,8 @@
 // compiled with the default machine scheduler (the rest of the library uses
 // the max-ilp one, with which the two inviscid sweeps spill or come close).
 //
-// One stage of 10^6 cells (curvilinear 96^3) takes 133 + 87 us; two gather
+// One stage of 10^6 cells (curvilinear 96^3) takes 142 + 88 us (133 + 87 with
+// reciprocal roots from seeds, whose squares round twice); two gather
 // kernels that passed 46 doubles per cell (three faces' state cotangents, the
 // viscous ones) took 223 + 184 us.  What bounds them now: k_vjp_j moves 42
 // doubles a cell that no other access could save (68 us at the 4.9 TB/s of a
@@ -283,7 +284,7 @@ __device__ __forceinline__ void cell_vjp_finish(const BlockDesc& b, const double
     lpv[v] += rd(b.fs + v * N, y);
   }
   cons_to_prim_fast(q, gas.gamma, pv);
-  // viscous: vs holds what k_vjp_visc summed (u, v, w, T) and the cotangents
+  // viscous: vs holds what sweep_visc summed (u, v, w, T) and the cotangents
   // of the cell's central differences along j
   const unsigned jm = y + (unsigned)((wrap_m(j, b.nj) - j) * b.nk), jp = y + (unsigned)((wrap_p(j, b.nj) - j) * b.nk);
 #pragma unroll

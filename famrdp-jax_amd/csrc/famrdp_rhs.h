@@ -154,10 +154,11 @@ __device__ __forceinline__ void invscd_tile(double* s_pv, double* s_f, int* odd,
 // grid beyond which they take several.  A thread per face of the tile, then a thread per
 // variable and cell.  Tiles that hold an invalid state are done again afterwards,
 // in registers that the first pass has anyway (PinFence): inside it, or without
-// the fences, its spills cost every tile 10-20 %.  Bound by FP64 issue: 68 x 52 x 84 cells 29.0 us (83.6 as
-// a thread per cell), 132^3 217.  (With six seeds a flux 28.6 and 207; the other
-// tiles then 4x4x8 29.7 and 224, 3x4x4 31.4 and 247, 2x4x8 29.4 and 225; six
-// waves per SIMD, spills, 28.0 and 225.)
+// the fences, its spills cost every tile 10-20 %.  Bound by FP64 issue: 68 x 52
+// x 84 cells 31.5 us in the trace (83.6 as a thread per cell), launches back to
+// back 27.1, 132^3 196.  (With the stage kernels' six seeds a flux 28.6 in the
+// trace, 132^3 207 there; the other tiles then 4x4x8 29.7 and 224, 3x4x4 31.4
+// and 247, 2x4x8 29.4 and 225; six waves per SIMD, spills, 28.0 and 225.)
 template <int TI, int TJ, int TK, int LIM>
 __global__ void __launch_bounds__((CrossGeom<TI, TJ, TK>::NTH)) __attribute__((amdgpu_waves_per_eu(5)))
 k_invscd_rhs(const double* __restrict__ q, const double* __restrict__ kxyz, const double* __restrict__ vol,

@@ -5,7 +5,7 @@
 // turns: viscous tensors, divergence, then the faces of each axis, every one
 // a pass and a remainder pass behind a barrier.  On a small block that chain
 // is the stage's time: one wave per SIMD or less, eight dependent passes,
-// 12.1 us for 20^3 cells, 13.2 for 36^3 (here 5.3 and 9.8; a launch is 2 of
+// 13.6 us for 20^3 cells, 13.5 for 36^3 (here 5.4 and 9.9; a launch is 2 of
 // them).  Here the first waves hold the tile's viscous
 // tensors, the others a face each, of all three axes; a thread's first loads
 // are all issued at the start and the stage has three barriers:
